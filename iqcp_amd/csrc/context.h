@@ -94,6 +94,7 @@ struct qcg_context {
     // J/K work plan: items per (class pair, precision part), rebuilt when options or tiles change
     struct Tile { int block = 64, reps = 1; };
     Tile tile[21][2];  // per quartet class and precision part (0 FP64, 1 FP32)
+    bool tiles_set = false;  // set or tuned by the caller; else chosen with the work plan (default_tiles)
     int class_nq[21] = {};  // Cartesian components per quartet class
     // mixed precision, per class: run its FP64 and FP32 items in one launch (jk_*_mp kernels, with
     // the FP64 part's tile) or in two; qcg_autotune_refine may split a class

@@ -164,10 +164,11 @@ QCG_HD void for_n(F&& body) {
 // into ck, the component normalisation is NOT applied here).  ppb: the bra's primitive pairs
 // (P.npp of them, from index 0: a copy staged in LDS or pp + P.pp_off), ppk: the ket's (Q.npp).
 // TAB_N: rys_tab already points at the coefficients of this class's Rys order (e.g. a copy
-// staged in LDS).
+// staged in LDS).  j0, js: the ket primitives taken, j0, j0 + js, ... (0, 1: all of them).
 template <int LA, int LB, int LC, int LD, typename R, bool TAB_N = false>
 QCG_HD void contract_quartet_pp(const PairRec& P, const PairRec& Q, const PrimPair<R>* __restrict__ ppb,
-                                const PrimPair<R>* __restrict__ ppk, const R* __restrict__ rys_tab, R* eri) {
+                                const PrimPair<R>* __restrict__ ppk, const R* __restrict__ rys_tab, R* eri, int j0 = 0,
+                                int js = 1) {
     using S = EriShape<LA, LB, LC, LD>;
     constexpr int N = S::NROOTS;
     const R abx = (R)P.abx, aby = (R)P.aby, abz = (R)P.abz;
@@ -178,7 +179,7 @@ QCG_HD void contract_quartet_pp(const PairRec& P, const PairRec& Q, const PrimPa
     // ket primitives outer: in the J/K kernels the bra pair is uniform over the block, so the inner
     // loop's bra primitive reads are uniform (an LDS broadcast) and each lane loads its ket
     // primitive once
-    for (int j = 0; j < Q.npp; ++j) {
+    for (int j = j0; j < Q.npp; j += js) {
         const PrimPair<R> c = ppk[j];
         const R q = c.p;
         const R hq = c.hp;

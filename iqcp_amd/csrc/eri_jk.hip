@@ -129,13 +129,22 @@ __device__ __forceinline__ void jk_item(
     });
     const double deg_p = (P.sa == P.sb) ? 0.5 : 1.0;
 
-    KetCursor cur{segs, it.y, it.z + tid};
-    for (int j = tid; j < item_kets(it); j += blockDim.x, cur.r += blockDim.x) {
+    // 2^lg lanes share a ket (uniform over the block): lane `sub` of them takes every 2^lg-th ket
+    // primitive and a fixed butterfly sums the partial quartets, so a heavily contracted quartet is
+    // no longer one lane's serial chain (alone, water (ss|ss) 335 -> 21 us, (pp|pp) 231 -> 50 us)
+    const int lg = item_lg(it), lanes = 1 << lg, sub = tid & (lanes - 1), step = blockDim.x >> lg;
+    KetCursor cur{segs, it.y, it.z + (tid >> lg)};
+    for (int j = tid >> lg; j < item_kets(it); j += step, cur.r += step) {
         const int q = cur.at();
         const PairRec Q = ket[q];
         R eri[S::NQ];
         for_n<U, S::NQ>([&](int i) { eri[i] = R(0); });
-        contract_quartet_pp<LA, LB, LC, LD, R, true>(P, Q, ppb, pp + Q.pp_off, rys_n, eri);
+        contract_quartet_pp<LA, LB, LC, LD, R, true>(P, Q, ppb, pp + Q.pp_off, rys_n, eri, sub, lanes);
+        if (lg) {
+            for (int off = 1; off < lanes; off <<= 1)
+                for_n<U, S::NQ>([&](int i) { eri[i] += __shfl_xor(eri[i], off, 64); });
+            if (sub) continue;  // the group's first lane digests
+        }
         const double deg = deg_p * ((Q.sa == Q.sb) ? 0.5 : 1.0) * ((diag && q == pidx) ? 0.5 : 1.0);
         if (do_j) {
             double Dqs[S::NCD];

@@ -13,46 +13,48 @@ namespace qcg {
 // concatenation into items (bra index, first segment, offset into it, w), so a block's lanes stay
 // busy across bucket boundaries instead of idling at the end of every bucket.
 //
-// w packs the ket count (bits 0-15) and an optional range of the bra's primitive pairs: first
-// (bits 16-23) and count (bits 24-31, 0 = all).  A bra pair with many primitive pairs is cut into
-// such ranges so that no lane runs the whole npp_bra x npp_ket primitive loop of a heavy quartet
-// alone; the integral is linear in the bra primitives, so the partial quartets are digested
-// (J and K) like whole ones.
-constexpr int kItemMaxKets = 0xffff;
+// w packs the ket count (bits 0-12), the lanes per ket of the per-lane J/K kernels as a power of two
+// (bits 13-15) and an optional range of the bra's primitive pairs: first (bits 16-23)
+// and count (bits 24-31, 0 = all).  A bra pair with many primitive pairs is cut into such ranges so
+// that no lane runs the whole npp_bra x npp_ket primitive loop of a heavy quartet alone; the integral
+// is linear in the bra primitives, so the partial quartets are digested (J and K) like whole ones.
+constexpr int kItemMaxKets = 0x1fff;
 constexpr int kItemMaxPrim = 0xff;
+constexpr int kItemMaxLg = 6;  // at most a whole wavefront per ket
 
-// items of at most ch kets over segments [g0, segs.size()) of bra `bra`, primitive range
-// (pbeg, pcnt) (pcnt = 0: all of them)
-inline void cut_items(std::vector<int4>& items, const std::vector<int2>& segs, int g0, int bra, int ch,
-                      int pbeg = 0, int pcnt = 0) {
+// items of at most ch kets over segments [g0, g1) of bra `bra`, 2^lg lanes per ket, primitive
+// range (pbeg, pcnt) (pcnt = 0: all of them)
+inline void cut_items(std::vector<int4>& items, const std::vector<int2>& segs, int g0, int g1, int bra, int ch,
+                      int lg = 0, int pbeg = 0, int pcnt = 0) {
     int total = 0;
-    for (size_t g = (size_t)g0; g < segs.size(); ++g) total += segs[g].y;
-    const int wbits = (pbeg << 16) | (pcnt << 24);
+    for (int g = g0; g < g1; ++g) total += segs[g].y;
+    const int wbits = (lg << 13) | (pbeg << 16) | (pcnt << 24);
     int g = g0, r = 0;
     for (int off = 0; off < total; off += ch) {
         const int n = std::min(ch, total - off);
         items.push_back(make_int4(bra, g, r, n | wbits));
         r += n;
-        while (g < (int)segs.size() && r >= segs[g].y) r -= segs[g++].y;
+        while (g < g1 && r >= segs[g].y) r -= segs[g++].y;
     }
 }
 
 // cut_items for every primitive range of a bra pair with npp primitive pairs: ranges of at most
 // split pairs (split <= 0 or npp <= split: one range, the whole pair), sizes balanced
-inline void cut_items_split(std::vector<int4>& items, const std::vector<int2>& segs, int g0, int bra, int ch,
-                            int npp, int split) {
+inline void cut_items_split(std::vector<int4>& items, const std::vector<int2>& segs, int g0, int g1, int bra, int ch,
+                            int npp, int split, int lg = 0) {
     if (split <= 0 || npp <= split || npp > kItemMaxPrim) {
-        cut_items(items, segs, g0, bra, ch);
+        cut_items(items, segs, g0, g1, bra, ch, lg);
         return;
     }
     const int nr = (npp + split - 1) / split;
     for (int k = 0; k < nr; ++k) {
         const int b = k * npp / nr, e = (k + 1) * npp / nr;
-        cut_items(items, segs, g0, bra, ch, b, e - b);
+        cut_items(items, segs, g0, g1, bra, ch, lg, b, e - b);
     }
 }
 
 inline QCG_HD int item_kets(const int4& it) { return it.w & kItemMaxKets; }
+inline QCG_HD int item_lg(const int4& it) { return (it.w >> 13) & 7; }
 
 // Most bra primitive pairs one per-lane J/K item may have: the kernel stages them in LDS (a block's
 // bra pair is uniform, so the inner primitive loop reads them as LDS broadcasts instead of scalar

@@ -28,8 +28,8 @@ int grad_plan(qcg_context* c) {
                 const int g0 = (int)segs.size();
                 for_ket_ranges(c, cb, ck, 0, p, c->schwarz_thr, c->schwarz_thr,
                                [&](int bs, int, int e) { segs.push_back(make_int2(bs, e - bs)); });
-                cut_items_split(items, segs, g0, p, grad_item_kets(cb, ck), c->pairs[c->class_off[cb] + p].npp,
-                                c->prim_split);
+                cut_items_split(items, segs, g0, (int)segs.size(), p, grad_item_kets(cb, ck),
+                                c->pairs[c->class_off[cb] + p].npp, c->prim_split);
             }
             c->grad_cnt[cls] = (int)items.size() - c->grad_off[cls];
         }

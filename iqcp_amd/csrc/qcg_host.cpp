@@ -419,6 +419,48 @@ static bool plan_fresh(const qcg_context* c) {
 
 bool qcg::jk_prepared(const qcg_context* c) { return plan_fresh(c) && !(c->profiling && !c->ev_made); }
 
+// Lanes per ket (eri_jk.hip): a lane that runs npp_bra x npp_ket primitive quartets of a contracted
+// core pair on its own takes 0.27 us (ss|ss) to 2.9 us (pp|pp) for each, so one C 1s-C 1s quartet
+// (36 x 36) takes 350 us whatever the molecule's size.  The plan gives such kets 2, 4, .. 64 lanes
+// until no chain is longer than kChainShare of what the whole build takes at kModelFlopsPerUs model
+// flops per us (decane: 90 us of 1.5 ms), but not below kChainMinUs, about one kernel's launch and
+// set-up.  One water 750 -> 290 us, benzene 1070 -> 500 us per build with the tiles below.
+constexpr double kChainMinUs = 12.0, kChainShare = 0.06, kModelFlopsPerUs = 16e6;
+
+// Tiles when the caller has set or tuned none.  Per-lane kernels: the block is widened from 64 to 256
+// threads until the waves that fit a CU's 160 KB of LDS next to each other (the K rows of one bra and
+// the Rys table are per block) reach what the kernel's registers allow (`want` per SIMD), as far as a
+// bra has kets for the block; a lane takes several kets once that still leaves 16384 waves.  (H2O)16
+// (304 functions): (ds|ss) 0.67 ms at 64 threads, 0.29 ms at 256; 64 alkanes (up to 160 functions):
+// (ps|ps) 6.7 ms at (64, 1), 4.7 ms at (128, 4), 5.8 ms at (256, 1).  Wave-cooperative kernels: up to
+// four kets per wavefront once that leaves about 6000 wavefronts ((H2O)16 (dp|ds): 0.67 / 0.54 / 0.50 ms
+// at 1 / 2 / 4).
+template <typename Bras>
+static void default_tiles(qcg_context* c, const int64_t (&quartets)[21][2], const Bras& bras) {
+    for (int cls = 0, cb = kNumPairClasses - 1; cb >= 0; --cb)
+        for (int ck = cb; ck >= 0; --ck, ++cls)
+            for (int part = 0; part < 2; ++part) {
+                const int64_t n = quartets[cls][part] + (part == 0 && c->fuse_cls[cls] ? quartets[cls][1] : 0);
+                qcg_context::Tile& t = c->tile[cls][part];
+                const int nq = c->class_nq[cls];
+                if (nq > kJkLaneMaxNQ) {
+                    t = {0, n > 24000 ? 4 : n > 8000 ? 2 : 1};
+                    continue;
+                }
+                const int64_t per_bra = n / std::max<int64_t>(1, (int64_t)bras[cls][part].size());
+                const int la = cb == 0 ? 0 : cb <= 2 ? 1 : 2, lb = (cb == 0 || cb == 1 || cb == 3) ? 0 : (cb == 2 || cb == 4) ? 1 : 2;
+                const int lc = ck == 0 ? 0 : ck <= 2 ? 1 : 2, ld = (ck == 0 || ck == 1 || ck == 3) ? 0 : (ck == 2 || ck == 4) ? 1 : 2;
+                const int nr = (la + lb + lc + ld) / 2 + 1;
+                const int lds = (nr <= 3 ? (qcg_rys_off[nr + 1] - qcg_rys_off[nr]) * 8 : 0) + (ncart(la) + ncart(lb)) * c->max_nbf * 8;
+                const int want = nq <= 1 ? 7 : nq <= 3 ? 5 : nq <= 9 ? 4 : nq <= 18 ? 3 : nq <= 36 ? 2 : 1;
+                int block = 64;
+                while (block < 256 && (163840 / std::max(lds, 1)) * (block / 64) < 4 * want) block *= 2;
+                while (block > 64 && per_bra < block * 3 / 4) block /= 2;
+                int64_t reps = std::min<int64_t>(n / 64 / 16384, per_bra / block);
+                t = {block, (int)std::max<int64_t>(1, std::min<int64_t>(8, reps))};
+            }
+}
+
 static int build_plan(qcg_context* c) {
     const bool mixed = c->precision == QCG_PREC_MIXED && c->fp32_cutoff > c->schwarz_thr;
     const double key[4] = {(double)c->precision, c->fp32_cutoff, c->schwarz_thr, (double)c->tile_sig};
@@ -437,6 +479,13 @@ static int build_plan(qcg_context* c) {
     c->segs.clear();
     const int nmol = c->nmol;
     const double cut = mixed ? c->fp32_cutoff : c->schwarz_thr;
+    // the surviving kets of every (class, precision part, bra), as segments
+    struct Bra {
+        int pair, npp, g0, g1, kbase;
+    };
+    std::vector<Bra> bras[21][2];
+    int64_t quartets[21][2] = {};
+    double fpq[21], total = 0.0;  // model flops per primitive quartet of a class, and of the build
     int cls = 0;
     for (int cb = kNumPairClasses - 1; cb >= 0; --cb)
         for (int ck = cb; ck >= 0; --ck, ++cls) {
@@ -446,17 +495,9 @@ static int build_plan(qcg_context* c) {
             const int la = cb == 0 ? 0 : cb <= 2 ? 1 : 2, lb = (cb == 0 || cb == 1 || cb == 3) ? 0 : (cb == 2 || cb == 4) ? 1 : 2;
             const int lc = ck == 0 ? 0 : ck <= 2 ? 1 : 2, ld = (ck == 0 || ck == 1 || ck == 3) ? 0 : (ck == 2 || ck == 4) ? 1 : 2;
             const double nq = (double)ncart(la) * ncart(lb) * ncart(lc) * ncart(ld);
-            const double fpq = ((la + lb + lc + ld) / 2 + 1) * (80.0 + 15.0 * (la + lb + 1) * (lc + ld + 1) + nq * (4.0 + 6.0 * (lb + ld)));
+            fpq[cls] = ((la + lb + lc + ld) / 2 + 1) * (80.0 + 15.0 * (la + lb + 1) * (lc + ld + 1) + nq * (4.0 + 6.0 * (lb + ld)));
             double cost = 0.0;
-            for (int part = 0; part < 2; ++part) {
-                // fused mixed launches run both parts with the FP64 part's tile
-                const qcg_context::Tile& t = c->tile[cls][(mixed && c->fuse_cls[cls]) ? 0 : part];
-                const int ch = std::min(kItemMaxKets, std::max(1, t.block > 0 ? t.block * t.reps : t.reps));
-                c->item_off[cls][part] = (int)c->items.size();
-                if (part == 1 && !mixed) {
-                    c->item_cnt[cls][part] = 0;
-                    continue;
-                }
+            for (int part = 0; part < (mixed ? 2 : 1); ++part)
                 for (int m = 0; m < nmol; ++m) {
                     const int pbase = c->ket_off_h[cb * nmol + m];
                     for (int p = 0; p < c->ket_cnt_h[cb * nmol + m]; ++p) {
@@ -467,18 +508,49 @@ static int build_plan(qcg_context* c) {
                             const int lo = part == 0 ? bs : sp, hi = part == 0 ? sp : e;
                             if (hi > lo) {
                                 c->segs.push_back(make_int2(lo, hi - lo));
+                                quartets[cls][part] += hi - lo;
                                 // a segment lies in one contraction bucket: one ket primitive count
-                                cost += (hi - lo) * (fpq * npp * c->pairs[kbase + lo].npp + 12.0 * nq);
+                                cost += (hi - lo) * (fpq[cls] * npp * c->pairs[kbase + lo].npp + 12.0 * nq);
                             }
                         });
-                        // bras above kBraPPMax primitive pairs are always cut into ranges
-                        const int split = (c->prim_split > 0 && c->prim_split < kBraPPMax) ? c->prim_split : kBraPPMax;
-                        cut_items_split(c->items, c->segs, g0, pbase + p, ch, npp, split);
+                        if ((int)c->segs.size() > g0) bras[cls][part].push_back({pbase + p, npp, g0, (int)c->segs.size(), kbase});
                     }
                 }
-                c->item_cnt[cls][part] = (int)c->items.size() - c->item_off[cls][part];
-            }
             c->plan_cost[cls] = cost;
+            total += cost;
+        }
+    if (!c->tiles_set) default_tiles(c, quartets, bras);
+    // the longest chain of primitive quartets one lane may run, in us
+    const double chain_us = std::max(kChainMinUs, kChainShare * total / kModelFlopsPerUs);
+    for (cls = 0; cls < 21; ++cls)
+        for (int part = 0; part < 2; ++part) {
+            // fused mixed launches run both parts with the FP64 part's tile
+            const qcg_context::Tile& t = c->tile[cls][(mixed && c->fuse_cls[cls]) ? 0 : part];
+            const bool lane_form = t.block > 0 ? c->class_nq[cls] <= kJkLaneMaxNQ : c->class_nq[cls] < 27;
+            const int ch = std::min(kItemMaxKets, std::max(1, t.block > 0 ? t.block * t.reps : t.reps));
+            // one lane's time per primitive quartet
+            const double step_us = 0.2 + 7.5e-4 * fpq[cls];
+            c->item_off[cls][part] = (int)c->items.size();
+            for (const Bra& b : bras[cls][part]) {
+                // bras above kBraPPMax primitive pairs are always cut into ranges
+                const int split = (c->prim_split > 0 && c->prim_split < kBraPPMax) ? c->prim_split : kBraPPMax;
+                const int nb = std::min(b.npp, split);
+                auto lg_of = [&](int g) {
+                    if (!lane_form) return 0;
+                    const int nk = c->pairs[b.kbase + c->segs[g].x].npp;
+                    int lg = 0;
+                    while (lg < kItemMaxLg && (1 << lg) < nk && nb * ((nk + (1 << lg) - 1) >> lg) * step_us > chain_us) ++lg;
+                    return lg;
+                };
+                for (int g = b.g0; g < b.g1;) {
+                    const int lg = lg_of(g);
+                    int e = g + 1;
+                    while (e < b.g1 && lg_of(e) == lg) ++e;
+                    cut_items_split(c->items, c->segs, g, e, b.pair, std::max(1, ch >> lg), b.npp, split, lg);
+                    g = e;
+                }
+            }
+            c->item_cnt[cls][part] = (int)c->items.size() - c->item_off[cls][part];
         }
     c->release(c->d_items);
     c->d_items = nullptr;
@@ -671,6 +743,7 @@ int qcg_autotune(qcg_context* c, const double* dD, int iters, int* chosen) {
     const int ncand = kTuneNCand;
     auto tile_of = [&](int k, int cls) { return tune_tile(c, k, cls); };
     for (int i = 0; i < 21; ++i) c->fuse_cls[i] = true;  // the per-class timings run fused launches
+    c->tiles_set = true;
     std::vector<double> best(42, 1e300);
     std::vector<int> pick(42, 0);
     const bool prof = c->profiling;
@@ -753,6 +826,7 @@ int qcg_autotune_refine(qcg_context* c, const double* dD, int builds, int* chose
         return fail(c, QCG_DEVICE, "autotune_refine: set-up");
     }
     c->use_graph = true;
+    c->tiles_set = true;  // the tiles in use, changed one at a time below
     auto measure = [&]() -> int {
         for (int w = 0; w < 2; ++w) {  // warm-up; the first also captures the graph for new tiles
             int r = qcg_build_fock_device(c, dH, dD, 0.5, dF, ts);
@@ -836,6 +910,7 @@ int qcg_set_tiles(qcg_context* c, const int* tiles) {
     for (int i = 0; i < 21; ++i)
         for (int part = 0; part < 2; ++part)
             c->tile[i][part] = {tiles[4 * i + 2 * part], tiles[4 * i + 2 * part + 1]};
+    c->tiles_set = true;
     c->tile_sig += 1;
     return QCG_OK;
 }

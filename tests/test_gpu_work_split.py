@@ -1,0 +1,44 @@
+"""How a build's quartets are dealt to lanes: several lanes per heavily contracted ket, one lane with
+several kets, blocks wider than a bra's kets.  J and K against the oracle's integral-direct build for
+the sizes where the split changes (one atom with a 36-primitive core pair, one water, a water dimer,
+benzene), every basis, both precisions.
+
+Tolerance: J and K are sums of at most a few thousand products of size <= 10 accumulated in fixed
+point with steps of 2^-50 or finer (fixacc.h), and the integrals are good to 1e-14 relative, so 1e-11
+absolute leaves two orders; mixed precision adds 2^-20 of quartets below 1e-6 each (test_gpu_eri.py),
+a few 1e-12 per quartet over at most 1e3 of them: 1e-9."""
+import numpy as np
+import pytest
+
+import oracle
+from helpers import bench_molecule, random_density
+from iqcp_amd import workloads
+from iqcp_amd.basis import build_basis
+from iqcp_amd.engine import Engine
+
+pytestmark = pytest.mark.gpu
+
+
+def _mol(name, basis):
+    if name == "Ne":
+        return build_basis([("Ne", (0.0, 0.0, 0.0))], basis)
+    if name == "water2":
+        return build_basis(workloads.water_cluster((2, 1, 1), 2.9, 3), basis, units="angstrom")
+    return bench_molecule(name, basis)
+
+
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-11), ("mixed", 1e-9)])
+@pytest.mark.parametrize("name,basis", [("Ne", "6-31g"), ("H2O", "sto-3g"), ("H2O", "6-31g*"), ("H2O", "6-31+g*"),
+                                        ("water2", "6-31g*"), ("C6H6", "6-31g")])
+def test_gpu_jk_split_over_lanes(name, basis, prec, tol):
+    b = _mol(name, basis)
+    D = random_density(b.nbf, seed=5, nocc=b.n_occ)
+    Jo, Ko, _ = oracle.jk_direct(b, D)
+    eng = Engine(b, precision=prec)
+    jk = eng.build_jk(D)
+    assert np.abs(jk.J - Jo).max() < tol and np.abs(jk.K - Ko).max() < tol
+    # another split of the same work (tiles set by the caller, bra primitives in ranges) agrees
+    eng.set_tiles([(64, 2)] * 21)
+    eng.set_prim_split(3)
+    jk2 = eng.build_jk(D)
+    assert np.abs(jk2.J - jk.J).max() < tol and np.abs(jk2.K - jk.K).max() < tol
