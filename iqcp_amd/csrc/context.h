@@ -51,8 +51,19 @@ struct qcg_context {
     int64_t mat_total = 0;
     // work buffers
     double *d_D = nullptr, *d_J = nullptr, *d_K = nullptr;
-    // J and K accumulators before symmetrisation, fixed-point (fixacc.h): one word per element
-    fix_t *d_Jacc = nullptr, *d_Kacc = nullptr;
+    // J and K accumulators before symmetrisation, fixed-point (fixacc.h): K one word per matrix element,
+    // J and the density it is contracted with (d_Dp) by shell pair and component (JkLaunch, d_jmap),
+    // the wave-cooperative kernels' J by matrix element (d_Jmat)
+    fix_t *d_Jacc = nullptr, *d_Jmat = nullptr, *d_Kacc = nullptr;
+    double *d_Dp = nullptr, *d_bf_norm = nullptr;
+    int* d_jmap = nullptr;
+    int jbase[kNumPairClasses] = {};
+    // the pairs and primitive pairs as arrays for the per-lane J/K kernels (KetPairs, KetPrims)
+    int4* d_kmeta = nullptr;
+    double2 *d_kcen = nullptr, *d_kprim = nullptr;
+    double* d_khp = nullptr;
+    float4* d_kprimf = nullptr;
+    int n_kprim = 0;
     // their scales per molecule (4 doubles each), recomputed at the start of every build from the
     // shell-pair Schwarz matrices (qsh, packed per molecule), the shell of every function and D
     double *d_fix = nullptr, *d_qsh = nullptr, *d_rowsum = nullptr, *d_qmax = nullptr;
@@ -126,7 +137,6 @@ struct qcg_context {
     std::vector<int4> items;  // J/K work items over the ket segments segs (cut_items)
     std::vector<int2> segs;
     int item_off[21][2] = {}, item_cnt[21][2] = {};
-    int bra_pp[kNumPairClasses] = {};  // per pair class: most primitive pairs of one item's bra
     int4* d_items = nullptr;
     int2* d_segs = nullptr;
     double plan_key[4] = {-1.0, -1.0, -1.0, -1.0};
@@ -188,9 +198,11 @@ struct qcg_context {
     void free_basis() {
         drop_fock_graph();
         for (void** p : {(void**)&d_pairs, (void**)&d_pp, (void**)&d_ppf, (void**)&d_D, (void**)&d_J, (void**)&d_K,
-                         (void**)&d_Jacc, (void**)&d_Kacc, (void**)&d_fix, (void**)&d_qsh, (void**)&d_rowsum,
+                         (void**)&d_Jacc, (void**)&d_Jmat, (void**)&d_Kacc, (void**)&d_fix, (void**)&d_qsh, (void**)&d_rowsum,
                          (void**)&d_qsh_off, (void**)&d_mol_ns, (void**)&d_bf_shell, (void**)&d_bf_off,
                          (void**)&d_qmax, (void**)&d_row_mol, (void**)&d_shell_first, (void**)&d_shell_first_off,
+                         (void**)&d_Dp, (void**)&d_bf_norm, (void**)&d_jmap, (void**)&d_kmeta, (void**)&d_kcen,
+                         (void**)&d_kprim, (void**)&d_khp, (void**)&d_kprimf,
                          (void**)&d_H, (void**)&d_F, (void**)&d_mol_nbf,
                          (void**)&d_mat_off, (void**)&d_ket_off, (void**)&d_ket_cnt, (void**)&d_items,
                          (void**)&d_segs, (void**)&d_grad_items, (void**)&d_grad_segs, (void**)&d_grad,
@@ -262,9 +274,11 @@ struct GraphHold {
 // symmetrize = false: leave J and K in the accumulators (a Fock build reads them there).
 struct JkAcc {
     fix_t* Jacc;
+    fix_t* Jmat;
     fix_t* Kacc;
     double* fix;
     double* rowsum;
+    double* Dp;
 };
 int run_jk(qcg_context* c, const double* dD, double* dJ, double* dK, hipStream_t st, const JkAcc* acc = nullptr,
            bool no_alloc = false, bool symmetrize = true);

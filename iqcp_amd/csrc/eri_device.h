@@ -162,13 +162,12 @@ QCG_HD void for_n(F&& body) {
 // Accumulate the contracted quartet (bra pair P | ket pair Q) into eri[NQ] (row-major
 // [a][b][c][d] over Cartesian components; the primitive-dependent normalisation is folded
 // into ck, the component normalisation is NOT applied here).  ppb: the bra's primitive pairs
-// (P.npp of them, from index 0: a copy staged in LDS or pp + P.pp_off), ppk: the ket's (Q.npp).
+// (P.npp of them, from index 0), ppk: ppk(j) is the ket's primitive pair j (Q.npp of them).
 // TAB_N: rys_tab already points at the coefficients of this class's Rys order (e.g. a copy
 // staged in LDS).  j0, js: the ket primitives taken, j0, j0 + js, ... (0, 1: all of them).
-template <int LA, int LB, int LC, int LD, typename R, bool TAB_N = false>
-QCG_HD void contract_quartet_pp(const PairRec& P, const PairRec& Q, const PrimPair<R>* __restrict__ ppb,
-                                const PrimPair<R>* __restrict__ ppk, const R* __restrict__ rys_tab, R* eri, int j0 = 0,
-                                int js = 1) {
+template <int LA, int LB, int LC, int LD, typename R, bool TAB_N = false, typename Ket>
+QCG_HD void contract_quartet_pp(const PairRec& P, const PairRec& Q, const PrimPair<R>* __restrict__ ppb, Ket&& ppk,
+                                const R* __restrict__ rys_tab, R* eri, int j0 = 0, int js = 1) {
     using S = EriShape<LA, LB, LC, LD>;
     constexpr int N = S::NROOTS;
     const R abx = (R)P.abx, aby = (R)P.aby, abz = (R)P.abz;
@@ -180,7 +179,7 @@ QCG_HD void contract_quartet_pp(const PairRec& P, const PairRec& Q, const PrimPa
     // loop's bra primitive reads are uniform (an LDS broadcast) and each lane loads its ket
     // primitive once
     for (int j = j0; j < Q.npp; j += js) {
-        const PrimPair<R> c = ppk[j];
+        const PrimPair<R> c = ppk(j);
         const R q = c.p;
         const R hq = c.hp;
         const R QCx = c.px - Cx, QCy = c.py - Cy, QCz = c.pz - Cz;
@@ -243,7 +242,8 @@ QCG_HD void contract_quartet_pp(const PairRec& P, const PairRec& Q, const PrimPa
 template <int LA, int LB, int LC, int LD, typename R, bool TAB_N = false>
 QCG_HD void contract_quartet(const PairRec& P, const PairRec& Q, const PrimPair<R>* __restrict__ pp,
                              const R* __restrict__ rys_tab, R* eri) {
-    contract_quartet_pp<LA, LB, LC, LD, R, TAB_N>(P, Q, pp + P.pp_off, pp + Q.pp_off, rys_tab, eri);
+    const PrimPair<R>* ppk = pp + Q.pp_off;
+    contract_quartet_pp<LA, LB, LC, LD, R, TAB_N>(P, Q, pp + P.pp_off, [ppk](int j) { return ppk[j]; }, rys_tab, eri);
 }
 
 }  // namespace qcg

@@ -29,19 +29,21 @@
 #ifndef QCG_CB
 #error "compile with -DQCG_CB=<bra pair class>"
 #endif
-// Per-lane kernel options, both off by default: the bra's primitive pairs staged in LDS (off: the
-// block-uniform reads go through the scalar cache), the D rows of the bra functions staged in LDS
-// next to the K rows (off: the K digestion reads D through the caches).  The smaller LDS footprint
-// keeps more blocks resident: decane, with tiles retuned for each, 643 -> 652 builds/s FP64 and
-// 631 -> 643 mixed without the D rows, then 652 -> 677 and 643 -> 659 without the bra staging.
-#ifndef QCG_JK_BRA_LDS
-#define QCG_JK_BRA_LDS 0
-#endif
-#ifndef QCG_JK_DROWS
-#define QCG_JK_DROWS 0
-#endif
-
 namespace qcg {
+
+// What every J/K kernel of a class takes by value (see JkLaunch).
+struct JkArgs {
+    const int2* segs;
+    const PairRec* bra;
+    const PairRec* ket;
+    KetPairs kpairs;
+    const double *D, *Dp, *fix;
+    fix_t *Jacc, *Jmat, *Kacc;
+    const int* ket_off;
+    const int64_t* mat_off;
+    const int* mol_nbf;
+    int diag, do_j, do_k, jb_bra, jb_ket, np_bra, np_ket;
+};
 
 // The Rys coefficients of order N for a block: staged in LDS (lds, at least rys_tab_size<N>()
 // elements) when N <= 3, where the per-lane kernels gather them at lane-dependent intervals once
@@ -60,63 +62,37 @@ constexpr int rys_lds_doubles() { return N <= 3 ? rys_tab_size<N>() : 1; }
 
 // One work item = (bra pair, run of its surviving kets over the ket segments, KetCursor); the
 // host builds the items with the exact screening predicate, so no quartet is tested twice or
-// skipped.  rys_n: the coefficients of this class's Rys order (rys_stage); bp: LDS room for the
-// bra's primitive pairs; rows: LDS room for the K rows of the bra functions a and b (krow bit 0:
-// (NA + NB) x nbf fixed-point words, fixacc.h, in which the four K terms of the item, all in the
-// rows of a and b, are summed and then flushed once per block) followed by their D rows (bit 1:
-// (NA + NB) x nbf doubles, read by the K digestion).  J and K go to the fixed-point accumulators
-// Jacc/Kacc with the scales fix[4 mol], fix[4 mol + 1], so the result does not depend on the order
-// in which blocks and lanes arrive.
-template <int LA, int LB, int LC, int LD, typename R, int ROWS>
-__device__ __forceinline__ void jk_item(
-    const int4 it, const int2* __restrict__ segs, const PairRec* __restrict__ bra, const PairRec* __restrict__ ket, int diag,
-    const PrimPair<R>* __restrict__ pp, const R* __restrict__ rys_n, const double* __restrict__ D,
-    fix_t* __restrict__ Jacc, fix_t* __restrict__ Kacc, const double* __restrict__ fix, int do_j, int do_k,
-    const int* __restrict__ ket_off, const int64_t* __restrict__ mat_off, const int* __restrict__ mol_nbf,
-    PrimPair<R>* bp, double* rows) {
-#if !QCG_JK_BRA_LDS
-    (void)bp;
-#endif
+// skipped.  rys_n: the coefficients of this class's Rys order (rys_stage); rows: with KROWS, LDS room
+// for the K rows of the bra functions a and b ((NA + NB) x nbf fixed-point words, fixacc.h), in which
+// the four K terms of the item, all in the rows of a and b, are summed and then flushed once per
+// block.  J and K go to the fixed-point accumulators Jacc (by shell pair) and Kacc with the scales
+// fix[4 mol], fix[4 mol + 1], so the result does not depend on the order in which blocks and lanes
+// arrive.  The bra's primitive pairs are uniform over the block and come through the scalar cache;
+// the D rows of K through the vector caches.
+template <int LA, int LB, int LC, int LD, typename R, bool KROWS>
+__device__ __forceinline__ void jk_item(const int4 it, const JkArgs& g, const KetPrims<R>& kprims,
+                                        const PrimPair<R>* __restrict__ pp, const R* __restrict__ rys_n, double* rows) {
     using S = EriShape<LA, LB, LC, LD>;
     constexpr bool U = S::kUnroll;
     constexpr int NR = S::NA + S::NB;
-    const PairRec P = item_bra(bra, it);
-    const int pidx = P.pos;
-    ket += ket_off[P.mol];
-    D += mat_off[P.mol];
-    Jacc += mat_off[P.mol];
-    Kacc += mat_off[P.mol];
-    const int nbf = mol_nbf[P.mol];
-    const double sJ = fix[4 * P.mol], sK = fix[4 * P.mol + 1];  // fixed-point scales of J and K
+    const PairRec P = item_bra(g.bra, it);
+    const int pidx = P.pos, ket0 = g.ket_off[P.mol];
+    const double* __restrict__ D = g.D + g.mat_off[P.mol];
+    fix_t* __restrict__ Jacc = g.Jacc;
+    fix_t* __restrict__ Kacc = g.Kacc + g.mat_off[P.mol];
+    const int nbf = g.mol_nbf[P.mol], do_j = g.do_j, do_k = g.do_k;
+    const double sJ = g.fix[4 * P.mol], sK = g.fix[4 * P.mol + 1];  // fixed-point scales of J and K
     const int tid = threadIdx.x;
-#if QCG_JK_BRA_LDS
-    for (int i = tid; i < P.npp; i += blockDim.x) bp[i] = pp[P.pp_off + i];
-    const PrimPair<R>* ppb = bp;
-#else
     const PrimPair<R>* ppb = pp + P.pp_off;
-#endif
-    // ROWS bit 0: K rows in LDS, bit 1: D rows in LDS after them (compile-time, so each
-    // instantiation holds one addressing path only)
-    constexpr bool kr = ROWS & 1, dr = ROWS & 2;
     const int nrow = NR * nbf;
     fix_t* kl = reinterpret_cast<fix_t*>(rows);
-    double* dl = rows + (kr ? nrow : 0);
-    if constexpr (ROWS != 0)
-        for (int i = tid; i < nrow; i += blockDim.x) {
-            if constexpr (dr) {
-                const int r = i / nbf, col = i - r * nbf;
-                dl[i] = D[(size_t)(r < S::NA ? P.bfa + r : P.bfb + (r - S::NA)) * nbf + col];
-            }
-            if constexpr (kr) kl[i] = 0;
-        }
+    if constexpr (KROWS)
+        for (int i = tid; i < nrow; i += blockDim.x) kl[i] = 0;
     __syncthreads();
     // D element (row function a + r of the bra's shell a, or b + r of shell b; column col)
-    auto drow = [&](bool row_b, int r, int col) -> double {
-        if constexpr (dr) return dl[(row_b ? S::NA + r : r) * nbf + col];
-        else return D[(size_t)((row_b ? P.bfb : P.bfa) + r) * nbf + col];
-    };
+    auto drow = [&](bool row_b, int r, int col) -> double { return D[(size_t)((row_b ? P.bfb : P.bfa) + r) * nbf + col]; };
     auto kadd = [&](bool row_b, int r, int col, double v) {
-        if constexpr (kr) fix_add_lds(kl, (row_b ? S::NA + r : r) * nbf + col, v, sK);
+        if constexpr (KROWS) fix_add_lds(kl, (row_b ? S::NA + r : r) * nbf + col, v, sK);
         else fix_add_global(Kacc, (size_t)((row_b ? P.bfb : P.bfa) + r) * nbf + col, v, sK);
     };
 
@@ -133,25 +109,36 @@ __device__ __forceinline__ void jk_item(
     // primitive and a fixed butterfly sums the partial quartets, so a heavily contracted quartet is
     // no longer one lane's serial chain (alone, water (ss|ss) 335 -> 21 us, (pp|pp) 231 -> 50 us)
     const int lg = item_lg(it), lanes = 1 << lg, sub = tid & (lanes - 1), step = blockDim.x >> lg;
-    KetCursor cur{segs, it.y, it.z + (tid >> lg)};
+    KetCursor cur{g.segs, it.y, it.z + (tid >> lg)};
     for (int j = tid >> lg; j < item_kets(it); j += step, cur.r += step) {
-        const int q = cur.at();
-        const PairRec Q = ket[q];
+        const int q = cur.at(), kq = ket0 + q;
+        const int4 km = g.kpairs.meta[kq];
+        PairRec Q;
+        Q.bfa = km.x & ~kKetSame;
+        Q.bfb = km.y;
+        Q.npp = (unsigned)km.w >> 24;
+        const int kstride = km.w & 0xffffff;
+        if constexpr (LC > 0) {
+            const double2 c0 = g.kpairs.cen[kq], c1 = g.kpairs.cen[g.kpairs.np + kq];
+            Q.ax = c0.x, Q.ay = c0.y, Q.az = c1.x, Q.abx = c1.y;
+            if constexpr (LD > 0) {
+                const double2 c2 = g.kpairs.cen[2 * g.kpairs.np + kq];
+                Q.aby = c2.x, Q.abz = c2.y;
+            }
+        }
         R eri[S::NQ];
         for_n<U, S::NQ>([&](int i) { eri[i] = R(0); });
-        contract_quartet_pp<LA, LB, LC, LD, R, true>(P, Q, ppb, pp + Q.pp_off, rys_n, eri, sub, lanes);
+        contract_quartet_pp<LA, LB, LC, LD, R, true>(
+            P, Q, ppb, [&](int i) { return kprims.at(km.z + i * kstride); }, rys_n, eri, sub, lanes);
         if (lg) {
             for (int off = 1; off < lanes; off <<= 1)
                 for_n<U, S::NQ>([&](int i) { eri[i] += __shfl_xor(eri[i], off, 64); });
             if (sub) continue;  // the group's first lane digests
         }
-        const double deg = deg_p * ((Q.sa == Q.sb) ? 0.5 : 1.0) * ((diag && q == pidx) ? 0.5 : 1.0);
+        const double deg = deg_p * ((km.x & kKetSame) ? 0.5 : 1.0) * ((g.diag && q == pidx) ? 0.5 : 1.0);
         if (do_j) {
             double Dqs[S::NCD];
-            for_n<U, S::NCD>([&](int cd) {
-                const int c = cd / S::ND, d = cd % S::ND;
-                Dqs[cd] = D[(size_t)(Q.bfa + c) * nbf + Q.bfb + d] * cnorm(LC, c) * cnorm(LD, d);
-            });
+            for_n<U, S::NCD>([&](int cd) { Dqs[cd] = g.Dp[g.jb_ket + cd * g.np_ket + kq]; });
             const double fj = 2.0 * deg;
             for_n<U, S::NAB>([&](int ab) {
                 double s = 0.0;
@@ -163,7 +150,7 @@ __device__ __forceinline__ void jk_item(
                 double s = 0.0;
                 for_n<U, S::NAB>([&](int ab) { s += Dps[ab] * (double)eri[ab * S::NCD + cd]; });
                 const int c = cd / S::ND, d = cd % S::ND;
-                fix_add_global(Jacc, (size_t)(Q.bfa + c) * nbf + Q.bfb + d, fj * cnorm(LC, c) * cnorm(LD, d) * s, sJ);
+                fix_add_global(Jacc, g.jb_ket + cd * g.np_ket + kq, fj * cnorm(LC, c) * cnorm(LD, d) * s, sJ);
             });
         }
         if (do_k) {
@@ -232,13 +219,10 @@ __device__ __forceinline__ void jk_item(
             double s = jp[ab];
 #pragma unroll
             for (int off = 32; off >= 1; off >>= 1) s += __shfl_xor(s, off, 64);
-            if ((tid & 63) == 0 && s != 0.0) {
-                const int a = ab / S::NB, b = ab % S::NB;
-                fix_add_global(Jacc, (size_t)(P.bfa + a) * nbf + P.bfb + b, s, sJ);
-            }
+            if ((tid & 63) == 0 && s != 0.0) fix_add_global(Jacc, g.jb_bra + ab * g.np_bra + it.x, s, sJ);
         });
     }
-    if constexpr (kr) {
+    if constexpr (KROWS) {
         __syncthreads();
         for (int i = tid; i < nrow; i += blockDim.x) {
             const int r = i / nbf, col = i - r * nbf;
@@ -248,70 +232,44 @@ __device__ __forceinline__ void jk_item(
     }
 }
 
-// LDS layout of the per-lane kernels' rows for nbf functions (the largest molecule's): K rows
-// as fixed-point words, (NA + NB) x nbf x 8 bytes, when they fit the budget left by the static
-// LDS (Rys coefficients, bra primitives), then the D rows, (NA + NB) x nbf x 8 bytes, when those
-// fit too.  Returns the krow flags (bit 0 K rows, bit 1 D rows) and the dynamic LDS bytes.
+// Dynamic LDS of a per-lane block: the K rows for nbf functions (the largest molecule's), when they
+// fit the budget left by the Rys coefficients; 0: K goes to memory directly.
 constexpr size_t kLdsBudget = 65536;
 template <int LA, int LB, int LC, int LD>
-inline int jk_row_flags(int nbf, int do_k, int bra_pp, size_t* bytes) {
+inline size_t jk_row_bytes(int nbf, int do_k) {
     using S = EriShape<LA, LB, LC, LD>;
-    const size_t fixed = (size_t)rys_lds_doubles<S::NROOTS>() * sizeof(double) + (size_t)bra_pp * sizeof(PrimPair<double>);
-    const size_t kb = (size_t)(S::NA + S::NB) * nbf * sizeof(fix_t), db = (size_t)(S::NA + S::NB) * nbf * sizeof(double);
-    int f = 0;
-    size_t n = 0;
-    if (do_k && fixed + kb <= kLdsBudget) {
-        f |= 1;
-        n += kb;
-    }
-    if (QCG_JK_DROWS && (f & 1) && fixed + n + db <= kLdsBudget) {
-        f |= 2;
-        n += db;
-    }
-    *bytes = n + (size_t)bra_pp * sizeof(PrimPair<double>);
-    return f;
+    const size_t kb = (size_t)(S::NA + S::NB) * nbf * sizeof(fix_t);
+    return do_k && (size_t)rys_lds_doubles<S::NROOTS>() * sizeof(double) + kb <= kLdsBudget ? kb : 0;
 }
 
-template <int LA, int LB, int LC, int LD, typename R, int ROWS>
-__global__ __launch_bounds__(256) void jk_kernel(
-    const int4* __restrict__ items, const int2* __restrict__ segs, const PairRec* __restrict__ bra, const PairRec* __restrict__ ket, int diag,
-    const PrimPair<R>* __restrict__ pp, const R* __restrict__ rys_tab, const double* __restrict__ D,
-    fix_t* __restrict__ Jacc, fix_t* __restrict__ Kacc, const double* __restrict__ fix, int do_j, int do_k,
-    const int* __restrict__ ket_off, const int64_t* __restrict__ mat_off, const int* __restrict__ mol_nbf,
-    int bra_pp) {
+template <int LA, int LB, int LC, int LD, typename R, bool KROWS>
+__global__ __launch_bounds__(256) void jk_kernel(const int4* __restrict__ items, const JkArgs g, const KetPrims<R> kprims,
+                                                 const PrimPair<R>* __restrict__ pp, const R* __restrict__ rys_tab) {
     constexpr int NR = EriShape<LA, LB, LC, LD>::NROOTS;
-    extern __shared__ double dyn[];  // bra primitive pairs (bra_pp), then the K / D rows
+    extern __shared__ double rows[];
     __shared__ double rys_raw[rys_lds_doubles<NR>()];
     const R* rys_n = rys_stage<R, NR>(rys_tab, reinterpret_cast<R*>(rys_raw));
-    jk_item<LA, LB, LC, LD, R, ROWS>(items[blockIdx.x], segs, bra, ket, diag, pp, rys_n, D, Jacc, Kacc, fix, do_j, do_k,
-                                     ket_off, mat_off, mol_nbf, reinterpret_cast<PrimPair<R>*>(dyn),
-                               dyn + bra_pp * sizeof(PrimPair<R>) / sizeof(double));
+    jk_item<LA, LB, LC, LD, R, KROWS>(items[blockIdx.x], g, kprims, pp, rys_n, rows);
 }
 
 // Mixed precision in one launch: items [0, n64) are FP64 quartets, the rest FP32 (one branch per
 // block); saves the second launch per class and its tail.
-template <int LA, int LB, int LC, int LD, int ROWS>
-__global__ __launch_bounds__(256) void jk_kernel_mp(
-    const int4* __restrict__ items, const int2* __restrict__ segs, int n64, const PairRec* __restrict__ bra, const PairRec* __restrict__ ket,
-    int diag, const PrimPair<double>* __restrict__ pp, const PrimPair<float>* __restrict__ ppf,
-    const double* __restrict__ rys_tab, const float* __restrict__ rys_tabf, const double* __restrict__ D,
-    fix_t* __restrict__ Jacc, fix_t* __restrict__ Kacc, const double* __restrict__ fix, int do_j, int do_k,
-    const int* __restrict__ ket_off, const int64_t* __restrict__ mat_off, const int* __restrict__ mol_nbf,
-    int bra_pp) {
+template <int LA, int LB, int LC, int LD, bool KROWS>
+__global__ __launch_bounds__(256) void jk_kernel_mp(const int4* __restrict__ items, int n64, const JkArgs g,
+                                                    const KetPrims<double> kprims, const KetPrims<float> kprimsf,
+                                                    const PrimPair<double>* __restrict__ pp,
+                                                    const PrimPair<float>* __restrict__ ppf,
+                                                    const double* __restrict__ rys_tab,
+                                                    const float* __restrict__ rys_tabf) {
     constexpr int NR = EriShape<LA, LB, LC, LD>::NROOTS;
-    extern __shared__ double dyn[];  // bra primitive pairs (bra_pp FP64 slots), then the K / D rows
+    extern __shared__ double rows[];
     __shared__ double rys_raw[rys_lds_doubles<NR>()];
-    double* rows = dyn + bra_pp * sizeof(PrimPair<double>) / sizeof(double);
     if ((int)blockIdx.x < n64) {
         const double* rys_n = rys_stage<double, NR>(rys_tab, rys_raw);
-        jk_item<LA, LB, LC, LD, double, ROWS>(items[blockIdx.x], segs, bra, ket, diag, pp, rys_n, D, Jacc, Kacc, fix,
-                                              do_j, do_k, ket_off, mat_off, mol_nbf,
-                                              reinterpret_cast<PrimPair<double>*>(dyn), rows);
+        jk_item<LA, LB, LC, LD, double, KROWS>(items[blockIdx.x], g, kprims, pp, rys_n, rows);
     } else {
         const float* rys_n = rys_stage<float, NR>(rys_tabf, reinterpret_cast<float*>(rys_raw));
-        jk_item<LA, LB, LC, LD, float, ROWS>(items[blockIdx.x], segs, bra, ket, diag, ppf, rys_n, D, Jacc, Kacc, fix,
-                                             do_j, do_k, ket_off, mat_off, mol_nbf,
-                                             reinterpret_cast<PrimPair<float>*>(dyn), rows);
+        jk_item<LA, LB, LC, LD, float, KROWS>(items[blockIdx.x], g, kprimsf, ppf, rys_n, rows);
     }
 }
 
@@ -336,10 +294,7 @@ struct JkWave {
 // One work item on one wavefront; V: the wave's LDS region (JkWave<..., R>::WAVE_D doubles).
 template <int LA, int LB, int LC, int LD, typename R>
 __device__ __forceinline__ void jk_wave_item(
-    const int4 it, const int2* __restrict__ segs, int lane, double* V, const PairRec* __restrict__ bra, const PairRec* __restrict__ ket,
-    int diag, const PrimPair<R>* __restrict__ pp, const R* __restrict__ rys_tab, const double* __restrict__ D,
-    fix_t* __restrict__ Jacc, fix_t* __restrict__ Kacc, const double* __restrict__ fix, int do_j, int do_k,
-    const int* __restrict__ ket_off, const int64_t* __restrict__ mat_off, const int* __restrict__ mol_nbf) {
+    const int4 it, int lane, double* V, const JkArgs& g, const PrimPair<R>* __restrict__ pp, const R* __restrict__ rys_tab) {
     using S = EriShape<LA, LB, LC, LD>;
     using W = JkWave<LA, LB, LC, LD, R>;
     using TB = typename W::T;
@@ -353,14 +308,15 @@ __device__ __forceinline__ void jk_wave_item(
     double* Dbc = Dad + NA * ND;
     double* Dac = Dbc + NB * NC;
 
-    const PairRec P = item_bra(bra, it);
+    const PairRec P = item_bra(g.bra, it);
     const int pidx = P.pos;
-    ket += ket_off[P.mol];
-    D += mat_off[P.mol];
-    Jacc += mat_off[P.mol];
-    Kacc += mat_off[P.mol];
-    const size_t nbf = (size_t)mol_nbf[P.mol];
-    const double sJ = fix[4 * P.mol], sK = fix[4 * P.mol + 1];  // fixed-point scales of J and K
+    const PairRec* __restrict__ ket = g.ket + g.ket_off[P.mol];
+    const double* __restrict__ D = g.D + g.mat_off[P.mol];
+    fix_t* __restrict__ Jmat = g.Jmat + g.mat_off[P.mol];
+    fix_t* __restrict__ Kacc = g.Kacc + g.mat_off[P.mol];
+    const size_t nbf = (size_t)g.mol_nbf[P.mol];
+    const int do_j = g.do_j, do_k = g.do_k;
+    const double sJ = g.fix[4 * P.mol], sK = g.fix[4 * P.mol + 1];  // fixed-point scales of J and K
 
     constexpr const CompTab<LA, LB, LC, LD>& ct = kCompTab<LA, LB, LC, LD>;
     int ox[KPL], oy[KPL], oz[KPL];
@@ -376,7 +332,7 @@ __device__ __forceinline__ void jk_wave_item(
     double jp = 0.0;  // J_ab of lane ab over the item's kets
     const double deg_p = (P.sa == P.sb) ? 0.5 : 1.0;
 
-    KetCursor cur{segs, it.y, it.z};
+    KetCursor cur{g.segs, it.y, it.z};
     for (int j = 0; j < item_kets(it); ++j, ++cur.r) {
         const int q = cur.at();
         const PairRec Q = ket[q];
@@ -396,7 +352,7 @@ __device__ __forceinline__ void jk_wave_item(
             }
         }
         wave_sync();
-        const double deg = deg_p * ((Q.sa == Q.sb) ? 0.5 : 1.0) * ((diag && q == pidx) ? 0.5 : 1.0);
+        const double deg = deg_p * ((Q.sa == Q.sb) ? 0.5 : 1.0) * ((g.diag && q == pidx) ? 0.5 : 1.0);
 #pragma unroll
         for (int j = 0; j < KPL; ++j) {
             const int k = lane + 64 * j;
@@ -424,7 +380,7 @@ __device__ __forceinline__ void jk_wave_item(
             for (int o = lane; o < NCD; o += 64) {
                 double s = 0.0;
                 for (int ab = 0; ab < S::NAB; ++ab) s += Dab[ab] * V[ab * NCD + o];
-                fix_add_global(Jacc, (Q.bfa + o / ND) * nbf + Q.bfb + o % ND, 2.0 * s, sJ);
+                fix_add_global(Jmat, (Q.bfa + o / ND) * nbf + Q.bfb + o % ND, 2.0 * s, sJ);
             }
         }
         if (do_k) {
@@ -459,45 +415,35 @@ __device__ __forceinline__ void jk_wave_item(
         }
 #undef VAT
     }
-    if (do_j && lane < S::NAB && jp != 0.0) fix_add_global(Jacc, (P.bfa + lane / NB) * nbf + P.bfb + lane % NB, jp, sJ);
+    if (do_j && lane < S::NAB && jp != 0.0) fix_add_global(Jmat, (P.bfa + lane / NB) * nbf + P.bfb + lane % NB, jp, sJ);
 }
 
 template <int LA, int LB, int LC, int LD, typename R>
-__global__ __launch_bounds__(256) void jk_wave_kernel(
-    const int4* __restrict__ items, const int2* __restrict__ segs, int nitems, const PairRec* __restrict__ bra, const PairRec* __restrict__ ket,
-    int diag, const PrimPair<R>* __restrict__ pp, const R* __restrict__ rys_tab, const double* __restrict__ D,
-    fix_t* __restrict__ Jacc, fix_t* __restrict__ Kacc, const double* __restrict__ fix, int do_j, int do_k,
-    const int* __restrict__ ket_off, const int64_t* __restrict__ mat_off, const int* __restrict__ mol_nbf) {
+__global__ __launch_bounds__(256) void jk_wave_kernel(const int4* __restrict__ items, int nitems, const JkArgs g,
+                                                      const PrimPair<R>* __restrict__ pp, const R* __restrict__ rys_tab) {
     constexpr int WD = JkWave<LA, LB, LC, LD, R>::WAVE_D;
     __shared__ double smem[4 * WD];
     const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int item = blockIdx.x * 4 + wid;
     if (item >= nitems) return;  // no block-wide barriers in the item: waves are independent
-    jk_wave_item<LA, LB, LC, LD, R>(items[item], segs, lane, smem + wid * WD, bra, ket, diag, pp, rys_tab, D, Jacc, Kacc,
-                                    fix, do_j, do_k, ket_off, mat_off, mol_nbf);
+    jk_wave_item<LA, LB, LC, LD, R>(items[item], lane, smem + wid * WD, g, pp, rys_tab);
 }
 
 // Mixed precision in one launch: items [0, n64) FP64, the rest FP32 (one branch per wavefront).
 template <int LA, int LB, int LC, int LD>
-__global__ __launch_bounds__(256) void jk_wave_kernel_mp(
-    const int4* __restrict__ items, const int2* __restrict__ segs, int nitems, int n64, const PairRec* __restrict__ bra,
-    const PairRec* __restrict__ ket, int diag, const PrimPair<double>* __restrict__ pp,
-    const PrimPair<float>* __restrict__ ppf, const double* __restrict__ rys_tab, const float* __restrict__ rys_tabf,
-    const double* __restrict__ D, fix_t* __restrict__ Jacc, fix_t* __restrict__ Kacc, const double* __restrict__ fix,
-    int do_j, int do_k, const int* __restrict__ ket_off, const int64_t* __restrict__ mat_off,
-    const int* __restrict__ mol_nbf) {
+__global__ __launch_bounds__(256) void jk_wave_kernel_mp(const int4* __restrict__ items, int nitems, int n64,
+                                                         const JkArgs g, const PrimPair<double>* __restrict__ pp,
+                                                         const PrimPair<float>* __restrict__ ppf,
+                                                         const double* __restrict__ rys_tab,
+                                                         const float* __restrict__ rys_tabf) {
     constexpr int WD64 = JkWave<LA, LB, LC, LD, double>::WAVE_D, WD32 = JkWave<LA, LB, LC, LD, float>::WAVE_D;
     constexpr int WD = WD64 > WD32 ? WD64 : WD32;
     __shared__ double smem[4 * WD];
     const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int item = blockIdx.x * 4 + wid;
     if (item >= nitems) return;
-    if (item < n64)
-        jk_wave_item<LA, LB, LC, LD, double>(items[item], segs, lane, smem + wid * WD, bra, ket, diag, pp, rys_tab, D, Jacc,
-                                             Kacc, fix, do_j, do_k, ket_off, mat_off, mol_nbf);
-    else
-        jk_wave_item<LA, LB, LC, LD, float>(items[item], segs, lane, smem + wid * WD, bra, ket, diag, ppf, rys_tabf, D, Jacc,
-                                            Kacc, fix, do_j, do_k, ket_off, mat_off, mol_nbf);
+    if (item < n64) jk_wave_item<LA, LB, LC, LD, double>(items[item], lane, smem + wid * WD, g, pp, rys_tab);
+    else jk_wave_item<LA, LB, LC, LD, float>(items[item], lane, smem + wid * WD, g, ppf, rys_tabf);
 }
 
 __device__ __forceinline__ int64_t pair_index64(int64_t i, int64_t j) {
@@ -546,6 +492,11 @@ __global__ __launch_bounds__(256) void eri_tensor_kernel(
 template <typename S>
 inline constexpr bool kLaneForm = S::NQ <= kJkLaneMaxNQ;
 
+static JkArgs jk_args(const JkLaunch& a) {
+    return {a.segs, a.bra, a.ket, a.kpairs, a.D, a.Dp, a.fix, a.Jacc, a.Jmat, a.Kacc, a.ket_off, a.mat_off, a.mol_nbf,
+            a.diag, a.do_j, a.do_k, a.jb_bra, a.jb_ket, a.np_bra, a.np_ket};
+}
+
 template <int CB, int CK, typename R>
 static hipError_t launch_jk_t(const JkLaunch& a, hipStream_t st) {
     constexpr int LA = QCG_LA(CB), LB = QCG_LB(CB), LC = QCG_LA(CK), LD = QCG_LB(CK);
@@ -554,27 +505,24 @@ static hipError_t launch_jk_t(const JkLaunch& a, hipStream_t st) {
     // wave-cooperative mode (four items per block); classes without a per-lane form always take it
     if (a.block == 0 || !kLaneForm<S>) {
         if constexpr (JkWave<LA, LB, LC, LD, R>::kEnabled) {
-            hipLaunchKernelGGL((jk_wave_kernel<LA, LB, LC, LD, R>), dim3((a.nitems + 3) / 4), dim3(256), 0, st,
-                               a.items, a.segs, a.nitems, a.bra, a.ket, a.diag, (const PrimPair<R>*)a.pp, (const R*)a.rys,
-                               a.D, a.Jacc, a.Kacc, a.fix, a.do_j, a.do_k, a.ket_off, a.mat_off, a.mol_nbf);
+            hipLaunchKernelGGL((jk_wave_kernel<LA, LB, LC, LD, R>), dim3((a.nitems + 3) / 4), dim3(256), 0, st, a.items,
+                               a.nitems, jk_args(a), (const PrimPair<R>*)a.pp, (const R*)a.rys);
             return hipGetLastError();
         }
     }
     if constexpr (kLaneForm<S>) {
-        // K and D rows of the bra functions in LDS when they fit (a.nbf is the largest molecule's nbf)
-        size_t dyn_bytes = 0;
-        const int bra_pp = QCG_JK_BRA_LDS ? a.bra_pp : 0;
-        const int krow = jk_row_flags<LA, LB, LC, LD>(a.nbf, a.do_k, bra_pp, &dyn_bytes);
-        auto go = [&](auto rows_c) {
-            constexpr int ROWS = decltype(rows_c)::value;
-            hipLaunchKernelGGL((jk_kernel<LA, LB, LC, LD, R, ROWS>), dim3(a.nitems), dim3(a.block > 0 ? a.block : 64),
-                               dyn_bytes, st, a.items, a.segs, a.bra, a.ket, a.diag, (const PrimPair<R>*)a.pp,
-                               (const R*)a.rys, a.D, a.Jacc, a.Kacc, a.fix, a.do_j, a.do_k, a.ket_off, a.mat_off,
-                               a.mol_nbf, bra_pp);
-        };
-        if (krow == 3) go(std::integral_constant<int, 3>{});
-        else if (krow == 1) go(std::integral_constant<int, 1>{});
-        else go(std::integral_constant<int, 0>{});
+        // K rows of the bra functions in LDS when they fit (a.nbf is the largest molecule's nbf)
+        const size_t rows = jk_row_bytes<LA, LB, LC, LD>(a.nbf, a.do_k);
+        const KetPrims<R>* kp;
+        if constexpr (sizeof(R) == 8) kp = &a.kprims;
+        else kp = &a.kprimsf;
+        const dim3 block(a.block > 0 ? a.block : 64);
+        if (rows)
+            hipLaunchKernelGGL((jk_kernel<LA, LB, LC, LD, R, true>), dim3(a.nitems), block, rows, st, a.items, jk_args(a),
+                               *kp, (const PrimPair<R>*)a.pp, (const R*)a.rys);
+        else
+            hipLaunchKernelGGL((jk_kernel<LA, LB, LC, LD, R, false>), dim3(a.nitems), block, 0, st, a.items, jk_args(a),
+                               *kp, (const PrimPair<R>*)a.pp, (const R*)a.rys);
         return hipGetLastError();
     } else {
         return hipErrorInvalidValue;  // not reached: large classes take the wave-cooperative form above
@@ -591,28 +539,22 @@ static hipError_t launch_jk_mp_t(const JkLaunch& a, hipStream_t st) {
     // classes without a per-lane form always take the wave-cooperative one
     if (a.block == 0 || !kLaneForm<S>) {
         if constexpr (JkWave<LA, LB, LC, LD, double>::kEnabled) {
-            hipLaunchKernelGGL((jk_wave_kernel_mp<LA, LB, LC, LD>), dim3((a.nitems + 3) / 4), dim3(256), 0, st,
-                               a.items, a.segs, a.nitems, a.n64, a.bra, a.ket, a.diag, (const PrimPair<double>*)a.pp,
-                               (const PrimPair<float>*)a.ppf, (const double*)a.rys, (const float*)a.rysf, a.D, a.Jacc,
-                               a.Kacc, a.fix, a.do_j, a.do_k, a.ket_off, a.mat_off, a.mol_nbf);
+            hipLaunchKernelGGL((jk_wave_kernel_mp<LA, LB, LC, LD>), dim3((a.nitems + 3) / 4), dim3(256), 0, st, a.items,
+                               a.nitems, a.n64, jk_args(a), (const PrimPair<double>*)a.pp, (const PrimPair<float>*)a.ppf,
+                               (const double*)a.rys, (const float*)a.rysf);
             return hipGetLastError();
         }
     }
     if constexpr (kLaneForm<S>) {
-        size_t dyn_bytes = 0;
-        const int bra_pp = QCG_JK_BRA_LDS ? a.bra_pp : 0;
-        const int krow = jk_row_flags<LA, LB, LC, LD>(a.nbf, a.do_k, bra_pp, &dyn_bytes);
+        const size_t rows = jk_row_bytes<LA, LB, LC, LD>(a.nbf, a.do_k);
         auto go = [&](auto rows_c) {
-            constexpr int ROWS = decltype(rows_c)::value;
-            hipLaunchKernelGGL((jk_kernel_mp<LA, LB, LC, LD, ROWS>), dim3(a.nitems), dim3(a.block > 0 ? a.block : 64),
-                               dyn_bytes, st, a.items, a.segs, a.n64, a.bra, a.ket, a.diag,
-                               (const PrimPair<double>*)a.pp, (const PrimPair<float>*)a.ppf, (const double*)a.rys,
-                               (const float*)a.rysf, a.D, a.Jacc, a.Kacc, a.fix, a.do_j, a.do_k, a.ket_off, a.mat_off,
-                               a.mol_nbf, bra_pp);
+            hipLaunchKernelGGL((jk_kernel_mp<LA, LB, LC, LD, decltype(rows_c)::value>), dim3(a.nitems),
+                               dim3(a.block > 0 ? a.block : 64), rows, st, a.items, a.n64, jk_args(a), a.kprims,
+                               a.kprimsf, (const PrimPair<double>*)a.pp, (const PrimPair<float>*)a.ppf,
+                               (const double*)a.rys, (const float*)a.rysf);
         };
-        if (krow == 3) go(std::integral_constant<int, 3>{});
-        else if (krow == 1) go(std::integral_constant<int, 1>{});
-        else go(std::integral_constant<int, 0>{});
+        if (rows) go(std::true_type{});
+        else go(std::false_type{});
         return hipGetLastError();
     } else {
         return hipErrorInvalidValue;  // not reached: large classes take the wave-cooperative form above

@@ -56,9 +56,8 @@ inline void cut_items_split(std::vector<int4>& items, const std::vector<int2>& s
 inline QCG_HD int item_kets(const int4& it) { return it.w & kItemMaxKets; }
 inline QCG_HD int item_lg(const int4& it) { return (it.w >> 13) & 7; }
 
-// Most bra primitive pairs one per-lane J/K item may have: the kernel stages them in LDS (a block's
-// bra pair is uniform, so the inner primitive loop reads them as LDS broadcasts instead of scalar
-// loads).  The planner cuts heavier bras into primitive ranges of at most this many.
+// Most bra primitive pairs one J/K item may have: the planner cuts heavier bras into primitive ranges
+// of at most this many.
 constexpr int kBraPPMax = 64;
 
 // Largest class (Cartesian components) with a per-lane J/K kernel; larger classes always run the
@@ -105,8 +104,18 @@ struct JkLaunch {
     const void* rys;    // Rys table (double or float)
     const double* D;    // density, nbf x nbf, symmetric
     int nbf;
-    fix_t* Jacc;        // fixed-point accumulators (fixacc.h), one word per element
-    fix_t* Kacc;
+    // J side by shell pair instead of by matrix element: component ab of pair i (index in its class)
+    // is word base + ab * (pairs of the class) + i of Dp (the density with the component norms) and
+    // Jacc (its accumulator), so the lanes of a wavefront, on consecutive kets, touch consecutive words
+    const double* Dp;
+    int jb_bra, jb_ket, np_bra, np_ket;  // bases and pair counts of the two classes
+    fix_t* Jacc;        // fixed-point accumulators (fixacc.h): J by shell pair
+    fix_t* Jmat;        // the wave-cooperative kernels' J, nbf x nbf: their few lanes per ket would all
+                        // add to the same lines of Jacc ((dd|ps) of benzene 52 -> 109 us)
+    fix_t* Kacc;        // nbf x nbf
+    KetPairs kpairs;    // the kets of the class as arrays (per-lane kernels); primitives in kprims / kprimsf
+    KetPrims<double> kprims;
+    KetPrims<float> kprimsf;
     const double* fix;  // per molecule: scale of J, scale of K, and their inverses (fix_scale_kernel)
     double thr_lo;      // process quartets with thr_lo <= Q_P Q_Q < thr_hi
     double thr_hi;
@@ -125,7 +134,6 @@ struct JkLaunch {
     const int2* segs;
     int nitems;
     int block;
-    int bra_pp;         // most primitive pairs of any bra of the items (<= kBraPPMax): LDS staging
     // mixed precision in one launch (n64 >= 0): the first n64 items are FP64, the rest FP32 with
     // the FP32 primitive pairs ppf and Rys table rysf; n64 < 0: one precision, given by the caller
     int n64 = -1;
@@ -239,20 +247,25 @@ struct FixData {
     const double* qmax;
     const int* shell_first;
     const int* shell_first_off;
+    // word of the pair-ordered J arrays (JkLaunch) that matrix element e belongs to, -1 for the
+    // elements of the pair's transposed block, and the component norm of every function
+    const int* jmap;
+    const double* bf_norm;
 };
 // Per molecule m the fixed-point scales fix[4m] (J) and fix[4m + 1] (K) and their inverses from a
 // bound on the accumulated magnitudes at density D: B_J = 2 Qmax sum_ls Q_ls |D_ls|,
 // B_K = 2 Qmax max_s sum_t Q_st sum_(n in t) sum_l |D_nl|.  Also zeroes the accumulators Jacc and
 // Kacc (either may be null).
-hipError_t launch_fix_scale(const double* D, const FixData& f, double* fix, int nmol, fix_t* Jacc, fix_t* Kacc,
-                            hipStream_t st);
-hipError_t launch_symmetrize(const fix_t* Jacc, const fix_t* Kacc, const double* fix, double* J, double* K, int nbf,
-                             hipStream_t st);
+// With Jacc also fills the pair-ordered density Dp.
+hipError_t launch_fix_scale(const double* D, const FixData& f, double* fix, int nmol, fix_t* Jacc, fix_t* Jmat,
+                            fix_t* Kacc, double* Dp, hipStream_t st);
+hipError_t launch_symmetrize(const fix_t* Jacc, const fix_t* Jmat, const fix_t* Kacc, const int* jmap, const double* fix,
+                             double* J, double* K, int nbf, hipStream_t st);
 // batched J = Jacc + Jacc^T, K = Kacc + Kacc^T over block-diagonal packed matrices
-hipError_t launch_symmetrize_batch(const fix_t* Jacc, const fix_t* Kacc, const double* fix, double* J, double* K, int nmol,
-                                   const int64_t* mat_off, const int* mol_nbf, int max_nbf, hipStream_t st);
-hipError_t launch_fock_combine(const double* H, const fix_t* Jacc, const fix_t* Kacc, const double* fix, double* F, int nbf,
-                               double kfac, hipStream_t st);
+hipError_t launch_symmetrize_batch(const fix_t* Jacc, const fix_t* Jmat, const fix_t* Kacc, const int* jmap,
+                                   const double* fix, double* J, double* K, int nmol, const int64_t* mat_off, const int* mol_nbf, int max_nbf, hipStream_t st);
+hipError_t launch_fock_combine(const double* H, const fix_t* Jacc, const fix_t* Jmat, const fix_t* Kacc, const int* jmap,
+                               const double* fix, double* F, int nbf, double kfac, hipStream_t st);
 hipError_t launch_boys_batch(int m, int n, const double* T, double* F, int* status, hipStream_t st);
 hipError_t launch_rys_batch(int nroots, int n, const double* T, const double* tab, double* x, double* w,
                             hipStream_t st);

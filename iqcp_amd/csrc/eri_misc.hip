@@ -67,7 +67,9 @@ __global__ __launch_bounds__(256) void fix_rows_kernel(
     const double* __restrict__ D, const int64_t* __restrict__ mat_off, const int* __restrict__ mol_nbf,
     const double* __restrict__ qsh, const int64_t* __restrict__ qsh_off, const int* __restrict__ mol_ns,
     const int* __restrict__ bf_shell, const int* __restrict__ bf_off, const int* __restrict__ row_mol, int nrows,
-    double* __restrict__ rowsum, fix_t* __restrict__ Jacc, fix_t* __restrict__ Kacc) {
+    double* __restrict__ rowsum, fix_t* __restrict__ Jacc, fix_t* __restrict__ Jmat, fix_t* __restrict__ Kacc,
+    const int* __restrict__ jmap,
+    const double* __restrict__ bf_norm, double* __restrict__ Dp) {
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (row >= nrows) return;
     const int m = row_mol[row], n = row - bf_off[m], nbf = mol_nbf[m], ns = mol_ns[m];
@@ -80,9 +82,17 @@ __global__ __launch_bounds__(256) void fix_rows_kernel(
         const double a = fabs(Drow[l]);
         r += a;
         j += Qrow[bs[l]] * a;
-        // the same row of the accumulators starts at zero (null: that matrix is not built)
-        if (Jacc) Jacc[ro + l] = 0;
+        // the accumulators start at zero (null: that matrix is not built); J's are in pair order
+        // next to the density with the component norms
         if (Kacc) Kacc[ro + l] = 0;
+        if (Jacc) {
+            Jmat[ro + l] = 0;
+            const int e = jmap[ro + l];
+            if (e >= 0) {
+                Jacc[e] = 0;
+                Dp[e] = Drow[l] * bf_norm[row] * bf_norm[bf_off[m] + l];
+            }
+        }
     }
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {
@@ -146,10 +156,11 @@ __global__ __launch_bounds__(1024) void fix_scale_kernel(FixData f, double* __re
     }
 }
 
-hipError_t launch_fix_scale(const double* D, const FixData& f, double* fix, int nmol, fix_t* Jacc, fix_t* Kacc,
-                            hipStream_t st) {
+hipError_t launch_fix_scale(const double* D, const FixData& f, double* fix, int nmol, fix_t* Jacc, fix_t* Jmat,
+                            fix_t* Kacc, double* Dp, hipStream_t st) {
     hipLaunchKernelGGL(fix_rows_kernel, dim3((f.nrows + 3) / 4), dim3(256), 0, st, D, f.mat_off, f.mol_nbf, f.qsh,
-                       f.qsh_off, f.mol_ns, f.bf_shell, f.bf_off, f.row_mol, f.nrows, f.rowsum, Jacc, Kacc);
+                       f.qsh_off, f.mol_ns, f.bf_shell, f.bf_off, f.row_mol, f.nrows, f.rowsum, Jacc, Jmat, Kacc,
+                       f.jmap, f.bf_norm, Dp);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(fix_scale_kernel, dim3(nmol), dim3(1024), 0, st, f, fix);
@@ -162,57 +173,70 @@ __device__ __forceinline__ double fix_sym(const fix_t* __restrict__ a, size_t ij
     return fix_value(a[ij] + a[ji], inv);
 }
 
+// The same for J, whose words are in shell-pair order: jmap holds the word of element e, or -1 where
+// only the transposed element has one (both do inside a pair of equal shells); mat: Jmat.
+__device__ __forceinline__ double fix_sym_pairs(const fix_t* __restrict__ a, const fix_t* __restrict__ mat,
+                                                const int* __restrict__ jmap, size_t ij, size_t ji, double inv) {
+    const int e = jmap[ij], f = jmap[ji];
+    return fix_value((e >= 0 ? a[e] : 0) + (f >= 0 ? a[f] : 0) + mat[ij] + mat[ji], inv);
+}
+
 // J = Jacc + Jacc^T, K = Kacc + Kacc^T
-__global__ void symmetrize_kernel(const fix_t* __restrict__ Jacc, const fix_t* __restrict__ Kacc,
-                                  const double* __restrict__ fix, double* __restrict__ J, double* __restrict__ K,
-                                  int nbf) {
+__global__ void symmetrize_kernel(const fix_t* __restrict__ Jacc, const fix_t* __restrict__ Jmat,
+                                  const fix_t* __restrict__ Kacc,
+                                  const int* __restrict__ jmap, const double* __restrict__ fix, double* __restrict__ J,
+                                  double* __restrict__ K, int nbf) {
     const int i = blockIdx.y, j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= nbf) return;
     const size_t ij = (size_t)i * nbf + j, ji = (size_t)j * nbf + i;
-    if (J) J[ij] = fix_sym(Jacc, ij, ji, fix[2]);
+    if (J) J[ij] = fix_sym_pairs(Jacc, Jmat, jmap, ij, ji, fix[2]);
     if (K) K[ij] = fix_sym(Kacc, ij, ji, fix[3]);
 }
 
-__global__ void symmetrize_batch_kernel(const fix_t* __restrict__ Jacc, const fix_t* __restrict__ Kacc,
-                                        const double* __restrict__ fix, double* __restrict__ J,
-                                        double* __restrict__ K, const int64_t* __restrict__ mat_off,
-                                        const int* __restrict__ mol_nbf) {
+__global__ void symmetrize_batch_kernel(const fix_t* __restrict__ Jacc, const fix_t* __restrict__ Jmat,
+                                        const fix_t* __restrict__ Kacc,
+                                        const int* __restrict__ jmap, const double* __restrict__ fix,
+                                        double* __restrict__ J, double* __restrict__ K,
+                                        const int64_t* __restrict__ mat_off, const int* __restrict__ mol_nbf) {
     const int m = blockIdx.z, n = mol_nbf[m];
     const int i = blockIdx.y, j = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n || j >= n) return;
     const size_t o = (size_t)mat_off[m];
     const size_t ij = o + (size_t)i * n + j, ji = o + (size_t)j * n + i;
-    if (J) J[ij] = fix_sym(Jacc, ij, ji, fix[4 * m + 2]);
+    if (J) J[ij] = fix_sym_pairs(Jacc, Jmat, jmap, ij, ji, fix[4 * m + 2]);
     if (K) K[ij] = fix_sym(Kacc, ij, ji, fix[4 * m + 3]);
 }
 
-hipError_t launch_symmetrize_batch(const fix_t* Jacc, const fix_t* Kacc, const double* fix, double* J, double* K,
-                                   int nmol, const int64_t* mat_off, const int* mol_nbf, int max_nbf, hipStream_t st) {
+hipError_t launch_symmetrize_batch(const fix_t* Jacc, const fix_t* Jmat, const fix_t* Kacc, const int* jmap,
+                                   const double* fix, double* J, double* K, int nmol, const int64_t* mat_off, const int* mol_nbf, int max_nbf,
+                                   hipStream_t st) {
     hipLaunchKernelGGL(symmetrize_batch_kernel, dim3((max_nbf + 127) / 128, max_nbf, nmol), dim3(128), 0, st, Jacc,
-                       Kacc, fix, J, K, mat_off, mol_nbf);
+                       Jmat, Kacc, jmap, fix, J, K, mat_off, mol_nbf);
     return hipGetLastError();
 }
 
-hipError_t launch_symmetrize(const fix_t* Jacc, const fix_t* Kacc, const double* fix, double* J, double* K, int nbf,
-                             hipStream_t st) {
-    hipLaunchKernelGGL(symmetrize_kernel, dim3((nbf + 127) / 128, nbf), dim3(128), 0, st, Jacc, Kacc, fix, J, K, nbf);
+hipError_t launch_symmetrize(const fix_t* Jacc, const fix_t* Jmat, const fix_t* Kacc, const int* jmap, const double* fix,
+                             double* J, double* K, int nbf, hipStream_t st) {
+    hipLaunchKernelGGL(symmetrize_kernel, dim3((nbf + 127) / 128, nbf), dim3(128), 0, st, Jacc, Jmat, Kacc, jmap, fix, J, K,
+                       nbf);
     return hipGetLastError();
 }
 
 // F = H + J - kfac K  (build_fock, scf/mod.rs:825-881 with kfac = 1/2; hybrid form dft/ks_scf.rs:1960)
 __global__ void fock_combine_kernel(const double* __restrict__ H, const fix_t* __restrict__ Jacc,
-                                    const fix_t* __restrict__ Kacc, const double* __restrict__ fix,
-                                    double* __restrict__ F, int nbf, double kfac) {
+                                    const fix_t* __restrict__ Jmat,
+                                    const fix_t* __restrict__ Kacc, const int* __restrict__ jmap,
+                                    const double* __restrict__ fix, double* __restrict__ F, int nbf, double kfac) {
     const int i = blockIdx.y, j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= nbf) return;
     const size_t ij = (size_t)i * nbf + j, ji = (size_t)j * nbf + i;
-    F[ij] = H[ij] + fix_sym(Jacc, ij, ji, fix[2]) - kfac * fix_sym(Kacc, ij, ji, fix[3]);
+    F[ij] = H[ij] + fix_sym_pairs(Jacc, Jmat, jmap, ij, ji, fix[2]) - kfac * fix_sym(Kacc, ij, ji, fix[3]);
 }
 
-hipError_t launch_fock_combine(const double* H, const fix_t* Jacc, const fix_t* Kacc, const double* fix, double* F,
-                               int nbf, double kfac, hipStream_t st) {
-    hipLaunchKernelGGL(fock_combine_kernel, dim3((nbf + 127) / 128, nbf), dim3(128), 0, st, H, Jacc, Kacc, fix, F, nbf,
-                       kfac);
+hipError_t launch_fock_combine(const double* H, const fix_t* Jacc, const fix_t* Jmat, const fix_t* Kacc, const int* jmap,
+                               const double* fix, double* F, int nbf, double kfac, hipStream_t st) {
+    hipLaunchKernelGGL(fock_combine_kernel, dim3((nbf + 127) / 128, nbf), dim3(128), 0, st, H, Jacc, Jmat, Kacc, jmap, fix, F,
+                       nbf, kfac);
     return hipGetLastError();
 }
 

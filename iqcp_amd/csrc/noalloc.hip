@@ -3,7 +3,8 @@
 // HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
 //
 // The array holds, for one molecule of at most kNoAllocMaxNbf functions, the fixed-point J and K
-// accumulators (nbf^2 words each), the four scale doubles and 2 nbf doubles of row sums: 4.2 MB,
+// accumulators (two for J) and the pair-ordered density (nbf^2 words each), the four scale doubles and
+// 2 nbf doubles of row sums: 8.4 MB,
 // resident on every GPU the library runs on until the process ends.  Every call on a GPU shares that
 // GPU's copy; the kernels clear the accumulators at the start of each call (fill kernels, no
 // hipMemsetAsync), and calls that overlap on one GPU race on it.
@@ -14,7 +15,7 @@
 namespace {
 
 constexpr int kNoAllocMaxNbf = 512;
-constexpr size_t kScratchWords = 2 * (size_t)kNoAllocMaxNbf * kNoAllocMaxNbf + 4 + 2 * (size_t)kNoAllocMaxNbf;
+constexpr size_t kScratchWords = 4 * (size_t)kNoAllocMaxNbf * kNoAllocMaxNbf + 4 + 2 * (size_t)kNoAllocMaxNbf;
 
 __device__ __align__(256) unsigned long long scratch[kScratchWords];
 
@@ -52,6 +53,7 @@ extern "C" int qcg_build_jk_device_noalloc(qcg_context* c, const double* dD, dou
     HIPCHK(c, hipSetDevice(c->device));
     fix_t* w = static_cast<fix_t*>(base);
     const size_t n2 = (size_t)nbf * nbf;
-    const JkAcc acc{w, w + n2, reinterpret_cast<double*>(w + 2 * n2), reinterpret_cast<double*>(w + 2 * n2 + 4)};
+    const JkAcc acc{w, w + n2, w + 2 * n2, reinterpret_cast<double*>(w + 4 * n2),
+                    reinterpret_cast<double*>(w + 4 * n2 + 4), reinterpret_cast<double*>(w + 3 * n2)};
     return run_jk(c, dD, dJ, dK, stream ? (hipStream_t)stream : c->stream, &acc, true);
 }

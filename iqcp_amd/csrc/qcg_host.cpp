@@ -364,6 +364,82 @@ int qcg_set_basis_batch(qcg_context* c, int nmol, const int* mol_nshell, const i
         }
     HIPCHK(c, hipMemcpy(c->d_pairs, all.data(), all.size() * sizeof(PairRec), hipMemcpyHostToDevice));
     c->pairs = all;
+    {
+        // the kets as arrays in list order (KetPairs, KetPrims), and the pair order of the J side
+        const int np = npairs, npr = (int)pp.size();
+        std::vector<int4> meta(np);
+        std::vector<double2> cen(3 * (size_t)np), kp(3 * (size_t)npr);
+        std::vector<double> khp(npr);
+        std::vector<float4> kpf(2 * (size_t)npr);
+        int first = 0;
+        for (int k = 0; k < kNumPairClasses; ++k)
+            for (int m = 0; m < nmol; ++m) {
+                const std::vector<int>& bnd = c->bucket_bnd[k * nmol + m];
+                const int base = c->class_off[k] + c->ket_off_h[k * nmol + m];
+                for (size_t b = 0; b + 1 < bnd.size(); ++b) {
+                    const int n = bnd[b + 1] - bnd[b], npp = all[base + bnd[b]].npp;
+                    for (int i = 0; i < n; ++i) {
+                        const int g = base + bnd[b] + i;
+                        const PairRec& r = all[g];
+                        meta[g] = make_int4(r.bfa | (r.sa == r.sb ? kKetSame : 0), r.bfb, first + i, (int)(((unsigned)npp << 24) | (unsigned)n));
+                        cen[g] = make_double2(r.ax, r.ay);
+                        cen[(size_t)np + g] = make_double2(r.az, r.abx);
+                        cen[2 * (size_t)np + g] = make_double2(r.aby, r.abz);
+                        for (int j = 0; j < npp; ++j) {
+                            const size_t e = (size_t)first + i + (size_t)j * n;
+                            const PrimPair<double>& q = pp[r.pp_off + j];
+                            const PrimPair<float>& f = ppf[r.pp_off + j];
+                            kp[e] = make_double2(q.px, q.py);
+                            kp[npr + e] = make_double2(q.pz, q.p);
+                            kp[2 * (size_t)npr + e] = make_double2(q.ckp, q.kab);
+                            khp[e] = q.hp;
+                            kpf[e] = make_float4(f.px, f.py, f.pz, f.p);
+                            kpf[npr + e] = make_float4(f.ckp, f.hp, f.kab, f.ea);
+                        }
+                    }
+                    first += n * npp;
+                }
+            }
+        std::vector<int> jmap((size_t)c->mat_total, -1);
+        std::vector<double> bfn;
+        for (const HostBasis& B : c->mols)
+            for (int s = 0; s < B.nshell; ++s)
+                for (int k = 0; k < ncart(B.l[s]); ++k) bfn.push_back(B.l[s] == 2 && (k == 0 || k == 3 || k == 5) ? 0.57735026918962576451 : 1.0);
+        int64_t words = 0;
+        for (int k = 0; k < kNumPairClasses; ++k) {
+            const int na = k == 0 ? 1 : k <= 2 ? 3 : 6, nb = (k == 0 || k == 1 || k == 3) ? 1 : (k == 2 || k == 4) ? 3 : 6;
+            const int n = c->class_off[k + 1] - c->class_off[k];
+            c->jbase[k] = (int)words;
+            for (int i = 0; i < n; ++i) {
+                const PairRec& r = all[c->class_off[k] + i];
+                const int64_t nbf = c->mol_nbf_h[r.mol];
+                for (int a = 0; a < na; ++a)
+                    for (int b = 0; b < nb; ++b)
+                        jmap[c->mat_off_h[r.mol] + (r.bfa + a) * nbf + r.bfb + b] = (int)(words + (int64_t)(a * nb + b) * n + i);
+            }
+            words += (int64_t)na * nb * n;
+        }
+        if (words > INT32_MAX || 3 * (int64_t)npr > INT32_MAX || 3 * (int64_t)np > INT32_MAX)
+            return fail(c, QCG_INVALID_ARG, "basis too large");
+        c->n_kprim = npr;
+        HIPCHK(c, c->alloc(&c->d_kmeta, meta.size()));
+        HIPCHK(c, c->alloc(&c->d_kcen, cen.size()));
+        HIPCHK(c, c->alloc(&c->d_kprim, kp.size()));
+        HIPCHK(c, c->alloc(&c->d_khp, khp.size()));
+        HIPCHK(c, c->alloc(&c->d_kprimf, kpf.size()));
+        HIPCHK(c, c->alloc(&c->d_jmap, jmap.size()));
+        HIPCHK(c, c->alloc(&c->d_bf_norm, bfn.size()));
+        HIPCHK(c, c->alloc(&c->d_Dp, (size_t)words));
+        HIPCHK(c, hipMemcpy(c->d_kmeta, meta.data(), meta.size() * sizeof(int4), hipMemcpyHostToDevice));
+        HIPCHK(c, hipMemcpy(c->d_kcen, cen.data(), cen.size() * sizeof(double2), hipMemcpyHostToDevice));
+        HIPCHK(c, hipMemcpy(c->d_kprim, kp.data(), kp.size() * sizeof(double2), hipMemcpyHostToDevice));
+        HIPCHK(c, hipMemcpy(c->d_khp, khp.data(), khp.size() * sizeof(double), hipMemcpyHostToDevice));
+        HIPCHK(c, hipMemcpy(c->d_kprimf, kpf.data(), kpf.size() * sizeof(float4), hipMemcpyHostToDevice));
+        HIPCHK(c, hipMemcpy(c->d_jmap, jmap.data(), jmap.size() * sizeof(int), hipMemcpyHostToDevice));
+        HIPCHK(c, hipMemcpy(c->d_bf_norm, bfn.data(), bfn.size() * sizeof(double), hipMemcpyHostToDevice));
+        c->fixdata.jmap = c->d_jmap;
+        c->fixdata.bf_norm = c->d_bf_norm;
+    }
     HIPCHK(c, c->alloc(&c->d_mol_nbf, nmol));
     HIPCHK(c, c->alloc(&c->d_mat_off, nmol));
     HIPCHK(c, c->alloc(&c->d_ket_off, kNumPairClasses * nmol));
@@ -377,6 +453,7 @@ int qcg_set_basis_batch(qcg_context* c, int nmol, const int* mol_nshell, const i
     HIPCHK(c, c->alloc(&c->d_J, n2));
     HIPCHK(c, c->alloc(&c->d_K, n2));
     HIPCHK(c, c->alloc(&c->d_Jacc, n2));
+    HIPCHK(c, c->alloc(&c->d_Jmat, n2));
     HIPCHK(c, c->alloc(&c->d_Kacc, n2));
     HIPCHK(c, c->alloc(&c->d_H, n2));
     HIPCHK(c, c->alloc(&c->d_F, n2));
@@ -469,12 +546,6 @@ static int build_plan(qcg_context* c) {
     for (const PairRec& pr : c->pairs)
         if (pr.npp > kItemMaxPrim)
             return fail(c, QCG_INVALID_ARG, "shell pair with more than 255 primitive pairs (at most 15 primitives per shell)");
-    for (int cb = 0; cb < kNumPairClasses; ++cb) {
-        int m = 1;
-        for (int i = c->class_off[cb]; i < c->class_off[cb + 1]; ++i) m = std::max(m, c->pairs[i].npp);
-        const int split = (c->prim_split > 0 && c->prim_split < kBraPPMax) ? c->prim_split : kBraPPMax;
-        c->bra_pp[cb] = std::min(m, split);
-    }
     c->items.clear();
     c->segs.clear();
     const int nmol = c->nmol;
@@ -595,7 +666,7 @@ int qcg::run_jk(qcg_context* c, const double* dD, double* dJ, double* dK, hipStr
         int rc = prepare_jk(c);
         if (rc) return rc;
     }
-    const JkAcc own{c->d_Jacc, c->d_Kacc, c->d_fix, c->d_rowsum};
+    const JkAcc own{c->d_Jacc, c->d_Jmat, c->d_Kacc, c->d_fix, c->d_rowsum, c->d_Dp};
     const JkAcc& A = acc ? *acc : own;
     HIPCHK(c, stream_begin(c, st));
     // the fixed-point scales come from a bound at this density; the same pass zeroes the
@@ -604,7 +675,8 @@ int qcg::run_jk(qcg_context* c, const double* dD, double* dJ, double* dK, hipStr
     fd.mat_off = c->d_mat_off;
     fd.mol_nbf = c->d_mol_nbf;
     fd.rowsum = A.rowsum;
-    HIPCHK(c, launch_fix_scale(dD, fd, A.fix, c->nmol, do_j ? A.Jacc : nullptr, do_k ? A.Kacc : nullptr, st));
+    HIPCHK(c, launch_fix_scale(dD, fd, A.fix, c->nmol, do_j ? A.Jacc : nullptr, A.Jmat, do_k ? A.Kacc : nullptr,
+                               A.Dp, st));
     const bool mixed = c->precision == QCG_PREC_MIXED && c->fp32_cutoff > c->schwarz_thr;
     if (c->profiling && !c->ev_made) {
         for (auto& e : c->ev) HIPCHK(c, hipEventCreate(&e));
@@ -655,7 +727,16 @@ int qcg::run_jk(qcg_context* c, const double* dD, double* dJ, double* dK, hipStr
             a.D = dD;
             a.nbf = nbf;
             a.Jacc = A.Jacc;
+            a.Jmat = A.Jmat;
             a.Kacc = A.Kacc;
+            a.Dp = A.Dp;
+            a.jb_bra = c->jbase[cb];
+            a.jb_ket = c->jbase[ck];
+            a.np_bra = c->class_off[cb + 1] - c->class_off[cb];
+            a.np_ket = c->class_off[ck + 1] - c->class_off[ck];
+            a.kpairs = {c->d_kmeta + c->class_off[ck], c->d_kcen + c->class_off[ck], (int)c->pairs.size()};
+            a.kprims = {c->d_kprim, c->d_khp, c->n_kprim};
+            a.kprimsf = {c->d_kprimf, c->n_kprim};
             a.fix = A.fix;
             a.do_j = do_j;
             a.do_k = do_k;
@@ -667,7 +748,6 @@ int qcg::run_jk(qcg_context* c, const double* dD, double* dJ, double* dK, hipStr
             a.segs = c->d_segs;
             a.nitems = c->item_cnt[cls][part];
             a.block = c->tile[cls][part].block;
-            a.bra_pp = c->bra_pp[cb];
             a.pp = part ? (const void*)c->d_ppf : (const void*)c->d_pp;
             a.rys = part ? (const void*)c->d_rys_f : (const void*)c->d_rys;
             if (fused) {
@@ -690,10 +770,10 @@ int qcg::run_jk(qcg_context* c, const double* dD, double* dJ, double* dK, hipStr
         }
     if (!symmetrize) {
         // the caller reads the accumulators itself (launch_fock_combine)
-    } else if (c->nmol == 1) HIPCHK(c, launch_symmetrize(A.Jacc, A.Kacc, A.fix, dJ, dK, nbf, st));
+    } else if (c->nmol == 1) HIPCHK(c, launch_symmetrize(A.Jacc, A.Jmat, A.Kacc, c->d_jmap, A.fix, dJ, dK, nbf, st));
     else
-        HIPCHK(c, launch_symmetrize_batch(A.Jacc, A.Kacc, A.fix, dJ, dK, c->nmol, c->d_mat_off, c->d_mol_nbf, nbf,
-                                          st));
+        HIPCHK(c, launch_symmetrize_batch(A.Jacc, A.Jmat, A.Kacc, c->d_jmap, A.fix, dJ, dK, c->nmol, c->d_mat_off,
+                                          c->d_mol_nbf, nbf, st));
     HIPCHK(c, stream_done(c, st));
     return QCG_OK;
 }
@@ -1019,7 +1099,7 @@ int qcg_build_fock_device(qcg_context* c, const double* dH, const double* dD, do
             if (rc) return rc;
             HIPCHK(c, hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
             rc = run_jk(c, dD, c->d_J, c->d_K, st, nullptr, false, false);
-            hipError_t e = rc ? hipSuccess : launch_fock_combine(dH, c->d_Jacc, c->d_Kacc, c->d_fix, dF, c->basis.nbf, k_factor, st);
+            hipError_t e = rc ? hipSuccess : launch_fock_combine(dH, c->d_Jacc, c->d_Jmat, c->d_Kacc, c->d_jmap, c->d_fix, dF, c->basis.nbf, k_factor, st);
             hipGraph_t g = nullptr;
             const hipError_t ec = hipStreamEndCapture(st, &g);
             if (rc || e != hipSuccess || ec != hipSuccess) {
@@ -1039,7 +1119,7 @@ int qcg_build_fock_device(qcg_context* c, const double* dH, const double* dD, do
     }
     int rc = run_jk(c, dD, c->d_J, c->d_K, st, nullptr, false, false);
     if (rc) return rc;
-    HIPCHK(c, launch_fock_combine(dH, c->d_Jacc, c->d_Kacc, c->d_fix, dF, c->basis.nbf, k_factor, st));
+    HIPCHK(c, launch_fock_combine(dH, c->d_Jacc, c->d_Jmat, c->d_Kacc, c->d_jmap, c->d_fix, dF, c->basis.nbf, k_factor, st));
     HIPCHK(c, stream_done(c, st));
     return QCG_OK;
 }
@@ -1105,7 +1185,7 @@ int qcg_build_fock(qcg_context* c, const double* H, const double* D, double* F) 
     HIPCHK(c, hipMemcpyAsync(c->d_H, H, n2 * sizeof(double), hipMemcpyHostToDevice, c->stream));
     int rc = run_jk(c, c->d_D, c->d_J, c->d_K, c->stream, nullptr, false, false);
     if (rc) return rc;
-    HIPCHK(c, launch_fock_combine(c->d_H, c->d_Jacc, c->d_Kacc, c->d_fix, c->d_F, nbf, 0.5, c->stream));
+    HIPCHK(c, launch_fock_combine(c->d_H, c->d_Jacc, c->d_Jmat, c->d_Kacc, c->d_jmap, c->d_fix, c->d_F, nbf, 0.5, c->stream));
     HIPCHK(c, hipMemcpyAsync(F, c->d_F, n2 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return QCG_OK;

@@ -51,4 +51,37 @@ struct alignas(16) PairRec {
     int pos;            // position in its molecule's sorted class list
 };
 
+// The kets of the per-lane J/K kernels as arrays over the pairs of a class, in list order: the lanes of
+// a wavefront take consecutive kets, so every load below is one run of consecutive words per wavefront
+// instead of 64 cache lines of PairRec / PrimPair structs.  Primitive j of a ket is element
+// meta.z + j * stride of the primitive arrays (the primitives of a contraction bucket are stored
+// primitive by primitive over the bucket's pairs).
+template <typename R>
+struct KetPrims;
+template <>
+struct KetPrims<double> {
+    const double2* v;   // n x (px, py), n x (pz, p), n x (ckp, kab)
+    const double* hp;
+    int n;
+    QCG_HD PrimPair<double> at(int i) const {
+        const double2 a = v[i], b = v[n + i], c = v[2 * n + i];
+        return {b.y, a.x, a.y, b.x, c.y, c.x, hp[i], 0.0};
+    }
+};
+template <>
+struct KetPrims<float> {
+    const float4* v;    // n x (px, py, pz, p), n x (ckp, hp, low and high word of the FP64 kab)
+    int n;
+    QCG_HD PrimPair<float> at(int i) const {
+        const float4 a = v[i], b = v[n + i];
+        return {a.w, a.x, a.y, a.z, b.z, b.x, b.y, b.w};
+    }
+};
+struct KetPairs {
+    const int4* meta;     // bfa | (sa == sb) << 30, bfb, first primitive, npp << 24 | stride
+    const double2* cen;   // np x (ax, ay), np x (az, abx), np x (aby, abz)
+    int np;               // pairs of all classes (the stride of cen)
+};
+constexpr int kKetSame = 1 << 30;
+
 }  // namespace qcg
