@@ -127,6 +127,11 @@ struct qcg_context {
     int grad_off[21] = {}, grad_cnt[21] = {};
     double grad_key[2] = {-1.0, -1.0};
     double* d_grad = nullptr;
+    // work items of the compressed tensor (made once per threshold)
+    int4* d_tensor_items = nullptr;
+    int2* d_tensor_segs = nullptr;
+    int tensor_off[21] = {}, tensor_cnt[21] = {};
+    double tensor_key = -1.0;
     double* d_W = nullptr;  // energy-weighted density of the gradient (nbf x nbf)
     // device basis copy and work list of the one-electron gradient kernel
     int* d_onee_int = nullptr;
@@ -205,7 +210,7 @@ struct qcg_context {
                          (void**)&d_kprim, (void**)&d_khp, (void**)&d_kprimf,
                          (void**)&d_H, (void**)&d_F, (void**)&d_mol_nbf,
                          (void**)&d_mat_off, (void**)&d_ket_off, (void**)&d_ket_cnt, (void**)&d_items,
-                         (void**)&d_segs, (void**)&d_grad_items, (void**)&d_grad_segs, (void**)&d_grad,
+                         (void**)&d_segs, (void**)&d_tensor_items, (void**)&d_tensor_segs, (void**)&d_grad_items, (void**)&d_grad_segs, (void**)&d_grad,
                          (void**)&d_W, (void**)&d_onee_int, (void**)&d_onee_dbl, (void**)&d_onee_work}) {
             release(*p);
             *p = nullptr;

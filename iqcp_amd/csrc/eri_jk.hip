@@ -60,6 +60,24 @@ __device__ __forceinline__ const R* rys_stage(const R* __restrict__ rys_tab, R* 
 template <int N>
 constexpr int rys_lds_doubles() { return N <= 3 ? rys_tab_size<N>() : 1; }
 
+// Ket kq of a class (km = its meta word): the fields that the class needs.
+template <int LC, int LD>
+__device__ __forceinline__ PairRec ket_pair(const KetPairs& k, int kq, const int4 km) {
+    PairRec Q;
+    Q.bfa = km.x & ~kKetSame;
+    Q.bfb = km.y;
+    Q.npp = (unsigned)km.w >> 24;
+    if constexpr (LC > 0) {
+        const double2 c0 = k.cen[kq], c1 = k.cen[k.np + kq];
+        Q.ax = c0.x, Q.ay = c0.y, Q.az = c1.x, Q.abx = c1.y;
+        if constexpr (LD > 0) {
+            const double2 c2 = k.cen[2 * k.np + kq];
+            Q.aby = c2.x, Q.abz = c2.y;
+        }
+    }
+    return Q;
+}
+
 // One work item = (bra pair, run of its surviving kets over the ket segments, KetCursor); the
 // host builds the items with the exact screening predicate, so no quartet is tested twice or
 // skipped.  rys_n: the coefficients of this class's Rys order (rys_stage); rows: with KROWS, LDS room
@@ -113,19 +131,8 @@ __device__ __forceinline__ void jk_item(const int4 it, const JkArgs& g, const Ke
     for (int j = tid >> lg; j < item_kets(it); j += step, cur.r += step) {
         const int q = cur.at(), kq = ket0 + q;
         const int4 km = g.kpairs.meta[kq];
-        PairRec Q;
-        Q.bfa = km.x & ~kKetSame;
-        Q.bfb = km.y;
-        Q.npp = (unsigned)km.w >> 24;
+        const PairRec Q = ket_pair<LC, LD>(g.kpairs, kq, km);
         const int kstride = km.w & 0xffffff;
-        if constexpr (LC > 0) {
-            const double2 c0 = g.kpairs.cen[kq], c1 = g.kpairs.cen[g.kpairs.np + kq];
-            Q.ax = c0.x, Q.ay = c0.y, Q.az = c1.x, Q.abx = c1.y;
-            if constexpr (LD > 0) {
-                const double2 c2 = g.kpairs.cen[2 * g.kpairs.np + kq];
-                Q.aby = c2.x, Q.abz = c2.y;
-            }
-        }
         R eri[S::NQ];
         for_n<U, S::NQ>([&](int i) { eri[i] = R(0); });
         contract_quartet_pp<LA, LB, LC, LD, R, true>(
@@ -291,16 +298,49 @@ struct JkWave {
     static constexpr bool kEnabled = S::NQ >= 27;
 };
 
+// The contracted quartet (P|Q) on one wavefront: component lane + 64 j in acc[j], without norms; tbl:
+// the wave's LDS table (JkWave<..., R>::T).
+template <int LA, int LB, int LC, int LD, typename R>
+__device__ __forceinline__ void wave_quartet(const PairRec& P, const PairRec& Q, const PrimPair<R>* __restrict__ pp,
+                                             const R* __restrict__ rys_tab, double* V, int lane, R* acc) {
+    using S = EriShape<LA, LB, LC, LD>;
+    using W = JkWave<LA, LB, LC, LD, R>;
+    using TB = typename W::T;
+    constexpr int N = S::NROOTS, HT = TB::HT, ES = TB::ES, KPL = W::KPL;
+    constexpr const CompTab<LA, LB, LC, LD>& ct = kCompTab<LA, LB, LC, LD>;
+    R* tbl = reinterpret_cast<R*>(V);
+    int ox[KPL], oy[KPL], oz[KPL];
+#pragma unroll
+    for (int j = 0; j < KPL; ++j) {
+        const int k = lane + 64 * j;
+        const int kk = k < S::NQ ? k : 0;
+        ox[j] = ct.hx[kk] * ES;
+        oy[j] = (HT + ct.hy[kk]) * ES;
+        oz[j] = (2 * HT + ct.hz[kk]) * ES;
+        acc[j] = R(0);
+    }
+    const int npq = P.npp * Q.npp;
+    for (int pq0 = 0; pq0 < npq; pq0 += TB::PQ_CAP) {
+        const int npc = min(TB::PQ_CAP, npq - pq0);
+        wave_sync();  // earlier readers of the table (and of what aliases it) are done
+        wave_tables<LA, LB, LC, LD, N, ES, R>(P, Q, pp, rys_tab, pq0, npc, tbl, lane);
+        wave_sync();
+        const int ne = npc * N;
+        for (int e = 0; e < ne; ++e) {
+#pragma unroll
+            for (int j = 0; j < KPL; ++j) acc[j] += tbl[ox[j] + e] * tbl[oy[j] + e] * tbl[oz[j] + e];
+        }
+    }
+}
+
 // One work item on one wavefront; V: the wave's LDS region (JkWave<..., R>::WAVE_D doubles).
 template <int LA, int LB, int LC, int LD, typename R>
 __device__ __forceinline__ void jk_wave_item(
     const int4 it, int lane, double* V, const JkArgs& g, const PrimPair<R>* __restrict__ pp, const R* __restrict__ rys_tab) {
     using S = EriShape<LA, LB, LC, LD>;
     using W = JkWave<LA, LB, LC, LD, R>;
-    using TB = typename W::T;
-    constexpr int N = S::NROOTS, HT = TB::HT, ES = TB::ES, KPL = W::KPL;
+    constexpr int KPL = W::KPL;
     constexpr int NA = S::NA, NB = S::NB, NC = S::NC, ND = S::ND, NCD = S::NCD;
-    R* tbl = reinterpret_cast<R*>(V);
     double* Dab = V + W::VD;
     double* Dcd = Dab + S::NAB;
     double* Dbd = Dcd + NCD;
@@ -318,16 +358,6 @@ __device__ __forceinline__ void jk_wave_item(
     const int do_j = g.do_j, do_k = g.do_k;
     const double sJ = g.fix[4 * P.mol], sK = g.fix[4 * P.mol + 1];  // fixed-point scales of J and K
 
-    constexpr const CompTab<LA, LB, LC, LD>& ct = kCompTab<LA, LB, LC, LD>;
-    int ox[KPL], oy[KPL], oz[KPL];
-#pragma unroll
-    for (int j = 0; j < KPL; ++j) {
-        const int k = lane + 64 * j;
-        const int kk = k < S::NQ ? k : 0;
-        ox[j] = ct.hx[kk] * ES;
-        oy[j] = (HT + ct.hy[kk]) * ES;
-        oz[j] = (2 * HT + ct.hz[kk]) * ES;
-    }
     for (int o = lane; o < S::NAB; o += 64) Dab[o] = D[(P.bfa + o / NB) * nbf + P.bfb + o % NB];
     double jp = 0.0;  // J_ab of lane ab over the item's kets
     const double deg_p = (P.sa == P.sb) ? 0.5 : 1.0;
@@ -337,20 +367,7 @@ __device__ __forceinline__ void jk_wave_item(
         const int q = cur.at();
         const PairRec Q = ket[q];
         R acc[KPL];
-#pragma unroll
-        for (int j = 0; j < KPL; ++j) acc[j] = R(0);
-        const int npq = P.npp * Q.npp;
-        for (int pq0 = 0; pq0 < npq; pq0 += TB::PQ_CAP) {
-            const int npc = min(TB::PQ_CAP, npq - pq0);
-            wave_sync();  // earlier readers of the table (and of V, which aliases it) are done
-            wave_tables<LA, LB, LC, LD, N, ES, R>(P, Q, pp, rys_tab, pq0, npc, tbl, lane);
-            wave_sync();
-            const int ne = npc * N;
-            for (int e = 0; e < ne; ++e) {
-#pragma unroll
-                for (int j = 0; j < KPL; ++j) acc[j] += tbl[ox[j] + e] * tbl[oy[j] + e] * tbl[oz[j] + e];
-            }
-        }
+        wave_quartet<LA, LB, LC, LD, R>(P, Q, pp, rys_tab, V, lane, acc);
         wave_sync();
         const double deg = deg_p * ((Q.sa == Q.sb) ? 0.5 : 1.0) * ((g.diag && q == pidx) ? 0.5 : 1.0);
 #pragma unroll
@@ -450,36 +467,88 @@ __device__ __forceinline__ int64_t pair_index64(int64_t i, int64_t j) {
     return i >= j ? i * (i + 1) / 2 + j : j * (j + 1) / 2 + i;
 }
 
-// The 8-fold compressed tensor (eri_compressed, integrals/eri/mod.rs:992-1070; index
-// pair_index/eri_index :946-960).  Every element of a surviving quartet is written once.
+// One element of the 8-fold compressed tensor (eri_compressed, integrals/eri/mod.rs:992-1070; index
+// pair_index/eri_index :946-960): component (a, b, c, d) of the quartet (P|Q), v with the norms.  Every
+// element of a surviving quartet is written once.
+__device__ __forceinline__ void tensor_put(double* __restrict__ out, int bfa, int bfb, bool same_p, int bfc, int bfd,
+                                           bool same_q, bool same_pq, int a, int b, int c, int d, double v) {
+    const int i = bfa + a, j = bfb + b, k = bfc + c, l = bfd + d;
+    if ((same_p && i < j) || (same_q && k < l)) return;
+    const int64_t ij = pair_index64(i, j), kl = pair_index64(k, l);
+    if (same_pq && ij < kl) return;
+    const int64_t hi = ij > kl ? ij : kl, lo = ij > kl ? kl : ij;
+    out[hi * (hi + 1) / 2 + lo] = v;
+}
+
+// The tensor by work items like those of J/K (lanes per ket, ket arrays), one block per item, for the
+// classes up to kTensorLaneMaxNQ components, whose quartet fits a lane's registers; one wavefront per
+// quartet above (eri_tensor_wave_kernel).  With one lane per quartet whatever its class the d classes'
+// quartets lived in scratch: propane/6-31G* (61 functions) took 16.9 ms per call, now 1.34 ms, of which
+// the kernels (35 us each, four streams) are a quarter and the 14 MB copy to the host most of the rest.
 template <int LA, int LB, int LC, int LD>
-__global__ __launch_bounds__(256) void eri_tensor_kernel(
-    const PairRec* __restrict__ bra, int nbra, const PairRec* __restrict__ ket, int nket, int diag,
-    const PrimPair<double>* __restrict__ pp, const double* __restrict__ rys_tab, double* __restrict__ out,
-    double thr) {
+__global__ __launch_bounds__(128) void eri_tensor_kernel(const int4* __restrict__ items, const JkArgs g,
+                                                         const KetPrims<double> kprims,
+                                                         const PrimPair<double>* __restrict__ pp,
+                                                         const double* __restrict__ rys_tab, double* __restrict__ out) {
     using S = EriShape<LA, LB, LC, LD>;
-    constexpr bool U = S::kUnroll;
-    const int pidx = diag ? (nbra - 1 - (int)blockIdx.x) : (int)blockIdx.x;
-    const PairRec P = bra[pidx];
-    const int q1 = diag ? pidx + 1 : nket;  // screened below with the reference's predicate
-    for (int q = threadIdx.x; q < q1; q += blockDim.x) {
-        const PairRec Q = ket[q];
-        if (P.Q * Q.Q < thr) continue;
+    __shared__ double rys_raw[rys_lds_doubles<S::NROOTS>()];
+    const double* rys_n = rys_stage<double, S::NROOTS>(rys_tab, rys_raw);
+    __syncthreads();
+    const int4 it = items[blockIdx.x];
+    const PairRec P = item_bra(g.bra, it);
+    const int tid = threadIdx.x, lg = item_lg(it), lanes = 1 << lg, sub = tid & (lanes - 1), step = blockDim.x >> lg;
+    KetCursor cur{g.segs, it.y, it.z + (tid >> lg)};
+    for (int j = tid >> lg; j < item_kets(it); j += step, cur.r += step) {
+        const int q = cur.at();
+        const int4 km = g.kpairs.meta[q];
+        const PairRec Q = ket_pair<LC, LD>(g.kpairs, q, km);
+        const int kstride = km.w & 0xffffff;
         double eri[S::NQ];
-        for_n<U, S::NQ>([&](int i) { eri[i] = 0.0; });
-        contract_quartet<LA, LB, LC, LD, double>(P, Q, pp, rys_tab, eri);
-#pragma unroll 1
-        for (int idx = 0; idx < S::NQ; ++idx) {
-            const int d = idx % S::ND, c = (idx / S::ND) % S::NC, b = (idx / S::NCD) % S::NB, a = idx / (S::NCD * S::NB);
-            const int i = P.bfa + a, j = P.bfb + b;
-            if (P.sa == P.sb && i < j) continue;
-            const int k = Q.bfa + c, l = Q.bfb + d;
-            if (Q.sa == Q.sb && k < l) continue;
-            const int64_t ij = pair_index64(i, j), kl = pair_index64(k, l);
-            if (diag && q == pidx && ij < kl) continue;
-            const int64_t hi = ij > kl ? ij : kl, lo = ij > kl ? kl : ij;
-            out[hi * (hi + 1) / 2 + lo] =
-                eri[idx] * cnorm(LA, a) * cnorm(LB, b) * cnorm(LC, c) * cnorm(LD, d);
+        for_n<true, S::NQ>([&](int i) { eri[i] = 0.0; });
+        contract_quartet_pp<LA, LB, LC, LD, double, true>(
+            P, Q, pp + P.pp_off, [&](int i) { return kprims.at(km.z + i * kstride); }, rys_n, eri, sub, lanes);
+        if (lg) {
+            for (int off = 1; off < lanes; off <<= 1)
+                for_n<true, S::NQ>([&](int i) { eri[i] += __shfl_xor(eri[i], off, 64); });
+            if (sub) continue;
+        }
+        const bool same_q = km.x & kKetSame, same_pq = g.diag && q == P.pos;
+        static_for<S::NQ>([&](auto kc) {
+            constexpr int k = decltype(kc)::value;
+            constexpr int d = k % S::ND, c = (k / S::ND) % S::NC, b = (k / S::NCD) % S::NB, a = k / (S::NCD * S::NB);
+            tensor_put(out, P.bfa, P.bfb, P.sa == P.sb, Q.bfa, Q.bfb, same_q, same_pq, a, b, c, d,
+                       eri[k] * (cnorm(LA, a) * cnorm(LB, b) * cnorm(LC, c) * cnorm(LD, d)));
+        });
+    }
+}
+
+template <int LA, int LB, int LC, int LD>
+__global__ __launch_bounds__(256) void eri_tensor_wave_kernel(const int4* __restrict__ items, int nitems, const JkArgs g,
+                                                              const PrimPair<double>* __restrict__ pp,
+                                                              const double* __restrict__ rys_tab,
+                                                              double* __restrict__ out) {
+    using W = JkWave<LA, LB, LC, LD, double>;
+    using S = EriShape<LA, LB, LC, LD>;
+    __shared__ double smem[4 * W::T::DOUBLES];
+    const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int item = blockIdx.x * 4 + wid;
+    if (item >= nitems) return;
+    const int4 it = items[item];
+    const PairRec P = item_bra(g.bra, it);
+    KetCursor cur{g.segs, it.y, it.z};
+    for (int j = 0; j < item_kets(it); ++j, ++cur.r) {
+        const int q = cur.at();
+        const PairRec Q = g.ket[q];
+        double acc[W::KPL];
+        wave_quartet<LA, LB, LC, LD, double>(P, Q, pp, rys_tab, smem + wid * W::T::DOUBLES, lane, acc);
+#pragma unroll
+        for (int m = 0; m < W::KPL; ++m) {
+            const int k = lane + 64 * m;
+            if (k < S::NQ) {
+                const int d = k % S::ND, c = (k / S::ND) % S::NC, b = (k / S::NCD) % S::NB, a = k / (S::NCD * S::NB);
+                tensor_put(out, P.bfa, P.bfb, P.sa == P.sb, Q.bfa, Q.bfb, Q.sa == Q.sb, g.diag && q == P.pos, a, b, c, d,
+                           acc[m] * (cnorm(LA, a) * cnorm(LB, b) * cnorm(LC, c) * cnorm(LD, d)));
+            }
         }
     }
 }
@@ -564,9 +633,14 @@ static hipError_t launch_jk_mp_t(const JkLaunch& a, hipStream_t st) {
 template <int CB, int CK>
 static hipError_t launch_tensor_t(const JkLaunch& a, double* out, hipStream_t st) {
     constexpr int LA = QCG_LA(CB), LB = QCG_LB(CB), LC = QCG_LA(CK), LD = QCG_LB(CK);
-    if (a.nbra <= 0 || a.nket <= 0) return hipSuccess;
-    hipLaunchKernelGGL((eri_tensor_kernel<LA, LB, LC, LD>), dim3(a.nbra), dim3(256), 0, st, a.bra, a.nbra, a.ket,
-                       a.nket, a.diag, (const PrimPair<double>*)a.pp, (const double*)a.rys, out, a.thr_lo);
+    using S = EriShape<LA, LB, LC, LD>;
+    if (a.nitems <= 0) return hipSuccess;
+    if constexpr (S::NQ <= kTensorLaneMaxNQ)
+        hipLaunchKernelGGL((eri_tensor_kernel<LA, LB, LC, LD>), dim3(a.nitems), dim3(a.block), 0, st, a.items, jk_args(a),
+                           a.kprims, (const PrimPair<double>*)a.pp, (const double*)a.rys, out);
+    else
+        hipLaunchKernelGGL((eri_tensor_wave_kernel<LA, LB, LC, LD>), dim3((a.nitems + 3) / 4), dim3(256), 0, st, a.items,
+                           a.nitems, jk_args(a), (const PrimPair<double>*)a.pp, (const double*)a.rys, out);
     return hipGetLastError();
 }
 

@@ -67,6 +67,9 @@ constexpr int kBraPPMax = 64;
 #endif
 constexpr int kJkLaneMaxNQ = QCG_JK_LANE_MAX_NQ;
 
+// The same limit for the compressed tensor's kernels.
+constexpr int kTensorLaneMaxNQ = 54;
+
 // the bra pair of an item, restricted to the item's primitive range
 inline QCG_HD PairRec item_bra(const PairRec* __restrict__ bra, const int4& it) {
     PairRec P = bra[it.x];
@@ -96,9 +99,7 @@ struct KetCursor {
 
 struct JkLaunch {
     const PairRec* bra;
-    int nbra;
     const PairRec* ket;
-    int nket;
     int diag;           // bra class == ket class: only ket positions <= bra position
     const void* pp;     // PrimPair<double> or PrimPair<float>
     const void* rys;    // Rys table (double or float)
@@ -117,8 +118,6 @@ struct JkLaunch {
     KetPrims<double> kprims;
     KetPrims<float> kprimsf;
     const double* fix;  // per molecule: scale of J, scale of K, and their inverses (fix_scale_kernel)
-    double thr_lo;      // process quartets with thr_lo <= Q_P Q_Q < thr_hi
-    double thr_hi;
     int do_j, do_k;
     // batch of molecules (nmol = 1 for a single molecule): kets of bra pair P are
     // ket[ket_off[P.mol] .. + ket_cnt[P.mol]); matrices of molecule m start at mat_off[m],

@@ -504,6 +504,28 @@ bool qcg::jk_prepared(const qcg_context* c) { return plan_fresh(c) && !(c->profi
 // set-up.  One water 750 -> 290 us, benzene 1070 -> 500 us per build with the tiles below.
 constexpr double kChainMinUs = 12.0, kChainShare = 0.06, kModelFlopsPerUs = 16e6;
 
+// One lane's time for npp_bra x npp_ket primitive quartets of fpq model flops each, in us, on 2^lg lanes
+// per ket, and the smallest lg that keeps it within chain_us.
+static double chain_time(int nb, int nk, double fpq, int lg) { return nb * ((nk + (1 << lg) - 1) >> lg) * (0.2 + 7.5e-4 * fpq); }
+static int lanes_per_ket(int nb, int nk, double fpq, double chain_us) {
+    int lg = 0;
+    while (lg < kItemMaxLg && (1 << lg) < nk && chain_time(nb, nk, fpq, lg) > chain_us) ++lg;
+    return lg;
+}
+
+// Angular momenta of a pair class; model flops per primitive quartet (qcg_class_stat).
+static void class_l(int k, int& la, int& lb) {
+    la = k == 0 ? 0 : k <= 2 ? 1 : 2;
+    lb = (k == 0 || k == 1 || k == 3) ? 0 : (k == 2 || k == 4) ? 1 : 2;
+}
+static double model_flops(int cb, int ck) {
+    int la, lb, lc, ld;
+    class_l(cb, la, lb);
+    class_l(ck, lc, ld);
+    const double nq = (double)ncart(la) * ncart(lb) * ncart(lc) * ncart(ld);
+    return ((la + lb + lc + ld) / 2 + 1) * (80.0 + 15.0 * (la + lb + 1) * (lc + ld + 1) + nq * (4.0 + 6.0 * (lb + ld)));
+}
+
 // Tiles when the caller has set or tuned none.  Per-lane kernels: the block is widened from 64 to 256
 // threads until the waves that fit a CU's 160 KB of LDS next to each other (the K rows of one bra and
 // the Rys table are per block) reach what the kernel's registers allow (`want` per SIMD), as far as a
@@ -525,8 +547,9 @@ static void default_tiles(qcg_context* c, const int64_t (&quartets)[21][2], cons
                     continue;
                 }
                 const int64_t per_bra = n / std::max<int64_t>(1, (int64_t)bras[cls][part].size());
-                const int la = cb == 0 ? 0 : cb <= 2 ? 1 : 2, lb = (cb == 0 || cb == 1 || cb == 3) ? 0 : (cb == 2 || cb == 4) ? 1 : 2;
-                const int lc = ck == 0 ? 0 : ck <= 2 ? 1 : 2, ld = (ck == 0 || ck == 1 || ck == 3) ? 0 : (ck == 2 || ck == 4) ? 1 : 2;
+                int la, lb, lc, ld;
+                class_l(cb, la, lb);
+                class_l(ck, lc, ld);
                 const int nr = (la + lb + lc + ld) / 2 + 1;
                 const int lds = (nr <= 3 ? (qcg_rys_off[nr + 1] - qcg_rys_off[nr]) * 8 : 0) + (ncart(la) + ncart(lb)) * c->max_nbf * 8;
                 const int want = nq <= 1 ? 7 : nq <= 3 ? 5 : nq <= 9 ? 4 : nq <= 18 ? 3 : nq <= 36 ? 2 : 1;
@@ -561,12 +584,9 @@ static int build_plan(qcg_context* c) {
     for (int cb = kNumPairClasses - 1; cb >= 0; --cb)
         for (int ck = cb; ck >= 0; --ck, ++cls) {
             // the class's model flops over its surviving quartets, before the primitive screen
-            // (the default launch schedule's cost): n_roots [80 + 15 (la+lb+1)(lc+ld+1)
-            // + N_q (4 + 6 (lb+ld))] per primitive quartet plus 12 N_q per quartet
-            const int la = cb == 0 ? 0 : cb <= 2 ? 1 : 2, lb = (cb == 0 || cb == 1 || cb == 3) ? 0 : (cb == 2 || cb == 4) ? 1 : 2;
-            const int lc = ck == 0 ? 0 : ck <= 2 ? 1 : 2, ld = (ck == 0 || ck == 1 || ck == 3) ? 0 : (ck == 2 || ck == 4) ? 1 : 2;
-            const double nq = (double)ncart(la) * ncart(lb) * ncart(lc) * ncart(ld);
-            fpq[cls] = ((la + lb + lc + ld) / 2 + 1) * (80.0 + 15.0 * (la + lb + 1) * (lc + ld + 1) + nq * (4.0 + 6.0 * (lb + ld)));
+            // (the default launch schedule's cost), plus 12 N_q per quartet
+            const double nq = c->class_nq[cls];
+            fpq[cls] = model_flops(cb, ck);
             double cost = 0.0;
             for (int part = 0; part < (mixed ? 2 : 1); ++part)
                 for (int m = 0; m < nmol; ++m) {
@@ -599,19 +619,13 @@ static int build_plan(qcg_context* c) {
             const qcg_context::Tile& t = c->tile[cls][(mixed && c->fuse_cls[cls]) ? 0 : part];
             const bool lane_form = t.block > 0 ? c->class_nq[cls] <= kJkLaneMaxNQ : c->class_nq[cls] < 27;
             const int ch = std::min(kItemMaxKets, std::max(1, t.block > 0 ? t.block * t.reps : t.reps));
-            // one lane's time per primitive quartet
-            const double step_us = 0.2 + 7.5e-4 * fpq[cls];
             c->item_off[cls][part] = (int)c->items.size();
             for (const Bra& b : bras[cls][part]) {
                 // bras above kBraPPMax primitive pairs are always cut into ranges
                 const int split = (c->prim_split > 0 && c->prim_split < kBraPPMax) ? c->prim_split : kBraPPMax;
                 const int nb = std::min(b.npp, split);
                 auto lg_of = [&](int g) {
-                    if (!lane_form) return 0;
-                    const int nk = c->pairs[b.kbase + c->segs[g].x].npp;
-                    int lg = 0;
-                    while (lg < kItemMaxLg && (1 << lg) < nk && nb * ((nk + (1 << lg) - 1) >> lg) * step_us > chain_us) ++lg;
-                    return lg;
+                    return lane_form ? lanes_per_ket(nb, c->pairs[b.kbase + c->segs[g].x].npp, fpq[cls], chain_us) : 0;
                 };
                 for (int g = b.g0; g < b.g1;) {
                     const int lg = lg_of(g);
@@ -636,9 +650,8 @@ static int build_plan(qcg_context* c) {
     return QCG_OK;
 }
 
-int qcg::prepare_jk(qcg_context* c) {
-    int rc = build_plan(c);
-    if (rc) return rc;
+// The auxiliary streams and the fork, join and order events.
+static int prepare_streams(qcg_context* c) {
     if (!c->ev_done) HIPCHK(c, hipEventCreateWithFlags(&c->ev_done, hipEventDisableTiming));
     if (!c->ev_fork) {
         HIPCHK(c, hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
@@ -648,6 +661,11 @@ int qcg::prepare_jk(qcg_context* c) {
         }
     }
     return QCG_OK;
+}
+
+int qcg::prepare_jk(qcg_context* c) {
+    const int rc = build_plan(c);
+    return rc ? rc : prepare_streams(c);
 }
 
 int qcg::run_jk(qcg_context* c, const double* dD, double* dJ, double* dK, hipStream_t st, const JkAcc* acc,
@@ -1191,33 +1209,91 @@ int qcg_build_fock(qcg_context* c, const double* H, const double* D, double* F) 
     return QCG_OK;
 }
 
+// Work items of the compressed tensor (qcg_eri_compressed): every bra's surviving kets in FP64, the
+// heavily contracted ones on several lanes; blocks of kTensorBlock lanes or, for the classes above
+// kTensorLaneMaxNQ components, wavefronts of one ket.  Made once per basis and threshold.
+constexpr int kTensorBlock = 64;
+static int tensor_plan(qcg_context* c) {
+    if (c->d_tensor_items && c->tensor_key == c->schwarz_thr) return QCG_OK;
+    for (const PairRec& pr : c->pairs)
+        if (pr.npp > kItemMaxPrim) return fail(c, QCG_INVALID_ARG, "shell pair with more than 255 primitive pairs");
+    std::vector<int4> items;
+    std::vector<int2> segs;
+    for (int cls = 0, cb = kNumPairClasses - 1; cb >= 0; --cb)
+        for (int ck = cb; ck >= 0; --ck, ++cls) {
+            c->tensor_off[cls] = (int)items.size();
+            const double fpq = model_flops(cb, ck);
+            const bool lane_form = c->class_nq[cls] <= kTensorLaneMaxNQ;
+            for (int p = 0; p < c->ket_cnt_h[cb * c->nmol]; ++p) {
+                const int npp = c->pairs[c->class_off[cb] + p].npp;
+                for_ket_ranges(c, cb, ck, 0, p, c->schwarz_thr, c->schwarz_thr, [&](int bs, int, int e) {
+                    const int lg = lane_form ? lanes_per_ket(npp, c->pairs[c->class_off[ck] + bs].npp, fpq, kChainMinUs) : 0;
+                    segs.push_back(make_int2(bs, e - bs));
+                    cut_items(items, segs, (int)segs.size() - 1, (int)segs.size(), p, lane_form ? kTensorBlock >> lg : 1, lg);
+                });
+            }
+            c->tensor_cnt[cls] = (int)items.size() - c->tensor_off[cls];
+        }
+    c->release(c->d_tensor_items);
+    c->release(c->d_tensor_segs);
+    c->d_tensor_items = nullptr;
+    c->d_tensor_segs = nullptr;
+    HIPCHK(c, c->alloc(&c->d_tensor_items, items.size()));
+    HIPCHK(c, c->alloc(&c->d_tensor_segs, segs.size()));
+    HIPCHK(c, hipMemcpy(c->d_tensor_items, items.data(), items.size() * sizeof(int4), hipMemcpyHostToDevice));
+    HIPCHK(c, hipMemcpy(c->d_tensor_segs, segs.data(), segs.size() * sizeof(int2), hipMemcpyHostToDevice));
+    c->tensor_key = c->schwarz_thr;
+    return QCG_OK;
+}
+
 int qcg_eri_compressed(qcg_context* c, double* out) {
     if (!c || !out) return QCG_INVALID_ARG;
     if (!c->has_basis) return fail(c, QCG_NO_BASIS, "no basis");
     HIPCHK(c, hipSetDevice(c->device));
+    int rc = tensor_plan(c);
+    if (rc) return rc;
+    rc = prepare_streams(c);
+    if (rc) return rc;
     const int64_t nbf = c->basis.nbf;
     const int64_t npair = nbf * (nbf + 1) / 2;
     const size_t neri = (size_t)(npair * (npair + 1) / 2);
     double* dout = nullptr;
     HIPCHK(c, c->alloc(&dout, neri));
-    HIPCHK(c, launch_fill(dout, neri, 0.0, c->stream));
-    for (int cb = 0; cb < kNumPairClasses; ++cb)
-        for (int ck = 0; ck <= cb; ++ck) {
-            JkLaunch a{};
-            a.bra = c->d_pairs + c->class_off[cb];
-            a.nbra = c->class_off[cb + 1] - c->class_off[cb];
-            a.ket = c->d_pairs + c->class_off[ck];
-            a.nket = c->class_off[ck + 1] - c->class_off[ck];
-            a.diag = cb == ck;
-            a.pp = c->d_pp;
-            a.rys = c->d_rys;
-            a.thr_lo = c->schwarz_thr;
-            HIPCHK(c, launch_eri_tensor(cb, ck, a, dout, c->stream));
+    auto build = [&]() -> int {
+        HIPCHK(c, stream_begin(c, c->stream));
+        HIPCHK(c, launch_fill(dout, neri, 0.0, c->stream));
+        // the classes over the auxiliary streams, forked from and joined back to the context's
+        HIPCHK(c, hipEventRecord(c->ev_fork, c->stream));
+        for (int i = 0; i < qcg_context::kStreams; ++i) HIPCHK(c, hipStreamWaitEvent(c->aux[i], c->ev_fork, 0));
+        for (int cls = 0, cb = kNumPairClasses - 1; cb >= 0; --cb)
+            for (int ck = cb; ck >= 0; --ck, ++cls) {
+                JkLaunch a{};
+                a.bra = c->d_pairs + c->class_off[cb];
+                a.ket = c->d_pairs + c->class_off[ck];
+                a.diag = cb == ck;
+                a.pp = c->d_pp;
+                a.rys = c->d_rys;
+                a.items = c->d_tensor_items + c->tensor_off[cls];
+                a.segs = c->d_tensor_segs;
+                a.nitems = c->tensor_cnt[cls];
+                a.block = kTensorBlock;
+                a.kpairs = {c->d_kmeta + c->class_off[ck], c->d_kcen + c->class_off[ck], (int)c->pairs.size()};
+                a.kprims = {c->d_kprim, c->d_khp, c->n_kprim};
+                HIPCHK(c, launch_eri_tensor(cb, ck, a, dout, c->aux[cls % qcg_context::kStreams]));
+            }
+        for (int i = 0; i < qcg_context::kStreams; ++i) {
+            HIPCHK(c, hipEventRecord(c->ev_join[i], c->aux[i]));
+            HIPCHK(c, hipStreamWaitEvent(c->stream, c->ev_join[i], 0));
         }
-    HIPCHK(c, hipMemcpyAsync(out, dout, neri * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+        HIPCHK(c, hipMemcpyAsync(out, dout, neri * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c, stream_done(c, c->stream));
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        return QCG_OK;
+    };
+    rc = build();
+    if (rc) (void)hipDeviceSynchronize();  // nothing may still write dout
     c->release(dout);
-    return QCG_OK;
+    return rc;
 }
 
 int qcg_boys_eval_all(qcg_context* c, int m_max, int n, const double* T, double* F) {

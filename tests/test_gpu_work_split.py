@@ -42,3 +42,18 @@ def test_gpu_jk_split_over_lanes(name, basis, prec, tol):
     eng.set_prim_split(3)
     jk2 = eng.build_jk(D)
     assert np.abs(jk2.J - jk.J).max() < tol and np.abs(jk2.K - jk.K).max() < tol
+
+
+@pytest.mark.parametrize("name,basis", [("Ne", "6-31g"), ("H2O", "sto-3g"), ("H2O", "6-31+g*"), ("water2", "6-31g*")])
+def test_gpu_tensor_split_over_lanes(name, basis):
+    """Every element of the compressed tensor (per-lane and wavefront kernels, lanes per ket), and again
+    after a change of the Schwarz threshold (the plan is made per threshold).  Elements are below 10 and
+    good to 1e-14 relative: 1e-12 absolute."""
+    b = _mol(name, basis)
+    eng = Engine(b)
+    eri, _ = oracle.eri_compressed(b)
+    assert np.abs(eng.eri_compressed() - eri).max() < 1e-12
+    eng.set_options("mixed", 1e-6, 1e-6)  # the tensor is FP64 in the mixed option too
+    dropped = eng.eri_compressed()
+    off = np.abs(dropped - eri) > 1e-12
+    assert off.any() and np.all(dropped[off] == 0.0) and np.abs(eri[off]).max() < 1e-6
