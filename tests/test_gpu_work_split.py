@@ -56,4 +56,5 @@ def test_gpu_tensor_split_over_lanes(name, basis):
     eng.set_options("mixed", 1e-6, 1e-6)  # the tensor is FP64 in the mixed option too
     dropped = eng.eri_compressed()
     off = np.abs(dropped - eri) > 1e-12
-    assert off.any() and np.all(dropped[off] == 0.0) and np.abs(eri[off]).max() < 1e-6
+    assert np.all(dropped[off] == 0.0) and np.all(np.abs(eri[off]) < 1e-6)
+    assert off.any() or name != "water2"  # an atom's quartets all survive, a dimer's do not
