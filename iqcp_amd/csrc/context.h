@@ -166,8 +166,8 @@ struct qcg_context {
            *d_dphz = nullptr, *d_X = nullptr, *d_aow = nullptr, *d_V = nullptr, *d_exc = nullptr,
            *d_Vparts = nullptr;  // split-K partial products of V = Phi^T aow
     int v_chunks = 0, v_chunks_mfma = 0, v_chunks_mfma32 = 0;
-    // XC build (qcg_set_xc_mode): 0 = FP32 MFMA kernels for the mixed option, FP64 MFMA kernels up
-    // to 352 functions and rocBLAS DGEMMs around point_kernel above; 1 = rocBLAS DGEMMs for both;
+    // XC build (qcg_set_xc_mode): 0 = FP32 MFMA kernels for the mixed option, packed FP64 MFMA kernels
+    // (rocBLAS DGEMMs around point_kernel where they do not apply); 1 = rocBLAS DGEMMs for both;
     // 2 = MFMA kernels for both
     int xc_mode = 0;
     // FP32 copies of Phi and grad Phi plus FP32 work arrays for the mixed-precision XC build,
@@ -176,14 +176,29 @@ struct qcg_context {
     float4* d_grid4 = nullptr;  // (Phi, dPhi/dx, dPhi/dy, dPhi/dz) per element, FP32
     GridShell* d_gshell = nullptr;
     double *d_gexp = nullptr, *d_gcn = nullptr;
+    // The packed FP64 form of the grid (xc_packed.h), made with the grid when the precision option is
+    // FP64, else on first use, like the dense arrays above (made with the grid in the mixed option);
+    // pk_state: 0 not made, 1 made, 2 some block has more than kPackedMaxLd functions
+    PackedGrid pk{};
+    int pk_state = 0;
+    int pk_ntile[3] = {};
+    int *d_pk_int = nullptr;       // ld, nfn, floff, fl
+    int64_t *d_pk_off = nullptr;   // off, voff
+    short* d_pk_pos = nullptr;
+    int4* d_pk_tiles = nullptr;
+    double *d_pk_pts = nullptr, *d_pk_val = nullptr, *d_pk_vparts = nullptr, *d_pk_vsum = nullptr;
+    int64_t pk_elems = 0;          // elements of one packed array; d_pk_val holds Phi, three grads and aow
     void free_grid() {
         for (void** p : {(void**)&d_pts, (void**)&d_w, (void**)&d_phi, (void**)&d_dphx, (void**)&d_dphy,
                          (void**)&d_dphz, (void**)&d_X, (void**)&d_aow, (void**)&d_V, (void**)&d_exc, (void**)&d_Vparts,
                          (void**)&d_gshell, (void**)&d_gexp, (void**)&d_gcn, (void**)&d_phi32, (void**)&d_grid4,
-                         (void**)&d_aow32, (void**)&d_D32}) {
+                         (void**)&d_aow32, (void**)&d_D32, (void**)&d_pk_int, (void**)&d_pk_off, (void**)&d_pk_pos,
+                         (void**)&d_pk_tiles, (void**)&d_pk_pts, (void**)&d_pk_val, (void**)&d_pk_vparts,
+                         (void**)&d_pk_vsum}) {
             release(*p);
             *p = nullptr;
         }
+        pk_state = 0;
         G = 0;
     }
     double stats_key[3] = {-1.0, -1.0, -1.0};

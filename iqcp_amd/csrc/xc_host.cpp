@@ -27,37 +27,22 @@ int ensure_blas(qcg_context* c) {
 }
 
 constexpr int64_t kVChunk = 16384;
-// Largest basis whose default FP64 XC build runs on the MFMA kernels: up to here the density kernel
-// holds all of X's columns per wavefront (16 x 22 MFMA column tiles); (H2O)16 (304 functions):
-// 11.5 ms per FP64 XC build against 12.1 ms for the library DGEMMs around point_kernel
-constexpr int kXcMfmaFp64MaxNbf = 352;
 
-int upload_grid(qcg_context* c) {
+// The dense arrays: Phi, grad Phi, X and aow as G x nbf row-major FP64, in the grid's own order (mixed
+// precision, the library form, the gradient, and grids the packed form does not take).
+int ensure_dense(qcg_context* c) {
+    if (c->d_phi) return QCG_OK;
     const HostBasis& B = c->basis;
-    c->free_grid();
-    const int64_t G = (int64_t)c->grid_w.size();
-    c->G = G;
-    if (G == 0) return QCG_OK;
+    const int64_t G = c->G;
     const size_t gn = (size_t)G * B.nbf;
-    HIPCHK(c, c->alloc(&c->d_pts, 3 * (size_t)G));
-    HIPCHK(c, c->alloc(&c->d_w, (size_t)G));
-    HIPCHK(c, c->alloc(&c->d_phi, gn));
-    HIPCHK(c, c->alloc(&c->d_dphx, gn));
-    HIPCHK(c, c->alloc(&c->d_dphy, gn));
-    HIPCHK(c, c->alloc(&c->d_dphz, gn));
-    HIPCHK(c, c->alloc(&c->d_X, gn));
-    HIPCHK(c, c->alloc(&c->d_aow, gn));
-    HIPCHK(c, c->alloc(&c->d_V, (size_t)B.nbf * B.nbf));
     // V = Phi^T aow has a long inner dimension (the grid): split it into chunks of about
     // kVChunk points, one strided-batched GEMM over the chunks plus a sum, so the GEMM has
     // chunks x tiles workgroups instead of a handful of tiles with a 10^6-long K loop
     c->v_chunks = (int)std::max<int64_t>(1, G / kVChunk);
     // the MFMA V kernel: grid chunks for two full rounds of (chunk, output tile) blocks at the
     // kernel's occupancy, at least 1024 points per chunk, and in FP32 (whose accumulators sum a
-    // chunk) at most 4096 points per chunk.  (H2O)16: FP64 160-wide tiles at one block per CU,
-    // 128 chunks of 8 200 points (2048 / 1024 / 512 blocks: 11.70 / 11.57 / 11.50 ms per FP64
-    // XC build); FP32 at two blocks per CU, 256 chunks of 4 100 points (512 blocks were 1 % faster
-    // with twice the FP32 summation length).
+    // chunk) at most 4096 points per chunk.  (H2O)16 FP32 at two blocks per CU: 256 chunks of 4 100
+    // points (512 blocks were 1 % faster with twice the FP32 summation length).
     {
         int cus = 0;
         HIPCHK(c, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
@@ -71,8 +56,179 @@ int upload_grid(qcg_context* c) {
         c->v_chunks_mfma = chunks(false);
         c->v_chunks_mfma32 = chunks(true);
     }
+    HIPCHK(c, c->alloc(&c->d_dphx, gn));
+    HIPCHK(c, c->alloc(&c->d_dphy, gn));
+    HIPCHK(c, c->alloc(&c->d_dphz, gn));
+    HIPCHK(c, c->alloc(&c->d_X, gn));
+    HIPCHK(c, c->alloc(&c->d_aow, gn));
+    HIPCHK(c, c->alloc(&c->d_V, (size_t)B.nbf * B.nbf));
     HIPCHK(c, c->alloc(&c->d_Vparts, (size_t)std::max({c->v_chunks, c->v_chunks_mfma, c->v_chunks_mfma32}) * B.nbf *
                                          B.nbf));
+    HIPCHK(c, c->alloc(&c->d_phi, gn));
+    HIPCHK(c, launch_basis_on_grid((int)G, B.nshell, c->d_gshell, c->d_gexp, c->d_gcn, c->d_pts, B.nbf, c->d_phi,
+                                   c->d_dphx, c->d_dphy, c->d_dphz, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return QCG_OK;
+}
+
+// The grid's points along a space-filling curve: cells of 1/32 of the molecule's extent (10 bohr around
+// it; points outside in its outermost cells) in Morton order, the grid's own order inside a cell.
+std::vector<int> spatial_order(const qcg_context* c) {
+    const int64_t G = c->G;
+    double lo[3] = {1e300, 1e300, 1e300}, ext = 0.0;
+    for (int x = 0; x < 3; ++x) {
+        double hi = -1e300;
+        for (int s = 0; s < c->basis.nshell; ++s) {
+            lo[x] = std::min(lo[x], c->basis.centers[3 * s + x]);
+            hi = std::max(hi, c->basis.centers[3 * s + x]);
+        }
+        lo[x] -= 10.0;
+        ext = std::max(ext, hi + 10.0 - lo[x]);
+    }
+    constexpr int kBits = 5, kCells = 1 << kBits;
+    const double inv = kCells / ext;
+    int spread[kCells];
+    for (int i = 0; i < kCells; ++i) {
+        spread[i] = 0;
+        for (int b = 0; b < kBits; ++b) spread[i] |= ((i >> b) & 1) << (3 * b);
+    }
+    std::vector<int> key((size_t)G), first((size_t)kCells * kCells * kCells + 1, 0), order((size_t)G);
+    const double* xyz = c->grid_xyz.data();
+#pragma omp parallel for schedule(static)
+    for (int64_t g = 0; g < G; ++g) {
+        int k = 0;
+        for (int x = 0; x < 3; ++x) {
+            const double v = (xyz[3 * g + x] - lo[x]) * inv;
+            k |= spread[v > 0.0 ? (int)std::min(v, kCells - 1.0) : 0] << x;
+        }
+        key[g] = k;
+    }
+    for (int64_t g = 0; g < G; ++g) ++first[key[g] + 1];
+    for (size_t k = 1; k < first.size(); ++k) first[k] += first[k - 1];
+    for (int64_t g = 0; g < G; ++g) order[first[key[g]]++] = (int)g;
+    return order;
+}
+
+// The packed form of the grid (xc_packed.h).  Points per block: about 512 blocks, two for every CU, so
+// the V kernel has a tile for each, but 64 to 1024 points ((H2O)16: 1024 blocks of 1024).
+int ensure_packed(qcg_context* c) {
+    if (c->pk_state) return QCG_OK;
+    const HostBasis& B = c->basis;
+    const int G = (int)c->G, ns = B.nshell, nbf = B.nbf;
+    PackedGrid& k = c->pk;
+    k = PackedGrid{};
+    k.G = G;
+    k.nbf = nbf;
+    k.S = 64;
+    while (k.S < 1024 && k.S * 512 < G) k.S *= 2;
+    const int nblk = k.nblk = (G + k.S - 1) / k.S;
+    const std::vector<int> order = spatial_order(c);
+    std::vector<double> pw(4 * (size_t)nblk * k.S, 0.0);  // 3 coordinates, then the weights
+    double* w = pw.data() + 3 * (size_t)nblk * k.S;
+    for (int i = 0; i < G; ++i) {
+        for (int x = 0; x < 3; ++x) pw[3 * (size_t)i + x] = c->grid_xyz[3 * (size_t)order[i] + x];
+        w[i] = c->grid_w[order[i]];
+    }
+    HIPCHK(c, c->alloc(&c->d_pk_pts, pw.size()));
+    HIPCHK(c, hipMemcpy(c->d_pk_pts, pw.data(), pw.size() * sizeof(double), hipMemcpyHostToDevice));
+    k.pts = c->d_pk_pts;
+    k.w = c->d_pk_pts + 3 * (size_t)nblk * k.S;
+    // the shells of each block
+    std::vector<unsigned char> act((size_t)nblk * ns);
+    std::vector<short> shcol((size_t)nblk * ns, -1);
+    unsigned char* d_act = nullptr;
+    short* d_col = nullptr;
+    HIPCHK(c, c->alloc(&d_act, act.size()));
+    hipError_t e = launch_packed_active(G, k.S, nblk, ns, c->d_gshell, k.pts, d_act, c->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(act.data(), d_act, act.size(), hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    c->release(d_act);
+    HIPCHK(c, e);
+    std::vector<int> ld(nblk), nfn(nblk), floff(nblk), fl;
+    std::vector<int64_t> off(2 * (size_t)nblk);
+    std::vector<short> pos((size_t)nblk * nbf, -1);
+    std::vector<int4> tiles[3];
+    int64_t elems = 0, velems = 0;
+    for (int b = 0; b < nblk; ++b) {
+        floff[b] = (int)fl.size();
+        int n = 0;
+        for (int s = 0; s < ns; ++s) {
+            if (!act[(size_t)b * ns + s]) continue;
+            shcol[(size_t)b * ns + s] = (short)n;
+            for (int i = 0; i < ncart(B.l[s]); ++i, ++n) {
+                pos[(size_t)b * nbf + B.bf_off[s] + i] = (short)n;
+                fl.push_back(B.bf_off[s] + i);
+            }
+        }
+        nfn[b] = n;
+        ld[b] = std::max(16, (n + 15) / 16 * 16);
+        fl.resize((size_t)floff[b] + ld[b], 0);
+        k.max_ld = std::max(k.max_ld, ld[b]);
+        off[b] = elems;
+        off[nblk + b] = velems;
+        elems += (int64_t)k.S * ld[b];
+        velems += (int64_t)ld[b] * ld[b];
+        const int vw = packed_v_width(ld[b]);
+        for (int m = 0; m < ld[b]; m += 32 * vw)
+            for (int n0 = 0; n0 < ld[b]; n0 += 32 * vw) tiles[vw - 3].push_back(make_int4(b, m, n0, 0));
+    }
+    if (k.max_ld > kPackedMaxLd || nbf > INT16_MAX) {
+        c->release(c->d_pk_pts);
+        c->d_pk_pts = nullptr;
+        c->pk_state = 2;
+        return QCG_OK;
+    }
+    std::vector<int4> all;
+    for (int i = 0; i < 3; ++i) {
+        c->pk_ntile[i] = (int)tiles[i].size();
+        all.insert(all.end(), tiles[i].begin(), tiles[i].end());
+    }
+    std::vector<int> iv(ld);
+    iv.insert(iv.end(), nfn.begin(), nfn.end());
+    iv.insert(iv.end(), floff.begin(), floff.end());
+    iv.insert(iv.end(), fl.begin(), fl.end());
+    c->pk_elems = elems;
+    HIPCHK(c, c->alloc(&c->d_pk_int, iv.size()));
+    HIPCHK(c, c->alloc(&c->d_pk_off, off.size()));
+    HIPCHK(c, c->alloc(&c->d_pk_pos, pos.size()));
+    HIPCHK(c, c->alloc(&c->d_pk_tiles, all.size()));
+    HIPCHK(c, c->alloc(&c->d_pk_val, 5 * (size_t)elems));
+    HIPCHK(c, c->alloc(&c->d_pk_vparts, (size_t)velems));
+    HIPCHK(c, c->alloc(&c->d_pk_vsum, (size_t)kPackedVGroups * nbf * nbf));
+    HIPCHK(c, c->alloc(&d_col, shcol.size()));
+    HIPCHK(c, hipMemcpy(c->d_pk_int, iv.data(), iv.size() * sizeof(int), hipMemcpyHostToDevice));
+    HIPCHK(c, hipMemcpy(c->d_pk_off, off.data(), off.size() * sizeof(int64_t), hipMemcpyHostToDevice));
+    HIPCHK(c, hipMemcpy(c->d_pk_pos, pos.data(), pos.size() * sizeof(short), hipMemcpyHostToDevice));
+    HIPCHK(c, hipMemcpy(c->d_pk_tiles, all.data(), all.size() * sizeof(int4), hipMemcpyHostToDevice));
+    HIPCHK(c, hipMemcpy(d_col, shcol.data(), shcol.size() * sizeof(short), hipMemcpyHostToDevice));
+    k.ld = c->d_pk_int;
+    k.nfn = k.ld + nblk;
+    k.floff = k.nfn + nblk;
+    k.fl = k.floff + nblk;
+    k.off = c->d_pk_off;
+    k.voff = k.off + nblk;
+    k.pos = c->d_pk_pos;
+    k.phi = c->d_pk_val;
+    k.dpx = k.phi + elems;
+    k.dpy = k.dpx + elems;
+    k.dpz = k.dpy + elems;
+    e = launch_packed_basis(k, ns, c->d_gshell, c->d_gexp, c->d_gcn, d_col, c->d_pk_val, c->d_pk_val + elems,
+                            c->d_pk_val + 2 * elems, c->d_pk_val + 3 * elems, c->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    c->release(d_col);
+    HIPCHK(c, e);
+    c->pk_state = 1;
+    return QCG_OK;
+}
+
+int upload_grid(qcg_context* c) {
+    const HostBasis& B = c->basis;
+    c->free_grid();
+    const int64_t G = (int64_t)c->grid_w.size();
+    c->G = G;
+    if (G == 0) return QCG_OK;
+    HIPCHK(c, c->alloc(&c->d_pts, 3 * (size_t)G));
+    HIPCHK(c, c->alloc(&c->d_w, (size_t)G));
     HIPCHK(c, c->alloc(&c->d_exc, 1));
     HIPCHK(c, hipMemcpy(c->d_pts, c->grid_xyz.data(), 3 * (size_t)G * sizeof(double), hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->d_w, c->grid_w.data(), (size_t)G * sizeof(double), hipMemcpyHostToDevice));
@@ -105,10 +261,10 @@ int upload_grid(qcg_context* c) {
     HIPCHK(c, hipMemcpy(c->d_gshell, gs.data(), gs.size() * sizeof(GridShell), hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->d_gexp, ex.data(), ex.size() * sizeof(double), hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->d_gcn, cn.data(), cn.size() * sizeof(double), hipMemcpyHostToDevice));
-    HIPCHK(c, launch_basis_on_grid((int)G, B.nshell, c->d_gshell, c->d_gexp, c->d_gcn, c->d_pts, B.nbf, c->d_phi,
-                                   c->d_dphx, c->d_dphy, c->d_dphz, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return QCG_OK;
+    // the arrays that the current options' XC build reads; the others follow on first use
+    if (c->precision == QCG_PREC_MIXED || c->xc_mode == 1) return ensure_dense(c);
+    const int rc = ensure_packed(c);
+    return rc || c->pk_state == 1 ? rc : ensure_dense(c);
 }
 
 // FP32 copies of Phi and grad Phi (and FP32 work arrays) for the mixed-precision XC build
@@ -149,13 +305,26 @@ int xc_build_mfma(qcg_context* c, const double* dD, double* dV, double* dExc, hi
 
 int xc_build(qcg_context* c, const double* dD, double* dV, double* dExc, hipStream_t st) {
     if (c->G <= 0) return fail(c, QCG_NO_GRID, "no grid: call qcg_build_grid or qcg_set_grid");
-    // mode 0: the MFMA kernels (FP32 products for the mixed option, FP64 otherwise), except FP64
-    // above kXcMfmaFp64MaxNbf functions, where the density kernel makes column passes and the
-    // library DGEMMs win; mode 1: library DGEMMs for both; mode 2: MFMA kernels for both
-    const bool mfma = c->xc_mode == 2 ||
-                      (c->xc_mode == 0 && (c->precision == QCG_PREC_MIXED || c->basis.nbf <= kXcMfmaFp64MaxNbf));
-    if (mfma) return xc_build_mfma(c, dD, dV, dExc, st);
-    int rc = ensure_blas(c);
+    // mode 0: the dense MFMA kernels with FP32 products in the mixed option, else the packed FP64 MFMA
+    // kernels, and the library DGEMMs for grids with blocks of more than kPackedMaxLd functions; mode 1:
+    // library DGEMMs for both; mode 2: MFMA kernels for both.  (A caller that captures its first FP64
+    // build on a grid made for the mixed option gets the dense FP64 kernels: the packed arrays cannot be
+    // made inside a capture.)
+    const bool mixed = c->precision == QCG_PREC_MIXED;
+    if (!mixed && c->xc_mode != 1 && !(c->pk_state == 0 && c->d_phi && capturing(st))) {
+        int rc = ensure_packed(c);
+        if (rc) return rc;
+        if (c->pk_state == 1) {
+            HIPCHK(c, launch_fill(dExc, 1, 0.0, st));
+            HIPCHK(c, launch_xc_packed(c->pk, dD, c->d_pk_val + 4 * c->pk_elems, c->d_pk_tiles, c->pk_ntile, c->d_pk_vparts,
+                                       c->d_pk_vsum, dV, dExc, st));
+            return QCG_OK;
+        }
+    }
+    int rc = ensure_dense(c);
+    if (rc) return rc;
+    if (c->xc_mode == 2 || (c->xc_mode == 0 && (mixed || c->pk_state == 0))) return xc_build_mfma(c, dD, dV, dExc, st);
+    rc = ensure_blas(c);
     if (rc) return rc;
     const int nbf = c->basis.nbf;
     const rocblas_int G = (rocblas_int)c->G;
@@ -190,7 +359,8 @@ int xc_build(qcg_context* c, const double* dD, double* dV, double* dExc, hipStre
 // XC nuclear gradient at the device density dD, ADDED into dgrad (natom x 3) on stream st.
 int xc_gradient(qcg_context* c, const double* dD, double* dgrad, hipStream_t st) {
     if (c->G <= 0) return fail(c, QCG_NO_GRID, "no grid: call qcg_build_grid or qcg_set_grid");
-    int rc = ensure_blas(c);
+    int rc = ensure_dense(c);
+    if (!rc) rc = ensure_blas(c);
     if (rc) return rc;
     const HostBasis& B = c->basis;
     const int nbf = B.nbf;

@@ -13,20 +13,15 @@
 
 namespace qcg {
 
-__global__ __launch_bounds__(256) void basis_kernel(int G, int nshell, const GridShell* __restrict__ shells,
-                                                    const double* __restrict__ exps, const double* __restrict__ cn,
-                                                    const double* __restrict__ pts, int nbf, double* __restrict__ phi,
-                                                    double* __restrict__ dphx, double* __restrict__ dphy,
-                                                    double* __restrict__ dphz) {
-    const size_t idx = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-    if (idx >= (size_t)G * nshell) return;
-    const int g = (int)(idx / nshell), s = (int)(idx % nshell);
-    const GridShell sh = shells[s];
-    const double dx = pts[3 * (size_t)g] - sh.cx, dy = pts[3 * (size_t)g + 1] - sh.cy, dz = pts[3 * (size_t)g + 2] - sh.cz;
+// Phi and grad Phi of one shell at one point, written to its consecutive elements from `row`.
+__device__ __forceinline__ void shell_on_point(const GridShell& sh, const double* __restrict__ exps,
+                                               const double* __restrict__ cn, double gx, double gy, double gz, size_t row,
+                                               double* __restrict__ phi, double* __restrict__ dphx,
+                                               double* __restrict__ dphy, double* __restrict__ dphz) {
+    const double dx = gx - sh.cx, dy = gy - sh.cy, dz = gz - sh.cz;
     const double r2 = dx * dx + dy * dy + dz * dz;
     const int nc = ncart(sh.l);
-    const size_t row = (size_t)g * nbf + sh.bf;
-    if (sh.amin * r2 > 34.5388) {  // GAUSSIAN_SCREENING_THRESHOLD (orbital/grid.rs:174)
+    if (sh.amin * r2 > kGridCut) {
         for (int c = 0; c < nc; ++c) phi[row + c] = dphx[row + c] = dphy[row + c] = dphz[row + c] = 0.0;
         return;
     }
@@ -60,6 +55,77 @@ __global__ __launch_bounds__(256) void basis_kernel(int G, int nshell, const Gri
         dphy[row + c] = gr[1];
         dphz[row + c] = gr[2];
     }
+}
+
+__global__ __launch_bounds__(256) void basis_kernel(int G, int nshell, const GridShell* __restrict__ shells,
+                                                    const double* __restrict__ exps, const double* __restrict__ cn,
+                                                    const double* __restrict__ pts, int nbf, double* __restrict__ phi,
+                                                    double* __restrict__ dphx, double* __restrict__ dphy,
+                                                    double* __restrict__ dphz) {
+    const size_t idx = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+    if (idx >= (size_t)G * nshell) return;
+    const int g = (int)(idx / nshell), s = (int)(idx % nshell);
+    const GridShell sh = shells[s];
+    shell_on_point(sh, exps, cn, pts[3 * (size_t)g], pts[3 * (size_t)g + 1], pts[3 * (size_t)g + 2],
+                   (size_t)g * nbf + sh.bf, phi, dphx, dphy, dphz);
+}
+
+// One thread block per grid block: does shell s reach any of its points?
+__global__ __launch_bounds__(256) void packed_active_kernel(int G, int S, int nshell, const GridShell* __restrict__ shells,
+                                                            const double* __restrict__ pts,
+                                                            unsigned char* __restrict__ active) {
+    const int b = blockIdx.x, g1 = min(G, (b + 1) * S);
+    for (int s = threadIdx.x; s < nshell; s += blockDim.x) {
+        const GridShell sh = shells[s];
+        bool on = false;
+        for (int g = b * S; g < g1 && !on; ++g) {  // every lane reads the same point
+            const double dx = pts[3 * (size_t)g] - sh.cx, dy = pts[3 * (size_t)g + 1] - sh.cy,
+                         dz = pts[3 * (size_t)g + 2] - sh.cz;
+            on = !(sh.amin * (dx * dx + dy * dy + dz * dz) > kGridCut);
+        }
+        active[(size_t)b * nshell + s] = on;
+    }
+}
+
+// The block's rows: threads over (point, shell); the zero padding (rows past the grid, columns past the
+// functions) is written too.
+__global__ __launch_bounds__(256) void packed_basis_kernel(const PackedGrid g, int nshell,
+                                                           const GridShell* __restrict__ shells,
+                                                           const double* __restrict__ exps, const double* __restrict__ cn,
+                                                           const short* __restrict__ shcol, double* __restrict__ phi,
+                                                           double* __restrict__ dphx, double* __restrict__ dphy,
+                                                           double* __restrict__ dphz) {
+    const int b = blockIdx.y, ld = g.ld[b];
+    const size_t base = (size_t)g.off[b];
+    const int n = g.S * (nshell + 1);
+    for (int idx = blockIdx.x * blockDim.x + threadIdx.x; idx < n; idx += gridDim.x * blockDim.x) {
+        const int p = idx / (nshell + 1), s = idx - p * (nshell + 1);
+        const size_t row = base + (size_t)p * ld, pt = (size_t)b * g.S + p;
+        if (s == nshell) {  // the padding: columns from the last function on, or the whole row
+            int c = pt < (size_t)g.G ? g.nfn[b] : 0;
+            for (; c < ld; ++c) phi[row + c] = dphx[row + c] = dphy[row + c] = dphz[row + c] = 0.0;
+            continue;
+        }
+        const int col = shcol[(size_t)b * nshell + s];
+        if (col < 0 || pt >= (size_t)g.G) continue;
+        shell_on_point(shells[s], exps, cn, g.pts[3 * pt], g.pts[3 * pt + 1], g.pts[3 * pt + 2], row + col, phi, dphx,
+                       dphy, dphz);
+    }
+}
+
+hipError_t launch_packed_active(int G, int S, int nblk, int nshell, const GridShell* shells, const double* pts,
+                                unsigned char* active, hipStream_t st) {
+    hipLaunchKernelGGL(packed_active_kernel, dim3(nblk), dim3(128), 0, st, G, S, nshell, shells, pts, active);
+    return hipGetLastError();
+}
+
+hipError_t launch_packed_basis(const PackedGrid& g, int nshell, const GridShell* shells, const double* exps,
+                               const double* cn, const short* shcol, double* phi, double* dpx, double* dpy, double* dpz,
+                               hipStream_t st) {
+    const unsigned per = (unsigned)((g.S * (nshell + 1) + 255) / 256);
+    hipLaunchKernelGGL(packed_basis_kernel, dim3(per, g.nblk), dim3(256), 0, st, g, nshell, shells, exps, cn, shcol, phi,
+                       dpx, dpy, dpz);
+    return hipGetLastError();
 }
 
 __global__ __launch_bounds__(256) void point_kernel(int G, int nbf, const double* __restrict__ w,

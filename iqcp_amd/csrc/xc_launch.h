@@ -1,14 +1,9 @@
 // Host-side launch interface of the XC kernels.
 #pragma once
 #include "qcg_common.h"
+#include "xc_packed.h"
 
 namespace qcg {
-
-struct GridShell {
-    double cx, cy, cz, amin;  // centre, smallest exponent (screening)
-    int l, nprim, poff, bf;
-    int atom, pad;
-};
 
 // Becke partition weights of np points (owner[p]: the point's atom), on the device
 hipError_t launch_becke_partition(int64_t np, const double* pts, const int* owner, int nat, const double* axyz,

@@ -4,8 +4,9 @@
 //                   grad rho (X never goes to HBM), then B3LYP per point (FP64), the aow rows and
 //                   E_xc -- the work of compute_density_and_gradient_matmul and the point part of
 //                   build_vxc_gga_matmul (dft/ks_scf.rs:1028-1093, :1150-1296) in one kernel;
-//   xc_rho_all_kernel : the same for nbf <= 352 with X for all columns held per wavefront, so Phi
-//                   is read once per K step instead of once per column pass;
+//   xc_rho_all_kernel : the same in FP32 for nbf <= 352 with X for all columns held per wavefront, so
+//                   Phi is read once per K step instead of once per column pass;
+//   xc_rho_packed_kernel, xc_v_packed_kernel : the FP64 build on the packed grid (xc_packed.h);
 //   xc_v_kernel   : V = Phi^T aow as 128x128 output tiles over grid chunks (split K), one partial
 //                   matrix per chunk, summed and symmetrised afterwards (sum_parts, sym_half).
 // rho, grad rho, E_xc and the functional are accumulated in FP64 whatever T is; with T = float the
@@ -76,19 +77,9 @@ constexpr int lds_pad(int n) {
     return sizeof(T) == 8 ? (16 - n % 32 + 32) % 32 : (16 - n % 64 + 64) % 64;
 }
 
-// All-columns rho kernel options.  PREFETCH_D: the next K step's D rows are loaded into registers
-// during the current step's MFMAs (FP32: on; FP64: off, the registers cost the second block per CU:
-// (H2O)16 FP64 rho 11.2 -> 9.3 ms without).  WPE64: waves per SIMD the kernel is compiled for (4
-// = two 512-thread blocks per CU, at most 128 VGPRs).
-#ifndef QCG_XC_RHO_PREFETCH_D
-#define QCG_XC_RHO_PREFETCH_D 1
-#endif
-#ifndef QCG_XC_RHO_PREFETCH_D64
-#define QCG_XC_RHO_PREFETCH_D64 0
-#endif
-#ifndef QCG_XC_RHO_WPE64
-#define QCG_XC_RHO_WPE64 4
-#endif
+// The density kernels of 512 threads are compiled for four waves per SIMD (two blocks per CU, at most
+// 128 VGPRs).
+#define QCG_XC_RHO_ATTR __attribute__((amdgpu_waves_per_eu(4)))
 
 // Most MFMA column tiles the all-columns kernel holds (nbf <= 352): D rows of one K step, all
 // columns, stay within the 64 KB of static LDS per block.
@@ -284,12 +275,6 @@ __global__ __launch_bounds__(256) void xc_rho_kernel(int G, int nbf, const doubl
     xc_point_tail<T, 4>(G, nbf, wv, l, g0, w, gv, aow, exc_sum, red, coef, part);
 }
 
-#if QCG_XC_RHO_WPE64
-#define QCG_XC_RHO_ATTR __attribute__((amdgpu_waves_per_eu(QCG_XC_RHO_WPE64)))
-#else
-#define QCG_XC_RHO_ATTR
-#endif
-
 // All-columns form of xc_rho_kernel for nbf <= 16 kRhoAllMaxNT, eight wavefronts per block of 64
 // points: wavefront wv keeps the X tile of the 16 points of row tile wv % 4 for column half wv / 4
 // (NH = ceil(NT / 2) MFMA column tiles, one accumulator each), so Phi is read from HBM once per K
@@ -320,10 +305,8 @@ __global__ __launch_bounds__(512) QCG_XC_RHO_ATTR void xc_rho_all_kernel(int G, 
     acc_t acc[NH];
 #pragma unroll
     for (int t = 0; t < NH; ++t) acc[t] = acc_t{T(0), T(0), T(0), T(0)};
-    // next K step's Phi (and, with QCG_XC_RHO_PREFETCH_D, D) elements, loaded while the current step
-    // is multiplied
-    constexpr bool kPrefD = sizeof(T) == 8 ? QCG_XC_RHO_PREFETCH_D64 : QCG_XC_RHO_PREFETCH_D;
-    constexpr int NBD = kPrefD ? (kRhoBK * BN + 511) / 512 : 1;
+    // next K step's Phi and D elements, loaded while the current step is multiplied
+    constexpr int NBD = (kRhoBK * BN + 511) / 512;
     T ra[NA], rb[NBD];
     auto load = [&](int k0) {
 #pragma unroll
@@ -331,12 +314,10 @@ __global__ __launch_bounds__(512) QCG_XC_RHO_ATTR void xc_rho_all_kernel(int G, 
             const int e = tid + 512 * i, r = e / kRhoBK, c = e % kRhoBK, g = g0 + r, k = k0 + c;
             ra[i] = (g < G && k < nbf) ? phi[(size_t)g * nbf + k] : T(0);
         }
-        if constexpr (kPrefD) {
 #pragma unroll
-            for (int i = 0; i < NBD; ++i) {
-                const int e = tid + 512 * i, r = e / BN, c = e - r * BN, k = k0 + r;
-                rb[i] = (e < kRhoBK * BN && k < nbf && c < nbf) ? Dm[(size_t)k * nbf + c] : T(0);
-            }
+        for (int i = 0; i < NBD; ++i) {
+            const int e = tid + 512 * i, r = e / BN, c = e - r * BN, k = k0 + r;
+            rb[i] = (e < kRhoBK * BN && k < nbf && c < nbf) ? Dm[(size_t)k * nbf + c] : T(0);
         }
     };
     load(0);
@@ -347,17 +328,10 @@ __global__ __launch_bounds__(512) QCG_XC_RHO_ATTR void xc_rho_all_kernel(int G, 
             const int e = tid + 512 * i;
             As[e % kRhoBK][e / kRhoBK] = ra[i];
         }
-        if constexpr (kPrefD) {
 #pragma unroll
-            for (int i = 0; i < NBD; ++i) {
-                const int e = tid + 512 * i, r = e / BN, c = e - r * BN;
-                if (e < kRhoBK * BN) Bs[r][c] = rb[i];
-            }
-        } else {
-            for (int e = tid; e < kRhoBK * BN; e += 512) {
-                const int r = e / BN, c = e - r * BN, k = k0 + r;
-                Bs[r][c] = (k < nbf && c < nbf) ? Dm[(size_t)k * nbf + c] : T(0);
-            }
+        for (int i = 0; i < NBD; ++i) {
+            const int e = tid + 512 * i, r = e / BN, c = e - r * BN;
+            if (e < kRhoBK * BN) Bs[r][c] = rb[i];
         }
         __syncthreads();
         if (k0 + kRhoBK < nbf) load(k0 + kRhoBK);
@@ -562,6 +536,269 @@ hipError_t launch_to_f32(const double* in, float* out, size_t n, hipStream_t st)
     return hipGetLastError();
 }
 
+// ---------------------------------------------------------------- packed FP64 form (xc_packed.h)
+// X = Phi D for 64 points of a block on MFMA, reduced into rho and grad rho, then the functional, the
+// aow rows and E_xc: xc_rho_all_kernel over the block's own functions.  Eight wavefronts, wavefront wv
+// holding the X tile of row tile wv % 4 and column half wv / 4 (at most NH of 16 columns); no bounds
+// checks, since rows and columns are padded with zeros.  D is gathered by function number straight into
+// LDS, 16 rows per K step, 32 threads per row; the next step's Phi and D elements are loaded during the
+// current MFMAs while the registers allow two blocks per CU (NH <= kPackedPrefNH).
+// Bound by memory: Phi for the product, Phi and grad Phi for the reduction and again for the aow rows.
+// (H2O)16, 1.05e6 points: density kernel 6.98 ms dense, 2.50 ms packed; V 3.67 -> 0.98 ms (three widths),
+// summing the partial V 0.05 -> 0.20 ms; benzene, 1.3e5 points: 0.29 -> 0.22 and 0.18 -> 0.13 ms.
+constexpr int kPackedPrefNH = 6;
+template <int NH>
+__global__ __launch_bounds__(512) QCG_XC_RHO_ATTR void xc_rho_packed_kernel(
+    const PackedGrid g, const double* __restrict__ Dm, double* __restrict__ aow, double* __restrict__ exc_sum) {
+    using M = Mfma<double>;
+    using acc_t = typename M::acc;
+    constexpr int BN = 32 * NH, SA = kRhoBM + 16, SB = BN + lds_pad<double>(BN);
+    constexpr bool kPref = NH <= kPackedPrefNH;
+    __shared__ double As[kRhoBK][SA];
+    __shared__ double Bs[kRhoBK][SB < 32 ? 32 : SB];
+    __shared__ double red[4][kRhoPW][4];
+    __shared__ double coef[4][kRhoPW][4];
+    __shared__ double part[4];
+    const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63, li = l & 15, lk = l >> 4;
+    const int per = g.S / kRhoBM, b = blockIdx.x / per, p0 = (blockIdx.x - b * per) * kRhoBM;
+    const int ld = g.ld[b], nt = ld >> 4, nh = (nt + 1) >> 1;
+    const int rt = wv & 3, half = wv >> 2, t0 = half * nh, mine = half ? nt - nh : nh;
+    const size_t base = (size_t)g.off[b] + (size_t)p0 * ld;
+    const int* fl = g.fl + g.floff[b];
+    const double* __restrict__ phi = g.phi + base;
+    acc_t acc[NH];
+#pragma unroll
+    for (int t = 0; t < NH; ++t) acc[t] = acc_t{0.0, 0.0, 0.0, 0.0};
+    // staging: A two functions of one point per thread, B columns (tid % 32) + 32 i of row tid / 32
+    const int ar = tid >> 3, ac = 2 * (tid & 7), br = tid >> 5, bc = tid & 31;
+    int fc[NH];
+#pragma unroll
+    for (int i = 0; i < NH; ++i) fc[i] = bc + 32 * i < ld ? fl[bc + 32 * i] : 0;
+    double2 ra;
+    double rb[kPref ? NH : 1];
+    auto load_b = [&](int k0) {
+        const double* row = Dm + (size_t)fl[k0 + br] * g.nbf;
+#pragma unroll
+        for (int i = 0; i < NH; ++i)
+            if (32 * i < ld) rb[kPref ? i : 0] = row[fc[i]];
+    };
+    auto load = [&](int k0) {
+        ra = *reinterpret_cast<const double2*>(phi + (size_t)ar * ld + k0 + ac);
+        if constexpr (kPref) load_b(k0);
+    };
+    load(0);
+    for (int k0 = 0; k0 < ld; k0 += kRhoBK) {
+        __syncthreads();  // the previous step's fragment reads are done
+        As[ac][ar] = ra.x;
+        As[ac + 1][ar] = ra.y;
+        if constexpr (kPref) {
+#pragma unroll
+            for (int i = 0; i < NH; ++i)
+                if (32 * i < ld) Bs[br][bc + 32 * i] = rb[i];
+        } else {
+            const double* row = Dm + (size_t)fl[k0 + br] * g.nbf;
+#pragma unroll
+            for (int i = 0; i < NH; ++i)
+                if (32 * i < ld) Bs[br][bc + 32 * i] = row[fc[i]];
+        }
+        __syncthreads();
+        if (k0 + kRhoBK < ld) load(k0 + kRhoBK);
+#pragma unroll 2
+        for (int ks = 0; ks < kRhoBK; ks += 4) {
+            const double a = As[ks + lk][kRhoPW * rt + li];
+#pragma unroll
+            for (int t = 0; t < NH; ++t)
+                if (t < mine) acc[t] = M::mma(a, Bs[ks + lk][16 * (t0 + t) + li], acc[t]);
+        }
+    }
+    double rs[4] = {}, xs[4] = {}, ys[4] = {}, zs[4] = {};
+    const GridVals<double> gv{g.phi + base, g.dpx + base, g.dpy + base, g.dpz + base, nullptr};
+#pragma unroll
+    for (int t = 0; t < NH; ++t) {
+        if (t < mine) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                double f, dx, dy, dz;
+                gv.get((size_t)(kRhoPW * rt + M::row(lk, r)) * ld + 16 * (t0 + t) + li, f, dx, dy, dz);
+                const double x = acc[t][r];
+                rs[r] += x * f;
+                xs[r] += x * dx;
+                ys[r] += x * dy;
+                zs[r] += x * dz;
+            }
+        }
+        // one tile's loads in flight at a time: hoisting all of them costs hundreds of VGPRs
+        asm volatile("" ::: "memory");
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+#pragma unroll
+        for (int off = 1; off < 16; off <<= 1) {
+            rs[r] += __shfl_xor(rs[r], off, 64);
+            xs[r] += __shfl_xor(xs[r], off, 64);
+            ys[r] += __shfl_xor(ys[r], off, 64);
+            zs[r] += __shfl_xor(zs[r], off, 64);
+        }
+    }
+    // per column half, row tile and point, in the D staging area (free now)
+    static_assert(sizeof(Bs) >= 2 * 4 * kRhoPW * 4 * sizeof(double), "red2 fits in Bs");
+    auto red2 = reinterpret_cast<double (*)[4][kRhoPW][4]>(&Bs[0][0]);
+    __syncthreads();  // every wavefront's last fragment reads are done
+    if (li == 0) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int p = M::row(lk, r);
+            red2[half][rt][p][0] = rs[r];
+            red2[half][rt][p][1] = xs[r];
+            red2[half][rt][p][2] = ys[r];
+            red2[half][rt][p][3] = zs[r];
+        }
+    }
+    __syncthreads();
+    if (tid < 4 * kRhoPW * 4) {  // the two column halves, in a fixed order
+        const int q = tid & 3, p = (tid >> 2) % kRhoPW, r4 = tid / (4 * kRhoPW);
+        red[r4][p][q] = red2[0][r4][p][q] + red2[1][r4][p][q];
+    }
+    __syncthreads();
+    xc_point_tail<double, 8, (NH + 1) / 2>(kRhoBM, ld, wv, l, 0, g.w + (size_t)b * g.S + p0, gv, aow + base, exc_sum, red,
+                                           coef, part);
+}
+
+// Partial V of one block: Phi^T aow over its S points by 32 VW square output tiles (xc_v_kernel's
+// tiling), written packed.
+template <int VW>
+__global__ __launch_bounds__(256) void xc_v_packed_kernel(const PackedGrid g, const int4* __restrict__ tiles,
+                                                          const double* __restrict__ aow, double* __restrict__ Vparts) {
+    using M = Mfma<double>;
+    using acc_t = typename M::acc;
+    constexpr int BM = 32 * VW;
+    __shared__ double As[kVBK][BM + kPad];
+    __shared__ double Bs[kVBK][BM + kPad];
+    const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63, li = l & 15, lk = l >> 4;
+    const int wr = wv >> 1, wc = wv & 1;
+    const int4 tl = tiles[blockIdx.x];
+    const int b = tl.x, m0 = tl.y, n0 = tl.z, ld = g.ld[b];
+    const double* __restrict__ A = g.phi + g.off[b] + m0;
+    const double* __restrict__ B = aow + g.off[b] + n0;
+    acc_t acc[VW][VW];
+#pragma unroll
+    for (int i = 0; i < VW; ++i)
+#pragma unroll
+        for (int j = 0; j < VW; ++j) acc[i][j] = acc_t{0.0, 0.0, 0.0, 0.0};
+    // staging: 16 threads per row of 16 points, two columns each per pass of 32
+    const int sr = tid >> 4, sc = 2 * (tid & 15);
+    double2 ra[VW], rb[VW];
+    auto load = [&](int k0) {
+        const size_t row = (size_t)(k0 + sr) * ld + sc;
+#pragma unroll
+        for (int i = 0; i < VW; ++i) {
+            ra[i] = m0 + 32 * i + sc < ld ? *reinterpret_cast<const double2*>(A + row + 32 * i) : make_double2(0.0, 0.0);
+            rb[i] = n0 + 32 * i + sc < ld ? *reinterpret_cast<const double2*>(B + row + 32 * i) : make_double2(0.0, 0.0);
+        }
+    };
+    load(0);
+    for (int k0 = 0; k0 < g.S; k0 += kVBK) {
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < VW; ++i) {
+            *reinterpret_cast<double2*>(&As[sr][32 * i + sc]) = ra[i];
+            *reinterpret_cast<double2*>(&Bs[sr][32 * i + sc]) = rb[i];
+        }
+        __syncthreads();
+        if (k0 + kVBK < g.S) load(k0 + kVBK);
+#pragma unroll
+        for (int ks = 0; ks < kVBK; ks += 4) {
+            double a[VW], c[VW];
+#pragma unroll
+            for (int i = 0; i < VW; ++i) {
+                a[i] = As[ks + lk][16 * VW * wr + 16 * i + li];
+                c[i] = Bs[ks + lk][16 * VW * wc + 16 * i + li];
+            }
+#pragma unroll
+            for (int i = 0; i < VW; ++i)
+#pragma unroll
+                for (int j = 0; j < VW; ++j)  // sub-tiles past the block's functions: uniform per wavefront
+                    if (m0 + 16 * VW * wr + 16 * i < ld && n0 + 16 * VW * wc + 16 * j < ld) acc[i][j] = M::mma(a[i], c[j], acc[i][j]);
+        }
+    }
+    double* out = Vparts + g.voff[b];
+#pragma unroll
+    for (int i = 0; i < VW; ++i)
+#pragma unroll
+        for (int j = 0; j < VW; ++j) {
+            const int col = n0 + 16 * VW * wc + 16 * j + li;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = m0 + 16 * VW * wr + 16 * i + M::row(lk, r);
+                if (row < ld && col < ld) out[(size_t)row * ld + col] = acc[i][j][r];
+            }
+        }
+}
+
+// Vsum[k] = sum of the partial matrices of the k-th run of blocks, one matrix row per thread block
+__global__ __launch_bounds__(128) void packed_vsum_kernel(const PackedGrid g, int per, const double* __restrict__ Vparts,
+                                                          double* __restrict__ Vsum) {
+    const int i = blockIdx.y, j = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.z;
+    const int b1 = min(g.nblk, (k + 1) * per);
+    const bool in = j < g.nbf;
+    double s = 0.0;
+    for (int b = k * per; b < b1; ++b) {
+        const int pi = g.pos[(size_t)b * g.nbf + i];
+        if (pi < 0) continue;  // uniform
+        const int pj = in ? g.pos[(size_t)b * g.nbf + j] : -1;
+        if (pj >= 0) s += Vparts[(size_t)g.voff[b] + (size_t)pi * g.ld[b] + pj];
+    }
+    if (in) Vsum[((size_t)k * g.nbf + i) * g.nbf + j] = s;
+}
+
+__global__ __launch_bounds__(128) void packed_vsym_kernel(int nbf, int ngrp, const double* __restrict__ Vsum,
+                                                          double* __restrict__ V) {
+    const int i = blockIdx.y, j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j >= nbf) return;
+    const size_t n2 = (size_t)nbf * nbf, ij = (size_t)i * nbf + j, ji = (size_t)j * nbf + i;
+    double s = 0.0, t = 0.0;
+#pragma unroll 8
+    for (int k = 0; k < ngrp; ++k) {
+        s += Vsum[k * n2 + ij];
+        t += Vsum[k * n2 + ji];
+    }
+    V[ij] = 0.5 * (s + t);
+}
+
+int packed_v_width(int ld) { return xc_v_width(ld, false); }
+
+hipError_t launch_xc_packed(const PackedGrid& g, const double* D, double* aow, const int4* tiles, const int ntile[3],
+                            double* Vparts, double* Vsum, double* V, double* exc_sum, hipStream_t st) {
+    const dim3 grid((unsigned)(g.nblk * (g.S / kRhoBM)));
+    switch ((g.max_ld / 16 + 1) / 2) {
+#define QCG_RHO_PACKED(n)                                                                                    \
+    case n:                                                                                                  \
+        hipLaunchKernelGGL((xc_rho_packed_kernel<n>), grid, dim3(512), 0, st, g, D, aow, exc_sum);           \
+        break;
+        QCG_RHO_PACKED(1) QCG_RHO_PACKED(2) QCG_RHO_PACKED(3) QCG_RHO_PACKED(4) QCG_RHO_PACKED(5) QCG_RHO_PACKED(6)
+        QCG_RHO_PACKED(7) QCG_RHO_PACKED(8) QCG_RHO_PACKED(9) QCG_RHO_PACKED(10) QCG_RHO_PACKED(11)
+#undef QCG_RHO_PACKED
+        default: return hipErrorInvalidValue;
+    }
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    const int4* t = tiles;
+    for (int w = 3; w <= 5; t += ntile[w - 3], ++w) {
+        if (ntile[w - 3] == 0) continue;
+        const dim3 tg((unsigned)ntile[w - 3]);
+        if (w == 3) hipLaunchKernelGGL((xc_v_packed_kernel<3>), tg, dim3(256), 0, st, g, t, aow, Vparts);
+        else if (w == 4) hipLaunchKernelGGL((xc_v_packed_kernel<4>), tg, dim3(256), 0, st, g, t, aow, Vparts);
+        else hipLaunchKernelGGL((xc_v_packed_kernel<5>), tg, dim3(256), 0, st, g, t, aow, Vparts);
+        e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    const int ngrp = g.nblk < kPackedVGroups ? g.nblk : kPackedVGroups, per = (g.nblk + ngrp - 1) / ngrp;
+    const dim3 vg((g.nbf + 127) / 128, g.nbf, ngrp);
+    hipLaunchKernelGGL(packed_vsum_kernel, vg, dim3(128), 0, st, g, per, Vparts, Vsum);
+    hipLaunchKernelGGL(packed_vsym_kernel, dim3((g.nbf + 127) / 128, g.nbf), dim3(128), 0, st, g.nbf, ngrp, Vsum, V);
+    return hipGetLastError();
+}
+
 template <typename T>
 static hipError_t launch_xc_mfma_t(int G, int nbf, int nchunk, const double* w, const T* phi, const T* dpx,
                                    const T* dpy, const T* dpz, const float4* g4, const T* Dm, T* aow, double* exc_sum,
@@ -575,12 +812,14 @@ static hipError_t launch_xc_mfma_t(int G, int nbf, int nchunk, const double* w, 
     constexpr int kMaxNT = sizeof(T) == 8 ? 4 : 5;
     const int tiles = (nbf + 15) / 16, passes = (tiles + kMaxNT - 1) / kMaxNT, nt = (tiles + passes - 1) / passes;
     const dim3 grid((G + kRhoBM - 1) / kRhoBM);
-    // up to kRhoAllMaxNT column tiles: the all-columns kernel (Phi read once per K step)
-    switch (tiles <= kRhoAllMaxNT ? 100 + tiles : nt) {
+    // FP32 up to kRhoAllMaxNT column tiles: the all-columns kernel (Phi read once per K step); FP64 runs
+    // here only where the packed form does not apply
+    switch (sizeof(T) == 4 && tiles <= kRhoAllMaxNT ? 100 + tiles : nt) {
 #define QCG_RHO_ALL(n)                                                                                  \
     case 100 + n:                                                                                       \
-        hipLaunchKernelGGL((xc_rho_all_kernel<T, n>), grid, dim3(512), 0, st, G, nbf, w, phi, gv, Dm, aow,  \
-                           exc_sum);                                                                    \
+        if constexpr (sizeof(T) == 4)                                                                   \
+            hipLaunchKernelGGL((xc_rho_all_kernel<T, n>), grid, dim3(512), 0, st, G, nbf, w, phi, gv, Dm, aow, \
+                               exc_sum);                                                                \
         break;
         QCG_RHO_ALL(1) QCG_RHO_ALL(2) QCG_RHO_ALL(3) QCG_RHO_ALL(4) QCG_RHO_ALL(5) QCG_RHO_ALL(6) QCG_RHO_ALL(7)
         QCG_RHO_ALL(8) QCG_RHO_ALL(9) QCG_RHO_ALL(10) QCG_RHO_ALL(11) QCG_RHO_ALL(12) QCG_RHO_ALL(13)
