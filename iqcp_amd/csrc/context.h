@@ -61,7 +61,8 @@ struct qcg_context {
     // the pairs and primitive pairs as arrays for the per-lane J/K kernels (KetPairs, KetPrims)
     int4* d_kmeta = nullptr;
     double2 *d_kcen = nullptr, *d_kprim = nullptr;
-    double* d_khp = nullptr;
+    double *d_khp = nullptr, *d_kea = nullptr;
+    int2* d_katoms = nullptr;
     float4* d_kprimf = nullptr;
     int n_kprim = 0;
     // their scales per molecule (4 doubles each), recomputed at the start of every build from the
@@ -184,9 +185,10 @@ struct qcg_context {
     int pk_ntile[3] = {};
     int *d_pk_int = nullptr;       // ld, nfn, floff, fl
     int64_t *d_pk_off = nullptr;   // off, voff
-    short* d_pk_pos = nullptr;
+    short *d_pk_pos = nullptr, *d_pk_shcol = nullptr;  // column of each function and shell in each block
     int4* d_pk_tiles = nullptr;
     double *d_pk_pts = nullptr, *d_pk_val = nullptr, *d_pk_vparts = nullptr, *d_pk_vsum = nullptr;
+    double* d_pk_grad = nullptr;   // X, M and t of the XC gradient, made on its first use
     int64_t pk_elems = 0;          // elements of one packed array; d_pk_val holds Phi, three grads and aow
     void free_grid() {
         for (void** p : {(void**)&d_pts, (void**)&d_w, (void**)&d_phi, (void**)&d_dphx, (void**)&d_dphy,
@@ -194,7 +196,7 @@ struct qcg_context {
                          (void**)&d_gshell, (void**)&d_gexp, (void**)&d_gcn, (void**)&d_phi32, (void**)&d_grid4,
                          (void**)&d_aow32, (void**)&d_D32, (void**)&d_pk_int, (void**)&d_pk_off, (void**)&d_pk_pos,
                          (void**)&d_pk_tiles, (void**)&d_pk_pts, (void**)&d_pk_val, (void**)&d_pk_vparts,
-                         (void**)&d_pk_vsum}) {
+                         (void**)&d_pk_vsum, (void**)&d_pk_shcol, (void**)&d_pk_grad}) {
             release(*p);
             *p = nullptr;
         }
@@ -222,7 +224,7 @@ struct qcg_context {
                          (void**)&d_qsh_off, (void**)&d_mol_ns, (void**)&d_bf_shell, (void**)&d_bf_off,
                          (void**)&d_qmax, (void**)&d_row_mol, (void**)&d_shell_first, (void**)&d_shell_first_off,
                          (void**)&d_Dp, (void**)&d_bf_norm, (void**)&d_jmap, (void**)&d_kmeta, (void**)&d_kcen,
-                         (void**)&d_kprim, (void**)&d_khp, (void**)&d_kprimf,
+                         (void**)&d_kprim, (void**)&d_khp, (void**)&d_kea, (void**)&d_katoms, (void**)&d_kprimf,
                          (void**)&d_H, (void**)&d_F, (void**)&d_mol_nbf,
                          (void**)&d_mat_off, (void**)&d_ket_off, (void**)&d_ket_cnt, (void**)&d_items,
                          (void**)&d_segs, (void**)&d_tensor_items, (void**)&d_tensor_segs, (void**)&d_grad_items, (void**)&d_grad_segs, (void**)&d_grad,
@@ -238,6 +240,17 @@ struct qcg_context {
 
 
 namespace qcg {
+
+// The kets of class ck as arrays (per-lane kernels).
+inline KetPairs ket_pairs(const qcg_context* c, int ck) {
+    const int o = c->class_off[ck];
+    return {c->d_kmeta + o, c->d_kcen + o, (int)c->pairs.size(), c->d_katoms + o};
+}
+
+// Lanes (as a power of two) that a ket of nk primitive pairs gets against a bra of nb so that no lane runs
+// longer than chain_us, fpq being the class's model flops per primitive quartet (qcg_host.cpp).
+int lanes_per_ket(int nb, int nk, double fpq, double chain_us);
+double model_flops(int cb, int ck);
 
 inline int fail(qcg_context* c, int code, const std::string& msg) {
     if (c) c->err = msg;

@@ -298,41 +298,6 @@ struct JkWave {
     static constexpr bool kEnabled = S::NQ >= 27;
 };
 
-// The contracted quartet (P|Q) on one wavefront: component lane + 64 j in acc[j], without norms; tbl:
-// the wave's LDS table (JkWave<..., R>::T).
-template <int LA, int LB, int LC, int LD, typename R>
-__device__ __forceinline__ void wave_quartet(const PairRec& P, const PairRec& Q, const PrimPair<R>* __restrict__ pp,
-                                             const R* __restrict__ rys_tab, double* V, int lane, R* acc) {
-    using S = EriShape<LA, LB, LC, LD>;
-    using W = JkWave<LA, LB, LC, LD, R>;
-    using TB = typename W::T;
-    constexpr int N = S::NROOTS, HT = TB::HT, ES = TB::ES, KPL = W::KPL;
-    constexpr const CompTab<LA, LB, LC, LD>& ct = kCompTab<LA, LB, LC, LD>;
-    R* tbl = reinterpret_cast<R*>(V);
-    int ox[KPL], oy[KPL], oz[KPL];
-#pragma unroll
-    for (int j = 0; j < KPL; ++j) {
-        const int k = lane + 64 * j;
-        const int kk = k < S::NQ ? k : 0;
-        ox[j] = ct.hx[kk] * ES;
-        oy[j] = (HT + ct.hy[kk]) * ES;
-        oz[j] = (2 * HT + ct.hz[kk]) * ES;
-        acc[j] = R(0);
-    }
-    const int npq = P.npp * Q.npp;
-    for (int pq0 = 0; pq0 < npq; pq0 += TB::PQ_CAP) {
-        const int npc = min(TB::PQ_CAP, npq - pq0);
-        wave_sync();  // earlier readers of the table (and of what aliases it) are done
-        wave_tables<LA, LB, LC, LD, N, ES, R>(P, Q, pp, rys_tab, pq0, npc, tbl, lane);
-        wave_sync();
-        const int ne = npc * N;
-        for (int e = 0; e < ne; ++e) {
-#pragma unroll
-            for (int j = 0; j < KPL; ++j) acc[j] += tbl[ox[j] + e] * tbl[oy[j] + e] * tbl[oz[j] + e];
-        }
-    }
-}
-
 // One work item on one wavefront; V: the wave's LDS region (JkWave<..., R>::WAVE_D doubles).
 template <int LA, int LB, int LC, int LD, typename R>
 __device__ __forceinline__ void jk_wave_item(

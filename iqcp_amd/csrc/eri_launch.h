@@ -184,6 +184,9 @@ struct GradLaunch {
     int nket;
     int diag;
     const PrimPair<double>* pp;  // ea and p - ea are the two primitive exponents
+    KetPairs kpairs;             // the kets as arrays (per-lane kernels), kea their first exponents
+    KetPrims<double> kprims;
+    const double* kea;
     const double* rys;
     const double* D;
     int nbf;
@@ -198,11 +201,25 @@ struct GradLaunch {
     int nitems;
 };
 
-// Work-item length (kets per item) the gradient kernel of a class expects: one block of threads
-// per item for the light classes (per-lane kernel), a few kets per wavefront otherwise.
-inline int grad_item_kets(int cb, int ck) {
-    auto nc = [](int c) { return c == 0 ? 1 : c == 1 ? 3 : c == 2 ? 9 : c == 3 ? 6 : c == 4 ? 18 : 36; };
-    return nc(cb) * nc(ck) <= 54 ? 128 : 8;
+// Components of the first shell that one launch of the per-lane gradient kernel of a class takes (0: the
+// class runs wave-cooperatively): as many as keep the weights and 1-D tables of a lane in registers
+// (measured at the kernel).
+constexpr int kGradLaneMaxNQ = 54;
+constexpr int grad_part(int cb, int ck) {
+    const int na = cb == 0 ? 1 : cb <= 2 ? 3 : 6;
+    const int nc[6] = {1, 3, 9, 6, 18, 36};
+    const int rest = nc[cb] / na * nc[ck];
+    for (int n = na; n >= 1; --n)
+        if (na % n == 0 && n * rest <= kGradLaneMaxNQ) return n;
+    return 0;
+}
+
+// Work-item length (kets per item) of a class with n quartets in the gradient: one block of 128 threads
+// per item for the per-lane kernel, up to eight kets per lane once that leaves 4096 blocks, and one to
+// eight kets per wavefront otherwise.
+inline int grad_item_kets(int cb, int ck, int64_t n) {
+    if (grad_part(cb, ck) > 0) return 128 * (int)std::max<int64_t>(1, std::min<int64_t>(8, n / (128 * 4096)));
+    return (int)std::max<int64_t>(1, std::min<int64_t>(8, n / 2048));
 }
 
 hipError_t launch_grad_cb0(int ck, const GradLaunch& a, hipStream_t st);

@@ -2,35 +2,52 @@
 #include "boys.h"
 #include "eri_device.h"
 #include "eri_launch.h"
+#include "eri_wave.h"
 
 namespace qcg {
 
-// Schwarz bound per pair: sqrt(max |(ab|ab)|) (compute_schwarz_bounds, integrals/eri/mod.rs:1263-1290)
+// Schwarz bound per pair: sqrt(max |(ab|ab)|) (compute_schwarz_bounds, integrals/eri/mod.rs:1263-1290).
+// One wavefront per pair: up to 81 components its lanes split the ket's primitives and sum the partial
+// quartets (a fixed butterfly), above it works as eri_wave.h.  One lane per pair had run every primitive
+// quartet in series, the (dp|dp) and (dd|dd) ones in scratch: 6.0 ms for any molecule with d shells.
 template <int LA, int LB>
-__global__ __launch_bounds__(128) void schwarz_kernel(const PairRec* __restrict__ pairs, int n,
+__global__ __launch_bounds__(256) void schwarz_kernel(const PairRec* __restrict__ pairs, int n,
                                                       const PrimPair<double>* __restrict__ pp,
                                                       const double* __restrict__ rys_tab, double* __restrict__ Q) {
     using S = EriShape<LA, LB, LA, LB>;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
+    const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (i >= n) return;  // the whole wavefront; no block-wide barrier below
     const PairRec P = pairs[i];
-    double eri[S::NQ];
-    for_n<S::kUnroll, S::NQ>([&](int k) { eri[k] = 0.0; });
-    contract_quartet<LA, LB, LA, LB, double>(P, P, pp, rys_tab, eri);
     double mx = 0.0;
-#pragma unroll 1
-    for (int k = 0; k < S::NQ; ++k) {
+    auto norm = [](int k) {
         const int d = k % S::NB, c = (k / S::NB) % S::NA, b = (k / S::NAB) % S::NB, a = k / (S::NAB * S::NB);
-        const double nrm = cnorm(LA, a) * cnorm(LB, b) * cnorm(LA, c) * cnorm(LB, d);
-        mx = fmax(mx, fabs(eri[k] * nrm));
+        return cnorm(LA, a) * cnorm(LB, b) * cnorm(LA, c) * cnorm(LB, d);
+    };
+    if constexpr (S::NQ <= 81) {
+        double eri[S::NQ];
+        for_n<true, S::NQ>([&](int k) { eri[k] = 0.0; });
+        const PrimPair<double>* ppk = pp + P.pp_off;
+        contract_quartet_pp<LA, LB, LA, LB, double>(P, P, ppk, [ppk](int j) { return ppk[j]; }, rys_tab, eri, lane, 64);
+        for (int off = 1; off < 64; off <<= 1) for_n<true, S::NQ>([&](int k) { eri[k] += __shfl_xor(eri[k], off, 64); });
+        for_n<true, S::NQ>([&](int k) { mx = fmax(mx, fabs(eri[k] * norm(k))); });
+    } else {
+        using TB = WaveTable<LA, LB, LA, LB, S::NROOTS, double>;
+        constexpr int KPL = (S::NQ + 63) / 64;
+        __shared__ double smem[4 * TB::DOUBLES];
+        double acc[KPL];
+        wave_quartet<LA, LB, LA, LB, double>(P, P, pp, rys_tab, smem + (threadIdx.x >> 6) * TB::DOUBLES, lane, acc);
+#pragma unroll
+        for (int j = 0; j < KPL; ++j)
+            if (lane + 64 * j < S::NQ) mx = fmax(mx, fabs(acc[j] * norm(lane + 64 * j)));
+        for (int off = 1; off < 64; off <<= 1) mx = fmax(mx, __shfl_xor(mx, off, 64));
     }
-    Q[i] = sqrt(mx);
+    if (lane == 0) Q[i] = sqrt(mx);
 }
 
 hipError_t launch_schwarz(int c, const PairRec* pairs, int n, const PrimPair<double>* pp, const double* rys,
                           double* Q, hipStream_t st) {
     if (n <= 0) return hipSuccess;
-    dim3 g((n + 127) / 128), b(128);
+    const dim3 g((n + 3) / 4), b(256);
     switch (c) {
         case 0: hipLaunchKernelGGL((schwarz_kernel<0, 0>), g, b, 0, st, pairs, n, pp, rys, Q); break;
         case 1: hipLaunchKernelGGL((schwarz_kernel<1, 0>), g, b, 0, st, pairs, n, pp, rys, Q); break;

@@ -24,24 +24,6 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Node r (runtime) of the N-point Rys rule at T: the same fits and asymptotic form as rys_eval.
-template <typename R, int N>
-__device__ __forceinline__ void rys_eval_one(R T, const R* __restrict__ tab, int r, R& x, R& w) {
-    if (T >= (R)qcg_rys_tmax[N]) {
-        const R rs = qrsqrt(T);
-        const R it = rs * rs;
-        x = (R)qcg_rys_hx[rys_tri(N) + r] * it;
-        w = (R)qcg_rys_hw[rys_tri(N) + r] * rs;
-        return;
-    }
-    const int k = (int)(T * (R)(1.0 / QCG_RYS_H));
-    const R s = (T - (R)(k * QCG_RYS_H)) * (R)(2.0 / QCG_RYS_H) - R(1);
-    const R* cx = tab + qcg_rys_off[N] + k * (2 * N * kRysStride) + r * kRysStride;
-    const R* cw = cx + N * kRysStride;
-    x = poly13(cx, s);
-    w = poly13(cw, s);
-}
-
 // LDS geometry of one wave for transfer tables with powers up to (TA, TB, TC, TD), N nodes,
 // element type R and a budget of kBytes per wave for the table.
 template <int TA, int TB, int TC, int TD, int N, typename R, int kBytes = 16384>
@@ -80,7 +62,7 @@ __device__ __forceinline__ void wave_tables(const PairRec& P, const PairRec& Q, 
         const R PQx = a.px - c.px, PQy = a.py - c.py, PQz = a.pz - c.pz;
         const R T = p * q * ipq * (PQx * PQx + PQy * PQy + PQz * PQz);
         R x, w;
-        rys_eval_one<R, N>(T, rys_tab, r, x, w);
+        rys_eval_node<R, N>(T, rys_tab + qcg_rys_off[N], r, x, w);
         const R qf = q * ipq, pf = p * ipq;
         const R b00 = R(0.5) * x * ipq;
         const R b10 = hp * (R(1) - x * qf);
@@ -100,6 +82,40 @@ __device__ __forceinline__ void wave_tables(const PairRec& P, const PairRec& Q, 
             sc = (prim_kab(a) * prim_kab(c) < kPrimScreen) ? R(0) : w * (two_pi_52 * rs * a.ckp * c.ckp);
         R* row = tbl + axis * HT * ES + pql * N + r;
         hrr1d_put<TA, TB, TC, TD, R>(g, AB, CD, [&](int h, R v) { row[h * ES] = v * sc; });
+    }
+}
+
+// The contracted quartet (P|Q) on one wavefront: component lane + 64 j in acc[j], without norms; V:
+// the wave's LDS table (WaveTable<LA, LB, LC, LD, S::NROOTS, R>).
+template <int LA, int LB, int LC, int LD, typename R>
+__device__ __forceinline__ void wave_quartet(const PairRec& P, const PairRec& Q, const PrimPair<R>* __restrict__ pp,
+                                             const R* __restrict__ rys_tab, double* V, int lane, R* acc) {
+    using S = EriShape<LA, LB, LC, LD>;
+    using TB = WaveTable<LA, LB, LC, LD, S::NROOTS, R>;
+    constexpr int N = S::NROOTS, HT = TB::HT, ES = TB::ES, KPL = (S::NQ + 63) / 64;
+    constexpr const CompTab<LA, LB, LC, LD>& ct = kCompTab<LA, LB, LC, LD>;
+    R* tbl = reinterpret_cast<R*>(V);
+    int ox[KPL], oy[KPL], oz[KPL];
+#pragma unroll
+    for (int j = 0; j < KPL; ++j) {
+        const int k = lane + 64 * j;
+        const int kk = k < S::NQ ? k : 0;
+        ox[j] = ct.hx[kk] * ES;
+        oy[j] = (HT + ct.hy[kk]) * ES;
+        oz[j] = (2 * HT + ct.hz[kk]) * ES;
+        acc[j] = R(0);
+    }
+    const int npq = P.npp * Q.npp;
+    for (int pq0 = 0; pq0 < npq; pq0 += TB::PQ_CAP) {
+        const int npc = min(TB::PQ_CAP, npq - pq0);
+        wave_sync();  // earlier readers of the table (and of what aliases it) are done
+        wave_tables<LA, LB, LC, LD, N, ES, R>(P, Q, pp, rys_tab, pq0, npc, tbl, lane);
+        wave_sync();
+        const int ne = npc * N;
+        for (int e = 0; e < ne; ++e) {
+#pragma unroll
+            for (int j = 0; j < KPL; ++j) acc[j] += tbl[ox[j] + e] * tbl[oy[j] + e] * tbl[oz[j] + e];
+        }
     }
 }
 

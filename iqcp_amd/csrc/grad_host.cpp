@@ -11,25 +11,46 @@ using namespace qcg;
 
 namespace {
 
+// Lanes per ket of the gradient kernels (lanes_per_ket): a primitive quartet costs about three of the J/K
+// builds' (0.5 us (ss|ss), 5 us (pp|ps) on one lane), and a chain may take 50 us
+constexpr double kGradFlops = 4.0, kGradChainUs = 50.0;
+
 // Work items of the gradient kernels: every bra pair's surviving kets (the exact screening
 // predicate Q_P Q_Q >= threshold, one segment per contraction bucket, as for J/K) cut into items
-// of grad_item_kets(class pair) kets.  Built once per basis, threshold and primitive split and kept
+// of grad_item_kets kets.  Built once per basis, threshold and primitive split and kept
 // on the device.
 int grad_plan(qcg_context* c) {
     const double key[2] = {c->schwarz_thr, (double)c->prim_split};
     if (c->d_grad_items && std::memcmp(key, c->grad_key, sizeof(key)) == 0) return QCG_OK;
+    for (const PairRec& pr : c->pairs)
+        if (pr.npp > kItemMaxPrim) return fail(c, QCG_INVALID_ARG, "shell pair with more than 255 primitive pairs");
     std::vector<int4> items;
     std::vector<int2> segs;
     int cls = 0;
     for (int cb = kNumPairClasses - 1; cb >= 0; --cb)
         for (int ck = cb; ck >= 0; --ck, ++cls) {
             c->grad_off[cls] = (int)items.size();
+            const bool lane_form = grad_part(cb, ck) > 0;
+            int64_t n_q = 0;
+            for (int p = 0; p < c->ket_cnt_h[cb]; ++p)
+                for_ket_ranges(c, cb, ck, 0, p, c->schwarz_thr, c->schwarz_thr, [&](int bs, int, int e) { n_q += e - bs; });
+            const int ch = grad_item_kets(cb, ck, n_q);
+            const double fpq = kGradFlops * model_flops(cb, ck);
             for (int p = 0; p < c->ket_cnt_h[cb]; ++p) {
-                const int g0 = (int)segs.size();
+                const int g0 = (int)segs.size(), npp = c->pairs[c->class_off[cb] + p].npp;
                 for_ket_ranges(c, cb, ck, 0, p, c->schwarz_thr, c->schwarz_thr,
                                [&](int bs, int, int e) { segs.push_back(make_int2(bs, e - bs)); });
-                cut_items_split(items, segs, g0, (int)segs.size(), p, grad_item_kets(cb, ck),
-                                c->pairs[c->class_off[cb] + p].npp, c->prim_split);
+                // runs of segments whose kets get the same number of lanes
+                auto lg_of = [&](int g) {
+                    return lane_form ? lanes_per_ket(npp, c->pairs[c->class_off[ck] + segs[g].x].npp, fpq, kGradChainUs) : 0;
+                };
+                for (int g = g0, n = (int)segs.size(); g < n;) {
+                    const int lg = lg_of(g);
+                    int e = g + 1;
+                    while (e < n && lg_of(e) == lg) ++e;
+                    cut_items_split(items, segs, g, e, p, std::max(1, ch >> lg), npp, c->prim_split, lg);
+                    g = e;
+                }
             }
             c->grad_cnt[cls] = (int)items.size() - c->grad_off[cls];
         }
@@ -84,6 +105,9 @@ int qcg::eri_grad_launch(qcg_context* c, const double* dD, double hf_frac, doubl
         a.nket = c->class_off[ck + 1] - c->class_off[ck];
         a.diag = cb == ck;
         a.pp = c->d_pp;
+        a.kpairs = ket_pairs(c, ck);
+        a.kprims = {c->d_kprim, c->d_khp, c->n_kprim};
+        a.kea = c->d_kea;
         a.rys = c->d_rys;
         a.D = dD;
         a.nbf = c->basis.nbf;

@@ -369,7 +369,8 @@ int qcg_set_basis_batch(qcg_context* c, int nmol, const int* mol_nshell, const i
         const int np = npairs, npr = (int)pp.size();
         std::vector<int4> meta(np);
         std::vector<double2> cen(3 * (size_t)np), kp(3 * (size_t)npr);
-        std::vector<double> khp(npr);
+        std::vector<double> khp(npr), kea(npr);
+        std::vector<int2> katoms(np);
         std::vector<float4> kpf(2 * (size_t)npr);
         int first = 0;
         for (int k = 0; k < kNumPairClasses; ++k)
@@ -382,6 +383,7 @@ int qcg_set_basis_batch(qcg_context* c, int nmol, const int* mol_nshell, const i
                         const int g = base + bnd[b] + i;
                         const PairRec& r = all[g];
                         meta[g] = make_int4(r.bfa | (r.sa == r.sb ? kKetSame : 0), r.bfb, first + i, (int)(((unsigned)npp << 24) | (unsigned)n));
+                        katoms[g] = make_int2(r.atom_a, r.atom_b);
                         cen[g] = make_double2(r.ax, r.ay);
                         cen[(size_t)np + g] = make_double2(r.az, r.abx);
                         cen[2 * (size_t)np + g] = make_double2(r.aby, r.abz);
@@ -393,6 +395,7 @@ int qcg_set_basis_batch(qcg_context* c, int nmol, const int* mol_nshell, const i
                             kp[npr + e] = make_double2(q.pz, q.p);
                             kp[2 * (size_t)npr + e] = make_double2(q.ckp, q.kab);
                             khp[e] = q.hp;
+                            kea[e] = q.ea;
                             kpf[e] = make_float4(f.px, f.py, f.pz, f.p);
                             kpf[npr + e] = make_float4(f.ckp, f.hp, f.kab, f.ea);
                         }
@@ -426,6 +429,8 @@ int qcg_set_basis_batch(qcg_context* c, int nmol, const int* mol_nshell, const i
         HIPCHK(c, c->alloc(&c->d_kcen, cen.size()));
         HIPCHK(c, c->alloc(&c->d_kprim, kp.size()));
         HIPCHK(c, c->alloc(&c->d_khp, khp.size()));
+        HIPCHK(c, c->alloc(&c->d_kea, kea.size()));
+        HIPCHK(c, c->alloc(&c->d_katoms, katoms.size()));
         HIPCHK(c, c->alloc(&c->d_kprimf, kpf.size()));
         HIPCHK(c, c->alloc(&c->d_jmap, jmap.size()));
         HIPCHK(c, c->alloc(&c->d_bf_norm, bfn.size()));
@@ -434,6 +439,8 @@ int qcg_set_basis_batch(qcg_context* c, int nmol, const int* mol_nshell, const i
         HIPCHK(c, hipMemcpy(c->d_kcen, cen.data(), cen.size() * sizeof(double2), hipMemcpyHostToDevice));
         HIPCHK(c, hipMemcpy(c->d_kprim, kp.data(), kp.size() * sizeof(double2), hipMemcpyHostToDevice));
         HIPCHK(c, hipMemcpy(c->d_khp, khp.data(), khp.size() * sizeof(double), hipMemcpyHostToDevice));
+        HIPCHK(c, hipMemcpy(c->d_kea, kea.data(), kea.size() * sizeof(double), hipMemcpyHostToDevice));
+        HIPCHK(c, hipMemcpy(c->d_katoms, katoms.data(), katoms.size() * sizeof(int2), hipMemcpyHostToDevice));
         HIPCHK(c, hipMemcpy(c->d_kprimf, kpf.data(), kpf.size() * sizeof(float4), hipMemcpyHostToDevice));
         HIPCHK(c, hipMemcpy(c->d_jmap, jmap.data(), jmap.size() * sizeof(int), hipMemcpyHostToDevice));
         HIPCHK(c, hipMemcpy(c->d_bf_norm, bfn.data(), bfn.size() * sizeof(double), hipMemcpyHostToDevice));
@@ -507,7 +514,7 @@ constexpr double kChainMinUs = 12.0, kChainShare = 0.06, kModelFlopsPerUs = 16e6
 // One lane's time for npp_bra x npp_ket primitive quartets of fpq model flops each, in us, on 2^lg lanes
 // per ket, and the smallest lg that keeps it within chain_us.
 static double chain_time(int nb, int nk, double fpq, int lg) { return nb * ((nk + (1 << lg) - 1) >> lg) * (0.2 + 7.5e-4 * fpq); }
-static int lanes_per_ket(int nb, int nk, double fpq, double chain_us) {
+int qcg::lanes_per_ket(int nb, int nk, double fpq, double chain_us) {
     int lg = 0;
     while (lg < kItemMaxLg && (1 << lg) < nk && chain_time(nb, nk, fpq, lg) > chain_us) ++lg;
     return lg;
@@ -518,7 +525,7 @@ static void class_l(int k, int& la, int& lb) {
     la = k == 0 ? 0 : k <= 2 ? 1 : 2;
     lb = (k == 0 || k == 1 || k == 3) ? 0 : (k == 2 || k == 4) ? 1 : 2;
 }
-static double model_flops(int cb, int ck) {
+double qcg::model_flops(int cb, int ck) {
     int la, lb, lc, ld;
     class_l(cb, la, lb);
     class_l(ck, lc, ld);
@@ -752,7 +759,7 @@ int qcg::run_jk(qcg_context* c, const double* dD, double* dJ, double* dK, hipStr
             a.jb_ket = c->jbase[ck];
             a.np_bra = c->class_off[cb + 1] - c->class_off[cb];
             a.np_ket = c->class_off[ck + 1] - c->class_off[ck];
-            a.kpairs = {c->d_kmeta + c->class_off[ck], c->d_kcen + c->class_off[ck], (int)c->pairs.size()};
+            a.kpairs = ket_pairs(c, ck);
             a.kprims = {c->d_kprim, c->d_khp, c->n_kprim};
             a.kprimsf = {c->d_kprimf, c->n_kprim};
             a.fix = A.fix;
@@ -1277,7 +1284,7 @@ int qcg_eri_compressed(qcg_context* c, double* out) {
                 a.segs = c->d_tensor_segs;
                 a.nitems = c->tensor_cnt[cls];
                 a.block = kTensorBlock;
-                a.kpairs = {c->d_kmeta + c->class_off[ck], c->d_kcen + c->class_off[ck], (int)c->pairs.size()};
+                a.kpairs = ket_pairs(c, ck);
                 a.kprims = {c->d_kprim, c->d_khp, c->n_kprim};
                 HIPCHK(c, launch_eri_tensor(cb, ck, a, dout, c->aux[cls % qcg_context::kStreams]));
             }

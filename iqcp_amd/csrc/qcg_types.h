@@ -81,6 +81,7 @@ struct KetPairs {
     const int4* meta;     // bfa | (sa == sb) << 30, bfb, first primitive, npp << 24 | stride
     const double2* cen;   // np x (ax, ay), np x (az, abx), np x (aby, abz)
     int np;               // pairs of all classes (the stride of cen)
+    const int2* atoms;    // the two shells' atoms (gradient kernels)
 };
 constexpr int kKetSame = 1 << 30;
 

@@ -57,6 +57,23 @@ QCG_HD void rys_eval_tab(R T, const R* __restrict__ tabN, R* x, R* w) {
     }
 }
 
+// Node r (runtime) of the rule: the same fits and asymptotic form.
+template <typename R, int N>
+QCG_HD void rys_eval_node(R T, const R* __restrict__ tabN, int r, R& x, R& w) {
+    if (T >= (R)qcg_rys_tmax[N]) {
+        const R rs = qrsqrt(T);
+        const R it = rs * rs;
+        x = (R)qcg_rys_hx[rys_tri(N) + r] * it;
+        w = (R)qcg_rys_hw[rys_tri(N) + r] * rs;
+        return;
+    }
+    const int k = (int)(T * (R)(1.0 / QCG_RYS_H));
+    const R s = (T - (R)(k * QCG_RYS_H)) * (R)(2.0 / QCG_RYS_H) - R(1);
+    const R* cx = tabN + k * (2 * N * kRysStride) + r * kRysStride;
+    x = poly13(cx, s);
+    w = poly13(cx + N * kRysStride, s);
+}
+
 // tab: qcg_rys_coef (double) or its float copy, resident in device memory.
 template <typename R, int N>
 QCG_HD void rys_eval(R T, const R* __restrict__ tab, R* x, R* w) {

@@ -58,3 +58,31 @@ def test_gpu_tensor_split_over_lanes(name, basis):
     off = np.abs(dropped - eri) > 1e-12
     assert np.all(dropped[off] == 0.0) and np.all(np.abs(eri[off]) < 1e-6)
     assert off.any() or name != "water2"  # an atom's quartets all survive, a dimer's do not
+
+
+@pytest.mark.parametrize("name,basis", [("H2O", "sto-3g"), ("H2O", "6-31+g*"), ("water2", "6-31g*"), ("C6H6", "6-31g")])
+def test_gpu_eri_gradient_split_over_lanes(name, basis):
+    """The ERI gradient (lanes per ket, parts of the first shell's components) against five-point
+    differences of 1/2 Tr D J - 1/4 Tr D K for one atom.  Step 0.02: the fourth-order remainder,
+    h^4 / 30 times a fifth derivative of order 10, is below 1e-7, and the energies (below 1e3, good to
+    1e-13) contribute 1e-10 / 0.02: 1e-6.  With the bra primitives in ranges the same sum is made of other
+    partial sums: 1e-10."""
+    b = _mol(name, basis)
+    D = random_density(b.nbf, seed=6, nocc=b.n_occ)
+    eng = Engine(b)
+    g = eng.eri_gradient(D)
+    assert np.abs(g.sum(axis=0)).max() < 1e-9
+    eng.set_prim_split(2)
+    assert np.abs(eng.eri_gradient(D) - g).max() < 1e-10
+    atoms = [(int(z), x.copy()) for z, x in zip(b.Z, b.xyz)]
+
+    def energy(step, axis):
+        moved = [(z, x + (step * np.eye(3)[axis] if i == 1 else 0.0)) for i, (z, x) in enumerate(atoms)]
+        jk = Engine(build_basis(moved, basis)).build_jk(D)
+        return 0.5 * np.sum(D * jk.J) - 0.25 * np.sum(D * jk.K)
+
+    h = 0.02
+    for axis in range(3):
+        e = {k: energy(k * h, axis) for k in (-2, -1, 1, 2)}
+        fd = (8 * (e[1] - e[-1]) - (e[2] - e[-2])) / (12 * h)
+        assert abs(fd - g[1, axis]) < 1e-6
