@@ -94,7 +94,6 @@ std::vector<int> spatial_order(const qcg_context* c) {
     }
     std::vector<int> key((size_t)G), first((size_t)kCells * kCells * kCells + 1, 0), order((size_t)G);
     const double* xyz = c->grid_xyz.data();
-#pragma omp parallel for schedule(static)
     for (int64_t g = 0; g < G; ++g) {
         int k = 0;
         for (int x = 0; x < 3; ++x) {
@@ -137,7 +136,6 @@ int ensure_packed(qcg_context* c) {
     std::vector<unsigned char> act((size_t)nblk * ns);
     std::vector<short> shcol((size_t)nblk * ns, -1);
     unsigned char* d_act = nullptr;
-    short* d_col = nullptr;
     HIPCHK(c, c->alloc(&d_act, act.size()));
     hipError_t e = launch_packed_active(G, k.S, nblk, ns, c->d_gshell, k.pts, d_act, c->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(act.data(), d_act, act.size(), hipMemcpyDeviceToHost, c->stream);
@@ -195,12 +193,12 @@ int ensure_packed(qcg_context* c) {
     HIPCHK(c, c->alloc(&c->d_pk_val, 5 * (size_t)elems));
     HIPCHK(c, c->alloc(&c->d_pk_vparts, (size_t)velems));
     HIPCHK(c, c->alloc(&c->d_pk_vsum, (size_t)kPackedVGroups * nbf * nbf));
-    HIPCHK(c, c->alloc(&d_col, shcol.size()));
+    HIPCHK(c, c->alloc(&c->d_pk_shcol, shcol.size()));
     HIPCHK(c, hipMemcpy(c->d_pk_int, iv.data(), iv.size() * sizeof(int), hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->d_pk_off, off.data(), off.size() * sizeof(int64_t), hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->d_pk_pos, pos.data(), pos.size() * sizeof(short), hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->d_pk_tiles, all.data(), all.size() * sizeof(int4), hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemcpy(d_col, shcol.data(), shcol.size() * sizeof(short), hipMemcpyHostToDevice));
+    HIPCHK(c, hipMemcpy(c->d_pk_shcol, shcol.data(), shcol.size() * sizeof(short), hipMemcpyHostToDevice));
     k.ld = c->d_pk_int;
     k.nfn = k.ld + nblk;
     k.floff = k.nfn + nblk;
@@ -212,10 +210,9 @@ int ensure_packed(qcg_context* c) {
     k.dpx = k.phi + elems;
     k.dpy = k.dpx + elems;
     k.dpz = k.dpy + elems;
-    e = launch_packed_basis(k, ns, c->d_gshell, c->d_gexp, c->d_gcn, d_col, c->d_pk_val, c->d_pk_val + elems,
+    e = launch_packed_basis(k, ns, c->d_gshell, c->d_gexp, c->d_gcn, c->d_pk_shcol, c->d_pk_val, c->d_pk_val + elems,
                             c->d_pk_val + 2 * elems, c->d_pk_val + 3 * elems, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    c->release(d_col);
     HIPCHK(c, e);
     c->pk_state = 1;
     return QCG_OK;
@@ -359,7 +356,18 @@ int xc_build(qcg_context* c, const double* dD, double* dV, double* dExc, hipStre
 // XC nuclear gradient at the device density dD, ADDED into dgrad (natom x 3) on stream st.
 int xc_gradient(qcg_context* c, const double* dD, double* dgrad, hipStream_t st) {
     if (c->G <= 0) return fail(c, QCG_NO_GRID, "no grid: call qcg_build_grid or qcg_set_grid");
-    int rc = ensure_dense(c);
+    // on the packed grid (FP64 in every precision option); the library form where it does not apply
+    int rc = ensure_packed(c);
+    if (rc) return rc;
+    if (c->pk_state == 1 && 3 * (size_t)c->basis.natom * sizeof(double) <= 65536) {
+        const size_t n = (size_t)c->pk_elems, rows = (size_t)c->pk.nblk * c->pk.S;
+        if (!c->d_pk_grad) HIPCHK(c, c->alloc(&c->d_pk_grad, 2 * n + 3 * rows));
+        HIPCHK(c, launch_xc_grad_packed(c->pk, c->basis.nshell, c->basis.natom, c->d_gshell, c->d_gexp, c->d_gcn,
+                                        c->d_pk_shcol, dD, c->d_pk_grad, c->d_pk_val + 4 * n, c->d_pk_grad + n,
+                                        c->d_pk_grad + 2 * n, dgrad, st));
+        return QCG_OK;
+    }
+    rc = ensure_dense(c);
     if (!rc) rc = ensure_blas(c);
     if (rc) return rc;
     const HostBasis& B = c->basis;

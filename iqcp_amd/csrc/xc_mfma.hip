@@ -89,10 +89,13 @@ constexpr int kRhoAllMaxNT = 22;
 // are in red[row tile][point]: B3LYP per point (FP64), the aow rows, E_xc.  NW wavefronts per block
 // (4 or 8); wavefront wv works on row tile wv % 4, and with 8 wavefronts each takes half its rows
 // in the aow pass.
+// tgrad: instead the rows of the gradient, w vrho Phi + 2 w vsigma (grad rho . grad Phi), and
+// t = 2 w vsigma grad rho (three per point) without E_xc.
 template <typename T, int NW, int MAXC = 0>
 __device__ __forceinline__ void xc_point_tail(int G, int nbf, int wv, int l, int g0, const double* __restrict__ w,
                                               const GridVals<T>& gv, T* __restrict__ aow, double* __restrict__ exc_sum,
-                                              double (*red)[kRhoPW][4], double (*coef)[kRhoPW][4], double* part) {
+                                              double (*red)[kRhoPW][4], double (*coef)[kRhoPW][4], double* part,
+                                              double* __restrict__ tgrad = nullptr) {
     static_assert(NW == 4 || NW == 8, "four or eight wavefronts per block");
     const int tid = 64 * wv + l, rt = wv & 3, gw = g0 + kRhoPW * rt;
     double contrib = 0.0;
@@ -104,7 +107,7 @@ __device__ __forceinline__ void xc_point_tail(int G, int nbf, int wv, int l, int
             const double grx = 2.0 * red[rt][l][1], gry = 2.0 * red[rt][l][2], grz = 2.0 * red[rt][l][3];
             double exc, vrho, vsig;
             xc_b3lyp(rho, grx * grx + gry * gry + grz * grz, exc, vrho, vsig);
-            const double wg = w[g], f4 = 4.0 * wg * vsig;
+            const double wg = w[g], f4 = (tgrad ? 2.0 : 4.0) * wg * vsig;
             c0 = wg * vrho;
             c1 = f4 * grx;
             c2 = f4 * gry;
@@ -115,6 +118,11 @@ __device__ __forceinline__ void xc_point_tail(int G, int nbf, int wv, int l, int
         coef[rt][l][1] = c1;
         coef[rt][l][2] = c2;
         coef[rt][l][3] = c3;
+        if (tgrad) {
+            tgrad[3 * (size_t)g] = c1;
+            tgrad[3 * (size_t)g + 1] = c2;
+            tgrad[3 * (size_t)g + 2] = c3;
+        }
     }
     __syncthreads();
     // aow = w vrho Phi + 4 w vsigma (grad rho . grad Phi), row by row of the wavefront's points
@@ -142,6 +150,7 @@ __device__ __forceinline__ void xc_point_tail(int G, int nbf, int wv, int l, int
             }
         }
     }
+    if (tgrad) return;
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) contrib += __shfl_xor(contrib, off, 64);
     if (l == 0 && wv < 4) part[wv] = contrib;
@@ -546,10 +555,14 @@ hipError_t launch_to_f32(const double* in, float* out, size_t n, hipStream_t st)
 // Bound by memory: Phi for the product, Phi and grad Phi for the reduction and again for the aow rows.
 // (H2O)16, 1.05e6 points: density kernel 6.98 ms dense, 2.50 ms packed; V 3.67 -> 0.98 ms (three widths),
 // summing the partial V 0.05 -> 0.20 ms; benzene, 1.3e5 points: 0.29 -> 0.22 and 0.18 -> 0.13 ms.
+// The gradient uses it twice: kPackedGrad stores X, the gradient's rows and t as well, kPackedProduct only
+// the product `out` = `in` D.
 constexpr int kPackedPrefNH = 6;
-template <int NH>
+enum { kPackedBuild, kPackedGrad, kPackedProduct };
+template <int NH, int MODE>
 __global__ __launch_bounds__(512) QCG_XC_RHO_ATTR void xc_rho_packed_kernel(
-    const PackedGrid g, const double* __restrict__ Dm, double* __restrict__ aow, double* __restrict__ exc_sum) {
+    const PackedGrid g, const double* __restrict__ in, const double* __restrict__ Dm, double* __restrict__ out,
+    double* __restrict__ aow, double* __restrict__ exc_sum) {
     using M = Mfma<double>;
     using acc_t = typename M::acc;
     constexpr int BN = 32 * NH, SA = kRhoBM + 16, SB = BN + lds_pad<double>(BN);
@@ -565,7 +578,7 @@ __global__ __launch_bounds__(512) QCG_XC_RHO_ATTR void xc_rho_packed_kernel(
     const int rt = wv & 3, half = wv >> 2, t0 = half * nh, mine = half ? nt - nh : nh;
     const size_t base = (size_t)g.off[b] + (size_t)p0 * ld;
     const int* fl = g.fl + g.floff[b];
-    const double* __restrict__ phi = g.phi + base;
+    const double* __restrict__ phi = in + base;
     acc_t acc[NH];
 #pragma unroll
     for (int t = 0; t < NH; ++t) acc[t] = acc_t{0.0, 0.0, 0.0, 0.0};
@@ -610,6 +623,15 @@ __global__ __launch_bounds__(512) QCG_XC_RHO_ATTR void xc_rho_packed_kernel(
             for (int t = 0; t < NH; ++t)
                 if (t < mine) acc[t] = M::mma(a, Bs[ks + lk][16 * (t0 + t) + li], acc[t]);
         }
+    }
+    if constexpr (MODE != kPackedBuild) {
+#pragma unroll
+        for (int t = 0; t < NH; ++t)
+            if (t < mine)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    out[base + (size_t)(kRhoPW * rt + M::row(lk, r)) * ld + 16 * (t0 + t) + li] = acc[t][r];
+        if constexpr (MODE == kPackedProduct) return;
     }
     double rs[4] = {}, xs[4] = {}, ys[4] = {}, zs[4] = {};
     const GridVals<double> gv{g.phi + base, g.dpx + base, g.dpy + base, g.dpz + base, nullptr};
@@ -661,7 +683,31 @@ __global__ __launch_bounds__(512) QCG_XC_RHO_ATTR void xc_rho_packed_kernel(
     }
     __syncthreads();
     xc_point_tail<double, 8, (NH + 1) / 2>(kRhoBM, ld, wv, l, 0, g.w + (size_t)b * g.S + p0, gv, aow + base, exc_sum, red,
-                                           coef, part);
+                                           coef, part, MODE == kPackedGrad ? exc_sum + 3 * ((size_t)b * g.S + p0) : nullptr);
+}
+
+// in D for every block (or the whole XC build / gradient step, MODE)
+template <int MODE>
+static hipError_t launch_packed_rows(const PackedGrid& g, const double* in, const double* D, double* out, double* aow,
+                                     double* sum, hipStream_t st) {
+    const dim3 grid((unsigned)(g.nblk * (g.S / kRhoBM)));
+    switch ((g.max_ld / 16 + 1) / 2) {
+#define QCG_RHO_PACKED(n)                                                                                       \
+    case n:                                                                                                     \
+        hipLaunchKernelGGL((xc_rho_packed_kernel<n, MODE>), grid, dim3(512), 0, st, g, in, D, out, aow, sum);   \
+        break;
+        QCG_RHO_PACKED(1) QCG_RHO_PACKED(2) QCG_RHO_PACKED(3) QCG_RHO_PACKED(4) QCG_RHO_PACKED(5) QCG_RHO_PACKED(6)
+        QCG_RHO_PACKED(7) QCG_RHO_PACKED(8) QCG_RHO_PACKED(9) QCG_RHO_PACKED(10) QCG_RHO_PACKED(11)
+#undef QCG_RHO_PACKED
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_packed_grad_rows(const PackedGrid& g, const double* D, double* X, double* aow, double* M, double* t,
+                                   hipStream_t st) {
+    const hipError_t e = launch_packed_rows<kPackedGrad>(g, g.phi, D, X, aow, t, st);
+    return e != hipSuccess ? e : launch_packed_rows<kPackedProduct>(g, aow, D, M, nullptr, nullptr, st);
 }
 
 // Partial V of one block: Phi^T aow over its S points by 32 VW square output tiles (xc_v_kernel's
@@ -769,18 +815,7 @@ int packed_v_width(int ld) { return xc_v_width(ld, false); }
 
 hipError_t launch_xc_packed(const PackedGrid& g, const double* D, double* aow, const int4* tiles, const int ntile[3],
                             double* Vparts, double* Vsum, double* V, double* exc_sum, hipStream_t st) {
-    const dim3 grid((unsigned)(g.nblk * (g.S / kRhoBM)));
-    switch ((g.max_ld / 16 + 1) / 2) {
-#define QCG_RHO_PACKED(n)                                                                                    \
-    case n:                                                                                                  \
-        hipLaunchKernelGGL((xc_rho_packed_kernel<n>), grid, dim3(512), 0, st, g, D, aow, exc_sum);           \
-        break;
-        QCG_RHO_PACKED(1) QCG_RHO_PACKED(2) QCG_RHO_PACKED(3) QCG_RHO_PACKED(4) QCG_RHO_PACKED(5) QCG_RHO_PACKED(6)
-        QCG_RHO_PACKED(7) QCG_RHO_PACKED(8) QCG_RHO_PACKED(9) QCG_RHO_PACKED(10) QCG_RHO_PACKED(11)
-#undef QCG_RHO_PACKED
-        default: return hipErrorInvalidValue;
-    }
-    hipError_t e = hipGetLastError();
+    hipError_t e = launch_packed_rows<kPackedBuild>(g, g.phi, D, nullptr, aow, exc_sum, st);
     if (e != hipSuccess) return e;
     const int4* t = tiles;
     for (int w = 3; w <= 5; t += ntile[w - 3], ++w) {

@@ -50,6 +50,11 @@ hipError_t launch_packed_basis(const PackedGrid& g, int nshell, const GridShell*
 constexpr int kPackedVGroups = 32;
 hipError_t launch_xc_packed(const PackedGrid& g, const double* D, double* aow, const int4* tiles, const int ntile[3],
                             double* Vparts, double* Vsum, double* V, double* exc_sum, hipStream_t st);
+// The XC nuclear gradient at density D, added into grad (natom x 3): X, M (packed work arrays), t (3 per
+// row), A rows in aow.  shcol as for launch_packed_basis.
+hipError_t launch_xc_grad_packed(const PackedGrid& g, int nshell, int natom, const GridShell* shells, const double* exps,
+                                 const double* cn, const short* shcol, const double* D, double* X, double* aow, double* M,
+                                 double* t, double* grad, hipStream_t st);
 // Output tile width of a block of ld functions, in MFMA tiles per wavefront and dimension (3, 4 or 5)
 int packed_v_width(int ld);
 

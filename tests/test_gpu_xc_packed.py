@@ -66,3 +66,18 @@ def test_gpu_packed_follows_the_options():
     eng.set_options("mixed")
     V2, _ = eng.xc(D)
     assert np.array_equal(V2, Vm)
+
+
+@pytest.mark.parametrize("n", [1, 65, 3000])
+def test_gpu_packed_xc_gradient(n):
+    """The XC gradient on the packed grid against the oracle's; the sums run over the same products as V
+    times basis derivatives below 1e2: 1e-8."""
+    b = bench_molecule("H2O", "6-31g*")
+    xyz, w = _points(b, n, n, 1.5)
+    D = random_density(b.nbf, seed=9, nocc=b.n_occ)
+    for prec in ("fp64", "mixed"):  # the gradient is FP64 in both
+        eng = Engine(b, precision=prec)
+        eng.set_grid(xyz, w)
+        g = eng.xc_gradient(D)
+        assert np.abs(g - oracle.xc_gradient(b, xyz, w, D)).max() < 1e-8
+        assert np.array_equal(eng.xc_gradient(D).shape, (b.natom, 3))
