@@ -56,18 +56,24 @@ int upload_basis(qcg_context* c, const HostBasis& B, int** di, double** dd, Basi
 
 }  // namespace
 
-// Device basis and (ordered shell pair, primitive pair) work list of the gradient kernel, made once
+// Device basis and (shell pair, primitive pair) work list of the gradient kernel, made once
 // per basis.
 int onee_setup(qcg_context* c) {
     if (c->d_onee_work) return QCG_OK;
     const HostBasis& B = c->basis;
     int rc = upload_basis(c, B, &c->d_onee_int, &c->d_onee_dbl, &c->onee_view);
     if (rc) return rc;
-    std::vector<int4> work;
+    std::vector<int4> work, by[kNumPairClasses];
     for (int si = 0; si < B.nshell; ++si)
-        for (int sj = 0; sj < B.nshell; ++sj)
-            for (int pi = 0; pi < B.nprim[si]; ++pi)
-                for (int pj = 0; pj < B.nprim[sj]; ++pj) work.push_back(make_int4(si, sj, pi, pj));
+        for (int sj = 0; sj <= si; ++sj) {
+            const int a = B.l[si] >= B.l[sj] ? si : sj, b = B.l[si] >= B.l[sj] ? sj : si;
+            for (int pi = 0; pi < B.nprim[a]; ++pi)
+                for (int pj = 0; pj < B.nprim[b]; ++pj) by[pair_class(B.l[a], B.l[b])].push_back(make_int4(a, b, pi, pj));
+        }
+    for (auto& v : by) {
+        v.resize((v.size() + kOneeBlock - 1) / kOneeBlock * kOneeBlock, make_int4(-1, -1, 0, 0));
+        work.insert(work.end(), v.begin(), v.end());
+    }
     HIPCHK(c, c->alloc(&c->d_onee_work, work.size()));
     HIPCHK(c, hipMemcpy(c->d_onee_work, work.data(), work.size() * sizeof(int4), hipMemcpyHostToDevice));
     c->onee_nwork = (int)work.size();

@@ -4,7 +4,10 @@
 
 namespace qcg {
 
-// work[u] = (si, sj, pi, pj): one ordered shell pair and one of its primitive pairs per entry; the
+constexpr int kOneeBlock = 128;  // threads per block of the gradient kernel
+
+// work[u] = (si, sj, pi, pj), l(si) >= l(sj): one shell pair and one of its primitive pairs per entry, the
+// entries of one pair class after the other, each padded to a multiple of kOneeBlock with si = -1; the
 // terms are ADDED into grad (natom x 3, device).  D, W: nbf x nbf on the device.
 // work[u] = (si, sj, ia, jb), si <= sj: one Cartesian component pair per entry; S, T, V (nbf x nbf,
 // device) receive every element of the listed shell pairs and of their mirror images.

@@ -1,14 +1,14 @@
-// One-electron gradient terms of one primitive pair, shared by the host loop (onee.cpp) and the
-// device kernel (onee_kernels.hip): the same operations in the same order on both sides.
+// One-electron integrals and gradient terms of one primitive pair (onee_kernels.hip).
 //
-// sum_ab D_ab dH_ab/dR - W_ab dS_ab/dR, H = T + V, for the primitive pair (pi, pj) of the ordered
-// shell pair (si, sj) (overlap_derivative_matrix, scf/gradient.rs:188, and hcore_derivative_matrix
+// sum_ab D_ab dH_ab/dR - W_ab dS_ab/dR, H = T + V, for the primitive pair (pi, pj) of the shell pair
+// (si, sj) (overlap_derivative_matrix, scf/gradient.rs:188, and hcore_derivative_matrix
 // :355, contracted as in rhf_gradient :930-950).  Basis-function derivatives:
 // d/dA_x phi_i = 2 alpha phi_(i+1) - i phi_(i-1); for V the operator centre C gets -(dA + dB) by
 // translational invariance of each three-centre integral.
 #pragma once
 #include <cmath>
 
+#include "eri_device.h"
 #include "qcg_common.h"
 #include "rys.h"
 
@@ -102,115 +102,137 @@ QCG_HD OneePair onee_pair_setup(const BasisView& B, int si, int sj, int pi, int 
     return q;
 }
 
-// Overlap and kinetic terms of the primitive pair (pi, pj) of the ordered shell pair (si, sj);
-// add(atom, axis, value) accumulates a gradient contribution.
-template <typename Add>
-QCG_HD void onee_grad_overlap_kinetic(const BasisView& B, int si, int sj, int pi, int pj, const double* D,
-                                      const double* W, Add&& add) {
-    constexpr int LD = kMaxL + 4;
-    const OneePair q = onee_pair_setup(B, si, sj, pi, pj);
-    const double a = q.a, b = q.b;
-    double s1[3][LD * LD];
-    for (int x = 0; x < 3; ++x) onee_overlap_1d(q.PA[x], q.PB[x], q.oo2p, q.la + 2, q.lb + 2, s1[x], LD);
-    auto sv = [&](int x, int i, int j) { return (i < 0 || j < 0) ? 0.0 : s1[x][i * LD + j]; };
-    auto tv = [&](int x, int i, int j) {
-        if (i < 0 || j < 0) return 0.0;
-        double v = 4.0 * a * b * sv(x, i + 1, j + 1);
-        if (i > 0) v -= 2.0 * b * i * sv(x, i - 1, j + 1);
-        if (j > 0) v -= 2.0 * a * j * sv(x, i + 1, j - 1);
-        if (i > 0 && j > 0) v += (double)(i * j) * sv(x, i - 1, j - 1);
-        return 0.5 * v;
-    };
-    const double pre = q.kab * pow(kPi / q.p, 1.5) * q.ca * q.cb;
-    double gA0[3] = {0, 0, 0}, gB0[3] = {0, 0, 0};
-    for (int ia = 0; ia < q.na; ++ia)
-        for (int jb = 0; jb < q.nb; ++jb) {
-            const int ip[3] = {cart_x(q.la, ia), cart_y(q.la, ia), cart_z(q.la, ia)};
-            const int jp[3] = {cart_x(q.lb, jb), cart_y(q.lb, jb), cart_z(q.lb, jb)};
-            const size_t idx = (size_t)(q.bfa + ia) * B.nbf + q.bfb + jb;
-            const double dv = D[idx], wv = W[idx];
-            if (dv == 0.0 && wv == 0.0) continue;
-            const double nrm = onee_norm_comp(q.la, ia) * onee_norm_comp(q.lb, jb);
-            for (int x = 0; x < 3; ++x) {
-                const int y = (x + 1) % 3, z = (x + 2) % 3;
-                const double sy = sv(y, ip[y], jp[y]), sz = sv(z, ip[z], jp[z]);
-                const double ty = tv(y, ip[y], jp[y]), tz = tv(z, ip[z], jp[z]);
-                // derivative with respect to A_x and B_x of S and T
-                const double dsA = 2.0 * a * sv(x, ip[x] + 1, jp[x]) - ip[x] * sv(x, ip[x] - 1, jp[x]);
-                const double dsB = 2.0 * b * sv(x, ip[x], jp[x] + 1) - jp[x] * sv(x, ip[x], jp[x] - 1);
-                const double dtA = 2.0 * a * tv(x, ip[x] + 1, jp[x]) - ip[x] * tv(x, ip[x] - 1, jp[x]);
-                const double dtB = 2.0 * b * tv(x, ip[x], jp[x] + 1) - jp[x] * tv(x, ip[x], jp[x] - 1);
-                const double SA = dsA * sy * sz, SB = dsB * sy * sz;
-                const double TA = dtA * sy * sz + dsA * (ty * sz + sy * tz);
-                const double TB = dtB * sy * sz + dsB * (ty * sz + sy * tz);
-                gA0[x] += pre * nrm * (dv * TA - wv * SA);
-                gB0[x] += pre * nrm * (dv * TB - wv * SB);
-            }
-        }
-    for (int x = 0; x < 3; ++x) {
-        add(q.atA, x, gA0[x]);
-        add(q.atB, x, gB0[x]);
-    }
+// Density element (or sum of the mirrored ones) of a component pair of the unordered shell pair.
+QCG_HD double onee_weight(const double* M, int nbf, int i, int j, bool mirror) {
+    const double v = M[(size_t)i * nbf + j];
+    return mirror ? v + M[(size_t)j * nbf + i] : v;
 }
 
-// Nuclear attraction terms of nucleus cnuc for the primitive pair: one Rys rule and one set of 1-D
-// tables (with one extra power on each side), shared by all component pairs.
-template <typename Add>
-QCG_HD void onee_grad_nuclear(const BasisView& B, int si, int sj, int pi, int pj, int cnuc, const double* D,
-                              const double* rys_tab, Add&& add) {
-    constexpr int LV = kMaxL + 2;                 // table dimension for i, j <= l + 1
-    constexpr int kNr = (2 * kMaxL + 1) / 2 + 1;  // nodes for la = lb = kMaxL
+// Overlap and kinetic terms of the primitive pair (pi, pj) of the shell pair (si, sj) of angular momenta
+// LA, LB; mirror: the pair stands for (sj, si) too.  gA, gB: the derivative sums of the two centres.
+template <int LA, int LB>
+QCG_HD void onee_grad_overlap_kinetic(const BasisView& B, int si, int sj, int pi, int pj, bool mirror, const double* D,
+                                      const double* W, double* gA, double* gB) {
+    constexpr int NB = ncart(LB), NQ = ncart(LA) * NB, LD = LB + 3;
     const OneePair q = onee_pair_setup(B, si, sj, pi, pj);
     const double a = q.a, b = q.b;
-    const int nr = (q.la + q.lb + 1) / 2 + 1;
-    const int nmax = q.la + q.lb + 2;
+    // per axis S(i, j), i <= LA + 2, j <= LB + 2, and T(i, j), i <= LA + 1, j <= LB + 1
+    double s[3][(LA + 3) * LD], t[3][(LA + 2) * LD];
+#pragma unroll
+    for (int x = 0; x < 3; ++x) {
+        double* sx = s[x];
+        sx[0] = 1.0;
+        static_for<(LA + 3) * LD - 1>([&](auto ec) {
+            constexpr int e = decltype(ec)::value + 1, i = e / LD, j = e % LD;
+            double v;
+            if constexpr (i > 0) {
+                v = q.PA[x] * sx[e - LD];
+                if constexpr (i > 1) v += (i - 1) * q.oo2p * sx[e - 2 * LD];
+                if constexpr (j > 0) v += j * q.oo2p * sx[e - LD - 1];
+            } else {
+                v = q.PB[x] * sx[e - 1];
+                if constexpr (j > 1) v += (j - 1) * q.oo2p * sx[e - 2];
+            }
+            sx[e] = v;
+        });
+        static_for<(LA + 2) * (LB + 2)>([&](auto ec) {
+            constexpr int i = decltype(ec)::value / (LB + 2), j = decltype(ec)::value % (LB + 2), e = i * LD + j;
+            double v = 4.0 * a * b * sx[e + LD + 1];
+            if constexpr (i > 0) v -= 2.0 * b * i * sx[e - LD + 1];
+            if constexpr (j > 0) v -= 2.0 * a * j * sx[e + LD - 1];
+            if constexpr (i > 0 && j > 0) v += (double)(i * j) * sx[e - LD - 1];
+            t[x][e] = 0.5 * v;
+        });
+    }
+    const double pre = q.kab * (kPi / q.p) * sqrt(kPi / q.p) * q.ca * q.cb;
+    static_for<NQ>([&](auto kc) {
+        constexpr int k = decltype(kc)::value, ca = k / NB, cb = k % NB;
+        constexpr int ip[3] = {cart_x(LA, ca), cart_y(LA, ca), cart_z(LA, ca)};
+        constexpr int jp[3] = {cart_x(LB, cb), cart_y(LB, cb), cart_z(LB, cb)};
+        constexpr int e[3] = {ip[0] * LD + jp[0], ip[1] * LD + jp[1], ip[2] * LD + jp[2]};
+        const double nrm = pre * cnorm(LA, ca) * cnorm(LB, cb);
+        const double dv = nrm * onee_weight(D, B.nbf, q.bfa + ca, q.bfb + cb, mirror);
+        const double wv = nrm * onee_weight(W, B.nbf, q.bfa + ca, q.bfb + cb, mirror);
+        static_for<3>([&](auto xc) {
+            constexpr int x = decltype(xc)::value, y = (x + 1) % 3, z = (x + 2) % 3;
+            const double sy = s[y][e[y]], sz = s[z][e[z]], syz = sy * sz, tyz = t[y][e[y]] * sz + sy * t[z][e[z]];
+            // derivative with respect to A_x and B_x of S and T
+            double dsA = 2.0 * a * s[x][e[x] + LD], dsB = 2.0 * b * s[x][e[x] + 1];
+            double dtA = 2.0 * a * t[x][e[x] + LD], dtB = 2.0 * b * t[x][e[x] + 1];
+            if constexpr (ip[x] > 0) {
+                dsA -= ip[x] * s[x][e[x] - LD];
+                dtA -= ip[x] * t[x][e[x] - LD];
+            }
+            if constexpr (jp[x] > 0) {
+                dsB -= jp[x] * s[x][e[x] - 1];
+                dtB -= jp[x] * t[x][e[x] - 1];
+            }
+            gA[x] += dv * (dtA * syz + dsA * tyz) - wv * dsA * syz;
+            gB[x] += dv * (dtB * syz + dsB * tyz) - wv * dsB * syz;
+        });
+    });
+}
+
+// Nuclear attraction terms of nucleus cnuc for the primitive pair (pi, pj) of the shell pair (si, sj) of
+// angular momenta LA, LB; mirror: the pair stands for (sj, si) too.  gA, gB: the derivative sums of the
+// two centres.  One Rys node at a time, everything in registers: per axis the 1-D factors I(i, j) for
+// i <= LA + 1, j <= LB, and I(i, j+1) = I(i+1, j) + AB I(i, j).
+template <int LA, int LB>
+QCG_HD void onee_grad_nuclear(const BasisView& B, int si, int sj, int pi, int pj, int cnuc, bool mirror,
+                              const double* D, const double* rys_tab, double* gA, double* gB) {
+    constexpr int N = (LA + LB + 1) / 2 + 1, NB = ncart(LB), NQ = ncart(LA) * NB, NM = LA + LB + 1;
+    const OneePair q = onee_pair_setup(B, si, sj, pi, pj);
     const double* C = &B.xyz[3 * cnuc];
     const double PC[3] = {q.P[0] - C[0], q.P[1] - C[1], q.P[2] - C[2]};
-    const double Tn = q.p * (PC[0] * PC[0] + PC[1] * PC[1] + PC[2] * PC[2]);
-    double rx[QCG_RYS_NMAX], rw[QCG_RYS_NMAX];
-    onee_rys(nr, Tn, rys_tab, rx, rw);
-    double g[kNr][3][LV * LV];
-    for (int r = 0; r < nr; ++r) {
-        const double u = rx[r];
-        for (int x = 0; x < 3; ++x) {
-            double h[2 * kMaxL + 3];
-            const double c0 = q.PA[x] - u * PC[x];
-            const double bb = (1.0 - u) * q.oo2p;
-            h[0] = 1.0;
-            if (nmax > 0) h[1] = c0;
-            for (int n = 1; n < nmax; ++n) h[n + 1] = c0 * h[n] + n * bb * h[n - 1];
-            double t2[(2 * kMaxL + 3) * LV];
-            for (int n = 0; n <= nmax; ++n) t2[n * LV] = h[n];
-            for (int j = 1; j <= q.lb + 1; ++j)
-                for (int n = 0; n + j <= nmax; ++n)
-                    t2[n * LV + j] = t2[(n + 1) * LV + j - 1] + q.AB[x] * t2[n * LV + j - 1];
-            for (int i = 0; i <= q.la + 1; ++i)
-                for (int j = 0; j <= q.lb + 1; ++j) g[r][x][i * LV + j] = (i + j <= nmax) ? t2[i * LV + j] : 0.0;
-        }
-    }
+    double rx[N], rw[N];
+    rys_eval<double, N>(q.p * (PC[0] * PC[0] + PC[1] * PC[1] + PC[2] * PC[2]), rys_tab, rx, rw);
     const double pz = -(double)B.Z[cnuc] * 2.0 * kPi / q.p * q.kab * q.ca * q.cb;
-    double gA[3] = {0, 0, 0}, gB[3] = {0, 0, 0};
-    for (int ia = 0; ia < q.na; ++ia)
-        for (int jb = 0; jb < q.nb; ++jb) {
-            const double dv = D[(size_t)(q.bfa + ia) * B.nbf + q.bfb + jb];
-            if (dv == 0.0) continue;
-            const int ip[3] = {cart_x(q.la, ia), cart_y(q.la, ia), cart_z(q.la, ia)};
-            const int jp[3] = {cart_x(q.lb, jb), cart_y(q.lb, jb), cart_z(q.lb, jb)};
-            const double pv = pz * onee_norm_comp(q.la, ia) * onee_norm_comp(q.lb, jb) * dv;
-            for (int r = 0; r < nr; ++r) {
-                auto gv = [&](int x, int i, int j) { return (i < 0 || j < 0) ? 0.0 : g[r][x][i * LV + j]; };
-                for (int x = 0; x < 3; ++x) {
-                    const int y = (x + 1) % 3, z = (x + 2) % 3;
-                    const double oth = rw[r] * pv * gv(y, ip[y], jp[y]) * gv(z, ip[z], jp[z]);
-                    gA[x] += oth * (2.0 * a * gv(x, ip[x] + 1, jp[x]) - ip[x] * gv(x, ip[x] - 1, jp[x]));
-                    gB[x] += oth * (2.0 * b * gv(x, ip[x], jp[x] + 1) - jp[x] * gv(x, ip[x], jp[x] - 1));
+    double W[NQ];
+    static_for<NQ>([&](auto kc) {
+        constexpr int k = decltype(kc)::value, a = k / NB, b = k % NB;
+        W[k] = pz * cnorm(LA, a) * cnorm(LB, b) * onee_weight(D, B.nbf, q.bfa + a, q.bfb + b, mirror);
+    });
+    const double two_a = 2.0 * q.a, two_b = 2.0 * q.b;
+#pragma unroll
+    for (int r = 0; r < N; ++r) {
+        const double u = rx[r], bb = (1.0 - u) * q.oo2p;
+        double I[3][(LA + 2) * (LB + 1)];
+#pragma unroll
+        for (int x = 0; x < 3; ++x) {
+            double h[NM + 1], t[NM + 1];
+            const double c0 = q.PA[x] - u * PC[x];
+            h[0] = 1.0;
+            h[1] = c0;
+#pragma unroll
+            for (int n = 1; n < NM; ++n) h[n + 1] = c0 * h[n] + n * bb * h[n - 1];
+#pragma unroll
+            for (int j = 0; j <= LB; ++j) {
+#pragma unroll
+                for (int n = 0; n + j <= NM; ++n) {
+                    t[n] = j == 0 ? h[n] : h[n + 1] + q.AB[x] * h[n];
+                    if (n <= LA + 1) I[x][n * (LB + 1) + j] = t[n];
                 }
+#pragma unroll
+                for (int n = 0; n + j <= NM; ++n) h[n] = t[n];
             }
         }
-    for (int x = 0; x < 3; ++x) {
-        add(q.atA, x, gA[x]);
-        add(q.atB, x, gB[x]);
-        add(cnuc, x, -(gA[x] + gB[x]));
+        static_for<NQ>([&](auto kc) {
+            constexpr int k = decltype(kc)::value, a = k / NB, b = k % NB;
+            constexpr int ip[3] = {cart_x(LA, a), cart_y(LA, a), cart_z(LA, a)};
+            constexpr int jp[3] = {cart_x(LB, b), cart_y(LB, b), cart_z(LB, b)};
+            constexpr int e[3] = {ip[0] * (LB + 1) + jp[0], ip[1] * (LB + 1) + jp[1], ip[2] * (LB + 1) + jp[2]};
+            const double w = rw[r] * W[k];
+            static_for<3>([&](auto xc) {
+                constexpr int x = decltype(xc)::value, y = (x + 1) % 3, z = (x + 2) % 3;
+                const double oth = w * (I[y][e[y]] * I[z][e[z]]);
+                const double up = I[x][e[x] + LB + 1];
+                double dA = two_a * up, dB = two_b * (up + q.AB[x] * I[x][e[x]]);
+                if constexpr (ip[x] > 0) dA -= ip[x] * I[x][e[x] - (LB + 1)];
+                if constexpr (jp[x] > 0) dB -= jp[x] * I[x][e[x] - 1];
+                gA[x] += oth * dA;
+                gB[x] += oth * dB;
+            });
+        });
     }
 }
 
