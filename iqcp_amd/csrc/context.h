@@ -108,6 +108,7 @@ struct qcg_context {
     Tile tile[21][2];  // per quartet class and precision part (0 FP64, 1 FP32)
     bool tiles_set = false;  // set or tuned by the caller; else chosen with the work plan (default_tiles)
     int class_nq[21] = {};  // Cartesian components per quartet class
+    int class_nas[21] = {};  // components of the first shell per launch of its per-lane kernel (jk_part)
     // mixed precision, per class: run its FP64 and FP32 items in one launch (jk_*_mp kernels, with
     // the FP64 part's tile) or in two; qcg_autotune_refine may split a class
     bool fuse_cls[21] = {true, true, true, true, true, true, true, true, true, true, true,

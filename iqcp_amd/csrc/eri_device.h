@@ -165,19 +165,20 @@ QCG_HD void for_n(F&& body) {
 // (P.npp of them, from index 0), ppk: ppk(j) is the ket's primitive pair j (Q.npp of them).
 // TAB_N: rys_tab already points at the coefficients of this class's Rys order (e.g. a copy
 // staged in LDS).  j0, js: the ket primitives taken, j0, j0 + js, ... (0, 1: all of them).
-template <int LA, int LB, int LC, int LD, typename R, bool TAB_N = false, typename Ket>
+// K0, NK: the components K0 .. K0 + NK - 1 only (NK = 0: all), in eri[0 .. NK).
+template <int LA, int LB, int LC, int LD, typename R, bool TAB_N = false, int K0 = 0, int NK = 0, typename Ket>
 QCG_HD void contract_quartet_pp(const PairRec& P, const PairRec& Q, const PrimPair<R>* __restrict__ ppb, Ket&& ppk,
                                 const R* __restrict__ rys_tab, R* eri, int j0 = 0, int js = 1) {
     using S = EriShape<LA, LB, LC, LD>;
-    constexpr int N = S::NROOTS;
+    constexpr int N = S::NROOTS, NQ = NK ? NK : S::NQ;
     const R abx = (R)P.abx, aby = (R)P.aby, abz = (R)P.abz;
     const R cdx = (R)Q.abx, cdy = (R)Q.aby, cdz = (R)Q.abz;
     const R Ax = (R)P.ax, Ay = (R)P.ay, Az = (R)P.az;
     const R Cx = (R)Q.ax, Cy = (R)Q.ay, Cz = (R)Q.az;
     const R two_pi_52 = (R)(2.0 * kPi * kPi * 1.7724538509055160273);
+    const R* __restrict__ tab = TAB_N ? rys_tab : rys_tab + qcg_rys_off[N];
     // ket primitives outer: in the J/K kernels the bra pair is uniform over the block, so the inner
-    // loop's bra primitive reads are uniform (an LDS broadcast) and each lane loads its ket
-    // primitive once
+    // loop's bra primitive reads are uniform (scalar loads) and each lane loads its ket primitive once
     for (int j = j0; j < Q.npp; j += js) {
         const PrimPair<R> c = ppk(j);
         const R q = c.p;
@@ -198,11 +199,10 @@ QCG_HD void contract_quartet_pp(const PairRec& P, const PairRec& Q, const PrimPa
             const R rho = p * q * ipq;
             const R T = rho * (PQx * PQx + PQy * PQy + PQz * PQz);
             const R pref = two_pi_52 * rs * a.ckp * c.ckp * keep;
-            R rx[N], rw[N];
-            if constexpr (TAB_N) rys_eval_tab<R, N>(T, rys_tab, rx, rw);
-            else rys_eval<R, N>(T, rys_tab, rx, rw);
             const R qf = q * ipq, pf = p * ipq;
             const R PAx = a.px - Ax, PAy = a.py - Ay, PAz = a.pz - Az;
+            R rx[N], rw[N];
+            rys_eval_tab<R, N>(T, tab, rx, rw);
 #pragma unroll
             for (int r = 0; r < N; ++r) {
                 const R u = rx[r];
@@ -221,12 +221,12 @@ QCG_HD void contract_quartet_pp(const PairRec& P, const PairRec& Q, const PrimPa
                 const R wp = rw[r] * pref;
 #pragma unroll
                 for (int h = 0; h < S::H4; ++h) iz[h] *= wp;
-                if constexpr (S::kUnroll) {
-                    static_for<S::NQ>([&](auto kc) {
+                if constexpr (NK > 0 || S::kUnroll) {
+                    static_for<NQ>([&](auto kc) {
                         constexpr int k = decltype(kc)::value;
-                        constexpr int hx = kCompTab<LA, LB, LC, LD>.hx[k];
-                        constexpr int hy = kCompTab<LA, LB, LC, LD>.hy[k];
-                        constexpr int hz = kCompTab<LA, LB, LC, LD>.hz[k];
+                        constexpr int hx = kCompTab<LA, LB, LC, LD>.hx[K0 + k];
+                        constexpr int hy = kCompTab<LA, LB, LC, LD>.hy[K0 + k];
+                        constexpr int hz = kCompTab<LA, LB, LC, LD>.hz[K0 + k];
                         eri[k] += ix[hx] * iy[hy] * iz[hz];
                     });
                 } else {

@@ -13,11 +13,12 @@
 //   * the host cuts every range into work items (bra pair, ket sub-range) of a per-class size;
 //     one block per item, one thread per ket (several for cheap classes), so every class
 //     launch has many more blocks than the GPU has CUs;
-//   * digestion: J_P in registers + wave reduction; J_Q by FP64 atomics; the four K terms all
-//     land in the rows of the bra functions, so they are summed in LDS rows (one block = one bra
-//     pair) and flushed with one global atomic per touched element at the end of the block (device
-//     atomics are performed memory-side on this GPU, so every global atomic is HBM write
-//     traffic).  J = Jacc + Jacc^T, K = Kacc + Kacc^T after.
+//   * digestion: J_P in registers + wave reduction; J_Q by fixed-point atomics on arrays ordered by
+//     ket pair, so a wavefront's adds are consecutive; the four K terms all land in the rows of the
+//     bra functions, so they are summed in LDS rows (one block = one bra pair) and flushed with one
+//     global atomic per touched element at the end of the block (device atomics are performed
+//     memory-side on this GPU, so every global atomic is HBM write traffic).  J is gathered from the
+//     pair-ordered sums, K = Kacc + Kacc^T after.
 //   * symmetry factors: 1/2 for a == b shells, 1/2 for c == d shells, 1/2 for P == Q, folded
 //     together with the component normalisation into the density sub-blocks.
 // With the symmetric density this reproduces build_fock's G = J - K/2 (scf/mod.rs:825-881) and
@@ -86,14 +87,15 @@ __device__ __forceinline__ PairRec ket_pair(const KetPairs& k, int kq, const int
 // block.  J and K go to the fixed-point accumulators Jacc (by shell pair) and Kacc with the scales
 // fix[4 mol], fix[4 mol + 1], so the result does not depend on the order in which blocks and lanes
 // arrive.  The bra's primitive pairs are uniform over the block and come through the scalar cache;
-// the D rows of K through the vector caches.
-template <int LA, int LB, int LC, int LD, typename R, bool KROWS>
+// the D rows of K through the vector caches.  A0, NA: the components of the first shell taken (jk_part);
+// J_Q, and the K terms in the rows of b, are sums over the parts, which the accumulators make of them.
+template <int LA, int LB, int LC, int LD, typename R, bool KROWS, int A0, int NA>
 __device__ __forceinline__ void jk_item(const int4 it, const JkArgs& g, const KetPrims<R>& kprims,
                                         const PrimPair<R>* __restrict__ pp, const R* __restrict__ rys_n, double* rows) {
     using S = EriShape<LA, LB, LC, LD>;
-    constexpr bool U = S::kUnroll;
-    constexpr int NR = S::NA + S::NB;
-    const PairRec P = item_bra(g.bra, it);
+    constexpr int NAB = NA * S::NB, NQ = NAB * S::NCD, NR = NA + S::NB;
+    PairRec P = item_bra(g.bra, it);
+    P.bfa += A0;  // the part's components are functions bfa .. bfa + NA - 1 from here on
     const int pidx = P.pos, ket0 = g.ket_off[P.mol];
     const double* __restrict__ D = g.D + g.mat_off[P.mol];
     fix_t* __restrict__ Jacc = g.Jacc;
@@ -110,15 +112,15 @@ __device__ __forceinline__ void jk_item(const int4 it, const JkArgs& g, const Ke
     // D element (row function a + r of the bra's shell a, or b + r of shell b; column col)
     auto drow = [&](bool row_b, int r, int col) -> double { return D[(size_t)((row_b ? P.bfb : P.bfa) + r) * nbf + col]; };
     auto kadd = [&](bool row_b, int r, int col, double v) {
-        if constexpr (KROWS) fix_add_lds(kl, (row_b ? S::NA + r : r) * nbf + col, v, sK);
+        if constexpr (KROWS) fix_add_lds(kl, (row_b ? NA + r : r) * nbf + col, v, sK);
         else fix_add_global(Kacc, (size_t)((row_b ? P.bfb : P.bfa) + r) * nbf + col, v, sK);
     };
 
     // bra density block scaled by the bra component norms
-    double Dps[S::NAB], jp[S::NAB];
-    for_n<U, S::NAB>([&](int ab) {
+    double Dps[NAB], jp[NAB];
+    for_n<true, NAB>([&](int ab) {
         const int a = ab / S::NB, b = ab % S::NB;
-        Dps[ab] = drow(false, a, P.bfb + b) * cnorm(LA, a) * cnorm(LB, b);
+        Dps[ab] = drow(false, a, P.bfb + b) * cnorm(LA, A0 + a) * cnorm(LB, b);
         jp[ab] = 0.0;
     });
     const double deg_p = (P.sa == P.sb) ? 0.5 : 1.0;
@@ -133,29 +135,29 @@ __device__ __forceinline__ void jk_item(const int4 it, const JkArgs& g, const Ke
         const int4 km = g.kpairs.meta[kq];
         const PairRec Q = ket_pair<LC, LD>(g.kpairs, kq, km);
         const int kstride = km.w & 0xffffff;
-        R eri[S::NQ];
-        for_n<U, S::NQ>([&](int i) { eri[i] = R(0); });
-        contract_quartet_pp<LA, LB, LC, LD, R, true>(
+        R eri[NQ];
+        for_n<true, NQ>([&](int i) { eri[i] = R(0); });
+        contract_quartet_pp<LA, LB, LC, LD, R, true, A0 * S::NB * S::NCD, NQ>(
             P, Q, ppb, [&](int i) { return kprims.at(km.z + i * kstride); }, rys_n, eri, sub, lanes);
         if (lg) {
             for (int off = 1; off < lanes; off <<= 1)
-                for_n<U, S::NQ>([&](int i) { eri[i] += __shfl_xor(eri[i], off, 64); });
+                for_n<true, NQ>([&](int i) { eri[i] += __shfl_xor(eri[i], off, 64); });
             if (sub) continue;  // the group's first lane digests
         }
         const double deg = deg_p * ((km.x & kKetSame) ? 0.5 : 1.0) * ((g.diag && q == pidx) ? 0.5 : 1.0);
         if (do_j) {
             double Dqs[S::NCD];
-            for_n<U, S::NCD>([&](int cd) { Dqs[cd] = g.Dp[g.jb_ket + cd * g.np_ket + kq]; });
+            for_n<true, S::NCD>([&](int cd) { Dqs[cd] = g.Dp[g.jb_ket + cd * g.np_ket + kq]; });
             const double fj = 2.0 * deg;
-            for_n<U, S::NAB>([&](int ab) {
+            for_n<true, NAB>([&](int ab) {
                 double s = 0.0;
-                for_n<U, S::NCD>([&](int cd) { s += Dqs[cd] * (double)eri[ab * S::NCD + cd]; });
+                for_n<true, S::NCD>([&](int cd) { s += Dqs[cd] * (double)eri[ab * S::NCD + cd]; });
                 const int a = ab / S::NB, b = ab % S::NB;
-                jp[ab] += fj * cnorm(LA, a) * cnorm(LB, b) * s;
+                jp[ab] += fj * cnorm(LA, A0 + a) * cnorm(LB, b) * s;
             });
-            for_n<U, S::NCD>([&](int cd) {
+            for_n<true, S::NCD>([&](int cd) {
                 double s = 0.0;
-                for_n<U, S::NAB>([&](int ab) { s += Dps[ab] * (double)eri[ab * S::NCD + cd]; });
+                for_n<true, NAB>([&](int ab) { s += Dps[ab] * (double)eri[ab * S::NCD + cd]; });
                 const int c = cd / S::ND, d = cd % S::ND;
                 fix_add_global(Jacc, g.jb_ket + cd * g.np_ket + kq, fj * cnorm(LC, c) * cnorm(LD, d) * s, sJ);
             });
@@ -163,55 +165,55 @@ __device__ __forceinline__ void jk_item(const int4 it, const JkArgs& g, const Ke
         if (do_k) {
             // Kacc_ik += D_jl v, Kacc_jk += D_il v, Kacc_il += D_jk v, Kacc_jl += D_ik v
             // (i in a, j in b, k in c, l in d); every D sub-block pre-scaled by the norms it sums over.
-            double Dbd[S::NB * S::ND], Dad[S::NA * S::ND], Dbc[S::NB * S::NC], Dac[S::NA * S::NC];
-            for_n<U, S::NB * S::ND>([&](int i) {
+            double Dbd[S::NB * S::ND], Dad[NA * S::ND], Dbc[S::NB * S::NC], Dac[NA * S::NC];
+            for_n<true, S::NB * S::ND>([&](int i) {
                 const int b = i / S::ND, d = i % S::ND;
                 Dbd[i] = drow(true, b, Q.bfb + d) * cnorm(LB, b) * cnorm(LD, d);
             });
-            for_n<U, S::NA * S::ND>([&](int i) {
+            for_n<true, NA * S::ND>([&](int i) {
                 const int a = i / S::ND, d = i % S::ND;
-                Dad[i] = drow(false, a, Q.bfb + d) * cnorm(LA, a) * cnorm(LD, d);
+                Dad[i] = drow(false, a, Q.bfb + d) * cnorm(LA, A0 + a) * cnorm(LD, d);
             });
-            for_n<U, S::NB * S::NC>([&](int i) {
+            for_n<true, S::NB * S::NC>([&](int i) {
                 const int b = i / S::NC, c = i % S::NC;
                 Dbc[i] = drow(true, b, Q.bfa + c) * cnorm(LB, b) * cnorm(LC, c);
             });
-            for_n<U, S::NA * S::NC>([&](int i) {
+            for_n<true, NA * S::NC>([&](int i) {
                 const int a = i / S::NC, c = i % S::NC;
-                Dac[i] = drow(false, a, Q.bfa + c) * cnorm(LA, a) * cnorm(LC, c);
+                Dac[i] = drow(false, a, Q.bfa + c) * cnorm(LA, A0 + a) * cnorm(LC, c);
             });
 #define VIDX(a, b, c, d) ((((a) * S::NB + (b)) * S::NC + (c)) * S::ND + (d))
-            for_n<U, S::NA * S::NC>([&](int ac) {
+            for_n<true, NA * S::NC>([&](int ac) {
                 const int a = ac / S::NC, c = ac % S::NC;
                 double s = 0.0;
-                for_n<U, S::NB * S::ND>([&](int bd) {
+                for_n<true, S::NB * S::ND>([&](int bd) {
                     const int b = bd / S::ND, d = bd % S::ND;
                     s += Dbd[bd] * (double)eri[VIDX(a, b, c, d)];
                 });
-                kadd(false, a, Q.bfa + c, deg * cnorm(LA, a) * cnorm(LC, c) * s);
+                kadd(false, a, Q.bfa + c, deg * cnorm(LA, A0 + a) * cnorm(LC, c) * s);
             });
-            for_n<U, S::NB * S::NC>([&](int bc) {
+            for_n<true, S::NB * S::NC>([&](int bc) {
                 const int b = bc / S::NC, c = bc % S::NC;
                 double s = 0.0;
-                for_n<U, S::NA * S::ND>([&](int ad) {
+                for_n<true, NA * S::ND>([&](int ad) {
                     const int a = ad / S::ND, d = ad % S::ND;
                     s += Dad[ad] * (double)eri[VIDX(a, b, c, d)];
                 });
                 kadd(true, b, Q.bfa + c, deg * cnorm(LB, b) * cnorm(LC, c) * s);
             });
-            for_n<U, S::NA * S::ND>([&](int ad) {
+            for_n<true, NA * S::ND>([&](int ad) {
                 const int a = ad / S::ND, d = ad % S::ND;
                 double s = 0.0;
-                for_n<U, S::NB * S::NC>([&](int bc) {
+                for_n<true, S::NB * S::NC>([&](int bc) {
                     const int b = bc / S::NC, c = bc % S::NC;
                     s += Dbc[bc] * (double)eri[VIDX(a, b, c, d)];
                 });
-                kadd(false, a, Q.bfb + d, deg * cnorm(LA, a) * cnorm(LD, d) * s);
+                kadd(false, a, Q.bfb + d, deg * cnorm(LA, A0 + a) * cnorm(LD, d) * s);
             });
-            for_n<U, S::NB * S::ND>([&](int bd) {
+            for_n<true, S::NB * S::ND>([&](int bd) {
                 const int b = bd / S::ND, d = bd % S::ND;
                 double s = 0.0;
-                for_n<U, S::NA * S::NC>([&](int ac) {
+                for_n<true, NA * S::NC>([&](int ac) {
                     const int a = ac / S::NC, c = ac % S::NC;
                     s += Dac[ac] * (double)eri[VIDX(a, b, c, d)];
                 });
@@ -222,18 +224,18 @@ __device__ __forceinline__ void jk_item(const int4 it, const JkArgs& g, const Ke
     }
     // J_P: wave reduction (a fixed shuffle tree), one fixed-point add per component per wave
     if (do_j) {
-        for_n<true, S::NAB>([&](int ab) {
+        for_n<true, NAB>([&](int ab) {
             double s = jp[ab];
 #pragma unroll
             for (int off = 32; off >= 1; off >>= 1) s += __shfl_xor(s, off, 64);
-            if ((tid & 63) == 0 && s != 0.0) fix_add_global(Jacc, g.jb_bra + ab * g.np_bra + it.x, s, sJ);
+            if ((tid & 63) == 0 && s != 0.0) fix_add_global(Jacc, g.jb_bra + (A0 * S::NB + ab) * g.np_bra + it.x, s, sJ);
         });
     }
     if constexpr (KROWS) {
         __syncthreads();
         for (int i = tid; i < nrow; i += blockDim.x) {
             const int r = i / nbf, col = i - r * nbf;
-            const int row = r < S::NA ? P.bfa + r : P.bfb + (r - S::NA);
+            const int row = r < NA ? P.bfa + r : P.bfb + (r - NA);
             fix_add_word_global(Kacc, (size_t)row * nbf + col, kl[i]);
         }
     }
@@ -243,25 +245,25 @@ __device__ __forceinline__ void jk_item(const int4 it, const JkArgs& g, const Ke
 // fit the budget left by the Rys coefficients; 0: K goes to memory directly.
 constexpr size_t kLdsBudget = 65536;
 template <int LA, int LB, int LC, int LD>
-inline size_t jk_row_bytes(int nbf, int do_k) {
+inline size_t jk_row_bytes(int nas, int nbf, int do_k) {
     using S = EriShape<LA, LB, LC, LD>;
-    const size_t kb = (size_t)(S::NA + S::NB) * nbf * sizeof(fix_t);
+    const size_t kb = (size_t)(nas + S::NB) * nbf * sizeof(fix_t);
     return do_k && (size_t)rys_lds_doubles<S::NROOTS>() * sizeof(double) + kb <= kLdsBudget ? kb : 0;
 }
 
-template <int LA, int LB, int LC, int LD, typename R, bool KROWS>
+template <int LA, int LB, int LC, int LD, typename R, bool KROWS, int A0, int NAS>
 __global__ __launch_bounds__(256) void jk_kernel(const int4* __restrict__ items, const JkArgs g, const KetPrims<R> kprims,
                                                  const PrimPair<R>* __restrict__ pp, const R* __restrict__ rys_tab) {
     constexpr int NR = EriShape<LA, LB, LC, LD>::NROOTS;
     extern __shared__ double rows[];
     __shared__ double rys_raw[rys_lds_doubles<NR>()];
     const R* rys_n = rys_stage<R, NR>(rys_tab, reinterpret_cast<R*>(rys_raw));
-    jk_item<LA, LB, LC, LD, R, KROWS>(items[blockIdx.x], g, kprims, pp, rys_n, rows);
+    jk_item<LA, LB, LC, LD, R, KROWS, A0, NAS>(items[blockIdx.x], g, kprims, pp, rys_n, rows);
 }
 
 // Mixed precision in one launch: items [0, n64) are FP64 quartets, the rest FP32 (one branch per
 // block); saves the second launch per class and its tail.
-template <int LA, int LB, int LC, int LD, bool KROWS>
+template <int LA, int LB, int LC, int LD, bool KROWS, int A0, int NAS>
 __global__ __launch_bounds__(256) void jk_kernel_mp(const int4* __restrict__ items, int n64, const JkArgs g,
                                                     const KetPrims<double> kprims, const KetPrims<float> kprimsf,
                                                     const PrimPair<double>* __restrict__ pp,
@@ -273,10 +275,10 @@ __global__ __launch_bounds__(256) void jk_kernel_mp(const int4* __restrict__ ite
     __shared__ double rys_raw[rys_lds_doubles<NR>()];
     if ((int)blockIdx.x < n64) {
         const double* rys_n = rys_stage<double, NR>(rys_tab, rys_raw);
-        jk_item<LA, LB, LC, LD, double, KROWS>(items[blockIdx.x], g, kprims, pp, rys_n, rows);
+        jk_item<LA, LB, LC, LD, double, KROWS, A0, NAS>(items[blockIdx.x], g, kprims, pp, rys_n, rows);
     } else {
         const float* rys_n = rys_stage<float, NR>(rys_tabf, reinterpret_cast<float*>(rys_raw));
-        jk_item<LA, LB, LC, LD, float, KROWS>(items[blockIdx.x], g, kprimsf, ppf, rys_n, rows);
+        jk_item<LA, LB, LC, LD, float, KROWS, A0, NAS>(items[blockIdx.x], g, kprimsf, ppf, rys_n, rows);
     }
 }
 
@@ -521,57 +523,69 @@ __global__ __launch_bounds__(256) void eri_tensor_wave_kernel(const int4* __rest
 #define QCG_LA(c) ((c) == 0 ? 0 : (c) <= 2 ? 1 : 2)
 #define QCG_LB(c) ((c) == 0 || (c) == 1 || (c) == 3 ? 0 : ((c) == 2 || (c) == 4) ? 1 : 2)
 
-// Classes that have a per-lane kernel: up to kJkLaneMaxNQ Cartesian components (above that the
-// wave-cooperative kernel always wins and the per-lane form is register-starved).
-template <typename S>
-inline constexpr bool kLaneForm = S::NQ <= kJkLaneMaxNQ;
-
 static JkArgs jk_args(const JkLaunch& a) {
     return {a.segs, a.bra, a.ket, a.kpairs, a.D, a.Dp, a.fix, a.Jacc, a.Jmat, a.Kacc, a.ket_off, a.mat_off, a.mol_nbf,
             a.diag, a.do_j, a.do_k, a.jb_bra, a.jb_ket, a.np_bra, a.np_ket};
 }
 
+// One launch per part of the first shell's components (jk_part).
+template <int LA, int LB, int LC, int LD, typename R, int NAS, int A0 = 0>
+static hipError_t launch_jk_parts(const JkLaunch& a, const JkArgs& g, hipStream_t st) {
+    // K rows of the bra functions in LDS when they fit (a.nbf is the largest molecule's nbf)
+    const size_t rows = jk_row_bytes<LA, LB, LC, LD>(NAS, a.nbf, a.do_k);
+    const KetPrims<R>* kp;
+    if constexpr (sizeof(R) == 8) kp = &a.kprims;
+    else kp = &a.kprimsf;
+    const dim3 block(a.block > 0 ? a.block : 64);
+    if (rows)
+        hipLaunchKernelGGL((jk_kernel<LA, LB, LC, LD, R, true, A0, NAS>), dim3(a.nitems), block, rows, st, a.items, g, *kp,
+                           (const PrimPair<R>*)a.pp, (const R*)a.rys);
+    else
+        hipLaunchKernelGGL((jk_kernel<LA, LB, LC, LD, R, false, A0, NAS>), dim3(a.nitems), block, 0, st, a.items, g, *kp,
+                           (const PrimPair<R>*)a.pp, (const R*)a.rys);
+    const hipError_t e = hipGetLastError();
+    if constexpr (A0 + NAS < ncart(LA)) return e != hipSuccess ? e : launch_jk_parts<LA, LB, LC, LD, R, NAS, A0 + NAS>(a, g, st);
+    else return e;
+}
+template <int LA, int LB, int LC, int LD, int NAS, int A0 = 0>
+static hipError_t launch_jk_mp_parts(const JkLaunch& a, const JkArgs& g, hipStream_t st) {
+    const size_t rows = jk_row_bytes<LA, LB, LC, LD>(NAS, a.nbf, a.do_k);
+    auto go = [&](auto rows_c) {
+        hipLaunchKernelGGL((jk_kernel_mp<LA, LB, LC, LD, decltype(rows_c)::value, A0, NAS>), dim3(a.nitems),
+                           dim3(a.block > 0 ? a.block : 64), rows, st, a.items, a.n64, g, a.kprims, a.kprimsf,
+                           (const PrimPair<double>*)a.pp, (const PrimPair<float>*)a.ppf, (const double*)a.rys,
+                           (const float*)a.rysf);
+    };
+    if (rows) go(std::true_type{});
+    else go(std::false_type{});
+    const hipError_t e = hipGetLastError();
+    if constexpr (A0 + NAS < ncart(LA)) return e != hipSuccess ? e : launch_jk_mp_parts<LA, LB, LC, LD, NAS, A0 + NAS>(a, g, st);
+    else return e;
+}
+
 template <int CB, int CK, typename R>
 static hipError_t launch_jk_t(const JkLaunch& a, hipStream_t st) {
-    constexpr int LA = QCG_LA(CB), LB = QCG_LB(CB), LC = QCG_LA(CK), LD = QCG_LB(CK);
-    using S = EriShape<LA, LB, LC, LD>;
+    constexpr int LA = QCG_LA(CB), LB = QCG_LB(CB), LC = QCG_LA(CK), LD = QCG_LB(CK), NAS = jk_part(CB, CK);
     if (a.nitems <= 0) return hipSuccess;
     // wave-cooperative mode (four items per block); classes without a per-lane form always take it
-    if (a.block == 0 || !kLaneForm<S>) {
+    if (a.block == 0 || NAS == 0) {
         if constexpr (JkWave<LA, LB, LC, LD, R>::kEnabled) {
             hipLaunchKernelGGL((jk_wave_kernel<LA, LB, LC, LD, R>), dim3((a.nitems + 3) / 4), dim3(256), 0, st, a.items,
                                a.nitems, jk_args(a), (const PrimPair<R>*)a.pp, (const R*)a.rys);
             return hipGetLastError();
         }
     }
-    if constexpr (kLaneForm<S>) {
-        // K rows of the bra functions in LDS when they fit (a.nbf is the largest molecule's nbf)
-        const size_t rows = jk_row_bytes<LA, LB, LC, LD>(a.nbf, a.do_k);
-        const KetPrims<R>* kp;
-        if constexpr (sizeof(R) == 8) kp = &a.kprims;
-        else kp = &a.kprimsf;
-        const dim3 block(a.block > 0 ? a.block : 64);
-        if (rows)
-            hipLaunchKernelGGL((jk_kernel<LA, LB, LC, LD, R, true>), dim3(a.nitems), block, rows, st, a.items, jk_args(a),
-                               *kp, (const PrimPair<R>*)a.pp, (const R*)a.rys);
-        else
-            hipLaunchKernelGGL((jk_kernel<LA, LB, LC, LD, R, false>), dim3(a.nitems), block, 0, st, a.items, jk_args(a),
-                               *kp, (const PrimPair<R>*)a.pp, (const R*)a.rys);
-        return hipGetLastError();
-    } else {
-        return hipErrorInvalidValue;  // not reached: large classes take the wave-cooperative form above
-    }
+    if constexpr (NAS > 0) return launch_jk_parts<LA, LB, LC, LD, R, NAS>(a, jk_args(a), st);
+    else return hipErrorInvalidValue;  // not reached: these classes take the wave-cooperative form above
 }
 
 // Mixed precision, both parts in one launch: a.items holds a.n64 FP64 items then the FP32 items,
 // all cut for the same tile (a.block); a.pp/a.rys are the FP64 data, a.ppf/a.rysf the FP32 copies.
 template <int CB, int CK>
 static hipError_t launch_jk_mp_t(const JkLaunch& a, hipStream_t st) {
-    constexpr int LA = QCG_LA(CB), LB = QCG_LB(CB), LC = QCG_LA(CK), LD = QCG_LB(CK);
-    using S = EriShape<LA, LB, LC, LD>;
+    constexpr int LA = QCG_LA(CB), LB = QCG_LB(CB), LC = QCG_LA(CK), LD = QCG_LB(CK), NAS = jk_part(CB, CK);
     if (a.nitems <= 0) return hipSuccess;
-    // classes without a per-lane form always take the wave-cooperative one
-    if (a.block == 0 || !kLaneForm<S>) {
+    if (a.block == 0 || NAS == 0) {
         if constexpr (JkWave<LA, LB, LC, LD, double>::kEnabled) {
             hipLaunchKernelGGL((jk_wave_kernel_mp<LA, LB, LC, LD>), dim3((a.nitems + 3) / 4), dim3(256), 0, st, a.items,
                                a.nitems, a.n64, jk_args(a), (const PrimPair<double>*)a.pp, (const PrimPair<float>*)a.ppf,
@@ -579,20 +593,8 @@ static hipError_t launch_jk_mp_t(const JkLaunch& a, hipStream_t st) {
             return hipGetLastError();
         }
     }
-    if constexpr (kLaneForm<S>) {
-        const size_t rows = jk_row_bytes<LA, LB, LC, LD>(a.nbf, a.do_k);
-        auto go = [&](auto rows_c) {
-            hipLaunchKernelGGL((jk_kernel_mp<LA, LB, LC, LD, decltype(rows_c)::value>), dim3(a.nitems),
-                               dim3(a.block > 0 ? a.block : 64), rows, st, a.items, a.n64, jk_args(a), a.kprims,
-                               a.kprimsf, (const PrimPair<double>*)a.pp, (const PrimPair<float>*)a.ppf,
-                               (const double*)a.rys, (const float*)a.rysf);
-        };
-        if (rows) go(std::true_type{});
-        else go(std::false_type{});
-        return hipGetLastError();
-    } else {
-        return hipErrorInvalidValue;  // not reached: large classes take the wave-cooperative form above
-    }
+    if constexpr (NAS > 0) return launch_jk_mp_parts<LA, LB, LC, LD, NAS>(a, jk_args(a), st);
+    else return hipErrorInvalidValue;  // not reached: these classes take the wave-cooperative form above
 }
 
 template <int CB, int CK>

@@ -60,12 +60,32 @@ inline QCG_HD int item_lg(const int4& it) { return (it.w >> 13) & 7; }
 // of at most this many.
 constexpr int kBraPPMax = 64;
 
-// Largest class (Cartesian components) with a per-lane J/K kernel; larger classes always run the
-// wave-cooperative one, classes from 27 components up to this limit may run either (tile block 0).
-#ifndef QCG_JK_LANE_MAX_NQ
-#define QCG_JK_LANE_MAX_NQ 81
-#endif
-constexpr int kJkLaneMaxNQ = QCG_JK_LANE_MAX_NQ;
+// Largest class (Cartesian components) whose per-lane J/K kernel holds a whole quartet in registers;
+// classes from 27 components on may also run the wave-cooperative kernel (tile block 0).
+constexpr int kJkLaneMaxNQ = 81;
+
+// Components of the first shell that one launch of the per-lane J/K kernel of a class takes: all of them up
+// to kJkLaneMaxNQ components, else as many as keep a part at kJkPartMaxNQ (0: no per-lane form).  Every
+// part evaluates the quartet's roots and 2D integrals anew, yet against the wave-cooperative kernel, whose
+// lanes share one quartet's components and leave half of the fused multiply-adds to index arithmetic, a
+// class with at most two or three parts is the faster one once a launch has lanes enough (default_tiles):
+// (H2O)16 6-31G* FP64 (dp|ds) 0.50 -> 0.18 ms, (dd|ps) 0.29 -> 0.20, (dp|pp) 0.25 -> 0.22, the build 3.40 ->
+// 2.73 ms.  At a total angular momentum of 6 the classes alone are slower ((dp|dp) 0.12 -> 0.28 ms), but run
+// beside others on the four streams they fill the chip better: build 2.80 ms without them, 2.73 with.
+// Above, (dd|dp) and (dd|dd) would need six or more parts.
+constexpr int kJkPartMaxNQ = 54;
+constexpr int kJkPartMaxL = 6;
+constexpr int jk_part(int cb, int ck) {
+    const int na = cb == 0 ? 1 : cb <= 2 ? 3 : 6;
+    const int nc[6] = {1, 3, 9, 6, 18, 36};
+    const int rest = nc[cb] / na * nc[ck];
+    if (na * rest <= kJkLaneMaxNQ) return na;
+    const int l[6] = {0, 1, 2, 2, 3, 4};
+    if (l[cb] + l[ck] > kJkPartMaxL) return 0;
+    for (int n = na; n >= 1; --n)
+        if (na % n == 0 && n * rest <= kJkPartMaxNQ) return n;
+    return 0;
+}
 
 // The same limit for the compressed tensor's kernels.
 constexpr int kTensorLaneMaxNQ = 54;

@@ -64,6 +64,7 @@ int qcg_create(qcg_context** out, int device) {
                 c->tile[cls][part].reps = nq >= 162 ? 1 : nq > kJkLaneMaxNQ ? 2 : nq >= 18 ? 4 : 1;
             }
             c->class_nq[cls] = nq;
+            c->class_nas[cls] = jk_part(cb, ck);
         }
     *out = c.release();
     return QCG_OK;
@@ -533,6 +534,12 @@ double qcg::model_flops(int cb, int ck) {
     return ((la + lb + lc + ld) / 2 + 1) * (80.0 + 15.0 * (la + lb + 1) * (lc + ld + 1) + nq * (4.0 + 6.0 * (lb + ld)));
 }
 
+// Quartets from which a class above kJkLaneMaxNQ components runs per lane in parts rather than
+// wave-cooperatively: one quartet per lane needs 256 wavefronts to touch every CU.  Whole builds, decane
+// 6-31G* mixed / (H2O)16 FP64: 1.70 / 2.80 ms from 4096 quartets on, 1.46 / 2.72 from 16384, 1.49 / 2.77
+// from 32768.
+constexpr int64_t kPartsMinQuartets = 16384;
+
 // Tiles when the caller has set or tuned none.  Per-lane kernels: the block is widened from 64 to 256
 // threads until the waves that fit a CU's 160 KB of LDS next to each other (the K rows of one bra and
 // the Rys table are per block) reach what the kernel's registers allow (`want` per SIMD), as far as a
@@ -549,7 +556,7 @@ static void default_tiles(qcg_context* c, const int64_t (&quartets)[21][2], cons
                 const int64_t n = quartets[cls][part] + (part == 0 && c->fuse_cls[cls] ? quartets[cls][1] : 0);
                 qcg_context::Tile& t = c->tile[cls][part];
                 const int nq = c->class_nq[cls];
-                if (nq > kJkLaneMaxNQ) {
+                if (nq > kJkLaneMaxNQ && (n < kPartsMinQuartets || jk_part(cb, ck) == 0)) {
                     t = {0, n > 24000 ? 4 : n > 8000 ? 2 : 1};
                     continue;
                 }
@@ -558,7 +565,7 @@ static void default_tiles(qcg_context* c, const int64_t (&quartets)[21][2], cons
                 class_l(cb, la, lb);
                 class_l(ck, lc, ld);
                 const int nr = (la + lb + lc + ld) / 2 + 1;
-                const int lds = (nr <= 3 ? (qcg_rys_off[nr + 1] - qcg_rys_off[nr]) * 8 : 0) + (ncart(la) + ncart(lb)) * c->max_nbf * 8;
+                const int lds = (nr <= 3 ? (qcg_rys_off[nr + 1] - qcg_rys_off[nr]) * 8 : 0) + (jk_part(cb, ck) + ncart(lb)) * c->max_nbf * 8;
                 const int want = nq <= 1 ? 7 : nq <= 3 ? 5 : nq <= 9 ? 4 : nq <= 18 ? 3 : nq <= 36 ? 2 : 1;
                 int block = 64;
                 while (block < 256 && (163840 / std::max(lds, 1)) * (block / 64) < 4 * want) block *= 2;
@@ -624,7 +631,7 @@ static int build_plan(qcg_context* c) {
         for (int part = 0; part < 2; ++part) {
             // fused mixed launches run both parts with the FP64 part's tile
             const qcg_context::Tile& t = c->tile[cls][(mixed && c->fuse_cls[cls]) ? 0 : part];
-            const bool lane_form = t.block > 0 ? c->class_nq[cls] <= kJkLaneMaxNQ : c->class_nq[cls] < 27;
+            const bool lane_form = t.block > 0 ? c->class_nas[cls] > 0 : c->class_nq[cls] < 27;
             const int ch = std::min(kItemMaxKets, std::max(1, t.block > 0 ? t.block * t.reps : t.reps));
             c->item_off[cls][part] = (int)c->items.size();
             for (const Bra& b : bras[cls][part]) {
@@ -816,11 +823,11 @@ constexpr int kTuneCand[][2] = {{64, 1}, {64, 2}, {64, 4}, {128, 1}, {256, 1}, {
 constexpr int kTuneNCand = sizeof(kTuneCand) / sizeof(kTuneCand[0]);
 
 // Candidate k mapped onto what class cls has: classes with fewer than 27 components have only the
-// per-lane kernel, those above kJkLaneMaxNQ only the wave-cooperative one.
+// per-lane kernel, those without a per-lane form only the wave-cooperative one.
 qcg_context::Tile tune_tile(const qcg_context* c, int k, int cls) {
     const int nq = c->class_nq[cls];
     if (nq < 27) return kTuneCand[k][0] == 0 ? qcg_context::Tile{64, 1} : qcg_context::Tile{kTuneCand[k][0], kTuneCand[k][1]};
-    if (nq > kJkLaneMaxNQ)
+    if (c->class_nas[cls] == 0)
         return kTuneCand[k][0] == 0 ? qcg_context::Tile{0, kTuneCand[k][1]}
                                     : qcg_context::Tile{0, std::min(8, kTuneCand[k][1] * 2)};
     return qcg_context::Tile{kTuneCand[k][0], kTuneCand[k][1]};

@@ -44,6 +44,23 @@ def test_gpu_jk_split_over_lanes(name, basis, prec, tol):
     assert np.abs(jk2.J - jk.J).max() < tol and np.abs(jk2.K - jk.K).max() < tol
 
 
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-11), ("mixed", 1e-9)])
+@pytest.mark.parametrize("name,basis", [("Ne", "6-31g*"), ("H2O", "6-31+g*"), ("water2", "6-31g*")])
+def test_gpu_jk_component_parts(name, basis, prec, tol):
+    """Per-lane kernels for every class that has one (the largest in parts of the first shell's
+    components) and wavefront kernels for every class that has one, J and K together and alone."""
+    b = _mol(name, basis)
+    D = random_density(b.nbf, seed=8, nocc=b.n_occ)
+    Jo, Ko, _ = oracle.jk_direct(b, D)
+    eng = Engine(b, precision=prec)
+    for tile in [(64, 1), (0, 1), (256, 2)]:
+        eng.set_tiles([tile] * 21)
+        jk = eng.build_jk(D)
+        assert np.abs(jk.J - Jo).max() < tol and np.abs(jk.K - Ko).max() < tol
+        assert np.abs(eng.build_jk(D, want_k=False).J - Jo).max() < tol
+        assert np.abs(eng.build_jk(D, want_j=False).K - Ko).max() < tol
+
+
 @pytest.mark.parametrize("name,basis", [("Ne", "6-31g"), ("H2O", "sto-3g"), ("H2O", "6-31+g*"), ("water2", "6-31g*")])
 def test_gpu_tensor_split_over_lanes(name, basis):
     """Every element of the compressed tensor (per-lane and wavefront kernels, lanes per ket), and again
