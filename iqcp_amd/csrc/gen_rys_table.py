@@ -3,20 +3,27 @@
 The n-point Rys rule for the weight exp(-T x) / (2 sqrt(x)) on x = t^2 in [0, 1]
 has moments mu_k = F_k(T) (Boys function).  For each n = 1..NMAX the exact nodes
 x_i(T) and weights w_i(T) are computed in 50-digit arithmetic (Golub-Welsch from
-the Hankel moment matrix), then fitted on intervals [k h, (k+1) h) of T by a
-degree-D polynomial in the local variable s = 2 (T - T_k)/h - 1 (Chebyshev
-least squares, converted to monomials; Horner evaluation on the device).
+the Hankel moment matrix), then fitted per interval [T_k, T_k + h_k) of T by a
+polynomial of degree D(n) in the local variable s = 2 (T - T_k)/h_k - 1 (truncated
+Chebyshev series of the exact values, converted to monomials in the same arithmetic).
+The functions flatten as T grows, so the intervals widen with it: they are those of
+T + T0(n) that share an exponent and the leading B(n) bits of the mantissa, which the
+device reads from the number's bits.  FITS holds (T0, B, D), chosen so that every fit
+is good to 1e-15 relative.
 Above T_max(n) the large-T limit is used: x_i = s_i^2 / T, w_i = W_i / sqrt(T)
 with s_i, W_i the positive nodes / weights of the 2n-point Gauss-Hermite rule
 (the truncation of the weight at t = 1 is below 1e-16 relative there).
 
 Output layout (double): for n, interval k: [x_0..x_{n-1} coeffs (D+1 each),
-w_0..w_{n-1} coeffs (D+1 each)], coefficient 0 = constant term.
+w_0..w_{n-1} coeffs (D+1 each), 2 unused], coefficient 0 = constant term.  The two
+unused words make the interval stride an odd multiple of 16 bytes (n <= 3), so the
+intervals start in all LDS banks.
 
     python iqcp_amd/csrc/gen_rys_table.py          # writes rys_table.inc next to this file
 """
 from __future__ import annotations
 
+import multiprocessing
 import sys
 from pathlib import Path
 
@@ -24,9 +31,10 @@ import mpmath as mp
 import numpy as np
 
 NMAX = 7
-H = 2.0           # interval width in T
-DEG = 13          # polynomial degree per interval
-NODES = 28        # Chebyshev sample nodes per interval
+H = 2.0           # step of the search for T_max
+FITS = {1: (8, 4, 9), 2: (8, 4, 9), 3: (4, 3, 11), 4: (8, 4, 11), 5: (8, 4, 11), 6: (8, 4, 11), 7: (8, 4, 11)}
+NODES = 24        # Chebyshev sample nodes per interval
+PAD = 2           # unused words per interval
 mp.mp.dps = 50
 
 
@@ -98,52 +106,77 @@ def tmax_for(n):
         T += H
 
 
-def fit_interval(n, T0):
-    # Chebyshev nodes on [-1, 1]
-    k = np.arange(NODES)
-    z = np.cos(np.pi * (k + 0.5) / NODES)
-    Ts = T0 + (z + 1.0) * 0.5 * H
-    X = np.zeros((NODES, n))
-    W = np.zeros((NODES, n))
-    for a, T in enumerate(Ts):
-        x, w = rys_exact(n, T)
-        X[a] = [float(v) for v in x]
-        W[a] = [float(v) for v in w]
-    coefs = []
-    for arr in (X, W):
-        for i in range(n):
-            c = np.polynomial.chebyshev.chebfit(z, arr[:, i], DEG)
-            coefs.append(np.polynomial.chebyshev.cheb2poly(c))
-    return np.array(coefs)
+def intervals(n, tmax):
+    """(T_k, h_k) of the fits, up to the one that holds tmax."""
+    T0, bits, _ = FITS[n]
+    out = []
+    lo = float(T0)
+    while lo <= tmax + T0:
+        h = 2.0 ** (int(np.floor(np.log2(lo))) - bits)
+        out.append((lo - T0, h))
+        lo += h
+    return out
+
+
+def fit_interval(job):
+    n, T0, h = job
+    mp.mp.dps = 50
+    deg = FITS[n][2]
+    th = [mp.pi * (k + mp.mpf(1) / 2) / NODES for k in range(NODES)]
+    vals = []
+    for t in th:
+        x, w = rys_exact(n, T0 + (mp.cos(t) + 1) * h / 2)
+        vals.append(list(x) + list(w))
+    cheb = [[mp.mpf(1)], [mp.mpf(0), mp.mpf(1)]]  # Chebyshev polynomials in monomials
+    while len(cheb) <= deg:
+        p = [mp.mpf(0)] + [2 * v for v in cheb[-1]]
+        for q, v in enumerate(cheb[-2]):
+            p[q] -= v
+        cheb.append(p)
+    out = []
+    for i in range(2 * n):
+        m = [mp.mpf(0)] * (deg + 1)
+        for j in range(deg + 1):
+            c = (1 if j == 0 else 2) * sum(vals[k][i] * mp.cos(j * th[k]) for k in range(NODES)) / NODES
+            for q, v in enumerate(cheb[j]):
+                m[q] += c * v
+        out += [float(v) for v in m]
+    return out + [0.0] * PAD
 
 
 def main():
     out = Path(__file__).with_name("rys_table.inc")
     tmax = {}
-    blocks = []
+    jobs = []
     offsets = []
+    nint = {}
     herm = {}
     total = 0
     for n in range(1, NMAX + 1):
-        tm = tmax_for(n)
-        tmax[n] = tm
-        nint = int(round(tm / H))
+        tmax[n] = tmax_for(n)
+        iv = intervals(n, tmax[n])
+        nint[n] = len(iv)
         offsets.append(total)
-        for kint in range(nint):
-            blocks.append(fit_interval(n, kint * H))
-            total += 2 * n * (DEG + 1)
+        jobs += [(n, t, h) for t, h in iv]
+        total += len(iv) * (2 * n * (FITS[n][2] + 1) + PAD)
         herm[n] = hermite_half(n)
-        print(f"n={n} tmax={tm} intervals={nint}", file=sys.stderr)
-    flat = np.concatenate([b.ravel() for b in blocks])
+        print(f"n={n} tmax={tmax[n]} intervals={nint[n]}", file=sys.stderr)
+    with multiprocessing.Pool() as pool:
+        flat = np.concatenate(pool.map(fit_interval, jobs, chunksize=1))
+    ns = range(1, NMAX + 1)
+
+    def table(ctype, name, values):
+        return f"constexpr {ctype} {name}[QCG_RYS_NMAX + 1] = {{0, " + ", ".join(str(v) for v in values) + "};"
+
     lines = ["// Generated by gen_rys_table.py: piecewise fits of Rys nodes/weights (see generator docstring).",
              f"#define QCG_RYS_NMAX {NMAX}",
-             f"#define QCG_RYS_DEG {DEG}",
-             f"#define QCG_RYS_H {H!r}",
-             "constexpr int qcg_rys_nint[QCG_RYS_NMAX + 1] = {0, " +
-             ", ".join(str(int(round(tmax[n] / H))) for n in range(1, NMAX + 1)) + "};",
-             "constexpr int qcg_rys_off[QCG_RYS_NMAX + 1] = {0, " + ", ".join(str(o) for o in offsets) + "};",
-             "constexpr double qcg_rys_tmax[QCG_RYS_NMAX + 1] = {0.0, " +
-             ", ".join(f"{tmax[n]!r}" for n in range(1, NMAX + 1)) + "};"]
+             f"#define QCG_RYS_PAD {PAD}",
+             table("int", "qcg_rys_deg", [FITS[n][2] for n in ns]),
+             table("int", "qcg_rys_log2t0", [int(np.log2(FITS[n][0])) for n in ns]),
+             table("int", "qcg_rys_bits", [FITS[n][1] for n in ns]),
+             table("int", "qcg_rys_nint", [nint[n] for n in ns]),
+             table("int", "qcg_rys_off", offsets),
+             table("double", "qcg_rys_tmax", [tmax[n] for n in ns])]
     hx = []
     hw = []
     for n in range(1, NMAX + 1):
