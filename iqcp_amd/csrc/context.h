@@ -183,21 +183,23 @@ struct qcg_context {
     // pk_state: 0 not made, 1 made, 2 some block has more than kPackedMaxLd functions
     PackedGrid pk{};
     int pk_state = 0;
-    int pk_ntile[3] = {};
-    int *d_pk_int = nullptr;       // ld, nfn, floff, fl
-    int64_t *d_pk_off = nullptr;   // off, voff
+    int pk_ntile = 0;
+    int *d_pk_int = nullptr;       // ld, nfn, floff, ldr, nl, fl, fs
+    int64_t *d_pk_off = nullptr;   // off, voff, roff
     short *d_pk_pos = nullptr, *d_pk_shcol = nullptr;  // column of each function and shell in each block
     int4* d_pk_tiles = nullptr;
+    double2* d_pk_rad = nullptr;   // radial parts per point and shell
+    GridFn* d_pk_fn = nullptr;
     double *d_pk_pts = nullptr, *d_pk_val = nullptr, *d_pk_vparts = nullptr, *d_pk_vsum = nullptr;
     double* d_pk_grad = nullptr;   // X, M and t of the XC gradient, made on its first use
-    int64_t pk_elems = 0;          // elements of one packed array; d_pk_val holds Phi, three grads and aow
+    int64_t pk_elems = 0;          // elements of one packed array; d_pk_val holds Phi and aow
     void free_grid() {
         for (void** p : {(void**)&d_pts, (void**)&d_w, (void**)&d_phi, (void**)&d_dphx, (void**)&d_dphy,
                          (void**)&d_dphz, (void**)&d_X, (void**)&d_aow, (void**)&d_V, (void**)&d_exc, (void**)&d_Vparts,
                          (void**)&d_gshell, (void**)&d_gexp, (void**)&d_gcn, (void**)&d_phi32, (void**)&d_grid4,
                          (void**)&d_aow32, (void**)&d_D32, (void**)&d_pk_int, (void**)&d_pk_off, (void**)&d_pk_pos,
                          (void**)&d_pk_tiles, (void**)&d_pk_pts, (void**)&d_pk_val, (void**)&d_pk_vparts,
-                         (void**)&d_pk_vsum, (void**)&d_pk_shcol, (void**)&d_pk_grad}) {
+                         (void**)&d_pk_vsum, (void**)&d_pk_shcol, (void**)&d_pk_grad, (void**)&d_pk_rad, (void**)&d_pk_fn}) {
             release(*p);
             *p = nullptr;
         }

@@ -9,6 +9,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <numeric>
 #include <string>
 #include <vector>
 
@@ -125,7 +126,8 @@ int ensure_packed(qcg_context* c) {
     std::vector<double> pw(4 * (size_t)nblk * k.S, 0.0);  // 3 coordinates, then the weights
     double* w = pw.data() + 3 * (size_t)nblk * k.S;
     for (int i = 0; i < G; ++i) {
-        for (int x = 0; x < 3; ++x) pw[3 * (size_t)i + x] = c->grid_xyz[3 * (size_t)order[i] + x];
+        // a point at infinity sees no function; kept finite, so that 0 times its powers is 0
+        for (int x = 0; x < 3; ++x) pw[3 * (size_t)i + x] = std::clamp(c->grid_xyz[3 * (size_t)order[i] + x], -1e100, 1e100);
         w[i] = c->grid_w[order[i]];
     }
     HIPCHK(c, c->alloc(&c->d_pk_pts, pw.size()));
@@ -134,7 +136,8 @@ int ensure_packed(qcg_context* c) {
     k.w = c->d_pk_pts + 3 * (size_t)nblk * k.S;
     // the shells of each block
     std::vector<unsigned char> act((size_t)nblk * ns);
-    std::vector<short> shcol((size_t)nblk * ns, -1);
+    std::vector<short> shcol(2 * (size_t)nblk * ns, -1);  // first column, then the place among the block's shells
+    short* shrad = shcol.data() + (size_t)nblk * ns;
     unsigned char* d_act = nullptr;
     HIPCHK(c, c->alloc(&d_act, act.size()));
     hipError_t e = launch_packed_active(G, k.S, nblk, ns, c->d_gshell, k.pts, d_act, c->stream);
@@ -142,33 +145,44 @@ int ensure_packed(qcg_context* c) {
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     c->release(d_act);
     HIPCHK(c, e);
-    std::vector<int> ld(nblk), nfn(nblk), floff(nblk), fl;
-    std::vector<int64_t> off(2 * (size_t)nblk);
+    std::vector<int> ld(nblk), nfn(nblk), floff(nblk), ldr(nblk), nl(2 * (size_t)nblk), fl, fs, by_l(ns);
+    std::iota(by_l.begin(), by_l.end(), 0);
+    std::stable_sort(by_l.begin(), by_l.end(), [&](int x, int y) { return B.l[x] < B.l[y]; });
+    std::vector<int64_t> off(3 * (size_t)nblk);
     std::vector<short> pos((size_t)nblk * nbf, -1);
     std::vector<int4> tiles[3];
-    int64_t elems = 0, velems = 0;
+    int64_t elems = 0, velems = 0, relems = 0;
     for (int b = 0; b < nblk; ++b) {
         floff[b] = (int)fl.size();
-        int n = 0;
-        for (int s = 0; s < ns; ++s) {
+        int n = 0, nr = 0;
+        for (int s : by_l) {
+            nl[2 * b] += B.l[s] < 1 ? act[(size_t)b * ns + s] : 0;
+            nl[2 * b + 1] += B.l[s] < 2 ? act[(size_t)b * ns + s] * ncart(B.l[s]) : 0;
             if (!act[(size_t)b * ns + s]) continue;
             shcol[(size_t)b * ns + s] = (short)n;
+            shrad[(size_t)b * ns + s] = (short)nr;
             for (int i = 0; i < ncart(B.l[s]); ++i, ++n) {
                 pos[(size_t)b * nbf + B.bf_off[s] + i] = (short)n;
                 fl.push_back(B.bf_off[s] + i);
+                fs.push_back(nr);
             }
+            ++nr;
         }
         nfn[b] = n;
         ld[b] = std::max(16, (n + 15) / 16 * 16);
         fl.resize((size_t)floff[b] + ld[b], 0);
+        fs.resize((size_t)floff[b] + ld[b], nr);
+        ldr[b] = nr + 1;
         k.max_ld = std::max(k.max_ld, ld[b]);
         off[b] = elems;
         off[nblk + b] = velems;
         elems += (int64_t)k.S * ld[b];
         velems += (int64_t)ld[b] * ld[b];
+        off[2 * nblk + b] = relems;
+        relems += (int64_t)k.S * ldr[b];
         const int vw = packed_v_width(ld[b]);
         for (int m = 0; m < ld[b]; m += 32 * vw)
-            for (int n0 = 0; n0 < ld[b]; n0 += 32 * vw) tiles[vw - 3].push_back(make_int4(b, m, n0, 0));
+            for (int n0 = 0; n0 < ld[b]; n0 += 32 * vw) tiles[vw - 3].push_back(make_int4(b, m, n0, vw));
     }
     if (k.max_ld > kPackedMaxLd || nbf > INT16_MAX) {
         c->release(c->d_pk_pts);
@@ -177,20 +191,35 @@ int ensure_packed(qcg_context* c) {
         return QCG_OK;
     }
     std::vector<int4> all;
-    for (int i = 0; i < 3; ++i) {
-        c->pk_ntile[i] = (int)tiles[i].size();
-        all.insert(all.end(), tiles[i].begin(), tiles[i].end());
-    }
+    for (int i = 2; i >= 0; --i) all.insert(all.end(), tiles[i].begin(), tiles[i].end());
+    c->pk_ntile = (int)all.size();
     std::vector<int> iv(ld);
     iv.insert(iv.end(), nfn.begin(), nfn.end());
     iv.insert(iv.end(), floff.begin(), floff.end());
+    iv.insert(iv.end(), ldr.begin(), ldr.end());
+    iv.insert(iv.end(), nl.begin(), nl.end());
     iv.insert(iv.end(), fl.begin(), fl.end());
+    iv.insert(iv.end(), fs.begin(), fs.end());
+    std::vector<GridFn> fn(nbf);
+    for (int s = 0; s < ns; ++s)
+        for (int i = 0; i < ncart(B.l[s]); ++i) {
+            const int l = B.l[s];
+            const double* A = B.centers.data() + 3 * s;
+            int axis[2] = {3, 3}, n = 0;
+            for (int k = 0; k < cart_x(l, i); ++k) axis[n++] = 0;
+            for (int k = 0; k < cart_y(l, i); ++k) axis[n++] = 1;
+            for (int k = 0; k < cart_z(l, i); ++k) axis[n++] = 2;
+            fn[B.bf_off[s] + i] = {A[0], A[1], A[2], axis[0] | axis[1] << 2, 0};
+        }
     c->pk_elems = elems;
     HIPCHK(c, c->alloc(&c->d_pk_int, iv.size()));
     HIPCHK(c, c->alloc(&c->d_pk_off, off.size()));
     HIPCHK(c, c->alloc(&c->d_pk_pos, pos.size()));
     HIPCHK(c, c->alloc(&c->d_pk_tiles, all.size()));
-    HIPCHK(c, c->alloc(&c->d_pk_val, 5 * (size_t)elems));
+    HIPCHK(c, c->alloc(&c->d_pk_val, 2 * (size_t)elems));
+    HIPCHK(c, c->alloc(&c->d_pk_rad, (size_t)relems));
+    HIPCHK(c, c->alloc(&c->d_pk_fn, fn.size()));
+    HIPCHK(c, hipMemcpy(c->d_pk_fn, fn.data(), fn.size() * sizeof(GridFn), hipMemcpyHostToDevice));
     HIPCHK(c, c->alloc(&c->d_pk_vparts, (size_t)velems));
     HIPCHK(c, c->alloc(&c->d_pk_vsum, (size_t)kPackedVGroups * nbf * nbf));
     HIPCHK(c, c->alloc(&c->d_pk_shcol, shcol.size()));
@@ -202,16 +231,19 @@ int ensure_packed(qcg_context* c) {
     k.ld = c->d_pk_int;
     k.nfn = k.ld + nblk;
     k.floff = k.nfn + nblk;
-    k.fl = k.floff + nblk;
+    k.ldr = k.floff + nblk;
+    k.nl = k.ldr + nblk;
+    k.fl = k.nl + 2 * nblk;
+    k.fs = k.fl + fl.size();
+    k.fn = c->d_pk_fn;
     k.off = c->d_pk_off;
     k.voff = k.off + nblk;
+    k.roff = k.voff + nblk;
     k.pos = c->d_pk_pos;
     k.phi = c->d_pk_val;
-    k.dpx = k.phi + elems;
-    k.dpy = k.dpx + elems;
-    k.dpz = k.dpy + elems;
-    e = launch_packed_basis(k, ns, c->d_gshell, c->d_gexp, c->d_gcn, c->d_pk_shcol, c->d_pk_val, c->d_pk_val + elems,
-                            c->d_pk_val + 2 * elems, c->d_pk_val + 3 * elems, c->stream);
+    k.rad = c->d_pk_rad;
+    e = launch_packed_basis(k, ns, c->d_gshell, c->d_gexp, c->d_gcn, c->d_pk_shcol, c->d_pk_shcol + (size_t)nblk * ns,
+                            c->d_pk_val, c->d_pk_rad, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     HIPCHK(c, e);
     c->pk_state = 1;
@@ -313,7 +345,7 @@ int xc_build(qcg_context* c, const double* dD, double* dV, double* dExc, hipStre
         if (rc) return rc;
         if (c->pk_state == 1) {
             HIPCHK(c, launch_fill(dExc, 1, 0.0, st));
-            HIPCHK(c, launch_xc_packed(c->pk, dD, c->d_pk_val + 4 * c->pk_elems, c->d_pk_tiles, c->pk_ntile, c->d_pk_vparts,
+            HIPCHK(c, launch_xc_packed(c->pk, dD, c->d_pk_val + c->pk_elems, c->d_pk_tiles, c->pk_ntile, c->d_pk_vparts,
                                        c->d_pk_vsum, dV, dExc, st));
             return QCG_OK;
         }
@@ -363,7 +395,7 @@ int xc_gradient(qcg_context* c, const double* dD, double* dgrad, hipStream_t st)
         const size_t n = (size_t)c->pk_elems, rows = (size_t)c->pk.nblk * c->pk.S;
         if (!c->d_pk_grad) HIPCHK(c, c->alloc(&c->d_pk_grad, 2 * n + 3 * rows));
         HIPCHK(c, launch_xc_grad_packed(c->pk, c->basis.nshell, c->basis.natom, c->d_gshell, c->d_gexp, c->d_gcn,
-                                        c->d_pk_shcol, dD, c->d_pk_grad, c->d_pk_val + 4 * n, c->d_pk_grad + n,
+                                        c->d_pk_shcol, dD, c->d_pk_grad, c->d_pk_val + n, c->d_pk_grad + n,
                                         c->d_pk_grad + 2 * n, dgrad, st));
         return QCG_OK;
     }

@@ -14,6 +14,18 @@
 
 namespace qcg {
 
+// The radial sums R0 = sum c_p e_p and R1 = sum c_p alpha_p e_p of a shell at squared distance r2.
+__device__ __forceinline__ void radial_sums(const GridShell& sh, const double* __restrict__ exps,
+                                            const double* __restrict__ cn, double r2, double& R0, double& R1) {
+    R0 = R1 = 0.0;
+    for (int p = 0; p < sh.nprim; ++p) {
+        const double a = exps[sh.poff + p];
+        const double e = cn[sh.poff + p] * exp(-a * r2);
+        R0 += e;
+        R1 += a * e;
+    }
+}
+
 // Phi and grad Phi of one shell at one point, written to its consecutive elements from `row`.
 __device__ __forceinline__ void shell_on_point(const GridShell& sh, const double* __restrict__ exps,
                                                const double* __restrict__ cn, double gx, double gy, double gz, size_t row,
@@ -26,14 +38,8 @@ __device__ __forceinline__ void shell_on_point(const GridShell& sh, const double
         for (int c = 0; c < nc; ++c) phi[row + c] = dphx[row + c] = dphy[row + c] = dphz[row + c] = 0.0;
         return;
     }
-    // radial sums: R0 = sum c_p e_p, R1 = sum c_p alpha_p e_p
-    double R0 = 0.0, R1 = 0.0;
-    for (int p = 0; p < sh.nprim; ++p) {
-        const double a = exps[sh.poff + p];
-        const double e = cn[sh.poff + p] * exp(-a * r2);
-        R0 += e;
-        R1 += a * e;
-    }
+    double R0, R1;
+    radial_sums(sh, exps, cn, r2, R0, R1);
     const double d[3] = {dx, dy, dz};
     for (int c = 0; c < nc; ++c) {
         const int px = cart_x(sh.l, c), py = cart_y(sh.l, c), pz = cart_z(sh.l, c);
@@ -93,24 +99,35 @@ __global__ __launch_bounds__(256) void packed_active_kernel(int G, int S, int ns
 __global__ __launch_bounds__(256) void packed_basis_kernel(const PackedGrid g, int nshell,
                                                            const GridShell* __restrict__ shells,
                                                            const double* __restrict__ exps, const double* __restrict__ cn,
-                                                           const short* __restrict__ shcol, double* __restrict__ phi,
-                                                           double* __restrict__ dphx, double* __restrict__ dphy,
-                                                           double* __restrict__ dphz) {
-    const int b = blockIdx.y, ld = g.ld[b];
+                                                           const short* __restrict__ shcol,
+                                                           const short* __restrict__ shrad, double* __restrict__ phi,
+                                                           double2* __restrict__ rad) {
+    const int b = blockIdx.y, ld = g.ld[b], ldr = g.ldr[b];
     const size_t base = (size_t)g.off[b];
     const int n = g.S * (nshell + 1);
     for (int idx = blockIdx.x * blockDim.x + threadIdx.x; idx < n; idx += gridDim.x * blockDim.x) {
         const int p = idx / (nshell + 1), s = idx - p * (nshell + 1);
-        const size_t row = base + (size_t)p * ld, pt = (size_t)b * g.S + p;
+        const size_t row = base + (size_t)p * ld, pt = (size_t)b * g.S + p, rrow = (size_t)g.roff[b] + (size_t)p * ldr;
         if (s == nshell) {  // the padding: columns from the last function on, or the whole row
-            int c = pt < (size_t)g.G ? g.nfn[b] : 0;
-            for (; c < ld; ++c) phi[row + c] = dphx[row + c] = dphy[row + c] = dphz[row + c] = 0.0;
+            for (int c = pt < (size_t)g.G ? g.nfn[b] : 0; c < ld; ++c) phi[row + c] = 0.0;
+            for (int c = pt < (size_t)g.G ? ldr - 1 : 0; c < ldr; ++c) rad[rrow + c] = make_double2(0.0, 0.0);
             continue;
         }
         const int col = shcol[(size_t)b * nshell + s];
         if (col < 0 || pt >= (size_t)g.G) continue;
-        shell_on_point(shells[s], exps, cn, g.pts[3 * pt], g.pts[3 * pt + 1], g.pts[3 * pt + 2], row + col, phi, dphx,
-                       dphy, dphz);
+        const GridShell sh = shells[s];
+        const double dx = g.pts[3 * pt] - sh.cx, dy = g.pts[3 * pt + 1] - sh.cy, dz = g.pts[3 * pt + 2] - sh.cz;
+        const double r2 = dx * dx + dy * dy + dz * dz;
+        double R0 = 0.0, R1 = 0.0;
+        if (!(sh.amin * r2 > kGridCut)) radial_sums(sh, exps, cn, r2, R0, R1);
+        rad[rrow + shrad[(size_t)b * nshell + s]] = make_double2(R0, -2.0 * R1);
+        auto pw = [](double v, int k) { return k == 0 ? 1.0 : (k == 1 ? v : v * v); };
+        for (int c = 0; c < ncart(sh.l); ++c) {
+            const int px = cart_x(sh.l, c), py = cart_y(sh.l, c), pz = cart_z(sh.l, c);
+            const double nrm = (sh.l == 2 && (px == 2 || py == 2 || pz == 2)) ? 0.57735026918962576451 : 1.0;
+            const double ang = pw(dx, px) * pw(dy, py) * pw(dz, pz);
+            phi[row + col + c] = fabs(ang) >= 1e-30 && R0 != 0.0 ? nrm * ang * R0 : 0.0;
+        }
     }
 }
 
@@ -121,11 +138,11 @@ hipError_t launch_packed_active(int G, int S, int nblk, int nshell, const GridSh
 }
 
 hipError_t launch_packed_basis(const PackedGrid& g, int nshell, const GridShell* shells, const double* exps,
-                               const double* cn, const short* shcol, double* phi, double* dpx, double* dpy, double* dpz,
+                               const double* cn, const short* shcol, const short* shrad, double* phi, double2* rad,
                                hipStream_t st) {
     const unsigned per = (unsigned)((g.S * (nshell + 1) + 255) / 256);
-    hipLaunchKernelGGL(packed_basis_kernel, dim3(per, g.nblk), dim3(256), 0, st, g, nshell, shells, exps, cn, shcol, phi,
-                       dpx, dpy, dpz);
+    hipLaunchKernelGGL(packed_basis_kernel, dim3(per, g.nblk), dim3(256), 0, st, g, nshell, shells, exps, cn, shcol,
+                       shrad, phi, rad);
     return hipGetLastError();
 }
 

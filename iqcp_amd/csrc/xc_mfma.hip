@@ -85,19 +85,13 @@ constexpr int lds_pad(int n) {
 // columns, stay within the 64 KB of static LDS per block.
 constexpr int kRhoAllMaxNT = 22;
 
-// The point part shared by both rho kernels, once the rho and grad rho sums of the block's 64 points
-// are in red[row tile][point]: B3LYP per point (FP64), the aow rows, E_xc.  NW wavefronts per block
-// (4 or 8); wavefront wv works on row tile wv % 4, and with 8 wavefronts each takes half its rows
-// in the aow pass.
-// tgrad: instead the rows of the gradient, w vrho Phi + 2 w vsigma (grad rho . grad Phi), and
-// t = 2 w vsigma grad rho (three per point) without E_xc.
-template <typename T, int NW, int MAXC = 0>
-__device__ __forceinline__ void xc_point_tail(int G, int nbf, int wv, int l, int g0, const double* __restrict__ w,
-                                              const GridVals<T>& gv, T* __restrict__ aow, double* __restrict__ exc_sum,
-                                              double (*red)[kRhoPW][4], double (*coef)[kRhoPW][4], double* part,
-                                              double* __restrict__ tgrad = nullptr) {
-    static_assert(NW == 4 || NW == 8, "four or eight wavefronts per block");
-    const int tid = 64 * wv + l, rt = wv & 3, gw = g0 + kRhoPW * rt;
+// The functional (B3LYP, FP64) at the block's 64 points, whose rho and grad rho sums are in red[row tile]
+// [point]: coef = w vrho, 4 w vsigma grad rho; returns the point's E_xc (wavefronts 0 to 3).
+// tgrad: instead w vrho and 2 w vsigma grad rho, the latter also in tgrad (three per point).
+__device__ __forceinline__ double xc_point_coef(int G, int wv, int l, int g0, const double* __restrict__ w,
+                                                double (*red)[kRhoPW][4], double (*coef)[kRhoPW][4], bool half,
+                                                double* __restrict__ tgrad) {
+    const int rt = wv & 3, gw = g0 + kRhoPW * rt;
     double contrib = 0.0;
     if (wv < 4 && l < kRhoPW) {
         const int g = gw + l;
@@ -107,7 +101,7 @@ __device__ __forceinline__ void xc_point_tail(int G, int nbf, int wv, int l, int
             const double grx = 2.0 * red[rt][l][1], gry = 2.0 * red[rt][l][2], grz = 2.0 * red[rt][l][3];
             double exc, vrho, vsig;
             xc_b3lyp(rho, grx * grx + gry * gry + grz * grz, exc, vrho, vsig);
-            const double wg = w[g], f4 = (tgrad ? 2.0 : 4.0) * wg * vsig;
+            const double wg = w[g], f4 = (half ? 2.0 : 4.0) * wg * vsig;
             c0 = wg * vrho;
             c1 = f4 * grx;
             c2 = f4 * gry;
@@ -124,6 +118,31 @@ __device__ __forceinline__ void xc_point_tail(int G, int nbf, int wv, int l, int
             tgrad[3 * (size_t)g + 2] = c3;
         }
     }
+    return contrib;
+}
+// E_xc of the block: part is four doubles of LDS.
+__device__ __forceinline__ void xc_point_exc(double contrib, int wv, int l, double* __restrict__ exc_sum, double* part) {
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) contrib += __shfl_xor(contrib, off, 64);
+    if (l == 0 && wv < 4) part[wv] = contrib;
+    __syncthreads();
+    if (wv == 0 && l == 0) {
+        const double s = part[0] + part[1] + part[2] + part[3];
+        if (s != 0.0) atomicAdd(exc_sum, s);
+    }
+}
+
+// The point part shared by both rho kernels, once the rho and grad rho sums of the block's 64 points
+// are in red[row tile][point]: B3LYP per point (FP64), the aow rows, E_xc.  NW wavefronts per block
+// (4 or 8); wavefront wv works on row tile wv % 4, and with 8 wavefronts each takes half its rows
+// in the aow pass.
+template <typename T, int NW, int MAXC = 0>
+__device__ __forceinline__ void xc_point_tail(int G, int nbf, int wv, int l, int g0, const double* __restrict__ w,
+                                              const GridVals<T>& gv, T* __restrict__ aow, double* __restrict__ exc_sum,
+                                              double (*red)[kRhoPW][4], double (*coef)[kRhoPW][4], double* part) {
+    static_assert(NW == 4 || NW == 8, "four or eight wavefronts per block");
+    const int rt = wv & 3, gw = g0 + kRhoPW * rt;
+    const double contrib = xc_point_coef(G, wv, l, g0, w, red, coef, false, nullptr);
     __syncthreads();
     // aow = w vrho Phi + 4 w vsigma (grad rho . grad Phi), row by row of the wavefront's points
     constexpr int kRows = kRhoPW / (NW / 4);
@@ -150,15 +169,7 @@ __device__ __forceinline__ void xc_point_tail(int G, int nbf, int wv, int l, int
             }
         }
     }
-    if (tgrad) return;
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) contrib += __shfl_xor(contrib, off, 64);
-    if (l == 0 && wv < 4) part[wv] = contrib;
-    __syncthreads();
-    if (tid == 0) {
-        const double s = part[0] + part[1] + part[2] + part[3];
-        if (s != 0.0) atomicAdd(exc_sum, s);
-    }
+    xc_point_exc(contrib, wv, l, exc_sum, part);
 }
 
 template <typename T, int NT>
@@ -546,18 +557,94 @@ hipError_t launch_to_f32(const double* in, float* out, size_t n, hipStream_t st)
 }
 
 // ---------------------------------------------------------------- packed FP64 form (xc_packed.h)
+// Functions of angular momentum up to L at a point without branches: the angular part is 1, u or n u v with
+// u and v the coordinates along the function's axes (meta: bits 0-1 and 2-3; L below the function's own
+// never asked for; axis 3 stands for the constant 1) and n the norm of the d components x^2, y^2, z^2.
+template <int L>
+struct FnAt {
+    double cx, cy, cz, n;
+    int shell;
+    double a[3], b[3], a1, b1;  // unit vectors of the axes, and 1 for the constant
+    __device__ __forceinline__ FnAt(double x, double y, double z, int meta) : cx(x), cy(y), cz(z), shell(meta >> 4) {
+        const int i = meta & 3, j = (meta >> 2) & 3;
+        if constexpr (L >= 1) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) a[k] = i == k ? 1.0 : 0.0;
+            a1 = i == 3 ? 1.0 : 0.0;
+        }
+        if constexpr (L >= 2) {
+            n = i == j && i < 3 ? 0.57735026918962576451 : 1.0;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) b[k] = j == k ? 1.0 : 0.0;
+            b1 = j == 3 ? 1.0 : 0.0;
+        }
+    }
+    __device__ __forceinline__ void angular(double x, double y, double z, double& ang, double& ax, double& ay,
+                                            double& az) const {
+        if constexpr (L == 0) {
+            ang = 1.0;
+            ax = ay = az = 0.0;
+        } else {
+            const double u = a1 + a[0] * x + a[1] * y + a[2] * z;
+            if constexpr (L == 1) {
+                ang = u;
+                ax = a[0];
+                ay = a[1];
+                az = a[2];
+            } else {
+                const double v = b1 + b[0] * x + b[1] * y + b[2] * z, nu = n * u, nv = n * v;
+                ang = nu * v;
+                ax = nv * a[0] + nu * b[0];
+                ay = nv * a[1] + nu * b[1];
+                az = nv * a[2] + nu * b[2];
+            }
+        }
+    }
+    // adds f * (Phi, grad Phi) into s
+    __device__ __forceinline__ void add(double x, double y, double z, const double2 R, double f, double (&s)[4]) const {
+        double ang, ax, ay, az;
+        angular(x, y, z, ang, ax, ay, az);
+        const double v0 = f * R.x;
+        if constexpr (L == 0) {
+            const double v1 = f * R.y;
+            s[0] += v0;
+            s[1] += v1 * x;
+            s[2] += v1 * y;
+            s[3] += v1 * z;
+        } else {
+            const double v1 = f * R.y * ang;
+            s[0] += v0 * ang;
+            s[1] += v0 * ax + v1 * x;
+            s[2] += v0 * ay + v1 * y;
+            s[3] += v0 * az + v1 * z;
+        }
+    }
+    // c0 Phi + (c1, c2, c3) . grad Phi
+    __device__ __forceinline__ double dot(double x, double y, double z, const double2 R, const double* c) const {
+        double ang, ax, ay, az;
+        angular(x, y, z, ang, ax, ay, az);
+        const double cd = c[1] * x + c[2] * y + c[3] * z;
+        if constexpr (L == 0) return R.x * c[0] + R.y * cd;
+        else return R.x * (c[0] * ang + c[1] * ax + c[2] * ay + c[3] * az) + R.y * ang * cd;
+    }
+};
+
 // X = Phi D for 64 points of a block on MFMA, reduced into rho and grad rho, then the functional, the
 // aow rows and E_xc: xc_rho_all_kernel over the block's own functions.  Eight wavefronts, wavefront wv
 // holding the X tile of row tile wv % 4 and column half wv / 4 (at most NH of 16 columns); no bounds
 // checks, since rows and columns are padded with zeros.  D is gathered by function number straight into
 // LDS, 16 rows per K step, 32 threads per row; the next step's Phi and D elements are loaded during the
 // current MFMAs while the registers allow two blocks per CU (NH <= kPackedPrefNH).
-// Bound by memory: Phi for the product, Phi and grad Phi for the reduction and again for the aow rows.
-// (H2O)16, 1.05e6 points: density kernel 6.98 ms dense, 2.50 ms packed; V 3.67 -> 0.98 ms (three widths),
-// summing the partial V 0.05 -> 0.20 ms; benzene, 1.3e5 points: 0.29 -> 0.22 and 0.18 -> 0.13 ms.
+// Reading Phi and grad Phi for the reduction and again for the aow rows it was bound by memory; both are made
+// from the radial parts instead (a sixth of the bytes; a block's functions are sorted by angular momentum,
+// so a tile of 16 s or p columns takes the shorter code), and what bounds it now is latency at the 16
+// wavefronts a CU that the accumulators leave (matrix cores 26 %, vector units 28 % busy).
+// (H2O)16, 1.05e6 points: density kernel 6.98 ms dense, 2.50 ms packed, 2.02 ms from radial parts; V 3.67 ->
+// 0.92 ms, summing the partial V 0.05 -> 0.17 ms; benzene, 1.3e5 points: density 0.29, 0.22, 0.18 ms (0.27 with
+// every tile treated as d), V 0.18 -> 0.085 ms.
 // The gradient uses it twice: kPackedGrad stores X, the gradient's rows and t as well, kPackedProduct only
 // the product `out` = `in` D.
-constexpr int kPackedPrefNH = 6;
+constexpr int kPackedPrefNH = 8;
 enum { kPackedBuild, kPackedGrad, kPackedProduct };
 template <int NH, int MODE>
 __global__ __launch_bounds__(512) QCG_XC_RHO_ATTR void xc_rho_packed_kernel(
@@ -633,48 +720,74 @@ __global__ __launch_bounds__(512) QCG_XC_RHO_ATTR void xc_rho_packed_kernel(
                     out[base + (size_t)(kRhoPW * rt + M::row(lk, r)) * ld + 16 * (t0 + t) + li] = acc[t][r];
         if constexpr (MODE == kPackedProduct) return;
     }
-    double rs[4] = {}, xs[4] = {}, ys[4] = {}, zs[4] = {};
-    const GridVals<double> gv{g.phi + base, g.dpx + base, g.dpy + base, g.dpz + base, nullptr};
-#pragma unroll
-    for (int t = 0; t < NH; ++t) {
-        if (t < mine) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                double f, dx, dy, dz;
-                gv.get((size_t)(kRhoPW * rt + M::row(lk, r)) * ld + 16 * (t0 + t) + li, f, dx, dy, dz);
-                const double x = acc[t][r];
-                rs[r] += x * f;
-                xs[r] += x * dx;
-                ys[r] += x * dy;
-                zs[r] += x * dz;
-            }
-        }
-        // one tile's loads in flight at a time: hoisting all of them costs hundreds of VGPRs
-        asm volatile("" ::: "memory");
+    // the block's functions, in the Phi staging area (free now)
+    static_assert(sizeof(As) >= BN * (3 * sizeof(double) + sizeof(int)), "the functions fit in As");
+    double(*fcen)[BN] = reinterpret_cast<double(*)[BN]>(&As[0][0]);
+    int* fmeta = reinterpret_cast<int*>(fcen + 3);
+    __syncthreads();  // every wavefront's last fragment reads are done
+    if (tid < ld) {
+        const GridFn f = g.fn[fl[tid]];
+        fcen[0][tid] = f.cx;
+        fcen[1][tid] = f.cy;
+        fcen[2][tid] = f.cz;
+        fmeta[tid] = f.axes | g.fs[g.floff[b] + tid] << 4;
     }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-#pragma unroll
-        for (int off = 1; off < 16; off <<= 1) {
-            rs[r] += __shfl_xor(rs[r], off, 64);
-            xs[r] += __shfl_xor(xs[r], off, 64);
-            ys[r] += __shfl_xor(ys[r], off, 64);
-            zs[r] += __shfl_xor(zs[r], off, 64);
-        }
-    }
+    const double2* __restrict__ rad = g.rad + g.roff[b] + (size_t)p0 * g.ldr[b];
+    const double* __restrict__ pts = g.pts + 3 * ((size_t)b * g.S + p0);
+    const int ldr = g.ldr[b];
+    if (tid < 3 * kRhoBM) coef[tid / (3 * kRhoPW)][tid / 3 % kRhoPW][tid % 3] = pts[tid];
+    __syncthreads();
     // per column half, row tile and point, in the D staging area (free now)
     static_assert(sizeof(Bs) >= 2 * 4 * kRhoPW * 4 * sizeof(double), "red2 fits in Bs");
     auto red2 = reinterpret_cast<double (*)[4][kRhoPW][4]>(&Bs[0][0]);
-    __syncthreads();  // every wavefront's last fragment reads are done
-    if (li == 0) {
+    // highest angular momentum among the columns c0 to c0 + n - 1 (a block's functions are sorted by it)
+    const int nfn = g.nfn[b], n0 = g.nl[2 * b], n1 = g.nl[2 * b + 1];
+    auto max_l = [&](int c0, int n) {
+        const int e = min(c0 + n, nfn);
+        return e <= n0 ? 0 : e <= n1 ? 1 : 2;
+    };
+    // RS of the lane's four points at a time, as many as the registers allow beside the accumulators
+    constexpr int RS = NH <= 1 ? 4 : NH <= 5 ? 2 : 1;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int p = M::row(lk, r);
-            red2[half][rt][p][0] = rs[r];
-            red2[half][rt][p][1] = xs[r];
-            red2[half][rt][p][2] = ys[r];
-            red2[half][rt][p][3] = zs[r];
+    for (int r0 = 0; r0 < 4; r0 += RS) {
+        double sum[RS][4] = {}, pt[RS][3];
+        const double2* row[RS];
+#pragma unroll
+        for (int r = 0; r < RS; ++r) {
+            const int p = M::row(lk, r0 + r);
+            row[r] = rad + (kRhoPW * rt + p) * ldr;
+#pragma unroll
+            for (int q = 0; q < 3; ++q) pt[r][q] = coef[rt][p][q];
         }
+#pragma unroll
+        for (int t = 0; t < NH; ++t) {
+            const int col = 16 * (t0 + t) + li;
+            auto tile = [&](auto lc) {
+                const FnAt<decltype(lc)::value> fn(fcen[0][col], fcen[1][col], fcen[2][col], fmeta[col]);
+                double2 R[RS];
+#pragma unroll
+                for (int r = 0; r < RS; ++r) R[r] = row[r][fn.shell];
+#pragma unroll
+                for (int r = 0; r < RS; ++r)
+                    fn.add(pt[r][0] - fn.cx, pt[r][1] - fn.cy, pt[r][2] - fn.cz, R[r], acc[t][r0 + r], sum[r]);
+            };
+            if (t < mine) {
+                const int lmax = max_l(16 * (t0 + t), 16);
+                if (lmax == 0) tile(std::integral_constant<int, 0>{});
+                else if (lmax == 1) tile(std::integral_constant<int, 1>{});
+                else tile(std::integral_constant<int, 2>{});
+            }
+            // one tile's loads in flight at a time: hoisting all of them costs hundreds of VGPRs
+            asm volatile("" ::: "memory");
+        }
+#pragma unroll
+        for (int r = 0; r < RS; ++r)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+#pragma unroll
+                for (int off = 1; off < 16; off <<= 1) sum[r][q] += __shfl_xor(sum[r][q], off, 64);
+                if (li == 0) red2[half][rt][M::row(lk, r0 + r)][q] = sum[r][q];
+            }
     }
     __syncthreads();
     if (tid < 4 * kRhoPW * 4) {  // the two column halves, in a fixed order
@@ -682,8 +795,31 @@ __global__ __launch_bounds__(512) QCG_XC_RHO_ATTR void xc_rho_packed_kernel(
         red[r4][p][q] = red2[0][r4][p][q] + red2[1][r4][p][q];
     }
     __syncthreads();
-    xc_point_tail<double, 8, (NH + 1) / 2>(kRhoBM, ld, wv, l, 0, g.w + (size_t)b * g.S + p0, gv, aow + base, exc_sum, red,
-                                           coef, part, MODE == kPackedGrad ? exc_sum + 3 * ((size_t)b * g.S + p0) : nullptr);
+    const size_t pt0 = (size_t)b * g.S + p0;
+    const double contrib = xc_point_coef(kRhoBM, wv, l, 0, g.w + pt0, red, coef, MODE == kPackedGrad,
+                                         MODE == kPackedGrad ? exc_sum + 3 * pt0 : nullptr);
+    __syncthreads();
+    // aow = w vrho Phi + 4 w vsigma (grad rho . grad Phi) (the gradient's rows: 2): lanes over the columns,
+    // each wavefront half the points of its row tile
+    constexpr int kRows = kRhoPW / 2;
+    const int q0 = kRhoPW * rt + kRows * half;
+    for (int c0 = 0; c0 < ld; c0 += 64) {
+        const int col = c0 + l;
+        auto rows = [&](auto lc) {
+            const FnAt<decltype(lc)::value> fn(fcen[0][col], fcen[1][col], fcen[2][col], fmeta[col]);
+#pragma unroll 4
+            for (int p = q0; p < q0 + kRows; ++p)
+                aow[base + (size_t)p * ld + col] = fn.dot(pts[3 * p] - fn.cx, pts[3 * p + 1] - fn.cy, pts[3 * p + 2] - fn.cz,
+                                                          rad[p * ldr + fn.shell], coef[rt][p - kRhoPW * rt]);
+        };
+        const int lmax = max_l(c0, 64);
+        if (col < ld) {
+            if (lmax == 0) rows(std::integral_constant<int, 0>{});
+            else if (lmax == 1) rows(std::integral_constant<int, 1>{});
+            else rows(std::integral_constant<int, 2>{});
+        }
+    }
+    if constexpr (MODE == kPackedBuild) xc_point_exc(contrib, wv, l, exc_sum, part);
 }
 
 // in D for every block (or the whole XC build / gradient step, MODE)
@@ -710,19 +846,18 @@ hipError_t launch_packed_grad_rows(const PackedGrid& g, const double* D, double*
     return e != hipSuccess ? e : launch_packed_rows<kPackedProduct>(g, aow, D, M, nullptr, nullptr, st);
 }
 
-// Partial V of one block: Phi^T aow over its S points by 32 VW square output tiles (xc_v_kernel's
+// One output tile of the partial V of a block: Phi^T aow over its S points, 32 VW square (xc_v_kernel's
 // tiling), written packed.
 template <int VW>
-__global__ __launch_bounds__(256) void xc_v_packed_kernel(const PackedGrid g, const int4* __restrict__ tiles,
-                                                          const double* __restrict__ aow, double* __restrict__ Vparts) {
+__device__ __forceinline__ void xc_v_packed_tile(const PackedGrid& g, const int4 tl, const double* __restrict__ aow,
+                                                 double* __restrict__ Vparts, double* smem) {
     using M = Mfma<double>;
     using acc_t = typename M::acc;
     constexpr int BM = 32 * VW;
-    __shared__ double As[kVBK][BM + kPad];
-    __shared__ double Bs[kVBK][BM + kPad];
+    auto As = reinterpret_cast<double (*)[BM + kPad]>(smem);
+    auto Bs = As + kVBK;
     const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63, li = l & 15, lk = l >> 4;
     const int wr = wv >> 1, wc = wv & 1;
-    const int4 tl = tiles[blockIdx.x];
     const int b = tl.x, m0 = tl.y, n0 = tl.z, ld = g.ld[b];
     const double* __restrict__ A = g.phi + g.off[b] + m0;
     const double* __restrict__ B = aow + g.off[b] + n0;
@@ -781,6 +916,17 @@ __global__ __launch_bounds__(256) void xc_v_packed_kernel(const PackedGrid g, co
         }
 }
 
+// The tiles of all widths in one launch, the widest first.  One launch per width left the chip half idle in
+// each: (H2O)16 0.47 + 0.28 + 0.24 ms (half a wavefront per SIMD in the widest), benzene 0.08 + 0.05.
+__global__ __launch_bounds__(256) void xc_v_packed_kernel(const PackedGrid g, const int4* __restrict__ tiles,
+                                                          const double* __restrict__ aow, double* __restrict__ Vparts) {
+    __shared__ double smem[2 * kVBK * (32 * 5 + kPad)];
+    const int4 tl = tiles[blockIdx.x];
+    if (tl.w == 3) xc_v_packed_tile<3>(g, tl, aow, Vparts, smem);
+    else if (tl.w == 4) xc_v_packed_tile<4>(g, tl, aow, Vparts, smem);
+    else xc_v_packed_tile<5>(g, tl, aow, Vparts, smem);
+}
+
 // Vsum[k] = sum of the partial matrices of the k-th run of blocks, one matrix row per thread block
 __global__ __launch_bounds__(128) void packed_vsum_kernel(const PackedGrid g, int per, const double* __restrict__ Vparts,
                                                           double* __restrict__ Vsum) {
@@ -813,20 +959,11 @@ __global__ __launch_bounds__(128) void packed_vsym_kernel(int nbf, int ngrp, con
 
 int packed_v_width(int ld) { return xc_v_width(ld, false); }
 
-hipError_t launch_xc_packed(const PackedGrid& g, const double* D, double* aow, const int4* tiles, const int ntile[3],
+hipError_t launch_xc_packed(const PackedGrid& g, const double* D, double* aow, const int4* tiles, int ntile,
                             double* Vparts, double* Vsum, double* V, double* exc_sum, hipStream_t st) {
     hipError_t e = launch_packed_rows<kPackedBuild>(g, g.phi, D, nullptr, aow, exc_sum, st);
     if (e != hipSuccess) return e;
-    const int4* t = tiles;
-    for (int w = 3; w <= 5; t += ntile[w - 3], ++w) {
-        if (ntile[w - 3] == 0) continue;
-        const dim3 tg((unsigned)ntile[w - 3]);
-        if (w == 3) hipLaunchKernelGGL((xc_v_packed_kernel<3>), tg, dim3(256), 0, st, g, t, aow, Vparts);
-        else if (w == 4) hipLaunchKernelGGL((xc_v_packed_kernel<4>), tg, dim3(256), 0, st, g, t, aow, Vparts);
-        else hipLaunchKernelGGL((xc_v_packed_kernel<5>), tg, dim3(256), 0, st, g, t, aow, Vparts);
-        e = hipGetLastError();
-        if (e != hipSuccess) return e;
-    }
+    hipLaunchKernelGGL(xc_v_packed_kernel, dim3((unsigned)ntile), dim3(256), 0, st, g, tiles, aow, Vparts);
     const int ngrp = g.nblk < kPackedVGroups ? g.nblk : kPackedVGroups, per = (g.nblk + ngrp - 1) / ngrp;
     const dim3 vg((g.nbf + 127) / 128, g.nbf, ngrp);
     hipLaunchKernelGGL(packed_vsum_kernel, vg, dim3(128), 0, st, g, per, Vparts, Vsum);

@@ -49,6 +49,20 @@ def test_gpu_packed_far_points_and_long_molecules():
     _check(b, far, w[:500])
 
 
+@pytest.mark.parametrize("name,basis", [("H2O", "sto-3g"), ("NH3", "6-31+g*"), ("C6H6", "6-31g*")])
+def test_gpu_packed_functions_from_radial_parts(name, basis):
+    """Blocks without d functions, with tiles of mixed angular momentum, and points out of every reach,
+    one of them at infinity, which add nothing."""
+    b = bench_molecule(name, basis)
+    xyz, w = _points(b, 2000, 5)
+    D, V, E, _ = _check(b, xyz, w)
+    out = np.array([[1e6, 0.0, 0.0], [0.0, -1e200, 3.0], [np.inf, 0.0, 0.0]])
+    eng = Engine(b)
+    eng.set_grid(np.concatenate([xyz, out]), np.concatenate([w, np.ones(3)]))
+    V2, E2 = eng.xc(D)
+    assert np.abs(V2 - V).max() < 1e-10 and abs(E2 - E) < 1e-10 * max(1.0, abs(E))
+
+
 def test_gpu_packed_follows_the_options():
     b = bench_molecule("H2O", "6-31g*")
     xyz, w = _points(b, 5000, 8)
