@@ -22,11 +22,6 @@ namespace qcg {
 std::vector<double> ScfRun::Diis::extrapolate() const {
     const int n = (int)f.size();
     if (n == 1) return f[0];
-    auto dot = [](const std::vector<double>& a, const std::vector<double>& b) {
-        double s = 0.0;
-        for (size_t i = 0; i < a.size(); ++i) s += a[i] * b[i];
-        return s;
-    };
     auto average = [&]() {
         std::vector<double> out(f[0].size(), 0.0);
         const double c = 1.0 / (double)n;
@@ -36,7 +31,7 @@ std::vector<double> ScfRun::Diis::extrapolate() const {
     };
     std::vector<double> B((size_t)(n + 1) * (n + 1), 0.0), rhs(n + 1, 0.0), c;
     for (int i = 0; i < n; ++i)
-        for (int j = 0; j <= i; ++j) B[(size_t)i * (n + 1) + j] = B[(size_t)j * (n + 1) + i] = dot(e[i], e[j]);
+        for (int j = 0; j <= i; ++j) B[(size_t)i * (n + 1) + j] = B[(size_t)j * (n + 1) + i] = dot(e[i].data(), e[j].data(), e[i].size());
     for (int i = 0; i < n; ++i) B[(size_t)i * (n + 1) + n] = B[(size_t)n * (n + 1) + i] = -1.0;
     rhs[n] = -1.0;
     if (!lu_solve(B, rhs, n + 1, c)) return average();
@@ -57,12 +52,8 @@ void ScfRun::diagonalize(const std::vector<double>& Fm) {
     sym_eigen(Fp, n, eps, Cp);
     C.assign((size_t)n * n, 0.0);
     matmul(X.data(), Cp.data(), C.data(), n);           // C = X C'
-    for (int i = 0; i < n; ++i)
-        for (int j = 0; j < n; ++j) {
-            double s = 0.0;
-            for (int k = 0; k < nocc; ++k) s += C[(size_t)i * n + k] * C[(size_t)j * n + k];
-            D[(size_t)i * n + j] = 2.0 * s;
-        }
+    gemm(C.data(), n, false, C.data(), n, true, D.data(), n, n, n, nocc);  // the occupied orbitals
+    for (double& d : D) d *= 2.0;
 }
 
 int ScfRun::init(int nbf_, int nocc_, const double* S_, const double* H_, double e_nuc_, const ScfConfig& cfg_,
@@ -132,16 +123,12 @@ bool ScfRun::accept_fock(const double* F_, double e_elec, bool may_converge, dou
         double ss = 0.0;
         for (size_t i = 0; i < n2; ++i) ss += (D[i] - Dold[i]) * (D[i] - Dold[i]);
         last_rms = std::sqrt(ss / (double)n2);
-        std::vector<double> tmp(n2);
-        matmul(F.data(), C.data(), tmp.data(), nbf);
-        double g2 = 0.0;
-        for (int v = nocc; v < nbf; ++v)
-            for (int o = 0; o < nocc; ++o) {
-                double s = 0.0;
-                for (int k = 0; k < nbf; ++k) s += C[(size_t)k * nbf + v] * tmp[(size_t)k * nbf + o];
-                g2 += s * s;
-            }
+        // occupied-virtual block of C^T F C
         const int nvir = nbf - nocc;
+        std::vector<double> tmp((size_t)nbf * nocc), Fov((size_t)nvir * nocc);
+        gemm(F.data(), nbf, false, C.data(), nbf, false, tmp.data(), nocc, nbf, nocc, nbf);
+        gemm(C.data() + nocc, nbf, true, tmp.data(), nocc, false, Fov.data(), nocc, nvir, nocc, nbf);
+        const double g2 = dot(Fov.data(), Fov.data(), Fov.size());
         const double gnorm = nvir > 0 ? std::sqrt(4.0 * g2) / std::sqrt((double)nvir * nocc) : 0.0;
         e_tot = e_new;
         last_g = gnorm;
