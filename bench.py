@@ -35,7 +35,7 @@ def kernel_name(la, lb, lc, ld, tile, f64, fused=False):
     """Name of the J/K kernel a class runs under a tile (block 0 = wave-cooperative kernel); fused:
     the mixed-precision launch that runs both parts (jk_kernel_mp / jk_wave_kernel_mp)."""
     nq = ncart(la) * ncart(lb) * ncart(lc) * ncart(ld)
-    k = "jk_wave_kernel" if (tile[0] == 0 and nq >= 27) else "jk_kernel"
+    k = "jk_wave_kernel" if (tile[0] == 0 and nq >= 27) or la + lb + lc + ld > 6 else "jk_kernel"
     if fused:
         return f"{k}_mp<{la}, {lb}, {lc}, {ld}>"
     return f"{k}<{la}, {lb}, {lc}, {ld}, {'double' if f64 else 'float'}>"

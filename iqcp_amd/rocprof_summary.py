@@ -35,7 +35,7 @@ PEAK_MFMA = {"F32": 157.3e12, "F64": 78.6e12}
 MFMA_FLOPS = 2 * 16 * 16 * 4
 
 KERNEL_RE = re.compile(r"(jk_wave_kernel_mp|jk_kernel_mp|jk_wave_kernel|jk_kernel)<(\d), (\d), (\d), (\d)"
-                       r"(?:, (double|float))?(?:, (\d))?>")
+                       r"(?:, (double|float))?(?:, (true|false|\d))?(?:, \d+)*>")
 
 
 def short_name(name: str) -> str:
@@ -44,7 +44,8 @@ def short_name(name: str) -> str:
 
 
 def bench_label(name: str) -> str | None:
-    """The name bench.py gives a J/K kernel (no LDS-row template argument), None for other kernels."""
+    """The name bench.py gives a J/K kernel (no arguments for LDS rows and parts of a
+    class, whose launches count as one kernel), None for other kernels."""
     m = KERNEL_RE.search(name)
     if not m:
         return None
