@@ -56,17 +56,34 @@ def hbm_traffic(name, tile):
 
 def grad_model_flops(stats):
     """Algorithmic flops of one ERI-gradient evaluation from the J/K class counts (same Schwarz and
-    primitive screens): per surviving primitive quartet n_g [80 + 15 (la+lb+2)(lc+ld+2)
-    + 13 N_q (4 + 6 (lb+ld+1))] with n_g = (L+2)//2 + 1 roots, plus 144 N_q per contracted quartet."""
+    primitive screens): per surviving primitive quartet n_g [80 + 15 (la+lb+2)(lc+ld+2) + 24 N_q] with
+    n_g = (L+2)//2 + 1 roots (a component takes three products of two 1-D factors, the density weight
+    on each, and nine multiply-adds into the derivatives of three centres), plus 144 N_q per contracted
+    quartet."""
     tot = 0.0
     for x in stats:
         la, lb, lc, ld = x["la"], x["lb"], x["lc"], x["ld"]
         nq = ncart(la) * ncart(lb) * ncart(lc) * ncart(ld)
         ng = (la + lb + lc + ld + 2) // 2 + 1
-        per_prim = ng * (80 + 15 * (la + lb + 2) * (lc + ld + 2) + 13 * nq * (4 + 6 * (lb + ld + 1)))
+        per_prim = ng * (80 + 15 * (la + lb + 2) * (lc + ld + 2) + 24 * nq)
         tot += per_prim * (x["prim_quartets_fp64"] + x["prim_quartets_fp32"])
         tot += 144 * nq * (x["quartets_fp64"] + x["quartets_fp32"])
     return tot
+
+
+def reaching_functions(b, pts):
+    """Per grid point the number of basis functions that reach it (smallest exponent times r^2 at most
+    34.5388, the grid's cut-off), as a device tensor."""
+    import numpy as np
+    import torch
+    x = torch.tensor(np.ascontiguousarray(pts), device="cuda")
+    n = torch.zeros(len(x), dtype=torch.float64, device="cuda")
+    for s in range(b.nshell):
+        o = int(b.shell_prim_off[s])
+        amin = float(np.min(b.exps[o:o + int(b.shell_nprim[s])]))
+        c = torch.tensor(b.xyz[int(b.shell_atom[s])], device="cuda")
+        n += ncart(int(b.shell_l[s])) * (amin * ((x - c) ** 2).sum(1) <= 34.5388)
+    return n
 
 
 def main():
@@ -345,13 +362,16 @@ def main():
             ks[f"{prec}_ms_per_build"] = round(1e3 * el_k / nk, 3)
             ks[f"{prec}_two_electron_plus_xc_energy"] = Ek
         ks["speedup_mixed_vs_fp64"] = round(ks["fp64_ms_per_build"] / ks["mixed_ms_per_build"], 3)
-        # XC roofline: 4 G nbf^2 (the two grid GEMMs) + 16 G nbf (rho, grad rho, aow rows) + 300 G
-        # (the functional) flops per build on MFMA (FP32 products in the mixed option, FP64 otherwise);
-        # algorithmic bytes: Phi and grad Phi read once (4 G nbf elements) + D, V (2 nbf^2 doubles)
-        xc_fl = 4.0 * npts * bw.nbf ** 2 + 16.0 * npts * bw.nbf + 300.0 * npts
-        for prec, peak, esz in (("mixed", 157.3, 4), ("fp64", 78.6, 8)):
+        # XC roofline: 4 n^2 (the two grid products) + 16 n (rho, grad rho, aow rows) + 300 (the
+        # functional) flops per point on MFMA (FP32 products in the mixed option, FP64 otherwise), n all
+        # functions in the mixed option's dense kernels and those that reach the point in the FP64 form;
+        # algorithmic bytes: Phi and grad Phi read once (4 n elements per point) + D, V (2 nbf^2 doubles)
+        n_pt = reaching_functions(bw, ew.get_grid()[0])
+        dense = torch.full_like(n_pt, bw.nbf)
+        for prec, peak, esz, n_ in (("mixed", 157.3, 4, dense), ("fp64", 78.6, 8, n_pt)):
             t_ = ks[f"{prec}_xc_ms"] * 1e-3
-            byts = 4.0 * npts * bw.nbf * esz + 2.0 * bw.nbf ** 2 * 8
+            xc_fl = float((4.0 * n_ * n_ + 16.0 * n_ + 300.0).sum())
+            byts = 4.0 * float(n_.sum()) * esz + 2.0 * bw.nbf ** 2 * 8
             ks[f"{prec}_xc_roofline"] = {"bound": "mfma", "achieved": round(xc_fl / t_ / 1e12, 3), "peak": peak,
                                          "unit": "TFLOP/s", "frac": round(xc_fl / t_ / 1e12 / peak, 4),
                                          "flops_model": xc_fl, "algorithmic_GBps": round(byts / t_ / 1e9, 1)}
