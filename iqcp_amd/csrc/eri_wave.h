@@ -2,7 +2,8 @@
 // at a time, with the Rys transfer tables in LDS instead of per-lane registers.
 //
 // The per-lane kernels (one quartet per lane) hold NQ accumulators plus three transfer tables per
-// lane; from about NQ = 81 on that no longer fits the register file and the arrays go to scratch.
+// lane; above NQ = 81 that no longer fits the register file and they run in parts (jk_part, grad_part),
+// which pays with quartets enough to fill the lanes of the chip.
 // Here the work of a quartet is split three ways over the wave:
 //   phase A  lanes over (primitive quartet, Rys node, axis): node/weight, 2-D VRR and the 1-D
 //            transfer of one axis, written to an LDS table tbl[(axis*HT + h)*ES + e] whose entry

@@ -2,7 +2,7 @@
 // cut into blocks of S consecutive points, and each block keeping only the functions that reach any of
 // its points (the others' Phi and grad Phi are exactly zero there, basis_kernel's cut-off).  (H2O)16 on
 // 1.05e6 points: a block of 1024 points keeps about 45 % of the 304 functions, so the two grid products
-// take a fifth to a quarter of the dense ones' flops and the arrays 45 % of the bytes; benzene keeps 80 %.
+// take a quarter of the dense ones' flops and the arrays a sixth of the bytes; benzene keeps 80 %.
 #pragma once
 #include "qcg_common.h"
 
