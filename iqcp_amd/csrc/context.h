@@ -176,6 +176,7 @@ struct qcg_context {
     // made on its first use for the current grid
     float *d_phi32 = nullptr, *d_aow32 = nullptr, *d_D32 = nullptr;
     float4* d_grid4 = nullptr;  // (Phi, dPhi/dx, dPhi/dy, dPhi/dz) per element, FP32
+    unsigned* d_tile_mask = nullptr;  // per 16 points: tiles of 16 functions that are not zero there
     GridShell* d_gshell = nullptr;
     double *d_gexp = nullptr, *d_gcn = nullptr;
     // The packed FP64 form of the grid (xc_packed.h), made with the grid when the precision option is
@@ -199,7 +200,7 @@ struct qcg_context {
                          (void**)&d_gshell, (void**)&d_gexp, (void**)&d_gcn, (void**)&d_phi32, (void**)&d_grid4,
                          (void**)&d_aow32, (void**)&d_D32, (void**)&d_pk_int, (void**)&d_pk_off, (void**)&d_pk_pos,
                          (void**)&d_pk_tiles, (void**)&d_pk_pts, (void**)&d_pk_val, (void**)&d_pk_vparts,
-                         (void**)&d_pk_vsum, (void**)&d_pk_shcol, (void**)&d_pk_grad, (void**)&d_pk_rad, (void**)&d_pk_fn}) {
+                         (void**)&d_pk_vsum, (void**)&d_pk_shcol, (void**)&d_pk_grad, (void**)&d_pk_rad, (void**)&d_pk_fn, (void**)&d_tile_mask}) {
             release(*p);
             *p = nullptr;
         }

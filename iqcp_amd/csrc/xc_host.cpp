@@ -306,6 +306,10 @@ int ensure_xc32(qcg_context* c, hipStream_t st) {
     HIPCHK(c, c->alloc(&c->d_D32, nn));
     HIPCHK(c, launch_to_f32(c->d_phi, c->d_phi32, gn, st));
     HIPCHK(c, launch_to_f32x4(c->d_phi, c->d_dphx, c->d_dphy, c->d_dphz, c->d_grid4, gn, st));
+    if (const size_t nm = xc_tile_mask_words((int)c->G, c->basis.nbf)) {
+        HIPCHK(c, c->alloc(&c->d_tile_mask, nm));
+        HIPCHK(c, launch_tile_mask((int)c->G, c->basis.nbf, c->d_grid4, c->d_tile_mask, st));
+    }
     return QCG_OK;
 }
 
@@ -319,7 +323,7 @@ int xc_build_mfma(qcg_context* c, const double* dD, double* dV, double* dExc, hi
         int rc = ensure_xc32(c, st);
         if (rc) return rc;
         HIPCHK(c, launch_to_f32(dD, c->d_D32, (size_t)nbf * nbf, st));
-        HIPCHK(c, launch_xc_mfma(G, nbf, c->v_chunks_mfma32, c->d_w, c->d_phi32, c->d_grid4, c->d_D32, c->d_aow32, dExc,
+        HIPCHK(c, launch_xc_mfma(G, nbf, c->v_chunks_mfma32, c->d_w, c->d_phi32, c->d_grid4, c->d_tile_mask, c->d_D32, c->d_aow32, dExc,
                                  c->d_Vparts, st));
     } else {
         HIPCHK(c, launch_xc_mfma(G, nbf, c->v_chunks_mfma, c->d_w, c->d_phi, c->d_dphx, c->d_dphy, c->d_dphz, dD, c->d_aow,

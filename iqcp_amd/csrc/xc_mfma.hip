@@ -84,6 +84,9 @@ constexpr int lds_pad(int n) {
 // Most MFMA column tiles the all-columns kernel holds (nbf <= 352): D rows of one K step, all
 // columns, stay within the 64 KB of static LDS per block.
 constexpr int kRhoAllMaxNT = 22;
+// From more column tiles than this on it leaves out the zero ones (octane 6-31G, 7 tiles: 313 us without, 317
+// with; (H2O)16, 19 tiles: see the kernel).
+constexpr int kRhoMaskNT = 12;
 
 // The functional (B3LYP, FP64) at the block's 64 points, whose rho and grad rho sums are in red[row tile]
 // [point]: coef = w vrho, 4 w vsigma grad rho; returns the point's E_xc (wavefronts 0 to 3).
@@ -139,7 +142,8 @@ __device__ __forceinline__ void xc_point_exc(double contrib, int wv, int l, doub
 template <typename T, int NW, int MAXC = 0>
 __device__ __forceinline__ void xc_point_tail(int G, int nbf, int wv, int l, int g0, const double* __restrict__ w,
                                               const GridVals<T>& gv, T* __restrict__ aow, double* __restrict__ exc_sum,
-                                              double (*red)[kRhoPW][4], double (*coef)[kRhoPW][4], double* part) {
+                                              double (*red)[kRhoPW][4], double (*coef)[kRhoPW][4], double* part,
+                                              unsigned tiles = ~0u) {
     static_assert(NW == 4 || NW == 8, "four or eight wavefronts per block");
     const int rt = wv & 3, gw = g0 + kRhoPW * rt;
     const double contrib = xc_point_coef(G, wv, l, g0, w, red, coef, false, nullptr);
@@ -154,13 +158,19 @@ __device__ __forceinline__ void xc_point_tail(int G, int nbf, int wv, int l, int
         const size_t row = (size_t)g * nbf;
         if constexpr (MAXC > 0) {
             // nbf <= 64 MAXC: the row's loads all in flight before the first use (unconditional, at
-            // columns clamped into the basis, so none waits inside a branch of its own)
+            // columns clamped into the basis, so none waits inside a branch of its own); the lanes of
+            // column tiles that are zero at these points (not in `tiles`) read the row's first element
             double f[MAXC], dx[MAXC], dy[MAXC], dz[MAXC];
 #pragma unroll
-            for (int i = 0; i < MAXC; ++i) gv.get(row + min(l + 64 * i, nbf - 1), f[i], dx[i], dy[i], dz[i]);
+            for (int i = 0; i < MAXC; ++i) {
+                const int col = min(l + 64 * i, nbf - 1);
+                gv.get(row + ((tiles >> (col >> 4)) & 1 ? col : 0), f[i], dx[i], dy[i], dz[i]);
+            }
 #pragma unroll
             for (int i = 0; i < MAXC; ++i)
-                if (l + 64 * i < nbf) aow[row + l + 64 * i] = (T)(c0 * f[i] + c1 * dx[i] + c2 * dy[i] + c3 * dz[i]);
+                if (l + 64 * i < nbf)
+                    aow[row + l + 64 * i] = (tiles >> ((l + 64 * i) >> 4)) & 1
+                                                ? (T)(c0 * f[i] + c1 * dx[i] + c2 * dy[i] + c3 * dz[i]) : T(0);
         } else {
             for (int col = l; col < nbf; col += 64) {
                 double f, dx, dy, dz;
@@ -300,13 +310,19 @@ __global__ __launch_bounds__(256) void xc_rho_kernel(int G, int nbf, const doubl
 // (NH = ceil(NT / 2) MFMA column tiles, one accumulator each), so Phi is read from HBM once per K
 // step instead of once per column pass; D rows k0..k0+15 (all columns) are staged in LDS per K step
 // (D stays L2-resident: every block reads all of it).
+// mask: per 16 points the tiles of 16 functions of which Phi or grad Phi has a nonzero element there
+// (tile_mask_kernel).  K steps that are zero at all 64 points are not staged, and a wavefront multiplies only
+// the K steps and column tiles that its 16 points see: what is left out are exact zeros, so every sum keeps
+// its bits.  (H2O)16, 1.05e6 points, FP32: 2.97 -> 2.50 ms.  (The
+// same in xc_v_kernel: 1.88 -> 3.44 ms, the scan for the next step and the registers cost more.)
 template <typename T, int NT>
 __global__ __launch_bounds__(512) QCG_XC_RHO_ATTR void xc_rho_all_kernel(int G, int nbf, const double* __restrict__ w,
                                                          const T* __restrict__ phi, const GridVals<T> gv,
                                                          const T* __restrict__ Dm, T* __restrict__ aow,
-                                                         double* __restrict__ exc_sum) {
+                                                         double* __restrict__ exc_sum, const unsigned* __restrict__ mask) {
     using M = Mfma<T>;
     using acc_t = typename M::acc;
+    static_assert(NT < 32, "one mask word");
     constexpr int NH = (NT + 1) / 2, BN = 16 * NT, SA = kRhoBM + lds_pad<T>(kRhoBM);
     // Bs row stride: padded for conflict-free fragment reads, and Bs large enough to hold red2 after
     // the K loop (2 x 4 x 16 x 4 doubles)
@@ -340,8 +356,17 @@ __global__ __launch_bounds__(512) QCG_XC_RHO_ATTR void xc_rho_all_kernel(int G, 
             rb[i] = (e < kRhoBK * BN && k < nbf && c < nbf) ? Dm[(size_t)k * nbf + c] : T(0);
         }
     };
-    load(0);
-    for (int k0 = 0; k0 < nbf; k0 += kRhoBK) {
+    static_assert(kRhoBK == 16, "a K step is a tile of the mask");
+    unsigned wm = (1u << NT) - 1, left = wm;  // the wavefront's tiles; the block's K steps still to do
+    if constexpr (NT > kRhoMaskNT) {
+        const unsigned* mk = mask + 4 * (size_t)blockIdx.x;
+        wm = __builtin_amdgcn_readfirstlane(mk[rt]);
+        left = __builtin_amdgcn_readfirstlane(mk[0] | mk[1] | mk[2] | mk[3]);
+    }
+    const auto on = [wm](int t) { return NT <= kRhoMaskNT || ((wm >> t) & 1); };
+    if (left) load(kRhoBK * __builtin_ctz(left));
+    for (; left; left &= left - 1) {
+        const int kt = __builtin_ctz(left);
         __syncthreads();  // the previous step's fragment reads are done
 #pragma unroll
         for (int i = 0; i < NA; ++i) {
@@ -354,20 +379,22 @@ __global__ __launch_bounds__(512) QCG_XC_RHO_ATTR void xc_rho_all_kernel(int G, 
             if (e < kRhoBK * BN) Bs[r][c] = rb[i];
         }
         __syncthreads();
-        if (k0 + kRhoBK < nbf) load(k0 + kRhoBK);
+        if (left & (left - 1)) load(kRhoBK * __builtin_ctz(left & (left - 1)));
+        if (!on(kt)) continue;
         // two k sub-steps per unrolled body: all four hoist 4 NH fragment reads (spills at NH = 8)
 #pragma unroll 2
         for (int ks = 0; ks < kRhoBK; ks += 4) {
             const T a = As[ks + lk][kRhoPW * rt + li];
 #pragma unroll
             for (int t = 0; t < NH; ++t)
-                if (t0 + t < NT) acc[t] = M::mma(a, Bs[ks + lk][16 * (t0 + t) + li], acc[t]);
+                if (t0 + t < NT && on(t0 + t)) acc[t] = M::mma(a, Bs[ks + lk][16 * (t0 + t) + li], acc[t]);
         }
     }
     // rho = sum_mu X Phi, grad rho / 2 = sum_mu X grad Phi over this half's columns
     double rs[4] = {}, xs[4] = {}, ys[4] = {}, zs[4] = {};
 #pragma unroll
     for (int t = 0; t < NH; ++t) {
+        if (!on(t0 + t)) continue;
         // the tile's loads are unconditional, at addresses clamped into the grid and the basis (X is
         // zero outside them, and the product is masked too), so the four rows' loads issue back to
         // back instead of each waiting inside its own branch: (H2O)16 XC, mixed 5.78 -> 5.41 ms,
@@ -420,7 +447,32 @@ __global__ __launch_bounds__(512) QCG_XC_RHO_ATTR void xc_rho_all_kernel(int G, 
         red[r4][p][q] = red2[0][r4][p][q] + red2[1][r4][p][q];
     }
     __syncthreads();
-    xc_point_tail<T, 8, (16 * NT + 63) / 64>(G, nbf, wv, l, g0, w, gv, aow, exc_sum, red, coef, part);
+    xc_point_tail<T, 8, (16 * NT + 63) / 64>(G, nbf, wv, l, g0, w, gv, aow, exc_sum, red, coef, part, NT > kRhoMaskNT ? wm : ~0u);
+}
+
+// One wavefront per 16 points: the tiles of 16 functions with a nonzero element there.
+__global__ __launch_bounds__(256) void tile_mask_kernel(int G, int nbf, int n, const float4* __restrict__ g4,
+                                                        unsigned* __restrict__ mask) {
+    const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (i >= n) return;
+    unsigned m = 0;
+    for (int p = 16 * i; p < min(G, 16 * i + 16); ++p)
+        for (int c = lane; c < nbf; c += 64) {
+            const float4 v = g4[(size_t)p * nbf + c];
+            if (v.x != 0.f || v.y != 0.f || v.z != 0.f || v.w != 0.f) m |= 1u << (c >> 4);
+        }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) m |= __shfl_xor(m, off, 64);
+    if (lane == 0) mask[i] = m;
+}
+
+size_t xc_tile_mask_words(int G, int nbf) { return nbf <= 16 * kRhoAllMaxNT ? 4 * ((size_t)(G + 63) / 64) + 4 : 0; }
+
+hipError_t launch_tile_mask(int G, int nbf, const float4* g4, unsigned* mask, hipStream_t st) {
+    const int n = (int)xc_tile_mask_words(G, nbf);
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL(tile_mask_kernel, dim3((n + 3) / 4), dim3(256), 0, st, G, nbf, n, g4, mask);
+    return hipGetLastError();
 }
 
 // Vparts[chunk] = Phi[chunk rows]^T aow[chunk rows] by 32 VW square output tiles (each wavefront a
@@ -974,7 +1026,7 @@ hipError_t launch_xc_packed(const PackedGrid& g, const double* D, double* aow, c
 template <typename T>
 static hipError_t launch_xc_mfma_t(int G, int nbf, int nchunk, const double* w, const T* phi, const T* dpx,
                                    const T* dpy, const T* dpz, const float4* g4, const T* Dm, T* aow, double* exc_sum,
-                                   double* Vparts, hipStream_t st) {
+                                   double* Vparts, const unsigned* mask, hipStream_t st) {
     const GridVals<T> gv{phi, dpx, dpy, dpz, g4};
     if (G <= 0 || nbf <= 0 || nchunk <= 0) return hipErrorInvalidValue;
     // column passes of at most 5 MFMA tiles (4 for FP64, whose accumulators take twice the
@@ -986,12 +1038,12 @@ static hipError_t launch_xc_mfma_t(int G, int nbf, int nchunk, const double* w, 
     const dim3 grid((G + kRhoBM - 1) / kRhoBM);
     // FP32 up to kRhoAllMaxNT column tiles: the all-columns kernel (Phi read once per K step); FP64 runs
     // here only where the packed form does not apply
-    switch (sizeof(T) == 4 && tiles <= kRhoAllMaxNT ? 100 + tiles : nt) {
+    switch (sizeof(T) == 4 && mask ? 100 + tiles : nt) {
 #define QCG_RHO_ALL(n)                                                                                  \
     case 100 + n:                                                                                       \
         if constexpr (sizeof(T) == 4)                                                                   \
             hipLaunchKernelGGL((xc_rho_all_kernel<T, n>), grid, dim3(512), 0, st, G, nbf, w, phi, gv, Dm, aow, \
-                               exc_sum);                                                                \
+                               exc_sum, mask);                                                              \
         break;
         QCG_RHO_ALL(1) QCG_RHO_ALL(2) QCG_RHO_ALL(3) QCG_RHO_ALL(4) QCG_RHO_ALL(5) QCG_RHO_ALL(6) QCG_RHO_ALL(7)
         QCG_RHO_ALL(8) QCG_RHO_ALL(9) QCG_RHO_ALL(10) QCG_RHO_ALL(11) QCG_RHO_ALL(12) QCG_RHO_ALL(13)
@@ -1048,15 +1100,16 @@ int xc_v_blocks_per_cu(int nbf, bool fp32) {
 }
 
 hipError_t launch_xc_mfma(int G, int nbf, int nchunk, const double* w, const float* phi, const float4* g4,
-                          const float* Dm, float* aow, double* exc_sum, double* Vparts, hipStream_t st) {
+                          const unsigned* mask, const float* Dm, float* aow, double* exc_sum, double* Vparts,
+                          hipStream_t st) {
     return launch_xc_mfma_t<float>(G, nbf, nchunk, w, phi, nullptr, nullptr, nullptr, g4, Dm, aow, exc_sum, Vparts,
-                                   st);
+                                   mask, st);
 }
 
 hipError_t launch_xc_mfma(int G, int nbf, int nchunk, const double* w, const double* phi, const double* dpx,
                           const double* dpy, const double* dpz, const double* Dm, double* aow, double* exc_sum,
                           double* Vparts, hipStream_t st) {
-    return launch_xc_mfma_t<double>(G, nbf, nchunk, w, phi, dpx, dpy, dpz, nullptr, Dm, aow, exc_sum, Vparts, st);
+    return launch_xc_mfma_t<double>(G, nbf, nchunk, w, phi, dpx, dpy, dpz, nullptr, Dm, aow, exc_sum, Vparts, nullptr, st);
 }
 
 }  // namespace qcg

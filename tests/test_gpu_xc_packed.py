@@ -63,6 +63,25 @@ def test_gpu_packed_functions_from_radial_parts(name, basis):
     assert np.abs(V2 - V).max() < 1e-10 and abs(E2 - E) < 1e-10 * max(1.0, abs(E))
 
 
+@pytest.mark.parametrize("n,far,atoms", [(1, 0, 10), (63, 0, 12), (3001, 0, 12), (3001, 700, 10), (3001, 700, 6)])
+def test_gpu_mixed_skips_zero_tiles(n, far, atoms):
+    """The mixed option's dense kernels leave out K steps and tiles that are zero at their points (a long
+    molecule, with points out of every reach in front).  V's elements are sums of FP32 products over at
+    most 4e3 points and 234 functions with weights up to 0.5: 6e-8 times a few tens, 1e-5; E_xc 1e-6."""
+    b = build_basis(workloads.alkane(atoms, 0.03, 4), "6-31g*", units="angstrom")
+    xyz, w = _points(b, n, 7)
+    if far:
+        xyz = np.concatenate([xyz[:far] + np.array([200.0, 0.0, 0.0]), xyz])
+        w = np.concatenate([w[:far], w])
+    D = random_density(b.nbf, seed=9, nocc=b.n_occ)
+    eng = Engine(b, precision="mixed")
+    eng.set_grid(xyz, w)
+    V, E = eng.xc(D)
+    chi, grad = oracle.basis_on_grid(b, xyz)
+    Vo, Eo, _ = oracle.vxc(chi, grad, w, D)
+    assert np.abs(V - Vo).max() < 1e-5 and abs(E - Eo) < 1e-6 * max(1.0, abs(Eo))
+
+
 def test_gpu_packed_follows_the_options():
     b = bench_molecule("H2O", "6-31g*")
     xyz, w = _points(b, 5000, 8)
