@@ -166,7 +166,9 @@ int qcg_build_fock_device(qcg_context* ctx, const double* dH, const double* dD, 
 /* Graph replay for qcg_build_fock_device: on != 0 captures the whole launch sequence of a device
  * Fock build (fill, class kernels on the auxiliary streams, combine) as one HIP graph the first
  * time and replays it afterwards; it is captured again when the buffers, stream, k factor,
- * precision options or tiles change.  Profiling mode always launches eagerly.  No counterpart in
+ * precision options or tiles change, or a call with other options has made the work plan anew in
+ * between.  (A capture of the caller's own holds the plan's lists too: it is good until the options,
+ * tiles or basis change.)  Profiling mode always launches eagerly.  No counterpart in
  * qc-core: launch mode only. */
 int qcg_set_graph(qcg_context* ctx, int on);
 

@@ -54,6 +54,7 @@ int grad_plan(qcg_context* c) {
             }
             c->grad_cnt[cls] = (int)items.size() - c->grad_off[cls];
         }
+    c->grad_key[0] = -1.0;  // no plan until both lists are on the device
     c->release(c->d_grad_items);
     c->release(c->d_grad_segs);
     c->d_grad_items = nullptr;

@@ -585,6 +585,11 @@ static int build_plan(qcg_context* c) {
     for (const PairRec& pr : c->pairs)
         if (pr.npp > kItemMaxPrim)
             return fail(c, QCG_INVALID_ARG, "shell pair with more than 255 primitive pairs (at most 15 primitives per shell)");
+    // the captured Fock graph holds the lists that are released below, and its key (options, tiles, buffers)
+    // cannot tell a plan made again for the same options from the one it was captured with; until the new
+    // lists are on the device there is no plan
+    c->drop_fock_graph();
+    c->plan_sig = 0;
     c->items.clear();
     c->segs.clear();
     const int nmol = c->nmol;
@@ -1250,6 +1255,7 @@ static int tensor_plan(qcg_context* c) {
             }
             c->tensor_cnt[cls] = (int)items.size() - c->tensor_off[cls];
         }
+    c->tensor_key = -1.0;  // no plan until both lists are on the device
     c->release(c->d_tensor_items);
     c->release(c->d_tensor_segs);
     c->d_tensor_items = nullptr;
