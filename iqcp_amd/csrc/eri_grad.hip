@@ -211,9 +211,9 @@ struct GradArgs {
 
 __device__ __forceinline__ PairRec grad_ket(const KetPairs& k, int kq, const int4 km) {
     PairRec Q;
-    Q.bfa = km.x & ~kKetSame;
-    Q.bfb = km.y;
-    Q.npp = (unsigned)km.w >> 24;
+    Q.bfa = km.x & kKetBfMask;
+    Q.bfb = (km.x >> kKetBfBits) & kKetBfMask;
+    Q.npp = km.y;
     const double2 c0 = k.cen[kq], c1 = k.cen[k.np + kq], c2 = k.cen[2 * k.np + kq];
     Q.ax = c0.x, Q.ay = c0.y, Q.az = c1.x, Q.abx = c1.y, Q.aby = c2.x, Q.abz = c2.y;
     return Q;
@@ -373,7 +373,7 @@ __global__ __launch_bounds__(kGradLaneBlock) void grad_lane_kernel(const int4* _
                    (cnorm(LA, a) * cnorm(LB, b) * cnorm(LC, c) * cnorm(LD, d));
         });
         double gq[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-        grad_quartet_lane<LA, LB, LC, LD, A0, NAS>(P, Q, ga, km.z, km.w & 0xffffff, sub, lanes, rys_n, W, gq);
+        grad_quartet_lane<LA, LB, LC, LD, A0, NAS>(P, Q, ga, km.z, km.w, sub, lanes, rys_n, W, gq);
         const int2 at = ga.kpairs.atoms[q];
 #pragma unroll
         for (int x = 0; x < 3; ++x) {

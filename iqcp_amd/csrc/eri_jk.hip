@@ -65,9 +65,9 @@ constexpr int rys_lds_doubles() { return N <= 3 ? rys_tab_size<N>() : 1; }
 template <int LC, int LD>
 __device__ __forceinline__ PairRec ket_pair(const KetPairs& k, int kq, const int4 km) {
     PairRec Q;
-    Q.bfa = km.x & ~kKetSame;
-    Q.bfb = km.y;
-    Q.npp = (unsigned)km.w >> 24;
+    Q.bfa = km.x & kKetBfMask;
+    Q.bfb = (km.x >> kKetBfBits) & kKetBfMask;
+    Q.npp = km.y;
     if constexpr (LC > 0) {
         const double2 c0 = k.cen[kq], c1 = k.cen[k.np + kq];
         Q.ax = c0.x, Q.ay = c0.y, Q.az = c1.x, Q.abx = c1.y;
@@ -134,7 +134,7 @@ __device__ __forceinline__ void jk_item(const int4 it, const JkArgs& g, const Ke
         const int q = cur.at(), kq = ket0 + q;
         const int4 km = g.kpairs.meta[kq];
         const PairRec Q = ket_pair<LC, LD>(g.kpairs, kq, km);
-        const int kstride = km.w & 0xffffff;
+        const int kstride = km.w;
         R eri[NQ];
         for_n<true, NQ>([&](int i) { eri[i] = R(0); });
         contract_quartet_pp<LA, LB, LC, LD, R, true, A0 * S::NB * S::NCD, NQ>(
@@ -469,7 +469,7 @@ __global__ __launch_bounds__(128) void eri_tensor_kernel(const int4* __restrict_
         const int q = cur.at();
         const int4 km = g.kpairs.meta[q];
         const PairRec Q = ket_pair<LC, LD>(g.kpairs, q, km);
-        const int kstride = km.w & 0xffffff;
+        const int kstride = km.w;
         double eri[S::NQ];
         for_n<true, S::NQ>([&](int i) { eri[i] = 0.0; });
         contract_quartet_pp<LA, LB, LC, LD, double, true>(

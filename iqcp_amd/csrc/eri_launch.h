@@ -39,10 +39,11 @@ inline void cut_items(std::vector<int4>& items, const std::vector<int2>& segs, i
 }
 
 // cut_items for every primitive range of a bra pair with npp primitive pairs: ranges of at most
-// split pairs (split <= 0 or npp <= split: one range, the whole pair), sizes balanced
+// split pairs (split <= 0 or npp <= split: one range, the whole pair), sizes balanced; npp is at most
+// kItemMaxPrim (the planners refuse longer contractions)
 inline void cut_items_split(std::vector<int4>& items, const std::vector<int2>& segs, int g0, int g1, int bra, int ch,
                             int npp, int split, int lg = 0) {
-    if (split <= 0 || npp <= split || npp > kItemMaxPrim) {
+    if (split <= 0 || npp <= split) {
         cut_items(items, segs, g0, g1, bra, ch, lg);
         return;
     }

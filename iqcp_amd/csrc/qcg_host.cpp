@@ -383,7 +383,7 @@ int qcg_set_basis_batch(qcg_context* c, int nmol, const int* mol_nshell, const i
                     for (int i = 0; i < n; ++i) {
                         const int g = base + bnd[b] + i;
                         const PairRec& r = all[g];
-                        meta[g] = make_int4(r.bfa | (r.sa == r.sb ? kKetSame : 0), r.bfb, first + i, (int)(((unsigned)npp << 24) | (unsigned)n));
+                        meta[g] = make_int4(r.bfa | r.bfb << kKetBfBits | (r.sa == r.sb ? kKetSame : 0), npp, first + i, n);
                         katoms[g] = make_int2(r.atom_a, r.atom_b);
                         cen[g] = make_double2(r.ax, r.ay);
                         cen[(size_t)np + g] = make_double2(r.az, r.abx);
@@ -1232,12 +1232,11 @@ int qcg_build_fock(qcg_context* c, const double* H, const double* D, double* F) 
 
 // Work items of the compressed tensor (qcg_eri_compressed): every bra's surviving kets in FP64, the
 // heavily contracted ones on several lanes; blocks of kTensorBlock lanes or, for the classes above
-// kTensorLaneMaxNQ components, wavefronts of one ket.  Made once per basis and threshold.
+// kTensorLaneMaxNQ components, wavefronts of one ket.  Bras are never cut into primitive ranges, so any
+// contraction length will do.  Made once per basis and threshold.
 constexpr int kTensorBlock = 64;
 static int tensor_plan(qcg_context* c) {
     if (c->d_tensor_items && c->tensor_key == c->schwarz_thr) return QCG_OK;
-    for (const PairRec& pr : c->pairs)
-        if (pr.npp > kItemMaxPrim) return fail(c, QCG_INVALID_ARG, "shell pair with more than 255 primitive pairs");
     std::vector<int4> items;
     std::vector<int2> segs;
     for (int cls = 0, cb = kNumPairClasses - 1; cb >= 0; --cb)

@@ -78,11 +78,13 @@ struct KetPrims<float> {
     }
 };
 struct KetPairs {
-    const int4* meta;     // bfa | (sa == sb) << 30, bfb, first primitive, npp << 24 | stride
+    const int4* meta;     // bfa | bfb << 15 | (sa == sb) << 30, npp, first primitive, stride
     const double2* cen;   // np x (ax, ay), np x (az, abx), np x (aby, abz)
     int np;               // pairs of all classes (the stride of cen)
     const int2* atoms;    // the two shells' atoms (gradient kernels)
 };
 constexpr int kKetSame = 1 << 30;
+constexpr int kKetBfBits = 15;  // a molecule has at most 4096 shells (qcg_set_basis), 24576 functions
+constexpr int kKetBfMask = (1 << kKetBfBits) - 1;
 
 }  // namespace qcg
