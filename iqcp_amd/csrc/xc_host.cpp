@@ -340,9 +340,11 @@ int xc_build(qcg_context* c, const double* dD, double* dV, double* dExc, hipStre
     if (c->G <= 0) return fail(c, QCG_NO_GRID, "no grid: call qcg_build_grid or qcg_set_grid");
     // mode 0: the dense MFMA kernels with FP32 products in the mixed option, else the packed FP64 MFMA
     // kernels, and the library DGEMMs for grids with blocks of more than kPackedMaxLd functions; mode 1:
-    // library DGEMMs for both; mode 2: MFMA kernels for both.  (A caller that captures its first FP64
-    // build on a grid made for the mixed option gets the dense FP64 kernels: the packed arrays cannot be
-    // made inside a capture.)
+    // library DGEMMs for both; mode 2: MFMA kernels for both.  A caller that captures its first FP64
+    // build on a grid made for the mixed option gets the dense FP64 kernels, since the packed arrays cannot
+    // be made inside a capture: (H2O)16, 286201 points, 3.3 ms with all columns of X held per wavefront and
+    // 4.6 ms in column passes; above kPackedMaxLd functions, where the MFMA kernels would make column
+    // passes, the library form if its handle is there.
     const bool mixed = c->precision == QCG_PREC_MIXED;
     if (!mixed && c->xc_mode != 1 && !(c->pk_state == 0 && c->d_phi && capturing(st))) {
         int rc = ensure_packed(c);
@@ -356,7 +358,8 @@ int xc_build(qcg_context* c, const double* dD, double* dV, double* dExc, hipStre
     }
     int rc = ensure_dense(c);
     if (rc) return rc;
-    if (c->xc_mode == 2 || (c->xc_mode == 0 && (mixed || c->pk_state == 0))) return xc_build_mfma(c, dD, dV, dExc, st);
+    const bool dense64 = c->pk_state == 0 && (c->basis.nbf <= kPackedMaxLd || !c->blas);
+    if (c->xc_mode == 2 || (c->xc_mode == 0 && (mixed || dense64))) return xc_build_mfma(c, dD, dV, dExc, st);
     rc = ensure_blas(c);
     if (rc) return rc;
     const int nbf = c->basis.nbf;

@@ -4,8 +4,8 @@
 //                   grad rho (X never goes to HBM), then B3LYP per point (FP64), the aow rows and
 //                   E_xc -- the work of compute_density_and_gradient_matmul and the point part of
 //                   build_vxc_gga_matmul (dft/ks_scf.rs:1028-1093, :1150-1296) in one kernel;
-//   xc_rho_all_kernel : the same in FP32 for nbf <= 352 with X for all columns held per wavefront, so
-//                   Phi is read once per K step instead of once per column pass;
+//   xc_rho_all_kernel : the same for nbf <= 352 with X for all columns held per wavefront, so Phi is read
+//                   once per K step instead of once per column pass;
 //   xc_rho_packed_kernel, xc_v_packed_kernel : the FP64 build on the packed grid (xc_packed.h);
 //   xc_v_kernel   : V = Phi^T aow as 128x128 output tiles over grid chunks (split K), one partial
 //                   matrix per chunk, summed and symmetrised afterwards (sum_parts, sym_half).
@@ -310,7 +310,10 @@ __global__ __launch_bounds__(256) void xc_rho_kernel(int G, int nbf, const doubl
 // (NH = ceil(NT / 2) MFMA column tiles, one accumulator each), so Phi is read from HBM once per K
 // step instead of once per column pass; D rows k0..k0+15 (all columns) are staged in LDS per K step
 // (D stays L2-resident: every block reads all of it).
-// mask: per 16 points the tiles of 16 functions of which Phi or grad Phi has a nonzero element there
+// FP64 products run here in a build that is captured on a grid made for the mixed option (xc_build); they
+// stage D without the look-ahead, whose registers would cost the second block per CU ((H2O)16, 1.05e6 points:
+// 11.2 -> 9.3 ms), and take no mask.
+// mask (FP32): per 16 points the tiles of 16 functions of which Phi or grad Phi has a nonzero element there
 // (tile_mask_kernel).  K steps that are zero at all 64 points are not staged, and a wavefront multiplies only
 // the K steps and column tiles that its 16 points see: what is left out are exact zeros, so every sum keeps
 // its bits.  (H2O)16, 1.05e6 points, FP32: 2.97 -> 2.50 ms.  (The
@@ -341,29 +344,32 @@ __global__ __launch_bounds__(512) QCG_XC_RHO_ATTR void xc_rho_all_kernel(int G, 
     acc_t acc[NH];
 #pragma unroll
     for (int t = 0; t < NH; ++t) acc[t] = acc_t{T(0), T(0), T(0), T(0)};
-    // next K step's Phi and D elements, loaded while the current step is multiplied
+    // next K step's Phi (FP32: and D) elements, loaded while the current step is multiplied
+    constexpr bool kAheadD = sizeof(T) == 4, kMask = sizeof(T) == 4 && NT > kRhoMaskNT;
     constexpr int NBD = (kRhoBK * BN + 511) / 512;
-    T ra[NA], rb[NBD];
+    T ra[NA], rb[kAheadD ? NBD : 1];
     auto load = [&](int k0) {
 #pragma unroll
         for (int i = 0; i < NA; ++i) {
             const int e = tid + 512 * i, r = e / kRhoBK, c = e % kRhoBK, g = g0 + r, k = k0 + c;
             ra[i] = (g < G && k < nbf) ? phi[(size_t)g * nbf + k] : T(0);
         }
+        if constexpr (kAheadD) {
 #pragma unroll
-        for (int i = 0; i < NBD; ++i) {
-            const int e = tid + 512 * i, r = e / BN, c = e - r * BN, k = k0 + r;
-            rb[i] = (e < kRhoBK * BN && k < nbf && c < nbf) ? Dm[(size_t)k * nbf + c] : T(0);
+            for (int i = 0; i < NBD; ++i) {
+                const int e = tid + 512 * i, r = e / BN, c = e - r * BN, k = k0 + r;
+                rb[i] = (e < kRhoBK * BN && k < nbf && c < nbf) ? Dm[(size_t)k * nbf + c] : T(0);
+            }
         }
     };
     static_assert(kRhoBK == 16, "a K step is a tile of the mask");
     unsigned wm = (1u << NT) - 1, left = wm;  // the wavefront's tiles; the block's K steps still to do
-    if constexpr (NT > kRhoMaskNT) {
+    if constexpr (kMask) {
         const unsigned* mk = mask + 4 * (size_t)blockIdx.x;
         wm = __builtin_amdgcn_readfirstlane(mk[rt]);
         left = __builtin_amdgcn_readfirstlane(mk[0] | mk[1] | mk[2] | mk[3]);
     }
-    const auto on = [wm](int t) { return NT <= kRhoMaskNT || ((wm >> t) & 1); };
+    const auto on = [wm](int t) { return !kMask || ((wm >> t) & 1); };
     if (left) load(kRhoBK * __builtin_ctz(left));
     for (; left; left &= left - 1) {
         const int kt = __builtin_ctz(left);
@@ -373,10 +379,17 @@ __global__ __launch_bounds__(512) QCG_XC_RHO_ATTR void xc_rho_all_kernel(int G, 
             const int e = tid + 512 * i;
             As[e % kRhoBK][e / kRhoBK] = ra[i];
         }
+        if constexpr (kAheadD) {
 #pragma unroll
-        for (int i = 0; i < NBD; ++i) {
-            const int e = tid + 512 * i, r = e / BN, c = e - r * BN;
-            if (e < kRhoBK * BN) Bs[r][c] = rb[i];
+            for (int i = 0; i < NBD; ++i) {
+                const int e = tid + 512 * i, r = e / BN, c = e - r * BN;
+                if (e < kRhoBK * BN) Bs[r][c] = rb[i];
+            }
+        } else {
+            for (int e = tid; e < kRhoBK * BN; e += 512) {
+                const int r = e / BN, c = e - r * BN, k = kRhoBK * kt + r;
+                Bs[r][c] = (k < nbf && c < nbf) ? Dm[(size_t)k * nbf + c] : T(0);
+            }
         }
         __syncthreads();
         if (left & (left - 1)) load(kRhoBK * __builtin_ctz(left & (left - 1)));
@@ -447,7 +460,7 @@ __global__ __launch_bounds__(512) QCG_XC_RHO_ATTR void xc_rho_all_kernel(int G, 
         red[r4][p][q] = red2[0][r4][p][q] + red2[1][r4][p][q];
     }
     __syncthreads();
-    xc_point_tail<T, 8, (16 * NT + 63) / 64>(G, nbf, wv, l, g0, w, gv, aow, exc_sum, red, coef, part, NT > kRhoMaskNT ? wm : ~0u);
+    xc_point_tail<T, 8, (16 * NT + 63) / 64>(G, nbf, wv, l, g0, w, gv, aow, exc_sum, red, coef, part, kMask ? wm : ~0u);
 }
 
 // One wavefront per 16 points: the tiles of 16 functions with a nonzero element there.
@@ -1036,14 +1049,12 @@ static hipError_t launch_xc_mfma_t(int G, int nbf, int nchunk, const double* w, 
     constexpr int kMaxNT = sizeof(T) == 8 ? 4 : 5;
     const int tiles = (nbf + 15) / 16, passes = (tiles + kMaxNT - 1) / kMaxNT, nt = (tiles + passes - 1) / passes;
     const dim3 grid((G + kRhoBM - 1) / kRhoBM);
-    // FP32 up to kRhoAllMaxNT column tiles: the all-columns kernel (Phi read once per K step); FP64 runs
-    // here only where the packed form does not apply
-    switch (sizeof(T) == 4 && mask ? 100 + tiles : nt) {
+    // up to kRhoAllMaxNT column tiles: the all-columns kernel (Phi read once per K step)
+    switch (tiles <= kRhoAllMaxNT && (sizeof(T) == 8 || mask) ? 100 + tiles : nt) {
 #define QCG_RHO_ALL(n)                                                                                  \
     case 100 + n:                                                                                       \
-        if constexpr (sizeof(T) == 4)                                                                   \
-            hipLaunchKernelGGL((xc_rho_all_kernel<T, n>), grid, dim3(512), 0, st, G, nbf, w, phi, gv, Dm, aow, \
-                               exc_sum, mask);                                                              \
+        hipLaunchKernelGGL((xc_rho_all_kernel<T, n>), grid, dim3(512), 0, st, G, nbf, w, phi, gv, Dm, aow,  \
+                           exc_sum, mask);                                                              \
         break;
         QCG_RHO_ALL(1) QCG_RHO_ALL(2) QCG_RHO_ALL(3) QCG_RHO_ALL(4) QCG_RHO_ALL(5) QCG_RHO_ALL(6) QCG_RHO_ALL(7)
         QCG_RHO_ALL(8) QCG_RHO_ALL(9) QCG_RHO_ALL(10) QCG_RHO_ALL(11) QCG_RHO_ALL(12) QCG_RHO_ALL(13)

@@ -1,0 +1,63 @@
+"""XC builds inside a caller's stream capture, where nothing can be allocated: which kernels run depends on
+the arrays that the grid has by then.
+
+Tolerance: V elements are sums over 1500 points of products of FP64 values of size <= 10 with weights up to
+0.5, rounded below 1e-15 of the largest term on either side; the oracle drops functions below 1e-10 on its
+512-point blocks, below the same bound after weighting: 1e-10 absolute, E_xc 1e-10 relative."""
+import numpy as np
+import pytest
+
+import oracle
+from helpers import bench_molecule, random_density
+from iqcp_amd import workloads
+from iqcp_amd.basis import build_basis
+from iqcp_amd.engine import Engine
+
+pytestmark = pytest.mark.gpu
+
+
+def _water(n):
+    return bench_molecule("H2O", "sto-3g") if n == 0 else build_basis(workloads.water_cluster((n, 1, 1), 2.9, 3), "6-31g*", units="angstrom")
+
+
+def _grid(b, n, seed):
+    rng = np.random.default_rng(seed)
+    return b.xyz[rng.integers(0, b.natom, n)] + rng.normal(0.0, 1.5, (n, 3)), rng.uniform(0.0, 0.5, n)
+
+
+def _captured(eng, D, prepare=lambda: None):
+    """V and E of three replays of a captured build, eager work of the device in between."""
+    import torch
+    st, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    dD = torch.tensor(D, device="cuda")
+    V, E = torch.full_like(dD, 7.0), torch.full((1,), 7.0, dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=st):
+        prepare()
+        eng.xc_device(dD.data_ptr(), V.data_ptr(), E.data_ptr(), st.cuda_stream)
+    out = []
+    for _ in range(3):
+        V.fill_(7.0)
+        E.fill_(7.0)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        out.append((V.cpu().numpy(), float(E[0])))
+    return out
+
+
+@pytest.mark.parametrize("nw", [0, 1, 4, 12, 13, 16, 18])
+def test_gpu_fp64_captured_on_a_mixed_grid(nw):
+    """A grid made for the mixed option, FP64 set, the first FP64 build captured: the dense FP64 kernels at 1
+    to 22 tiles of 16 functions ((H2O)n, 19 functions each)."""
+    b = _water(nw)
+    xyz, w = _grid(b, 1500, nw)
+    D = random_density(b.nbf, seed=9, nocc=b.n_occ)
+    Vo, Eo, _ = oracle.vxc(*oracle.basis_on_grid(b, xyz), w, D)
+    eng = Engine(b, precision="mixed")
+    eng.set_grid(xyz, w)
+    eng.set_options("fp64")
+    for V, E in _captured(eng, D):
+        assert np.abs(V - Vo).max() < 1e-10 and abs(E - Eo) < 1e-10 * max(1.0, abs(Eo))
+    V, E = eng.xc(D)  # eager on the same grid: the packed kernels
+    assert np.abs(V - Vo).max() < 1e-10 and abs(E - Eo) < 1e-10 * max(1.0, abs(Eo))
