@@ -250,7 +250,10 @@ int qcg_xc_device(qcg_context* ctx, const double* dD, double* dVxc, double* dExc
  * precision option, and MFMA kernels with FP64 products for FP64 on spatial blocks of the grid that keep
  * only the functions reaching them (the library form for a grid with a block of more than 352
  * functions); mode 1: library form for both options; mode 2: MFMA kernels for both
- * (FP64 products for FP64).  No counterpart in qc-core: kernel selection only. */
+ * (FP64 products for FP64).  Inside a stream capture a build runs on the arrays that the grid has by
+ * then: the library form wants one build in mode 1 outside it first, and on a grid made under FP64 a
+ * captured build of mode 1 without one runs the packed MFMA kernels.  No counterpart in qc-core: kernel
+ * selection only. */
 int qcg_set_xc_mode(qcg_context* ctx, int mode);
 /* ks_scf (dft/ks_scf.rs:1567) for B3LYP on the current grid: F = H + J - (a/2) K + V_xc. */
 int qcg_ks_scf(qcg_context* ctx, const qcg_scf_config* cfg, const double* D_init, qcg_scf_result* res, double* D,

@@ -344,9 +344,12 @@ int xc_build(qcg_context* c, const double* dD, double* dV, double* dExc, hipStre
     // build on a grid made for the mixed option gets the dense FP64 kernels, since the packed arrays cannot
     // be made inside a capture: (H2O)16, 286201 points, 3.3 ms with all columns of X held per wavefront and
     // 4.6 ms in column passes; above kPackedMaxLd functions, where the MFMA kernels would make column
-    // passes, the library form if its handle is there.
+    // passes, the library form if its handle is there.  Likewise the library form of FP64 needs the dense
+    // arrays, which a grid made for FP64 gets from the first build in mode 1 outside a capture: until then a
+    // captured build runs the packed kernels.
     const bool mixed = c->precision == QCG_PREC_MIXED;
-    if (!mixed && c->xc_mode != 1 && !(c->pk_state == 0 && c->d_phi && capturing(st))) {
+    const bool cap = capturing(st);
+    if (!mixed && (c->xc_mode != 1 ? !(c->pk_state == 0 && c->d_phi && cap) : c->pk_state == 1 && !c->d_phi && cap)) {
         int rc = ensure_packed(c);
         if (rc) return rc;
         if (c->pk_state == 1) {

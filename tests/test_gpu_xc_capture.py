@@ -61,3 +61,25 @@ def test_gpu_fp64_captured_on_a_mixed_grid(nw):
         assert np.abs(V - Vo).max() < 1e-10 and abs(E - Eo) < 1e-10 * max(1.0, abs(Eo))
     V, E = eng.xc(D)  # eager on the same grid: the packed kernels
     assert np.abs(V - Vo).max() < 1e-10 and abs(E - Eo) < 1e-10 * max(1.0, abs(Eo))
+
+
+@pytest.mark.parametrize("when", ["before", "inside", "after_gradient", "after_build"])
+def test_gpu_library_form_captured_on_an_fp64_grid(when):
+    """Mode 1 on a grid made for FP64, its first build captured: set before or inside the capture, after an XC
+    gradient, and after an eager build of mode 1 (which makes the dense arrays)."""
+    b = _water(4)
+    xyz, w = _grid(b, 1500, 5)
+    D = random_density(b.nbf, seed=9, nocc=b.n_occ)
+    Vo, Eo, _ = oracle.vxc(*oracle.basis_on_grid(b, xyz), w, D)
+    eng = Engine(b)
+    eng.set_grid(xyz, w)
+    if when == "after_gradient":
+        eng.xc_gradient(D)
+    if when != "inside":
+        eng.set_xc_mode(1)
+    if when == "after_build":
+        eng.xc(D)
+    for V, E in _captured(eng, D, (lambda: eng.set_xc_mode(1)) if when == "inside" else (lambda: None)):
+        assert np.abs(V - Vo).max() < 1e-10 and abs(E - Eo) < 1e-10 * max(1.0, abs(Eo))
+    V, E = eng.xc(D)
+    assert np.abs(V - Vo).max() < 1e-10 and abs(E - Eo) < 1e-10 * max(1.0, abs(Eo))
