@@ -241,16 +241,6 @@ __device__ __forceinline__ void jk_item(const int4 it, const JkArgs& g, const Ke
     }
 }
 
-// Dynamic LDS of a per-lane block: the K rows for nbf functions (the largest molecule's), when they
-// fit the budget left by the Rys coefficients; 0: K goes to memory directly.
-constexpr size_t kLdsBudget = 65536;
-template <int LA, int LB, int LC, int LD>
-inline size_t jk_row_bytes(int nas, int nbf, int do_k) {
-    using S = EriShape<LA, LB, LC, LD>;
-    const size_t kb = (size_t)(nas + S::NB) * nbf * sizeof(fix_t);
-    return do_k && (size_t)rys_lds_doubles<S::NROOTS>() * sizeof(double) + kb <= kLdsBudget ? kb : 0;
-}
-
 template <int LA, int LB, int LC, int LD, typename R, bool KROWS, int A0, int NAS>
 __global__ __launch_bounds__(256) void jk_kernel(const int4* __restrict__ items, const JkArgs g, const KetPrims<R> kprims,
                                                  const PrimPair<R>* __restrict__ pp, const R* __restrict__ rys_tab) {
@@ -532,7 +522,7 @@ static JkArgs jk_args(const JkLaunch& a) {
 template <int LA, int LB, int LC, int LD, typename R, int NAS, int A0 = 0>
 static hipError_t launch_jk_parts(const JkLaunch& a, const JkArgs& g, hipStream_t st) {
     // K rows of the bra functions in LDS when they fit (a.nbf is the largest molecule's nbf)
-    const size_t rows = jk_row_bytes<LA, LB, LC, LD>(NAS, a.nbf, a.do_k);
+    const size_t rows = a.do_k ? jk_row_bytes(NAS + ncart(LB), jk_table_bytes(EriShape<LA, LB, LC, LD>::NROOTS), a.nbf) : 0;
     const KetPrims<R>* kp;
     if constexpr (sizeof(R) == 8) kp = &a.kprims;
     else kp = &a.kprimsf;
@@ -549,7 +539,7 @@ static hipError_t launch_jk_parts(const JkLaunch& a, const JkArgs& g, hipStream_
 }
 template <int LA, int LB, int LC, int LD, int NAS, int A0 = 0>
 static hipError_t launch_jk_mp_parts(const JkLaunch& a, const JkArgs& g, hipStream_t st) {
-    const size_t rows = jk_row_bytes<LA, LB, LC, LD>(NAS, a.nbf, a.do_k);
+    const size_t rows = a.do_k ? jk_row_bytes(NAS + ncart(LB), jk_table_bytes(EriShape<LA, LB, LC, LD>::NROOTS), a.nbf) : 0;
     auto go = [&](auto rows_c) {
         hipLaunchKernelGGL((jk_kernel_mp<LA, LB, LC, LD, decltype(rows_c)::value, A0, NAS>), dim3(a.nitems),
                            dim3(a.block > 0 ? a.block : 64), rows, st, a.items, a.n64, g, a.kprims, a.kprimsf,

@@ -5,6 +5,7 @@
 
 #include "fixacc.h"
 #include "qcg_types.h"
+#include "rys.h"
 
 namespace qcg {
 
@@ -86,6 +87,16 @@ constexpr int jk_part(int cb, int ck) {
     for (int n = na; n >= 1; --n)
         if (na % n == 0 && n * rest <= kJkPartMaxNQ) return n;
     return 0;
+}
+
+// LDS of a per-lane J/K block: the Rys coefficients of nr nodes when they are staged (else one word), and the K rows of the
+// bra's functions (nrow of them in a part) for nbf functions (the largest molecule's) when they fit the
+// budget that the coefficients leave; 0 rows: K goes to memory directly.
+constexpr size_t kJkLdsBudget = 65536;
+inline size_t jk_table_bytes(int nr) { return nr <= 3 ? (size_t)(qcg_rys_off[nr + 1] - qcg_rys_off[nr]) * sizeof(double) : sizeof(double); }
+inline size_t jk_row_bytes(int nrow, size_t table, int nbf) {
+    const size_t kb = (size_t)nrow * nbf * sizeof(fix_t);
+    return table + kb <= kJkLdsBudget ? kb : 0;
 }
 
 // The same limit for the compressed tensor's kernels.

@@ -541,8 +541,8 @@ double qcg::model_flops(int cb, int ck) {
 constexpr int64_t kPartsMinQuartets = 16384;
 
 // Tiles when the caller has set or tuned none.  Per-lane kernels: the block is widened from 64 to 256
-// threads until the waves that fit a CU's 160 KB of LDS next to each other (the K rows of one bra and
-// the Rys table are per block) reach what the kernel's registers allow (`want` per SIMD), as far as a
+// threads until the waves that fit a CU's 160 KB of LDS next to each other (the K rows of one bra, where
+// they are kept there, and the Rys table are per block) reach what the kernel's registers allow (`want` per SIMD), as far as a
 // bra has kets for the block, and never below 128 from 65536 quartets on (two blocks of them per CU: fewer
 // K-row flushes and table copies, (H2O)16 (dp|ps) 0.27 -> 0.23 ms, (dd|ps) 0.19 -> 0.16, build 2.64 -> 2.49 ms;
 // with 128 from any size on decane's mixed build went 1.30 -> 1.31 ms); a lane takes several kets once that still leaves 16384 waves.  (H2O)16
@@ -567,10 +567,10 @@ static void default_tiles(qcg_context* c, const int64_t (&quartets)[21][2], cons
                 class_l(cb, la, lb);
                 class_l(ck, lc, ld);
                 const int nr = (la + lb + lc + ld) / 2 + 1;
-                const int lds = (nr <= 3 ? (qcg_rys_off[nr + 1] - qcg_rys_off[nr]) * 8 : 0) + (jk_part(cb, ck) + ncart(lb)) * c->max_nbf * 8;
+                const size_t table = jk_table_bytes(nr), lds = table + jk_row_bytes(jk_part(cb, ck) + ncart(lb), table, c->max_nbf);
                 const int want = nq <= 1 ? 7 : nq <= 3 ? 5 : nq <= 9 ? 4 : nq <= 18 ? 3 : nq <= 36 ? 2 : 1;
                 int block = n >= 65536 ? 128 : 64;
-                while (block < 256 && (163840 / std::max(lds, 1)) * (block / 64) < 4 * want) block *= 2;
+                while (block < 256 && (int)(163840 / std::max<size_t>(lds, 1)) * (block / 64) < 4 * want) block *= 2;
                 while (block > 64 && per_bra < block * 3 / 4) block /= 2;
                 int64_t reps = std::min<int64_t>(n / 64 / 16384, per_bra / block);
                 t = {block, (int)std::max<int64_t>(1, std::min<int64_t>(8, reps))};

@@ -140,3 +140,20 @@ def test_gpu_tensor_of_long_contractions(n):
         for call in (eng.build_jk, eng.eri_gradient):
             with pytest.raises(QcgError, match="255 primitive pairs"):
                 call(D)
+
+
+@pytest.mark.parametrize("n", [35, 45, 62])
+def test_gpu_jk_rows_of_k_out_of_lds(n):
+    """J and K of 525, 675 and 930 functions (neon atoms 40 bohr apart), where first (dd|ss), then the classes
+    with nine rows and a staged table, last those without a table keep their K rows in memory; per-lane
+    kernels forced for the classes in parts too."""
+    b = build_basis([("Ne", (40.0 * (i % 8), 40.0 * (i // 8), 0.0)) for i in range(n)], "6-31g*")
+    D = random_density(b.nbf, seed=3, nocc=b.n_occ)
+    Jo, Ko, _ = oracle.jk_direct(b, D)
+    eng = Engine(b)
+    for tile in (None, (64, 1), (256, 2)):
+        if tile:
+            eng.set_tiles([tile] * 21)
+        jk = eng.build_jk(D)
+        assert np.abs(jk.J - Jo).max() < 1e-11 * np.abs(Jo).max() and np.abs(jk.K - Ko).max() < 1e-11 * np.abs(Ko).max()
+    assert np.abs(eng.build_jk(D, want_j=False).K - Ko).max() < 1e-11 * np.abs(Ko).max()
