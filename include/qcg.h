@@ -203,7 +203,8 @@ int qcg_autotune_refine(qcg_context* ctx, const double* dD, int builds, int* cho
  * Block 0 on a class with fewer than 27 components runs the per-lane kernel with 64 threads; classes
  * with more than 81 components run the per-lane kernel in several launches, each for a part of the
  * first shell's components, and (dd|dp) and (dd|dd) always the wave-cooperative one (kets per wave =
- * the tile's kets for block 0, block x kets otherwise). */
+ * the tile's kets for block 0, block x kets otherwise).  Until they are set or tuned, tiles are chosen for
+ * the basis and the options; qcg_get_tiles then returns those of the next build with the current options. */
 int qcg_set_tiles(qcg_context* ctx, const int* tiles);
 int qcg_get_tiles(qcg_context* ctx, int* tiles);
 /* Launch schedule of the J/K class kernels.  A build launches the 21 class kernels longest first,

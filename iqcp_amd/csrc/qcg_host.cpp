@@ -57,8 +57,7 @@ int qcg_create(qcg_context** out, int device) {
             const int la = cb == 0 ? 0 : cb <= 2 ? 1 : 2, lb = (cb == 0 || cb == 1 || cb == 3) ? 0 : (cb == 2 || cb == 4) ? 1 : 2;
             const int lc = ck == 0 ? 0 : ck <= 2 ? 1 : 2, ld = (ck == 0 || ck == 1 || ck == 3) ? 0 : (ck == 2 || ck == 4) ? 1 : 2;
             const int nq = ncart(la) * ncart(lb) * ncart(lc) * ncart(ld);
-            // defaults close to what the autotuner picks on alkanes: the wave-cooperative kernel
-            // (block 0) above kJkLaneMaxNQ components, the per-lane kernel up to it
+            // what qcg_get_tiles returns until there is a basis to choose tiles for (default_tiles)
             for (int part = 0; part < 2; ++part) {
                 c->tile[cls][part].block = nq > kJkLaneMaxNQ ? 0 : (nq <= 3 ? 256 : 64);
                 c->tile[cls][part].reps = nq >= 162 ? 1 : nq > kJkLaneMaxNQ ? 2 : nq >= 18 ? 4 : 1;
@@ -496,11 +495,12 @@ int qcg_screen_counts(qcg_context* c, int64_t* n_kept, int64_t* n_fp32) {
 
 }  // extern "C"
 
-static bool plan_fresh(const qcg_context* c) {
+// The work plan is that of the current options and tiles.
+static bool plan_current(const qcg_context* c) {
     const double key[4] = {(double)c->precision, c->fp32_cutoff, c->schwarz_thr, (double)c->tile_sig};
-    return c->plan_sig == 1 && std::memcmp(key, c->plan_key, sizeof(key)) == 0 && c->ev_fork != nullptr &&
-           c->ev_done != nullptr;
+    return c->plan_sig == 1 && std::memcmp(key, c->plan_key, sizeof(key)) == 0;
 }
+static bool plan_fresh(const qcg_context* c) { return plan_current(c) && c->ev_fork != nullptr && c->ev_done != nullptr; }
 
 bool qcg::jk_prepared(const qcg_context* c) { return plan_fresh(c) && !(c->profiling && !c->ev_made); }
 
@@ -540,6 +540,53 @@ double qcg::model_flops(int cb, int ck) {
 // from 32768.
 constexpr int64_t kPartsMinQuartets = 16384;
 
+// The surviving kets of every bra of a class and precision part, as segments, for the current options.
+struct KetLists {
+    struct Bra {
+        int pair, npp, g0, g1, kbase;
+    };
+    std::vector<int2> segs;
+    std::vector<Bra> bras[21][2];
+    int64_t quartets[21][2] = {};
+    double fpq[21] = {}, cost[21] = {};  // model flops per primitive quartet of a class, and of the class
+};
+
+static bool mixed_plan(const qcg_context* c) { return c->precision == QCG_PREC_MIXED && c->fp32_cutoff > c->schwarz_thr; }
+
+static KetLists list_kets(const qcg_context* c) {
+    KetLists k;
+    const bool mixed = mixed_plan(c);
+    const int nmol = c->nmol;
+    const double cut = mixed ? c->fp32_cutoff : c->schwarz_thr;
+    int cls = 0;
+    for (int cb = kNumPairClasses - 1; cb >= 0; --cb)
+        for (int ck = cb; ck >= 0; --ck, ++cls) {
+            // the class's model flops over its surviving quartets, before the primitive screen
+            // (the default launch schedule's cost), plus 12 N_q per quartet
+            const double nq = c->class_nq[cls];
+            k.fpq[cls] = model_flops(cb, ck);
+            for (int part = 0; part < (mixed ? 2 : 1); ++part)
+                for (int m = 0; m < nmol; ++m) {
+                    const int pbase = c->ket_off_h[cb * nmol + m];
+                    for (int p = 0; p < c->ket_cnt_h[cb * nmol + m]; ++p) {
+                        const int g0 = (int)k.segs.size(), npp = c->pairs[c->class_off[cb] + pbase + p].npp;
+                        const int kbase = c->class_off[ck] + c->ket_off_h[ck * nmol + m];
+                        for_ket_ranges(c, cb, ck, m, p, c->schwarz_thr, cut, [&](int bs, int sp, int e) {
+                            const int lo = part == 0 ? bs : sp, hi = part == 0 ? sp : e;
+                            if (hi > lo) {
+                                k.segs.push_back(make_int2(lo, hi - lo));
+                                k.quartets[cls][part] += hi - lo;
+                                // a segment lies in one contraction bucket: one ket primitive count
+                                k.cost[cls] += (hi - lo) * (k.fpq[cls] * npp * c->pairs[kbase + lo].npp + 12.0 * nq);
+                            }
+                        });
+                        if ((int)k.segs.size() > g0) k.bras[cls][part].push_back({pbase + p, npp, g0, (int)k.segs.size(), kbase});
+                    }
+                }
+        }
+    return k;
+}
+
 // Tiles when the caller has set or tuned none.  Per-lane kernels: the block is widened from 64 to 256
 // threads until the waves that fit a CU's 160 KB of LDS next to each other (the K rows of one bra, where
 // they are kept there, and the Rys table are per block) reach what the kernel's registers allow (`want` per SIMD), as far as a
@@ -550,19 +597,18 @@ constexpr int64_t kPartsMinQuartets = 16384;
 // (ps|ps) 6.7 ms at (64, 1), 4.7 ms at (128, 4), 5.8 ms at (256, 1).  Wave-cooperative kernels: up to
 // four kets per wavefront once that leaves about 6000 wavefronts ((H2O)16 (dp|ds): 0.67 / 0.54 / 0.50 ms
 // at 1 / 2 / 4).
-template <typename Bras>
-static void default_tiles(qcg_context* c, const int64_t (&quartets)[21][2], const Bras& bras) {
+static void default_tiles(const qcg_context* c, const KetLists& k, qcg_context::Tile (&tile)[21][2]) {
     for (int cls = 0, cb = kNumPairClasses - 1; cb >= 0; --cb)
         for (int ck = cb; ck >= 0; --ck, ++cls)
             for (int part = 0; part < 2; ++part) {
-                const int64_t n = quartets[cls][part] + (part == 0 && c->fuse_cls[cls] ? quartets[cls][1] : 0);
-                qcg_context::Tile& t = c->tile[cls][part];
+                const int64_t n = k.quartets[cls][part] + (part == 0 && c->fuse_cls[cls] ? k.quartets[cls][1] : 0);
+                qcg_context::Tile& t = tile[cls][part];
                 const int nq = c->class_nq[cls];
                 if (nq > kJkLaneMaxNQ && (n < kPartsMinQuartets || jk_part(cb, ck) == 0)) {
                     t = {0, n > 24000 ? 4 : n > 8000 ? 2 : 1};
                     continue;
                 }
-                const int64_t per_bra = n / std::max<int64_t>(1, (int64_t)bras[cls][part].size());
+                const int64_t per_bra = n / std::max<int64_t>(1, (int64_t)k.bras[cls][part].size());
                 int la, lb, lc, ld;
                 class_l(cb, la, lb);
                 class_l(ck, lc, ld);
@@ -578,9 +624,8 @@ static void default_tiles(qcg_context* c, const int64_t (&quartets)[21][2], cons
 }
 
 static int build_plan(qcg_context* c) {
-    const bool mixed = c->precision == QCG_PREC_MIXED && c->fp32_cutoff > c->schwarz_thr;
-    const double key[4] = {(double)c->precision, c->fp32_cutoff, c->schwarz_thr, (double)c->tile_sig};
-    if (c->plan_sig == 1 && std::memcmp(key, c->plan_key, sizeof(key)) == 0) return QCG_OK;
+    const bool mixed = mixed_plan(c);
+    if (plan_current(c)) return QCG_OK;
     // a work item encodes its bra's primitive range in 8 bits (cut_items_split)
     for (const PairRec& pr : c->pairs)
         if (pr.npp > kItemMaxPrim)
@@ -591,62 +636,26 @@ static int build_plan(qcg_context* c) {
     c->drop_fock_graph();
     c->plan_sig = 0;
     c->items.clear();
-    c->segs.clear();
-    const int nmol = c->nmol;
-    const double cut = mixed ? c->fp32_cutoff : c->schwarz_thr;
-    // the surviving kets of every (class, precision part, bra), as segments
-    struct Bra {
-        int pair, npp, g0, g1, kbase;
-    };
-    std::vector<Bra> bras[21][2];
-    int64_t quartets[21][2] = {};
-    double fpq[21], total = 0.0;  // model flops per primitive quartet of a class, and of the build
-    int cls = 0;
-    for (int cb = kNumPairClasses - 1; cb >= 0; --cb)
-        for (int ck = cb; ck >= 0; --ck, ++cls) {
-            // the class's model flops over its surviving quartets, before the primitive screen
-            // (the default launch schedule's cost), plus 12 N_q per quartet
-            const double nq = c->class_nq[cls];
-            fpq[cls] = model_flops(cb, ck);
-            double cost = 0.0;
-            for (int part = 0; part < (mixed ? 2 : 1); ++part)
-                for (int m = 0; m < nmol; ++m) {
-                    const int pbase = c->ket_off_h[cb * nmol + m];
-                    for (int p = 0; p < c->ket_cnt_h[cb * nmol + m]; ++p) {
-                        const int g0 = (int)c->segs.size();
-                        const int npp = c->pairs[c->class_off[cb] + pbase + p].npp;
-                        const int kbase = c->class_off[ck] + c->ket_off_h[ck * nmol + m];
-                        for_ket_ranges(c, cb, ck, m, p, c->schwarz_thr, cut, [&](int bs, int sp, int e) {
-                            const int lo = part == 0 ? bs : sp, hi = part == 0 ? sp : e;
-                            if (hi > lo) {
-                                c->segs.push_back(make_int2(lo, hi - lo));
-                                quartets[cls][part] += hi - lo;
-                                // a segment lies in one contraction bucket: one ket primitive count
-                                cost += (hi - lo) * (fpq[cls] * npp * c->pairs[kbase + lo].npp + 12.0 * nq);
-                            }
-                        });
-                        if ((int)c->segs.size() > g0) bras[cls][part].push_back({pbase + p, npp, g0, (int)c->segs.size(), kbase});
-                    }
-                }
-            c->plan_cost[cls] = cost;
-            total += cost;
-        }
-    if (!c->tiles_set) default_tiles(c, quartets, bras);
+    KetLists k = list_kets(c);
+    c->segs = std::move(k.segs);
+    double total = 0.0;
+    for (int i = 0; i < 21; ++i) total += c->plan_cost[i] = k.cost[i];
+    if (!c->tiles_set) default_tiles(c, k, c->tile);
     // the longest chain of primitive quartets one lane may run, in us
     const double chain_us = std::max(kChainMinUs, kChainShare * total / kModelFlopsPerUs);
-    for (cls = 0; cls < 21; ++cls)
+    for (int cls = 0; cls < 21; ++cls)
         for (int part = 0; part < 2; ++part) {
             // fused mixed launches run both parts with the FP64 part's tile
             const qcg_context::Tile& t = c->tile[cls][(mixed && c->fuse_cls[cls]) ? 0 : part];
             const bool lane_form = t.block > 0 ? c->class_nas[cls] > 0 : c->class_nq[cls] < 27;
             const int ch = std::min(kItemMaxKets, std::max(1, t.block > 0 ? t.block * t.reps : t.reps));
             c->item_off[cls][part] = (int)c->items.size();
-            for (const Bra& b : bras[cls][part]) {
+            for (const KetLists::Bra& b : k.bras[cls][part]) {
                 // bras above kBraPPMax primitive pairs are always cut into ranges
                 const int split = (c->prim_split > 0 && c->prim_split < kBraPPMax) ? c->prim_split : kBraPPMax;
                 const int nb = std::min(b.npp, split);
                 auto lg_of = [&](int g) {
-                    return lane_form ? lanes_per_ket(nb, c->pairs[b.kbase + c->segs[g].x].npp, fpq[cls], chain_us) : 0;
+                    return lane_form ? lanes_per_ket(nb, c->pairs[b.kbase + c->segs[g].x].npp, k.fpq[cls], chain_us) : 0;
                 };
                 for (int g = b.g0; g < b.g1;) {
                     const int lg = lg_of(g);
@@ -666,6 +675,7 @@ static int build_plan(qcg_context* c) {
     c->d_segs = nullptr;
     HIPCHK(c, c->alloc(&c->d_segs, c->segs.size()));
     HIPCHK(c, hipMemcpy(c->d_segs, c->segs.data(), c->segs.size() * sizeof(int2), hipMemcpyHostToDevice));
+    const double key[4] = {(double)c->precision, c->fp32_cutoff, c->schwarz_thr, (double)c->tile_sig};
     std::memcpy(c->plan_key, key, sizeof(key));
     c->plan_sig = 1;
     return QCG_OK;
@@ -716,7 +726,7 @@ int qcg::run_jk(qcg_context* c, const double* dD, double* dJ, double* dK, hipStr
     fd.rowsum = A.rowsum;
     HIPCHK(c, launch_fix_scale(dD, fd, A.fix, c->nmol, do_j ? A.Jacc : nullptr, A.Jmat, do_k ? A.Kacc : nullptr,
                                A.Dp, st));
-    const bool mixed = c->precision == QCG_PREC_MIXED && c->fp32_cutoff > c->schwarz_thr;
+    const bool mixed = mixed_plan(c);
     if (c->profiling && !c->ev_made) {
         for (auto& e : c->ev) HIPCHK(c, hipEventCreate(&e));
         c->ev_made = true;
@@ -840,12 +850,12 @@ qcg_context::Tile tune_tile(const qcg_context* c, int k, int cls) {
     return qcg_context::Tile{kTuneCand[k][0], kTuneCand[k][1]};
 }
 
-void export_tiles(const qcg_context* c, int* chosen) {
+void export_tiles(const qcg_context::Tile (&tile)[21][2], int* chosen) {
     if (!chosen) return;
     for (int i = 0; i < 21; ++i)
         for (int part = 0; part < 2; ++part) {
-            chosen[4 * i + 2 * part] = c->tile[i][part].block;
-            chosen[4 * i + 2 * part + 1] = c->tile[i][part].reps;
+            chosen[4 * i + 2 * part] = tile[i][part].block;
+            chosen[4 * i + 2 * part + 1] = tile[i][part].reps;
         }
 }
 
@@ -892,7 +902,7 @@ int qcg_autotune(qcg_context* c, const double* dD, int iters, int* chosen) {
     c->class_cost_set = true;
     for (int i = 0; i < 21; ++i)
         for (int part = 0; part < 2; ++part) c->tile[i][part] = tile_of(pick[2 * i + part], i);
-    export_tiles(c, chosen);
+    export_tiles(c->tile, chosen);
     c->tile_sig += 1;
     c->profiling = prof;
     return QCG_OK;
@@ -1016,7 +1026,7 @@ int qcg_autotune_refine(qcg_context* c, const double* dD, int builds, int* chose
     }
     cleanup();
     if (rc) return rc;
-    export_tiles(c, chosen);
+    export_tiles(c->tile, chosen);
     return QCG_OK;
 }
 
@@ -1036,11 +1046,11 @@ int qcg_set_tiles(qcg_context* c, const int* tiles) {
 
 int qcg_get_tiles(qcg_context* c, int* tiles) {
     if (!c || !tiles) return QCG_INVALID_ARG;
-    for (int i = 0; i < 21; ++i)
-        for (int part = 0; part < 2; ++part) {
-            tiles[4 * i + 2 * part] = c->tile[i][part].block;
-            tiles[4 * i + 2 * part + 1] = c->tile[i][part].reps;
-        }
+    // tiles that are chosen with the plan: those of the plan that the next build makes or has
+    qcg_context::Tile t[21][2];
+    std::copy(&c->tile[0][0], &c->tile[0][0] + 42, &t[0][0]);
+    if (!c->tiles_set && c->has_basis && !plan_current(c)) default_tiles(c, list_kets(c), t);
+    export_tiles(t, tiles);
     return QCG_OK;
 }
 
@@ -1053,7 +1063,7 @@ int qcg_set_profiling(qcg_context* c, int on) {
 int qcg_class_stats(qcg_context* c, qcg_class_stat* out, int* n) {
     if (!c || !out) return QCG_INVALID_ARG;
     if (!c->has_basis) return fail(c, QCG_NO_BASIS, "no basis");
-    const bool mixed = c->precision == QCG_PREC_MIXED && c->fp32_cutoff > c->schwarz_thr;
+    const bool mixed = mixed_plan(c);
     const double thr = c->schwarz_thr, cut = mixed ? c->fp32_cutoff : thr;
     const bool cached = c->stats.size() == 21 && c->stats_key[0] == (double)c->precision &&
                         c->stats_key[1] == c->fp32_cutoff && c->stats_key[2] == c->schwarz_thr;

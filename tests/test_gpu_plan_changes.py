@@ -40,3 +40,26 @@ def test_gpu_fock_graph_follows_the_plan(between):
         # memory freed with the old lists is used by others
         junk = [torch.full((n,), -1, dtype=torch.int32, device="cuda") for n in (1 << 10, 1 << 14, 1 << 18)]
         del junk
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+def test_gpu_tiles_read_before_the_first_build(prec):
+    """The tiles read before any build are those that the builds choose, so setting them back changes
+    nothing: not the tiles, and not a bit of J and K; and they follow the options."""
+    b = bench_molecule("C6H6", "6-31g*")
+    D = random_density(b.nbf, seed=4, nocc=b.n_occ)
+    eng = Engine(b, precision=prec)
+    first = eng.get_tiles()
+    jk = eng.build_jk(D)
+    assert eng.get_tiles() == first
+    other = Engine(b, precision=prec)
+    other.set_tiles(other.get_tiles())
+    jk2 = other.build_jk(D)
+    assert other.get_tiles() == first
+    assert np.array_equal(jk2.J, jk.J) and np.array_equal(jk2.K, jk.K)
+    eng.set_options(prec, 1e-6, 1e-2)  # far fewer quartets, other tiles; read, then back without a build
+    changed = eng.get_tiles()
+    eng.set_options(prec)
+    assert eng.get_tiles() == first and changed != first
+    jk3 = eng.build_jk(D)
+    assert np.array_equal(jk3.J, jk.J) and np.array_equal(jk3.K, jk.K)
