@@ -1,6 +1,7 @@
 // The qcg_context object shared by the host translation units.
 #pragma once
 #include <algorithm>
+#include <initializer_list>
 #include <string>
 #include <vector>
 
@@ -181,7 +182,8 @@ struct qcg_context {
     double *d_gexp = nullptr, *d_gcn = nullptr;
     // The packed FP64 form of the grid (xc_packed.h), made with the grid when the precision option is
     // FP64, else on first use, like the dense arrays above (made with the grid in the mixed option);
-    // pk_state: 0 not made, 1 made, 2 some block has more than kPackedMaxLd functions
+    // pk_state: 0 not made, 1 made, 2 none for this grid (some block has more than kPackedMaxLd functions, or
+    // the memory does not hold it)
     PackedGrid pk{};
     int pk_state = 0;
     int pk_ntile = 0;
@@ -194,17 +196,30 @@ struct qcg_context {
     double *d_pk_pts = nullptr, *d_pk_val = nullptr, *d_pk_vparts = nullptr, *d_pk_vsum = nullptr;
     double* d_pk_grad = nullptr;   // X, M and t of the XC gradient, made on its first use
     int64_t pk_elems = 0;          // elements of one packed array; d_pk_val holds Phi and aow
-    void free_grid() {
-        for (void** p : {(void**)&d_pts, (void**)&d_w, (void**)&d_phi, (void**)&d_dphx, (void**)&d_dphy,
-                         (void**)&d_dphz, (void**)&d_X, (void**)&d_aow, (void**)&d_V, (void**)&d_exc, (void**)&d_Vparts,
-                         (void**)&d_gshell, (void**)&d_gexp, (void**)&d_gcn, (void**)&d_phi32, (void**)&d_grid4,
-                         (void**)&d_aow32, (void**)&d_D32, (void**)&d_pk_int, (void**)&d_pk_off, (void**)&d_pk_pos,
-                         (void**)&d_pk_tiles, (void**)&d_pk_pts, (void**)&d_pk_val, (void**)&d_pk_vparts,
-                         (void**)&d_pk_vsum, (void**)&d_pk_shcol, (void**)&d_pk_grad, (void**)&d_pk_rad, (void**)&d_pk_fn, (void**)&d_tile_mask}) {
+    void free_all(std::initializer_list<void**> list) {
+        for (void** p : list) {
             release(*p);
             *p = nullptr;
         }
+    }
+    void free_dense() {
+        free_all({(void**)&d_phi, (void**)&d_dphx, (void**)&d_dphy, (void**)&d_dphz, (void**)&d_X, (void**)&d_aow, (void**)&d_V,
+                  (void**)&d_Vparts});
+    }
+    void free_xc32() {
+        free_all({(void**)&d_phi32, (void**)&d_grid4, (void**)&d_aow32, (void**)&d_D32, (void**)&d_tile_mask});
+    }
+    void free_packed() {
+        free_all({(void**)&d_pk_int, (void**)&d_pk_off, (void**)&d_pk_pos, (void**)&d_pk_tiles, (void**)&d_pk_pts,
+                  (void**)&d_pk_val, (void**)&d_pk_vparts, (void**)&d_pk_vsum, (void**)&d_pk_shcol, (void**)&d_pk_grad,
+                  (void**)&d_pk_rad, (void**)&d_pk_fn});
         pk_state = 0;
+    }
+    void free_grid() {
+        free_dense();
+        free_xc32();
+        free_packed();
+        free_all({(void**)&d_pts, (void**)&d_w, (void**)&d_exc, (void**)&d_gshell, (void**)&d_gexp, (void**)&d_gcn});
         G = 0;
     }
     double stats_key[3] = {-1.0, -1.0, -1.0};

@@ -31,8 +31,7 @@ constexpr int64_t kVChunk = 16384;
 
 // The dense arrays: Phi, grad Phi, X and aow as G x nbf row-major FP64, in the grid's own order (mixed
 // precision, the library form, the gradient, and grids the packed form does not take).
-int ensure_dense(qcg_context* c) {
-    if (c->d_phi) return QCG_OK;
+int make_dense(qcg_context* c) {
     const HostBasis& B = c->basis;
     const int64_t G = c->G;
     const size_t gn = (size_t)G * B.nbf;
@@ -70,6 +69,12 @@ int ensure_dense(qcg_context* c) {
                                    c->d_dphx, c->d_dphy, c->d_dphz, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return QCG_OK;
+}
+int ensure_dense(qcg_context* c) {
+    if (c->d_phi) return QCG_OK;
+    const int rc = make_dense(c);
+    if (rc) c->free_dense();
+    return rc;
 }
 
 // The grid's points along a space-filling curve: cells of 1/32 of the molecule's extent (10 bohr around
@@ -110,9 +115,14 @@ std::vector<int> spatial_order(const qcg_context* c) {
 }
 
 // The packed form of the grid (xc_packed.h).  Points per block: about 512 blocks, two for every CU, so
-// the V kernel has a tile for each, but 64 to 1024 points ((H2O)16: 1024 blocks of 1024).
-int ensure_packed(qcg_context* c) {
-    if (c->pk_state) return QCG_OK;
+// the V kernel has a tile for each, but 64 to 1024 points ((H2O)16: 1024 blocks of 1024).  *oom: it failed
+// for want of device memory.
+int make_packed(qcg_context* c, bool* oom) {
+    auto get = [&](auto** p, size_t n) {
+        const hipError_t e = c->alloc(p, n);
+        *oom = *oom || e == hipErrorOutOfMemory;
+        return e;
+    };
     const HostBasis& B = c->basis;
     const int G = (int)c->G, ns = B.nshell, nbf = B.nbf;
     PackedGrid& k = c->pk;
@@ -130,7 +140,7 @@ int ensure_packed(qcg_context* c) {
         for (int x = 0; x < 3; ++x) pw[3 * (size_t)i + x] = std::clamp(c->grid_xyz[3 * (size_t)order[i] + x], -1e100, 1e100);
         w[i] = c->grid_w[order[i]];
     }
-    HIPCHK(c, c->alloc(&c->d_pk_pts, pw.size()));
+    HIPCHK(c, get(&c->d_pk_pts, pw.size()));
     HIPCHK(c, hipMemcpy(c->d_pk_pts, pw.data(), pw.size() * sizeof(double), hipMemcpyHostToDevice));
     k.pts = c->d_pk_pts;
     k.w = c->d_pk_pts + 3 * (size_t)nblk * k.S;
@@ -139,7 +149,7 @@ int ensure_packed(qcg_context* c) {
     std::vector<short> shcol(2 * (size_t)nblk * ns, -1);  // first column, then the place among the block's shells
     short* shrad = shcol.data() + (size_t)nblk * ns;
     unsigned char* d_act = nullptr;
-    HIPCHK(c, c->alloc(&d_act, act.size()));
+    HIPCHK(c, get(&d_act, act.size()));
     hipError_t e = launch_packed_active(G, k.S, nblk, ns, c->d_gshell, k.pts, d_act, c->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(act.data(), d_act, act.size(), hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
@@ -184,12 +194,7 @@ int ensure_packed(qcg_context* c) {
         for (int m = 0; m < ld[b]; m += 32 * vw)
             for (int n0 = 0; n0 < ld[b]; n0 += 32 * vw) tiles[vw - 3].push_back(make_int4(b, m, n0, vw));
     }
-    if (k.max_ld > kPackedMaxLd || nbf > INT16_MAX) {
-        c->release(c->d_pk_pts);
-        c->d_pk_pts = nullptr;
-        c->pk_state = 2;
-        return QCG_OK;
-    }
+    if (k.max_ld > kPackedMaxLd || nbf > INT16_MAX) return QCG_OK;  // pk_state stays 0
     std::vector<int4> all;
     for (int i = 2; i >= 0; --i) all.insert(all.end(), tiles[i].begin(), tiles[i].end());
     c->pk_ntile = (int)all.size();
@@ -212,17 +217,17 @@ int ensure_packed(qcg_context* c) {
             fn[B.bf_off[s] + i] = {A[0], A[1], A[2], axis[0] | axis[1] << 2, 0};
         }
     c->pk_elems = elems;
-    HIPCHK(c, c->alloc(&c->d_pk_int, iv.size()));
-    HIPCHK(c, c->alloc(&c->d_pk_off, off.size()));
-    HIPCHK(c, c->alloc(&c->d_pk_pos, pos.size()));
-    HIPCHK(c, c->alloc(&c->d_pk_tiles, all.size()));
-    HIPCHK(c, c->alloc(&c->d_pk_val, 2 * (size_t)elems));
-    HIPCHK(c, c->alloc(&c->d_pk_rad, (size_t)relems));
-    HIPCHK(c, c->alloc(&c->d_pk_fn, fn.size()));
+    HIPCHK(c, get(&c->d_pk_int, iv.size()));
+    HIPCHK(c, get(&c->d_pk_off, off.size()));
+    HIPCHK(c, get(&c->d_pk_pos, pos.size()));
+    HIPCHK(c, get(&c->d_pk_tiles, all.size()));
+    HIPCHK(c, get(&c->d_pk_val, 2 * (size_t)elems));
+    HIPCHK(c, get(&c->d_pk_rad, (size_t)relems));
+    HIPCHK(c, get(&c->d_pk_fn, fn.size()));
     HIPCHK(c, hipMemcpy(c->d_pk_fn, fn.data(), fn.size() * sizeof(GridFn), hipMemcpyHostToDevice));
-    HIPCHK(c, c->alloc(&c->d_pk_vparts, (size_t)velems));
-    HIPCHK(c, c->alloc(&c->d_pk_vsum, (size_t)kPackedVGroups * nbf * nbf));
-    HIPCHK(c, c->alloc(&c->d_pk_shcol, shcol.size()));
+    HIPCHK(c, get(&c->d_pk_vparts, (size_t)velems));
+    HIPCHK(c, get(&c->d_pk_vsum, (size_t)kPackedVGroups * nbf * nbf));
+    HIPCHK(c, get(&c->d_pk_shcol, shcol.size()));
     HIPCHK(c, hipMemcpy(c->d_pk_int, iv.data(), iv.size() * sizeof(int), hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->d_pk_off, off.data(), off.size() * sizeof(int64_t), hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->d_pk_pos, pos.data(), pos.size() * sizeof(short), hipMemcpyHostToDevice));
@@ -247,6 +252,19 @@ int ensure_packed(qcg_context* c) {
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     HIPCHK(c, e);
     c->pk_state = 1;
+    return QCG_OK;
+}
+// A grid that cannot be packed, also one whose packed arrays do not fit beside what is allocated (the dense
+// arrays of the mixed option, another program's), does with the dense ones.
+int ensure_packed(qcg_context* c) {
+    if (c->pk_state) return QCG_OK;
+    bool oom = false;
+    const int rc = make_packed(c, &oom);
+    if (c->pk_state == 1) return QCG_OK;
+    c->free_packed();
+    if (rc && !oom) return rc;
+    (void)hipGetLastError();  // a failed allocation is not the next launch's error
+    c->pk_state = 2;
     return QCG_OK;
 }
 
@@ -297,8 +315,7 @@ int upload_grid(qcg_context* c) {
 }
 
 // FP32 copies of Phi and grad Phi (and FP32 work arrays) for the mixed-precision XC build
-int ensure_xc32(qcg_context* c, hipStream_t st) {
-    if (c->d_phi32 && c->d_grid4 && c->d_aow32 && c->d_D32) return QCG_OK;
+int make_xc32(qcg_context* c, hipStream_t st) {
     const size_t gn = (size_t)c->G * c->basis.nbf, nn = (size_t)c->basis.nbf * c->basis.nbf;
     HIPCHK(c, c->alloc(&c->d_phi32, gn));
     HIPCHK(c, c->alloc(&c->d_grid4, gn));
@@ -311,6 +328,12 @@ int ensure_xc32(qcg_context* c, hipStream_t st) {
         HIPCHK(c, launch_tile_mask((int)c->G, c->basis.nbf, c->d_grid4, c->d_tile_mask, st));
     }
     return QCG_OK;
+}
+int ensure_xc32(qcg_context* c, hipStream_t st) {
+    if (c->d_phi32) return QCG_OK;
+    const int rc = make_xc32(c, st);
+    if (rc) c->free_xc32();
+    return rc;
 }
 
 // V_xc and E_xc with the MFMA kernels (xc_mfma.hip): FP32 products in mixed precision, FP64 otherwise
@@ -361,7 +384,7 @@ int xc_build(qcg_context* c, const double* dD, double* dV, double* dExc, hipStre
     }
     int rc = ensure_dense(c);
     if (rc) return rc;
-    const bool dense64 = c->pk_state == 0 && (c->basis.nbf <= kPackedMaxLd || !c->blas);
+    const bool dense64 = c->basis.nbf <= kPackedMaxLd || (c->pk_state == 0 && !c->blas);
     if (c->xc_mode == 2 || (c->xc_mode == 0 && (mixed || dense64))) return xc_build_mfma(c, dD, dV, dExc, st);
     rc = ensure_blas(c);
     if (rc) return rc;
@@ -399,15 +422,27 @@ int xc_build(qcg_context* c, const double* dD, double* dV, double* dExc, hipStre
 int xc_gradient(qcg_context* c, const double* dD, double* dgrad, hipStream_t st) {
     if (c->G <= 0) return fail(c, QCG_NO_GRID, "no grid: call qcg_build_grid or qcg_set_grid");
     // on the packed grid (FP64 in every precision option); the library form where it does not apply
+    const bool fresh = c->pk_state == 0;
     int rc = ensure_packed(c);
     if (rc) return rc;
     if (c->pk_state == 1 && 3 * (size_t)c->basis.natom * sizeof(double) <= 65536) {
         const size_t n = (size_t)c->pk_elems, rows = (size_t)c->pk.nblk * c->pk.S;
-        if (!c->d_pk_grad) HIPCHK(c, c->alloc(&c->d_pk_grad, 2 * n + 3 * rows));
-        HIPCHK(c, launch_xc_grad_packed(c->pk, c->basis.nshell, c->basis.natom, c->d_gshell, c->d_gexp, c->d_gcn,
-                                        c->d_pk_shcol, dD, c->d_pk_grad, c->d_pk_val + n, c->d_pk_grad + n,
-                                        c->d_pk_grad + 2 * n, dgrad, st));
-        return QCG_OK;
+        hipError_t e = c->d_pk_grad ? hipSuccess : c->alloc(&c->d_pk_grad, 2 * n + 3 * rows);
+        if (e == hipSuccess) {
+            HIPCHK(c, launch_xc_grad_packed(c->pk, c->basis.nshell, c->basis.natom, c->d_gshell, c->d_gexp, c->d_gcn,
+                                            c->d_pk_shcol, dD, c->d_pk_grad, c->d_pk_val + n, c->d_pk_grad + n,
+                                            c->d_pk_grad + 2 * n, dgrad, st));
+            return QCG_OK;
+        }
+        c->d_pk_grad = nullptr;
+        if (e != hipErrorOutOfMemory || !c->d_phi) HIPCHK(c, e);
+        // no room for the packed gradient beside the dense arrays: the library form on these; packed arrays
+        // made just now make way (older ones may be part of a caller's captured build)
+        (void)hipGetLastError();
+        if (fresh) {
+            c->free_packed();
+            c->pk_state = 2;
+        }
     }
     rc = ensure_dense(c);
     if (!rc) rc = ensure_blas(c);

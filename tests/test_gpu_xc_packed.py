@@ -114,3 +114,39 @@ def test_gpu_packed_xc_gradient(n):
         g = eng.xc_gradient(D)
         assert np.abs(g - oracle.xc_gradient(b, xyz, w, D)).max() < 1e-8
         assert np.array_equal(eng.xc_gradient(D).shape, (b.natom, 3))
+
+
+def test_gpu_packed_form_without_room():
+    """A grid made for the mixed option whose dense arrays leave no room for the packed ones: the gradient and the
+    FP64 build run on the dense arrays.  The card's memory is taken up to 1.9 GB beyond 9 matrices of points by
+    functions (Phi, its gradient, X, aow and the FP32 copies); the packed form and its gradient take at least 4 of
+    1 GB each.  Tolerances as above."""
+    import torch
+    b = bench_molecule("C6H6", "6-31g*")
+    n = 1_230_000
+    unit = 8 * n * b.nbf
+    xyz, w = _points(b, 2000, 6)
+    D = random_density(b.nbf, seed=9, nocc=b.n_occ)
+    ref = Engine(b)
+    ref.set_grid(xyz, w)
+    (V, E), g = ref.xc(D), ref.xc_gradient(D)
+    ref.close()
+    eng = Engine(b, precision="mixed")
+    eng.eri_gradient(D)
+    rep = n // 2000
+    big, wb = np.tile(xyz, (rep, 1)), np.tile(w / rep, rep)
+    torch.cuda.empty_cache()
+    keep = 9 * unit + (14 << 27)
+    hog = torch.empty(torch.cuda.mem_get_info()[0] - keep, dtype=torch.uint8, device="cuda")
+    try:
+        eng.set_grid(big, wb)
+        Vm, Em = eng.xc(D)
+        g2 = eng.xc_gradient(D)
+        eng.set_options("fp64")
+        V2, E2 = eng.xc(D)
+    finally:
+        del hog
+        torch.cuda.empty_cache()
+    assert np.abs(g2 - g).max() < 1e-8
+    assert np.abs(V2 - V).max() < 1e-10 and abs(E2 - E) < 1e-10 * max(1.0, abs(E))
+    assert np.abs(Vm - V).max() < 1e-4 and abs(Em - E) < 1e-4
