@@ -7,6 +7,8 @@ Tolerance: V elements are sums over the grid of products of FP64 values of size 
 up to the electron number scale; both sides accumulate with rounding below 1e-15 of the largest term
 and at most 1e5 terms: 1e-10 absolute, E_xc 1e-10 relative.  The oracle also drops functions below 1e-10
 on its 512-point blocks, which is below the same bound after weighting."""
+from dataclasses import replace
+
 import numpy as np
 import pytest
 
@@ -150,3 +152,48 @@ def test_gpu_packed_form_without_room():
     assert np.abs(g2 - g).max() < 1e-8
     assert np.abs(V2 - V).max() < 1e-10 and abs(E2 - E) < 1e-10 * max(1.0, abs(E))
     assert np.abs(Vm - V).max() < 1e-4 and abs(Em - E) < 1e-4
+
+
+def test_gpu_block_of_more_functions_than_the_packed_kernels_take():
+    """One block of 60 points that 380 functions reach: no packed form, so the library form (modes 0 and 1), the
+    column-pass MFMA kernels (mode 2) and the library gradient; then points that a part of them reaches."""
+    b = build_basis(workloads.water_cluster((5, 2, 2), 2.9, 3), "6-31g*", units="angstrom")
+    rng = np.random.default_rng(2)
+    D = random_density(b.nbf, seed=9, nocc=b.n_occ)
+    eng = Engine(b)
+    for _ in range(2):
+        xyz, w = b.xyz + rng.normal(0.0, 0.3, b.xyz.shape), rng.uniform(0.0, 0.5, b.natom)
+        Vo, Eo, _ = oracle.vxc(*oracle.basis_on_grid(b, xyz), w, D)
+        eng.set_grid(xyz, w)
+        for mode in (0, 2, 1, 0):
+            eng.set_xc_mode(mode)
+            V, E = eng.xc(D)
+            assert np.abs(V - Vo).max() < 1e-10 and abs(E - Eo) < 1e-10 * max(1.0, abs(Eo)), mode
+        assert np.abs(eng.xc_gradient(D) - oracle.xc_gradient(b, xyz, w, D)).max() < 1e-8
+        near = b.xyz[0] + rng.normal(0.0, 0.5, (100, 3))
+        _check(b, near, rng.uniform(0.0, 0.5, 100), eng)
+        assert np.abs(eng.xc_gradient(D) - oracle.xc_gradient(b, near, eng.get_grid()[1], D)).max() < 1e-8
+
+
+def _reordered(b, order):
+    """The basis with its shells in another order."""
+    o = np.asarray(order)
+    nc = (b.shell_l[o] + 1) * (b.shell_l[o] + 2) // 2
+    return replace(b, shell_l=b.shell_l[o], shell_nprim=b.shell_nprim[o], shell_prim_off=b.shell_prim_off[o],
+                   shell_atom=b.shell_atom[o], shell_center=np.ascontiguousarray(b.shell_center[o]),
+                   shell_bf_off=np.concatenate([[0], np.cumsum(nc)[:-1]]).astype(np.int32))
+
+
+@pytest.mark.parametrize("first", [1, 2])
+def test_gpu_packed_shell_orders(first):
+    """Function 0, which stands in for the padding columns of a block, as a p or d function: the p (or d) shells
+    first, then the others.  V and E_xc, and the XC gradient twice (its work arrays are kept)."""
+    b = bench_molecule("NH3", "6-31+g*")
+    b = _reordered(b, np.argsort(b.shell_l != first, kind="stable"))
+    assert b.shell_l[0] == first
+    xyz, w = _points(b, 2000, 5)
+    D, _, _, eng = _check(b, xyz, w)
+    g = eng.xc_gradient(D)
+    assert np.abs(g - oracle.xc_gradient(b, xyz, w, D)).max() < 1e-8
+    eng.xc(random_density(b.nbf, seed=10, nocc=b.n_occ))
+    assert np.abs(eng.xc_gradient(D) - g).max() < 1e-10  # its atomic sums arrive in any order
