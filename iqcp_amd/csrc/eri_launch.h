@@ -55,8 +55,8 @@ inline void cut_items_split(std::vector<int4>& items, const std::vector<int2>& s
     }
 }
 
-inline QCG_HD int item_kets(const int4& it) { return it.w & kItemMaxKets; }
-inline QCG_HD int item_lg(const int4& it) { return (it.w >> 13) & 7; }
+QCG_HD int item_kets(const int4& it) { return it.w & kItemMaxKets; }
+QCG_HD int item_lg(const int4& it) { return (it.w >> 13) & 7; }
 
 // Most bra primitive pairs one J/K item may have: the planner cuts heavier bras into primitive ranges
 // of at most this many.
@@ -103,7 +103,7 @@ inline size_t jk_row_bytes(int nrow, size_t table, int nbf) {
 constexpr int kTensorLaneMaxNQ = 54;
 
 // the bra pair of an item, restricted to the item's primitive range
-inline QCG_HD PairRec item_bra(const PairRec* __restrict__ bra, const int4& it) {
+QCG_HD PairRec item_bra(const PairRec* __restrict__ bra, const int4& it) {
     PairRec P = bra[it.x];
     const int pcnt = (it.w >> 24) & kItemMaxPrim;
     if (pcnt) {
