@@ -187,15 +187,13 @@ struct qcg_context {
     PackedGrid pk{};
     int pk_state = 0;
     int pk_ntile = 0;
-    int *d_pk_int = nullptr;       // ld, nfn, floff, ldr, nl, fl, fs
-    int64_t *d_pk_off = nullptr;   // off, voff, roff
-    short *d_pk_pos = nullptr, *d_pk_shcol = nullptr;  // column of each function and shell in each block
-    int4* d_pk_tiles = nullptr;
-    double2* d_pk_rad = nullptr;   // radial parts per point and shell
-    GridFn* d_pk_fn = nullptr;
-    double *d_pk_pts = nullptr, *d_pk_val = nullptr, *d_pk_vparts = nullptr, *d_pk_vsum = nullptr;
+    char* d_pk_lists = nullptr;    // the lists that pk points to, and the next two
+    const int4* d_pk_tiles = nullptr;
+    const short* d_pk_shcol = nullptr;  // column of each shell in each block
+    double* d_pk_pts = nullptr;
+    double *d_pk_val = nullptr, *d_pk_vparts = nullptr, *d_pk_vsum = nullptr;  // d_pk_val owns the work arrays
     double* d_pk_grad = nullptr;   // X, M and t of the XC gradient, made on its first use
-    int64_t pk_elems = 0;          // elements of one packed array; d_pk_val holds Phi and aow
+    int64_t pk_elems = 0;          // elements of one packed array; d_pk_val holds Phi, aow, the radial parts, partial and summed V
     void free_all(std::initializer_list<void**> list) {
         for (void** p : list) {
             release(*p);
@@ -210,9 +208,7 @@ struct qcg_context {
         free_all({(void**)&d_phi32, (void**)&d_grid4, (void**)&d_aow32, (void**)&d_D32, (void**)&d_tile_mask});
     }
     void free_packed() {
-        free_all({(void**)&d_pk_int, (void**)&d_pk_off, (void**)&d_pk_pos, (void**)&d_pk_tiles, (void**)&d_pk_pts,
-                  (void**)&d_pk_val, (void**)&d_pk_vparts, (void**)&d_pk_vsum, (void**)&d_pk_shcol, (void**)&d_pk_grad,
-                  (void**)&d_pk_rad, (void**)&d_pk_fn});
+        free_all({(void**)&d_pk_lists, (void**)&d_pk_pts, (void**)&d_pk_val, (void**)&d_pk_grad});
         pk_state = 0;
     }
     void free_grid() {

@@ -98,7 +98,9 @@ std::vector<int> spatial_order(const qcg_context* c) {
         spread[i] = 0;
         for (int b = 0; b < kBits; ++b) spread[i] |= ((i >> b) & 1) << (3 * b);
     }
-    std::vector<int> key((size_t)G), first((size_t)kCells * kCells * kCells + 1, 0), order((size_t)G);
+    constexpr int kAll = kCells * kCells * kCells;
+    std::vector<unsigned short> key((size_t)G);
+    std::vector<int> first((size_t)kAll + 1, 0), order((size_t)G);
     const double* xyz = c->grid_xyz.data();
     for (int64_t g = 0; g < G; ++g) {
         int k = 0;
@@ -106,10 +108,10 @@ std::vector<int> spatial_order(const qcg_context* c) {
             const double v = (xyz[3 * g + x] - lo[x]) * inv;
             k |= spread[v > 0.0 ? (int)std::min(v, kCells - 1.0) : 0] << x;
         }
-        key[g] = k;
+        key[g] = (unsigned short)k;
+        ++first[k + 1];
     }
-    for (int64_t g = 0; g < G; ++g) ++first[key[g] + 1];
-    for (size_t k = 1; k < first.size(); ++k) first[k] += first[k - 1];
+    for (int k = 0; k < kAll; ++k) first[k + 1] += first[k];
     for (int64_t g = 0; g < G; ++g) order[first[key[g]]++] = (int)g;
     return order;
 }
@@ -117,6 +119,9 @@ std::vector<int> spatial_order(const qcg_context* c) {
 // The packed form of the grid (xc_packed.h).  Points per block: about 512 blocks, two for every CU, so
 // the V kernel has a tile for each, but 64 to 1024 points ((H2O)16: 1024 blocks of 1024).  *oom: it failed
 // for want of device memory.
+// A grid is made once per geometry, so this counts beside its XC builds: qcg_build_grid takes 1.3 ms for benzene
+// (72314 points) and 12.4 ms for (H2O)16 (286081), 1.2 and 13.0 ms with the dense arrays; gathering the points
+// on the host, thirteen allocations and eight copies made that 2.6 and 15.4 ms.
 int make_packed(qcg_context* c, bool* oom) {
     auto get = [&](auto** p, size_t n) {
         const hipError_t e = c->alloc(p, n);
@@ -133,27 +138,23 @@ int make_packed(qcg_context* c, bool* oom) {
     while (k.S < 1024 && k.S * 512 < G) k.S *= 2;
     const int nblk = k.nblk = (G + k.S - 1) / k.S;
     const std::vector<int> order = spatial_order(c);
-    std::vector<double> pw(4 * (size_t)nblk * k.S, 0.0);  // 3 coordinates, then the weights
-    double* w = pw.data() + 3 * (size_t)nblk * k.S;
-    for (int i = 0; i < G; ++i) {
-        // a point at infinity sees no function; kept finite, so that 0 times its powers is 0
-        for (int x = 0; x < 3; ++x) pw[3 * (size_t)i + x] = std::clamp(c->grid_xyz[3 * (size_t)order[i] + x], -1e100, 1e100);
-        w[i] = c->grid_w[order[i]];
-    }
-    HIPCHK(c, get(&c->d_pk_pts, pw.size()));
-    HIPCHK(c, hipMemcpy(c->d_pk_pts, pw.data(), pw.size() * sizeof(double), hipMemcpyHostToDevice));
-    k.pts = c->d_pk_pts;
-    k.w = c->d_pk_pts + 3 * (size_t)nblk * k.S;
-    // the shells of each block
+    // the points in that order, and the shells of each block
+    const size_t rows = (size_t)nblk * k.S;
     std::vector<unsigned char> act((size_t)nblk * ns);
     std::vector<short> shcol(2 * (size_t)nblk * ns, -1);  // first column, then the place among the block's shells
     short* shrad = shcol.data() + (size_t)nblk * ns;
-    unsigned char* d_act = nullptr;
-    HIPCHK(c, get(&d_act, act.size()));
-    hipError_t e = launch_packed_active(G, k.S, nblk, ns, c->d_gshell, k.pts, d_act, c->stream);
+    HIPCHK(c, get(&c->d_pk_pts, 4 * rows));
+    k.pts = c->d_pk_pts;
+    k.w = c->d_pk_pts + 3 * rows;
+    int* d_order = nullptr;
+    HIPCHK(c, get(&d_order, (size_t)G + (act.size() + 3) / 4));
+    unsigned char* d_act = reinterpret_cast<unsigned char*>(d_order + G);
+    hipError_t e = hipMemcpyAsync(d_order, order.data(), (size_t)G * sizeof(int), hipMemcpyHostToDevice, c->stream);
+    if (e == hipSuccess) e = launch_packed_points(G, rows, d_order, c->d_pts, c->d_w, c->d_pk_pts, c->stream);
+    if (e == hipSuccess) e = launch_packed_active(G, k.S, nblk, ns, c->d_gshell, k.pts, d_act, c->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(act.data(), d_act, act.size(), hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    c->release(d_act);
+    c->release(d_order);
     HIPCHK(c, e);
     std::vector<int> ld(nblk), nfn(nblk), floff(nblk), ldr(nblk), nl(2 * (size_t)nblk), fl, fs, by_l(ns);
     std::iota(by_l.begin(), by_l.end(), 0);
@@ -195,16 +196,6 @@ int make_packed(qcg_context* c, bool* oom) {
             for (int n0 = 0; n0 < ld[b]; n0 += 32 * vw) tiles[vw - 3].push_back(make_int4(b, m, n0, vw));
     }
     if (k.max_ld > kPackedMaxLd || nbf > INT16_MAX) return QCG_OK;  // pk_state stays 0
-    std::vector<int4> all;
-    for (int i = 2; i >= 0; --i) all.insert(all.end(), tiles[i].begin(), tiles[i].end());
-    c->pk_ntile = (int)all.size();
-    std::vector<int> iv(ld);
-    iv.insert(iv.end(), nfn.begin(), nfn.end());
-    iv.insert(iv.end(), floff.begin(), floff.end());
-    iv.insert(iv.end(), ldr.begin(), ldr.end());
-    iv.insert(iv.end(), nl.begin(), nl.end());
-    iv.insert(iv.end(), fl.begin(), fl.end());
-    iv.insert(iv.end(), fs.begin(), fs.end());
     std::vector<GridFn> fn(nbf);
     for (int s = 0; s < ns; ++s)
         for (int i = 0; i < ncart(B.l[s]); ++i) {
@@ -216,39 +207,46 @@ int make_packed(qcg_context* c, bool* oom) {
             for (int k = 0; k < cart_z(l, i); ++k) axis[n++] = 2;
             fn[B.bf_off[s] + i] = {A[0], A[1], A[2], axis[0] | axis[1] << 2, 0};
         }
+    // the block lists in one allocation and one copy, the work arrays in another
+    std::vector<char> lists;
+    auto put = [&](const auto& v) {
+        const size_t o = lists.size(), n = v.size() * sizeof(v[0]);
+        lists.resize(o + (n + 15) / 16 * 16);
+        std::memcpy(lists.data() + o, v.data(), n);
+        return o;
+    };
+    c->pk_ntile = (int)(tiles[0].size() + tiles[1].size() + tiles[2].size());
+    std::vector<int4> all(tiles[2]);
+    all.insert(all.end(), tiles[1].begin(), tiles[1].end());
+    all.insert(all.end(), tiles[0].begin(), tiles[0].end());
+    const size_t at[] = {put(all), put(fn), put(off), put(ld), put(nfn), put(floff), put(ldr), put(nl), put(fl), put(fs),
+                         put(pos), put(shcol)};
     c->pk_elems = elems;
-    HIPCHK(c, get(&c->d_pk_int, iv.size()));
-    HIPCHK(c, get(&c->d_pk_off, off.size()));
-    HIPCHK(c, get(&c->d_pk_pos, pos.size()));
-    HIPCHK(c, get(&c->d_pk_tiles, all.size()));
-    HIPCHK(c, get(&c->d_pk_val, 2 * (size_t)elems));
-    HIPCHK(c, get(&c->d_pk_rad, (size_t)relems));
-    HIPCHK(c, get(&c->d_pk_fn, fn.size()));
-    HIPCHK(c, hipMemcpy(c->d_pk_fn, fn.data(), fn.size() * sizeof(GridFn), hipMemcpyHostToDevice));
-    HIPCHK(c, get(&c->d_pk_vparts, (size_t)velems));
-    HIPCHK(c, get(&c->d_pk_vsum, (size_t)kPackedVGroups * nbf * nbf));
-    HIPCHK(c, get(&c->d_pk_shcol, shcol.size()));
-    HIPCHK(c, hipMemcpy(c->d_pk_int, iv.data(), iv.size() * sizeof(int), hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemcpy(c->d_pk_off, off.data(), off.size() * sizeof(int64_t), hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemcpy(c->d_pk_pos, pos.data(), pos.size() * sizeof(short), hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemcpy(c->d_pk_tiles, all.data(), all.size() * sizeof(int4), hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemcpy(c->d_pk_shcol, shcol.data(), shcol.size() * sizeof(short), hipMemcpyHostToDevice));
-    k.ld = c->d_pk_int;
-    k.nfn = k.ld + nblk;
-    k.floff = k.nfn + nblk;
-    k.ldr = k.floff + nblk;
-    k.nl = k.ldr + nblk;
-    k.fl = k.nl + 2 * nblk;
-    k.fs = k.fl + fl.size();
-    k.fn = c->d_pk_fn;
-    k.off = c->d_pk_off;
+    HIPCHK(c, get(&c->d_pk_lists, lists.size()));
+    HIPCHK(c, get(&c->d_pk_val, 2 * (size_t)(elems + relems) + (size_t)velems + (size_t)kPackedVGroups * nbf * nbf));
+    HIPCHK(c, hipMemcpy(c->d_pk_lists, lists.data(), lists.size(), hipMemcpyHostToDevice));
+    auto get_list = [&](auto* t, int i) { return reinterpret_cast<decltype(t)>(c->d_pk_lists + at[i]); };
+    c->d_pk_tiles = get_list((const int4*)nullptr, 0);
+    k.fn = get_list((const GridFn*)nullptr, 1);
+    k.off = get_list((const int64_t*)nullptr, 2);
     k.voff = k.off + nblk;
     k.roff = k.voff + nblk;
-    k.pos = c->d_pk_pos;
+    k.ld = get_list((const int*)nullptr, 3);
+    k.nfn = get_list((const int*)nullptr, 4);
+    k.floff = get_list((const int*)nullptr, 5);
+    k.ldr = get_list((const int*)nullptr, 6);
+    k.nl = get_list((const int*)nullptr, 7);
+    k.fl = get_list((const int*)nullptr, 8);
+    k.fs = get_list((const int*)nullptr, 9);
+    k.pos = get_list((const short*)nullptr, 10);
+    c->d_pk_shcol = get_list((const short*)nullptr, 11);
     k.phi = c->d_pk_val;
-    k.rad = c->d_pk_rad;
+    double2* rad = reinterpret_cast<double2*>(c->d_pk_val + 2 * elems);
+    k.rad = rad;
+    c->d_pk_vparts = c->d_pk_val + 2 * (elems + relems);
+    c->d_pk_vsum = c->d_pk_vparts + velems;
     e = launch_packed_basis(k, ns, c->d_gshell, c->d_gexp, c->d_gcn, c->d_pk_shcol, c->d_pk_shcol + (size_t)nblk * ns,
-                            c->d_pk_val, c->d_pk_rad, c->stream);
+                            c->d_pk_val, rad, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     HIPCHK(c, e);
     c->pk_state = 1;

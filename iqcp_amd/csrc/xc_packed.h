@@ -55,6 +55,9 @@ struct PackedGrid {
 // the accumulators of two wavefronts (2 x 11 MFMA tiles of 16 columns).
 constexpr int kPackedMaxLd = 352;
 
+// out: 3 n coordinates, then n weights, of the points order[0 .. G), zero from G to n
+hipError_t launch_packed_points(int G, size_t n, const int* order, const double* pts, const double* w, double* out,
+                                hipStream_t st);
 // active[b * nshell + s] = 1 if shell s reaches a point of block b
 hipError_t launch_packed_active(int G, int S, int nblk, int nshell, const GridShell* shells, const double* pts,
                                 unsigned char* active, hipStream_t st);

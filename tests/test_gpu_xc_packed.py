@@ -197,3 +197,25 @@ def test_gpu_packed_shell_orders(first):
     assert np.abs(g - oracle.xc_gradient(b, xyz, w, D)).max() < 1e-8
     eng.xc(random_density(b.nbf, seed=10, nocc=b.n_occ))
     assert np.abs(eng.xc_gradient(D) - g).max() < 1e-10  # its atomic sums arrive in any order
+
+
+@pytest.mark.parametrize("n", [32767, 32768, 32769, 65537, 131073, 262145, 300000])
+def test_gpu_packed_block_sizes(n):
+    """Blocks of 64 to 1024 points, the last one full, almost empty or partly filled: V, E_xc and the XC gradient of
+    the packed form against the library form on the dense arrays, and the same bits of V from a second set_grid.
+    Both are sums of n <= 3e5 terms of size <= 1 rounded below 1e-15 of the largest: 1e-10."""
+    b = bench_molecule("H2O", "6-31g*")
+    xyz, w = _points(b, n, 3, spread=4.0)
+    w = w * (2000.0 / n)
+    D = random_density(b.nbf, seed=9, nocc=b.n_occ)
+    eng = Engine(b)
+    eng.set_grid(xyz, w)
+    V, E = eng.xc(D)
+    g = eng.xc_gradient(D)
+    eng.set_xc_mode(1)
+    Vl, El = eng.xc(D)
+    assert np.abs(V - Vl).max() < 1e-10 and abs(E - El) < 1e-10 * max(1.0, abs(El))
+    eng.set_xc_mode(0)
+    eng.set_grid(xyz, w)
+    V2, _ = eng.xc(D)
+    assert np.array_equal(V2, V) and np.abs(eng.xc_gradient(D) - g).max() < 1e-10
