@@ -4,6 +4,7 @@
 #include <cstdint>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -31,6 +32,61 @@ double qcg::nuclear_repulsion(const HostBasis& B) {
     return e;
 }
 
+namespace {
+
+// Streams outlive their contexts: a destroyed context leaves its set to the next one on the device.  The runtime
+// frees a stream's queue object in hipStreamDestroy while its completion thread may still be leaving that object's
+// lock for the last command, however well the stream has been waited for: now and then a word of the freed
+// heap block was decremented and another zeroed afterwards, once the low half of a contraction coefficient of the
+// context made next, whose V_xc was then off by 1.5e-8.  At most kIdleSets sets wait (six streams each); the
+// streams of further ones are destroyed.
+struct StreamSet {
+    int device = 0;
+    hipStream_t main = nullptr, aux[qcg_context::kStreams] = {}, xc = nullptr;
+};
+constexpr size_t kIdleSets = 16;
+struct IdleStreams {
+    std::mutex m;
+    std::vector<StreamSet> sets;
+    IdleStreams() { sets.reserve(kIdleSets); }
+};
+IdleStreams& idle_streams() {
+    static IdleStreams* p = new IdleStreams;  // never destroyed: at exit the runtime may be gone
+    return *p;
+}
+
+StreamSet take_streams(int device) {
+    IdleStreams& I = idle_streams();
+    const std::lock_guard<std::mutex> lock(I.m);
+    for (size_t i = I.sets.size(); i-- > 0;)
+        if (I.sets[i].device == device) {
+            const StreamSet s = I.sets[i];
+            I.sets.erase(I.sets.begin() + i);
+            return s;
+        }
+    StreamSet s;
+    s.device = device;
+    return s;
+}
+
+// drained: every stream of the set has been waited for without an error
+void give_streams(const StreamSet& s, bool drained) {
+    if (drained) {
+        IdleStreams& I = idle_streams();
+        const std::lock_guard<std::mutex> lock(I.m);
+        if (I.sets.size() < kIdleSets) {
+            I.sets.push_back(s);
+            return;
+        }
+    }
+    for (hipStream_t a : s.aux)
+        if (a) (void)hipStreamDestroy(a);
+    if (s.xc) (void)hipStreamDestroy(s.xc);
+    if (s.main) (void)hipStreamDestroy(s.main);
+}
+
+}  // namespace
+
 extern "C" {
 
 int qcg_create(qcg_context** out, int device) {
@@ -42,7 +98,11 @@ int qcg_create(qcg_context** out, int device) {
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev <= 0) return QCG_DEVICE;
     if (device < 0 || device >= ndev) return QCG_INVALID_ARG;
     if (hipSetDevice(device) != hipSuccess) return QCG_DEVICE;
-    if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) return QCG_DEVICE;
+    const StreamSet streams = take_streams(device);
+    c->stream = streams.main;
+    std::copy(streams.aux, streams.aux + qcg_context::kStreams, c->aux);
+    c->xc_stream = streams.xc;
+    if (!c->stream && hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) return QCG_DEVICE;
     // the static scratch of qcg_build_jk_device_noalloc; a failure surfaces in that entry point
     (void)noalloc_setup(device);
     const size_t nt = sizeof(qcg_rys_coef) / sizeof(double);
@@ -73,30 +133,28 @@ void qcg_destroy(qcg_context* c) {
     if (!c) return;
     (void)hipSetDevice(c->device);
     c->drop_fock_graph();  // waits for the exec's last launch
-    (void)hipStreamSynchronize(c->stream);
+    bool drained = hipStreamSynchronize(c->stream) == hipSuccess;
     if (c->ev_done) (void)hipEventSynchronize(c->ev_done);  // the last entry point's work on any stream
-    for (int i = 0; i < qcg_context::kStreams; ++i)
-        if (c->aux[i]) (void)hipStreamSynchronize(c->aux[i]);
-    if (c->xc_stream) (void)hipStreamSynchronize(c->xc_stream);
+    StreamSet streams;
+    streams.device = c->device;
+    streams.main = c->stream;
+    streams.xc = c->xc_stream;
+    std::copy(c->aux, c->aux + qcg_context::kStreams, streams.aux);
+    for (hipStream_t a : c->aux)
+        if (a) drained = hipStreamSynchronize(a) == hipSuccess && drained;
+    if (c->xc_stream) drained = hipStreamSynchronize(c->xc_stream) == hipSuccess && drained;
     for (void* p : c->owned) (void)hipFree(p);
     c->owned.clear();
     if (c->ev_made)
         for (auto& e : c->ev) (void)hipEventDestroy(e);
-    if (c->ev_fork) {
-        (void)hipEventDestroy(c->ev_fork);
-        for (int i = 0; i < qcg_context::kStreams; ++i) {
-            (void)hipEventDestroy(c->ev_join[i]);
-            (void)hipStreamDestroy(c->aux[i]);
-        }
-    }
+    if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
+    for (hipEvent_t e : c->ev_join)
+        if (e) (void)hipEventDestroy(e);
     if (c->ev_done) (void)hipEventDestroy(c->ev_done);
-    if (c->xc_stream) {
-        (void)hipEventDestroy(c->ev_xc_fork);
-        (void)hipEventDestroy(c->ev_xc_join);
-        (void)hipStreamDestroy(c->xc_stream);
-    }
+    if (c->ev_xc_fork) (void)hipEventDestroy(c->ev_xc_fork);
+    if (c->ev_xc_join) (void)hipEventDestroy(c->ev_xc_join);
     if (c->blas) (void)rocblas_destroy_handle(c->blas);
-    if (c->stream) (void)hipStreamDestroy(c->stream);
+    give_streams(streams, drained);
     delete c;
 }
 
@@ -687,7 +745,7 @@ static int prepare_streams(qcg_context* c) {
     if (!c->ev_fork) {
         HIPCHK(c, hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
         for (int i = 0; i < qcg_context::kStreams; ++i) {
-            HIPCHK(c, hipStreamCreateWithFlags(&c->aux[i], hipStreamNonBlocking));
+            if (!c->aux[i]) HIPCHK(c, hipStreamCreateWithFlags(&c->aux[i], hipStreamNonBlocking));
             HIPCHK(c, hipEventCreateWithFlags(&c->ev_join[i], hipEventDisableTiming));
         }
     }
@@ -934,14 +992,15 @@ int qcg_autotune_refine(qcg_context* c, const double* dD, int builds, int* chose
     // hipStreamBeginCapture); run_jk refuses to rebuild it inside a capture.
     const size_t n2 = (size_t)c->basis.nbf * c->basis.nbf;
     double *dH = nullptr, *dF = nullptr;
-    hipStream_t ts = nullptr;
+    StreamSet own = take_streams(c->device);
+    hipStream_t& ts = own.main;
     const bool graph = c->use_graph;
     auto cleanup = [&]() {
         c->drop_fock_graph();  // waits for its launches on ts, before ts goes away
         if (ts) {
-            (void)hipStreamSynchronize(ts);
+            const bool drained = hipStreamSynchronize(ts) == hipSuccess;
             if (c->last_stream == ts) c->last_stream = nullptr;  // drained: nothing to order after
-            (void)hipStreamDestroy(ts);
+            give_streams(own, drained);
         }
         c->release(dH);
         c->release(dF);
@@ -949,7 +1008,7 @@ int qcg_autotune_refine(qcg_context* c, const double* dD, int builds, int* chose
         c->profiling = prof;
     };
     if (c->alloc(&dH, n2) != hipSuccess || c->alloc(&dF, n2) != hipSuccess ||
-        hipStreamCreateWithFlags(&ts, hipStreamNonBlocking) != hipSuccess ||
+        (!ts && hipStreamCreateWithFlags(&ts, hipStreamNonBlocking) != hipSuccess) ||
         launch_fill(dH, n2, 0.0, ts) != hipSuccess) {
         cleanup();
         return fail(c, QCG_DEVICE, "autotune_refine: set-up");

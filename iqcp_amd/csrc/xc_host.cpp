@@ -654,8 +654,8 @@ int ks_fock_cb(void* u, const double* D, double* F, double* e_elec) {
     // V_xc on a stream of its own, concurrent with the J/K class kernels (the two share no buffer
     // and both only read D): the vector-ALU-bound integrals and the MFMA / HBM-bound grid products
     // overlap ((H2O)16: 9.80 -> 9.36 ms per mixed build, 16.35 -> 15.58 ms FP64)
-    if (!c->xc_stream) {
-        HIPCHK(c, hipStreamCreateWithFlags(&c->xc_stream, hipStreamNonBlocking));
+    if (!c->xc_stream) HIPCHK(c, hipStreamCreateWithFlags(&c->xc_stream, hipStreamNonBlocking));
+    if (!c->ev_xc_join) {
         HIPCHK(c, hipEventCreateWithFlags(&c->ev_xc_fork, hipEventDisableTiming));
         HIPCHK(c, hipEventCreateWithFlags(&c->ev_xc_join, hipEventDisableTiming));
     }
