@@ -363,12 +363,12 @@ def main():
             ks[f"{prec}_two_electron_plus_xc_energy"] = Ek
         ks["speedup_mixed_vs_fp64"] = round(ks["fp64_ms_per_build"] / ks["mixed_ms_per_build"], 3)
         # XC roofline: 4 n^2 (the two grid products) + 16 n (rho, grad rho, aow rows) + 300 (the
-        # functional) flops per point on MFMA (FP32 products in the mixed option, FP64 otherwise), n all
-        # functions in the mixed option's dense kernels and those that reach the point in the FP64 form;
+        # functional) flops per point on MFMA (FP32 products in the mixed option, FP64 otherwise), n the
+        # functions that reach the point (the mixed option's V product takes the zeros of the others too,
+        # which is no work that counts);
         # algorithmic bytes: Phi and grad Phi read once (4 n elements per point) + D, V (2 nbf^2 doubles)
-        n_pt = reaching_functions(bw, ew.get_grid()[0])
-        dense = torch.full_like(n_pt, bw.nbf)
-        for prec, peak, esz, n_ in (("mixed", 157.3, 4, dense), ("fp64", 78.6, 8, n_pt)):
+        n_ = reaching_functions(bw, ew.get_grid()[0])
+        for prec, peak, esz in (("mixed", 157.3, 4), ("fp64", 78.6, 8)):
             t_ = ks[f"{prec}_xc_ms"] * 1e-3
             xc_fl = float((4.0 * n_ * n_ + 16.0 * n_ + 300.0).sum())
             byts = 4.0 * float(n_.sum()) * esz + 2.0 * bw.nbf ** 2 * 8

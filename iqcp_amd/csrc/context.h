@@ -48,7 +48,6 @@ struct qcg_context {
     int* d_mol_nbf = nullptr;
     int64_t* d_mat_off = nullptr;
     int* d_ket_off = nullptr;
-    int* d_ket_cnt = nullptr;
     int64_t mat_total = 0;
     // work buffers
     double *d_D = nullptr, *d_J = nullptr, *d_K = nullptr;
@@ -241,7 +240,7 @@ struct qcg_context {
                          (void**)&d_Dp, (void**)&d_bf_norm, (void**)&d_jmap, (void**)&d_kmeta, (void**)&d_kcen,
                          (void**)&d_kprim, (void**)&d_khp, (void**)&d_kea, (void**)&d_katoms, (void**)&d_kprimf,
                          (void**)&d_H, (void**)&d_F, (void**)&d_mol_nbf,
-                         (void**)&d_mat_off, (void**)&d_ket_off, (void**)&d_ket_cnt, (void**)&d_items,
+                         (void**)&d_mat_off, (void**)&d_ket_off, (void**)&d_items,
                          (void**)&d_segs, (void**)&d_tensor_items, (void**)&d_tensor_segs, (void**)&d_grad_items, (void**)&d_grad_segs, (void**)&d_grad,
                          (void**)&d_W, (void**)&d_onee_int, (void**)&d_onee_dbl, (void**)&d_onee_work}) {
             release(*p);

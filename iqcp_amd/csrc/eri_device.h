@@ -15,10 +15,6 @@
 #include "qcg_types.h"
 #include "rys.h"
 
-#ifndef QCG_UNROLL_NQ
-#define QCG_UNROLL_NQ 128
-#endif
-
 namespace qcg {
 
 template <int LA, int LB, int LC, int LD>
@@ -29,7 +25,6 @@ struct EriShape {
     static constexpr int NROOTS = (LA + LB + LC + LD) / 2 + 1;
     static constexpr int G = (LAB + 1) * (LCD + 1);
     static constexpr int H4 = (LA + 1) * (LB + 1) * (LC + 1) * (LD + 1);
-    static constexpr bool kUnroll = NQ <= QCG_UNROLL_NQ;
 };
 
 // Component normalisation 1/sqrt((2i-1)!!(2j-1)!!(2k-1)!!) of component c of shell l
@@ -147,16 +142,10 @@ QCG_HD void static_for(F&& f) {
     static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
-// Run body(i) for i in [0, N): fully unrolled (constant i) when the class is small enough to live
-// in registers, a plain loop otherwise (large classes keep their arrays in scratch).
-template <bool UNROLL, int N, typename F>
+// body(i) for i in [0, N), fully unrolled: i is a constant after inlining.
+template <int N, typename F>
 QCG_HD void for_n(F&& body) {
-    if constexpr (UNROLL) {
-        static_for<N>([&](auto ic) { body((int)decltype(ic)::value); });
-    } else {
-#pragma unroll 1
-        for (int i = 0; i < N; ++i) body(i);
-    }
+    static_for<N>([&](auto ic) { body((int)decltype(ic)::value); });
 }
 
 // Accumulate the contracted quartet (bra pair P | ket pair Q) into eri[NQ] (row-major
@@ -221,29 +210,16 @@ QCG_HD void contract_quartet_pp(const PairRec& P, const PairRec& Q, const PrimPa
                 const R wp = rw[r] * pref;
 #pragma unroll
                 for (int h = 0; h < S::H4; ++h) iz[h] *= wp;
-                if constexpr (NK > 0 || S::kUnroll) {
-                    static_for<NQ>([&](auto kc) {
-                        constexpr int k = decltype(kc)::value;
-                        constexpr int hx = kCompTab<LA, LB, LC, LD>.hx[K0 + k];
-                        constexpr int hy = kCompTab<LA, LB, LC, LD>.hy[K0 + k];
-                        constexpr int hz = kCompTab<LA, LB, LC, LD>.hz[K0 + k];
-                        eri[k] += ix[hx] * iy[hy] * iz[hz];
-                    });
-                } else {
-                    constexpr const CompTab<LA, LB, LC, LD>& ct = kCompTab<LA, LB, LC, LD>;
-                    for_n<false, S::NQ>([&](int k) { eri[k] += ix[ct.hx[k]] * iy[ct.hy[k]] * iz[ct.hz[k]]; });
-                }
+                static_for<NQ>([&](auto kc) {
+                    constexpr int k = decltype(kc)::value;
+                    constexpr int hx = kCompTab<LA, LB, LC, LD>.hx[K0 + k];
+                    constexpr int hy = kCompTab<LA, LB, LC, LD>.hy[K0 + k];
+                    constexpr int hz = kCompTab<LA, LB, LC, LD>.hz[K0 + k];
+                    eri[k] += ix[hx] * iy[hy] * iz[hz];
+                });
             }
         }
     }
-}
-
-// contract_quartet_pp with both pairs' primitives read from the one array pp.
-template <int LA, int LB, int LC, int LD, typename R, bool TAB_N = false>
-QCG_HD void contract_quartet(const PairRec& P, const PairRec& Q, const PrimPair<R>* __restrict__ pp,
-                             const R* __restrict__ rys_tab, R* eri) {
-    const PrimPair<R>* ppk = pp + Q.pp_off;
-    contract_quartet_pp<LA, LB, LC, LD, R, TAB_N>(P, Q, pp + P.pp_off, [ppk](int j) { return ppk[j]; }, rys_tab, eri);
 }
 
 }  // namespace qcg

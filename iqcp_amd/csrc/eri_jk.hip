@@ -118,7 +118,7 @@ __device__ __forceinline__ void jk_item(const int4 it, const JkArgs& g, const Ke
 
     // bra density block scaled by the bra component norms
     double Dps[NAB], jp[NAB];
-    for_n<true, NAB>([&](int ab) {
+    for_n<NAB>([&](int ab) {
         const int a = ab / S::NB, b = ab % S::NB;
         Dps[ab] = drow(false, a, P.bfb + b) * cnorm(LA, A0 + a) * cnorm(LB, b);
         jp[ab] = 0.0;
@@ -136,28 +136,28 @@ __device__ __forceinline__ void jk_item(const int4 it, const JkArgs& g, const Ke
         const PairRec Q = ket_pair<LC, LD>(g.kpairs, kq, km);
         const int kstride = km.w;
         R eri[NQ];
-        for_n<true, NQ>([&](int i) { eri[i] = R(0); });
+        for_n<NQ>([&](int i) { eri[i] = R(0); });
         contract_quartet_pp<LA, LB, LC, LD, R, true, A0 * S::NB * S::NCD, NQ>(
             P, Q, ppb, [&](int i) { return kprims.at(km.z + i * kstride); }, rys_n, eri, sub, lanes);
         if (lg) {
             for (int off = 1; off < lanes; off <<= 1)
-                for_n<true, NQ>([&](int i) { eri[i] += __shfl_xor(eri[i], off, 64); });
+                for_n<NQ>([&](int i) { eri[i] += __shfl_xor(eri[i], off, 64); });
             if (sub) continue;  // the group's first lane digests
         }
         const double deg = deg_p * ((km.x & kKetSame) ? 0.5 : 1.0) * ((g.diag && q == pidx) ? 0.5 : 1.0);
         if (do_j) {
             double Dqs[S::NCD];
-            for_n<true, S::NCD>([&](int cd) { Dqs[cd] = g.Dp[g.jb_ket + cd * g.np_ket + kq]; });
+            for_n<S::NCD>([&](int cd) { Dqs[cd] = g.Dp[g.jb_ket + cd * g.np_ket + kq]; });
             const double fj = 2.0 * deg;
-            for_n<true, NAB>([&](int ab) {
+            for_n<NAB>([&](int ab) {
                 double s = 0.0;
-                for_n<true, S::NCD>([&](int cd) { s += Dqs[cd] * (double)eri[ab * S::NCD + cd]; });
+                for_n<S::NCD>([&](int cd) { s += Dqs[cd] * (double)eri[ab * S::NCD + cd]; });
                 const int a = ab / S::NB, b = ab % S::NB;
                 jp[ab] += fj * cnorm(LA, A0 + a) * cnorm(LB, b) * s;
             });
-            for_n<true, S::NCD>([&](int cd) {
+            for_n<S::NCD>([&](int cd) {
                 double s = 0.0;
-                for_n<true, NAB>([&](int ab) { s += Dps[ab] * (double)eri[ab * S::NCD + cd]; });
+                for_n<NAB>([&](int ab) { s += Dps[ab] * (double)eri[ab * S::NCD + cd]; });
                 const int c = cd / S::ND, d = cd % S::ND;
                 fix_add_global(Jacc, g.jb_ket + cd * g.np_ket + kq, fj * cnorm(LC, c) * cnorm(LD, d) * s, sJ);
             });
@@ -166,54 +166,54 @@ __device__ __forceinline__ void jk_item(const int4 it, const JkArgs& g, const Ke
             // Kacc_ik += D_jl v, Kacc_jk += D_il v, Kacc_il += D_jk v, Kacc_jl += D_ik v
             // (i in a, j in b, k in c, l in d); every D sub-block pre-scaled by the norms it sums over.
             double Dbd[S::NB * S::ND], Dad[NA * S::ND], Dbc[S::NB * S::NC], Dac[NA * S::NC];
-            for_n<true, S::NB * S::ND>([&](int i) {
+            for_n<S::NB * S::ND>([&](int i) {
                 const int b = i / S::ND, d = i % S::ND;
                 Dbd[i] = drow(true, b, Q.bfb + d) * cnorm(LB, b) * cnorm(LD, d);
             });
-            for_n<true, NA * S::ND>([&](int i) {
+            for_n<NA * S::ND>([&](int i) {
                 const int a = i / S::ND, d = i % S::ND;
                 Dad[i] = drow(false, a, Q.bfb + d) * cnorm(LA, A0 + a) * cnorm(LD, d);
             });
-            for_n<true, S::NB * S::NC>([&](int i) {
+            for_n<S::NB * S::NC>([&](int i) {
                 const int b = i / S::NC, c = i % S::NC;
                 Dbc[i] = drow(true, b, Q.bfa + c) * cnorm(LB, b) * cnorm(LC, c);
             });
-            for_n<true, NA * S::NC>([&](int i) {
+            for_n<NA * S::NC>([&](int i) {
                 const int a = i / S::NC, c = i % S::NC;
                 Dac[i] = drow(false, a, Q.bfa + c) * cnorm(LA, A0 + a) * cnorm(LC, c);
             });
 #define VIDX(a, b, c, d) ((((a) * S::NB + (b)) * S::NC + (c)) * S::ND + (d))
-            for_n<true, NA * S::NC>([&](int ac) {
+            for_n<NA * S::NC>([&](int ac) {
                 const int a = ac / S::NC, c = ac % S::NC;
                 double s = 0.0;
-                for_n<true, S::NB * S::ND>([&](int bd) {
+                for_n<S::NB * S::ND>([&](int bd) {
                     const int b = bd / S::ND, d = bd % S::ND;
                     s += Dbd[bd] * (double)eri[VIDX(a, b, c, d)];
                 });
                 kadd(false, a, Q.bfa + c, deg * cnorm(LA, A0 + a) * cnorm(LC, c) * s);
             });
-            for_n<true, S::NB * S::NC>([&](int bc) {
+            for_n<S::NB * S::NC>([&](int bc) {
                 const int b = bc / S::NC, c = bc % S::NC;
                 double s = 0.0;
-                for_n<true, NA * S::ND>([&](int ad) {
+                for_n<NA * S::ND>([&](int ad) {
                     const int a = ad / S::ND, d = ad % S::ND;
                     s += Dad[ad] * (double)eri[VIDX(a, b, c, d)];
                 });
                 kadd(true, b, Q.bfa + c, deg * cnorm(LB, b) * cnorm(LC, c) * s);
             });
-            for_n<true, NA * S::ND>([&](int ad) {
+            for_n<NA * S::ND>([&](int ad) {
                 const int a = ad / S::ND, d = ad % S::ND;
                 double s = 0.0;
-                for_n<true, S::NB * S::NC>([&](int bc) {
+                for_n<S::NB * S::NC>([&](int bc) {
                     const int b = bc / S::NC, c = bc % S::NC;
                     s += Dbc[bc] * (double)eri[VIDX(a, b, c, d)];
                 });
                 kadd(false, a, Q.bfb + d, deg * cnorm(LA, A0 + a) * cnorm(LD, d) * s);
             });
-            for_n<true, S::NB * S::ND>([&](int bd) {
+            for_n<S::NB * S::ND>([&](int bd) {
                 const int b = bd / S::ND, d = bd % S::ND;
                 double s = 0.0;
-                for_n<true, NA * S::NC>([&](int ac) {
+                for_n<NA * S::NC>([&](int ac) {
                     const int a = ac / S::NC, c = ac % S::NC;
                     s += Dac[ac] * (double)eri[VIDX(a, b, c, d)];
                 });
@@ -224,7 +224,7 @@ __device__ __forceinline__ void jk_item(const int4 it, const JkArgs& g, const Ke
     }
     // J_P: wave reduction (a fixed shuffle tree), one fixed-point add per component per wave
     if (do_j) {
-        for_n<true, NAB>([&](int ab) {
+        for_n<NAB>([&](int ab) {
             double s = jp[ab];
 #pragma unroll
             for (int off = 32; off >= 1; off >>= 1) s += __shfl_xor(s, off, 64);
@@ -461,12 +461,12 @@ __global__ __launch_bounds__(128) void eri_tensor_kernel(const int4* __restrict_
         const PairRec Q = ket_pair<LC, LD>(g.kpairs, q, km);
         const int kstride = km.w;
         double eri[S::NQ];
-        for_n<true, S::NQ>([&](int i) { eri[i] = 0.0; });
+        for_n<S::NQ>([&](int i) { eri[i] = 0.0; });
         contract_quartet_pp<LA, LB, LC, LD, double, true>(
             P, Q, pp + P.pp_off, [&](int i) { return kprims.at(km.z + i * kstride); }, rys_n, eri, sub, lanes);
         if (lg) {
             for (int off = 1; off < lanes; off <<= 1)
-                for_n<true, S::NQ>([&](int i) { eri[i] += __shfl_xor(eri[i], off, 64); });
+                for_n<S::NQ>([&](int i) { eri[i] += __shfl_xor(eri[i], off, 64); });
             if (sub) continue;
         }
         const bool same_q = km.x & kKetSame, same_pq = g.diag && q == P.pos;

@@ -152,10 +152,9 @@ struct JkLaunch {
     const double* fix;  // per molecule: scale of J, scale of K, and their inverses (fix_scale_kernel)
     int do_j, do_k;
     // batch of molecules (nmol = 1 for a single molecule): kets of bra pair P are
-    // ket[ket_off[P.mol] .. + ket_cnt[P.mol]); matrices of molecule m start at mat_off[m],
+    // those of the items from ket[ket_off[P.mol]] on; matrices of molecule m start at mat_off[m],
     // dimension mol_nbf[m]; nbf above is the largest mol_nbf.
     const int* ket_off;
-    const int* ket_cnt;
     const int64_t* mat_off;
     const int* mol_nbf;
     // J/K work items (index in the bra class list, first segment, offset into it, ket count) over
@@ -211,9 +210,7 @@ inline hipError_t launch_eri_tensor(int cb, int ck, const JkLaunch& a, double* o
 
 struct GradLaunch {
     const PairRec* bra;
-    int nbra;
     const PairRec* ket;
-    int nket;
     int diag;
     const PrimPair<double>* pp;  // ea and p - ea are the two primitive exponents
     KetPairs kpairs;             // the kets as arrays (per-lane kernels), kea their first exponents
@@ -223,7 +220,6 @@ struct GradLaunch {
     const double* D;
     int nbf;
     double xfac;  // exchange weight c = hf_frac / 4 (eri_gradient_fused, scf/gradient.rs:1438)
-    double thr;
     int natom;
     double* grad;  // 3 * natom, accumulated
     // work items (index in the bra class list, first segment, offset into it, ket count) over the

@@ -25,11 +25,11 @@ __global__ __launch_bounds__(256) void schwarz_kernel(const PairRec* __restrict_
     };
     if constexpr (S::NQ <= 81) {
         double eri[S::NQ];
-        for_n<true, S::NQ>([&](int k) { eri[k] = 0.0; });
+        for_n<S::NQ>([&](int k) { eri[k] = 0.0; });
         const PrimPair<double>* ppk = pp + P.pp_off;
         contract_quartet_pp<LA, LB, LA, LB, double>(P, P, ppk, [ppk](int j) { return ppk[j]; }, rys_tab, eri, lane, 64);
-        for (int off = 1; off < 64; off <<= 1) for_n<true, S::NQ>([&](int k) { eri[k] += __shfl_xor(eri[k], off, 64); });
-        for_n<true, S::NQ>([&](int k) { mx = fmax(mx, fabs(eri[k] * norm(k))); });
+        for (int off = 1; off < 64; off <<= 1) for_n<S::NQ>([&](int k) { eri[k] += __shfl_xor(eri[k], off, 64); });
+        for_n<S::NQ>([&](int k) { mx = fmax(mx, fabs(eri[k] * norm(k))); });
     } else {
         using TB = WaveTable<LA, LB, LA, LB, S::NROOTS, double>;
         constexpr int KPL = (S::NQ + 63) / 64;

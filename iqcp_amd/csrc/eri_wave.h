@@ -12,7 +12,7 @@
 //            prefactor are folded into the z rows;
 //   phase B  lanes over Cartesian components: I(abcd) += Ix Iy Iz over the entries of the chunk;
 //   phase C  (caller) digestion of the contracted quartet.
-// The integrals are the same as contract_quartet's (eri_device.h), summed in the same order.
+// The integrals are contract_quartet_pp's (eri_device.h), with the bra's primitives outermost in the sum.
 #pragma once
 #include "eri_device.h"
 
@@ -41,7 +41,7 @@ struct WaveTable {
 
 // Phase A for the chunk of primitive quartets [pq0, pq0 + npc) of (P|Q): every lane of the wave
 // takes (primitive quartet, node, axis) units.  Primitive pair i of P and j of Q form primitive
-// quartet i * Q.npp + j (the loop order of contract_quartet).  Quartets failing the primitive
+// quartet i * Q.npp + j (bra primitives outer).  Quartets failing the primitive
 // screen k_ab k_cd >= 1e-15 get zero z rows.
 template <int TA, int TB, int TC, int TD, int N, int ES, typename R>
 __device__ __forceinline__ void wave_tables(const PairRec& P, const PairRec& Q, const PrimPair<R>* __restrict__ pp,

@@ -101,9 +101,7 @@ int qcg::eri_grad_launch(qcg_context* c, const double* dD, double hf_frac, doubl
         const int cls = order[k], cb = cls_cb[cls], ck = cls_ck[cls];
         GradLaunch a{};
         a.bra = c->d_pairs + c->class_off[cb];
-        a.nbra = c->class_off[cb + 1] - c->class_off[cb];
         a.ket = c->d_pairs + c->class_off[ck];
-        a.nket = c->class_off[ck + 1] - c->class_off[ck];
         a.diag = cb == ck;
         a.pp = c->d_pp;
         a.kpairs = ket_pairs(c, ck);
@@ -113,7 +111,6 @@ int qcg::eri_grad_launch(qcg_context* c, const double* dD, double hf_frac, doubl
         a.D = dD;
         a.nbf = c->basis.nbf;
         a.xfac = 0.25 * hf_frac;
-        a.thr = c->schwarz_thr;
         a.natom = c->basis.natom;
         a.grad = dgrad;
         a.items = c->d_grad_items + c->grad_off[cls];

@@ -508,11 +508,9 @@ int qcg_set_basis_batch(qcg_context* c, int nmol, const int* mol_nshell, const i
     HIPCHK(c, c->alloc(&c->d_mol_nbf, nmol));
     HIPCHK(c, c->alloc(&c->d_mat_off, nmol));
     HIPCHK(c, c->alloc(&c->d_ket_off, kNumPairClasses * nmol));
-    HIPCHK(c, c->alloc(&c->d_ket_cnt, kNumPairClasses * nmol));
     HIPCHK(c, hipMemcpy(c->d_mol_nbf, c->mol_nbf_h.data(), nmol * sizeof(int), hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->d_mat_off, c->mat_off_h.data(), nmol * sizeof(int64_t), hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->d_ket_off, c->ket_off_h.data(), c->ket_off_h.size() * sizeof(int), hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemcpy(c->d_ket_cnt, c->ket_cnt_h.data(), c->ket_cnt_h.size() * sizeof(int), hipMemcpyHostToDevice));
     const size_t n2 = (size_t)c->mat_total;
     HIPCHK(c, c->alloc(&c->d_D, n2));
     HIPCHK(c, c->alloc(&c->d_J, n2));
@@ -848,7 +846,6 @@ int qcg::run_jk(qcg_context* c, const double* dD, double* dJ, double* dK, hipStr
             a.do_j = do_j;
             a.do_k = do_k;
             a.ket_off = c->d_ket_off + ck * c->nmol;
-            a.ket_cnt = c->d_ket_cnt + ck * c->nmol;
             a.mat_off = c->d_mat_off;
             a.mol_nbf = c->d_mol_nbf;
             a.items = c->d_items + c->item_off[cls][part];

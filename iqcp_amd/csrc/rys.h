@@ -23,7 +23,8 @@ constexpr int rys_tab_size() { return qcg_rys_nint[N] * rys_stride<N>(); }
 // per primitive quartet, and for the classes of low angular momentum that is what bounds them: with 14
 // coefficients per polynomial on equal intervals the kernels of a (H2O)16 6-31G* FP64 build took 4.33 ms
 // one after the other and the 64-alkane batch 20.8 ms, with 10 (N <= 2) or 12 on intervals that widen with
-// T, strides that spread the intervals over the banks and tables of about the same size 4.01 and 19.0 ms.
+// T and strides that spread the intervals over the banks 4.01 and 19.0 ms.  (The staged tables are of 902, 1848
+// and 2294 words for one to three nodes; 560, 1288 and 2268 before.)
 // c[0] + c[1] s + ... + c[DEG] s^DEG in Estrin's scheme: dependency depth 5 instead of Horner's DEG
 // (the FP64 FMA latency, not the issue rate, bounds a lone Horner chain per lane).
 template <int DEG, typename R>
