@@ -1,11 +1,13 @@
 // Host side of the qcg library: context, basis/pair setup, C ABI (include/qcg.h).
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
 #include <memory>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "context.h"
@@ -34,55 +36,65 @@ double qcg::nuclear_repulsion(const HostBasis& B) {
 
 namespace {
 
-// Streams outlive their contexts: a destroyed context leaves its set to the next one on the device.  The runtime
-// frees a stream's queue object in hipStreamDestroy while its completion thread may still be leaving that object's
-// lock for the last command, however well the stream has been waited for: now and then a word of the freed
-// heap block was decremented and another zeroed afterwards, once the low half of a contraction coefficient of the
-// context made next, whose V_xc was then off by 1.5e-8.  At most kIdleSets sets wait (six streams each); the
-// streams of further ones are destroyed.
+// Streams outlive their contexts by kRetired.  The runtime frees a stream's queue object in hipStreamDestroy while
+// its completion thread may still be leaving that object's lock for the last command, however well the stream has
+// been waited for: now and then a word of the freed heap block was decremented and another zeroed afterwards, once the
+// low half of a contraction coefficient of the context made next, whose V_xc was then off by 1.5e-8.  So a destroyed
+// context's streams wait here until a later call finds them old enough, at most kRetiredSets sets of six (the oldest
+// goes at once for one more).  qcg_create waits for those that are not: the runtime deals new streams over the hardware
+// queues by what is alive, and with a set still there two auxiliary streams came to share one (J/K of (H2O)2 215 ->
+// 350 us; benzene, mixed, 515 -> 590 us with the old streams taken over instead of new ones).
+using Clock = std::chrono::steady_clock;
 struct StreamSet {
+    Clock::time_point since;
     int device = 0;
-    hipStream_t main = nullptr, aux[qcg_context::kStreams] = {}, xc = nullptr;
+    hipStream_t s[qcg_context::kStreams + 2] = {};
 };
-constexpr size_t kIdleSets = 16;
-struct IdleStreams {
+constexpr auto kRetired = std::chrono::milliseconds(1);
+constexpr size_t kRetiredSets = 32;
+struct Retired {
     std::mutex m;
-    std::vector<StreamSet> sets;
-    IdleStreams() { sets.reserve(kIdleSets); }
+    std::vector<StreamSet> sets;  // oldest first
+    Retired() { sets.reserve(kRetiredSets + 1); }
 };
-IdleStreams& idle_streams() {
-    static IdleStreams* p = new IdleStreams;  // never destroyed: at exit the runtime may be gone
+Retired& retired() {
+    static Retired* p = new Retired;  // never destroyed: at exit the runtime may be gone
     return *p;
 }
 
-StreamSet take_streams(int device) {
-    IdleStreams& I = idle_streams();
-    const std::lock_guard<std::mutex> lock(I.m);
-    for (size_t i = I.sets.size(); i-- > 0;)
-        if (I.sets[i].device == device) {
-            const StreamSet s = I.sets[i];
-            I.sets.erase(I.sets.begin() + i);
-            return s;
-        }
-    StreamSet s;
-    s.device = device;
-    return s;
+// Destroys the sets that are old enough.
+void destroy_retired(Retired& R) {
+    const auto now = Clock::now();
+    size_t n = 0;
+    for (; n < R.sets.size() && (R.sets.size() - n > kRetiredSets || now - R.sets[n].since >= kRetired); ++n) {
+        (void)hipSetDevice(R.sets[n].device);
+        for (hipStream_t a : R.sets[n].s)
+            if (a) (void)hipStreamDestroy(a);
+    }
+    R.sets.erase(R.sets.begin(), R.sets.begin() + n);
 }
 
-// drained: every stream of the set has been waited for without an error
-void give_streams(const StreamSet& s, bool drained) {
-    if (drained) {
-        IdleStreams& I = idle_streams();
-        const std::lock_guard<std::mutex> lock(I.m);
-        if (I.sets.size() < kIdleSets) {
-            I.sets.push_back(s);
-            return;
-        }
+void retire_streams(StreamSet add) {
+    Retired& R = retired();
+    const std::lock_guard<std::mutex> lock(R.m);
+    add.since = Clock::now();
+    R.sets.push_back(add);
+    destroy_retired(R);
+}
+
+// Waits until the sets that are retired now are old enough and destroys them; device: the current one.
+void flush_retired(int device) {
+    Retired& R = retired();
+    std::unique_lock<std::mutex> lock(R.m);
+    if (R.sets.empty()) return;
+    const auto until = R.sets.back().since + kRetired;
+    if (Clock::now() < until) {
+        lock.unlock();
+        std::this_thread::sleep_until(until);
+        lock.lock();
     }
-    for (hipStream_t a : s.aux)
-        if (a) (void)hipStreamDestroy(a);
-    if (s.xc) (void)hipStreamDestroy(s.xc);
-    if (s.main) (void)hipStreamDestroy(s.main);
+    destroy_retired(R);
+    (void)hipSetDevice(device);
 }
 
 }  // namespace
@@ -98,11 +110,8 @@ int qcg_create(qcg_context** out, int device) {
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev <= 0) return QCG_DEVICE;
     if (device < 0 || device >= ndev) return QCG_INVALID_ARG;
     if (hipSetDevice(device) != hipSuccess) return QCG_DEVICE;
-    const StreamSet streams = take_streams(device);
-    c->stream = streams.main;
-    std::copy(streams.aux, streams.aux + qcg_context::kStreams, c->aux);
-    c->xc_stream = streams.xc;
-    if (!c->stream && hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) return QCG_DEVICE;
+    flush_retired(device);
+    if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) return QCG_DEVICE;
     // the static scratch of qcg_build_jk_device_noalloc; a failure surfaces in that entry point
     (void)noalloc_setup(device);
     const size_t nt = sizeof(qcg_rys_coef) / sizeof(double);
@@ -133,16 +142,15 @@ void qcg_destroy(qcg_context* c) {
     if (!c) return;
     (void)hipSetDevice(c->device);
     c->drop_fock_graph();  // waits for the exec's last launch
-    bool drained = hipStreamSynchronize(c->stream) == hipSuccess;
+    (void)hipStreamSynchronize(c->stream);
     if (c->ev_done) (void)hipEventSynchronize(c->ev_done);  // the last entry point's work on any stream
     StreamSet streams;
     streams.device = c->device;
-    streams.main = c->stream;
-    streams.xc = c->xc_stream;
-    std::copy(c->aux, c->aux + qcg_context::kStreams, streams.aux);
-    for (hipStream_t a : c->aux)
-        if (a) drained = hipStreamSynchronize(a) == hipSuccess && drained;
-    if (c->xc_stream) drained = hipStreamSynchronize(c->xc_stream) == hipSuccess && drained;
+    std::copy(c->aux, c->aux + qcg_context::kStreams, streams.s);
+    streams.s[qcg_context::kStreams] = c->xc_stream;
+    streams.s[qcg_context::kStreams + 1] = c->stream;
+    for (hipStream_t a : streams.s)
+        if (a) (void)hipStreamSynchronize(a);
     for (void* p : c->owned) (void)hipFree(p);
     c->owned.clear();
     if (c->ev_made)
@@ -154,7 +162,7 @@ void qcg_destroy(qcg_context* c) {
     if (c->ev_xc_fork) (void)hipEventDestroy(c->ev_xc_fork);
     if (c->ev_xc_join) (void)hipEventDestroy(c->ev_xc_join);
     if (c->blas) (void)rocblas_destroy_handle(c->blas);
-    give_streams(streams, drained);
+    retire_streams(streams);
     delete c;
 }
 
@@ -743,7 +751,7 @@ static int prepare_streams(qcg_context* c) {
     if (!c->ev_fork) {
         HIPCHK(c, hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
         for (int i = 0; i < qcg_context::kStreams; ++i) {
-            if (!c->aux[i]) HIPCHK(c, hipStreamCreateWithFlags(&c->aux[i], hipStreamNonBlocking));
+            HIPCHK(c, hipStreamCreateWithFlags(&c->aux[i], hipStreamNonBlocking));
             HIPCHK(c, hipEventCreateWithFlags(&c->ev_join[i], hipEventDisableTiming));
         }
     }
@@ -989,15 +997,17 @@ int qcg_autotune_refine(qcg_context* c, const double* dD, int builds, int* chose
     // hipStreamBeginCapture); run_jk refuses to rebuild it inside a capture.
     const size_t n2 = (size_t)c->basis.nbf * c->basis.nbf;
     double *dH = nullptr, *dF = nullptr;
-    StreamSet own = take_streams(c->device);
-    hipStream_t& ts = own.main;
+    hipStream_t ts = nullptr;
     const bool graph = c->use_graph;
     auto cleanup = [&]() {
         c->drop_fock_graph();  // waits for its launches on ts, before ts goes away
         if (ts) {
-            const bool drained = hipStreamSynchronize(ts) == hipSuccess;
+            (void)hipStreamSynchronize(ts);
             if (c->last_stream == ts) c->last_stream = nullptr;  // drained: nothing to order after
-            give_streams(own, drained);
+            StreamSet own;
+            own.device = c->device;
+            own.s[0] = ts;
+            retire_streams(own);
         }
         c->release(dH);
         c->release(dF);
@@ -1005,7 +1015,7 @@ int qcg_autotune_refine(qcg_context* c, const double* dD, int builds, int* chose
         c->profiling = prof;
     };
     if (c->alloc(&dH, n2) != hipSuccess || c->alloc(&dF, n2) != hipSuccess ||
-        (!ts && hipStreamCreateWithFlags(&ts, hipStreamNonBlocking) != hipSuccess) ||
+        hipStreamCreateWithFlags(&ts, hipStreamNonBlocking) != hipSuccess ||
         launch_fill(dH, n2, 0.0, ts) != hipSuccess) {
         cleanup();
         return fail(c, QCG_DEVICE, "autotune_refine: set-up");

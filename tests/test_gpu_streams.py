@@ -1,5 +1,5 @@
-"""Contexts made and destroyed one after the other, many at a time and from several threads: a destroyed
-context's streams go to the next one.  J and K are integer sums, so every context's have the same bits; V_xc and
+"""Contexts made and destroyed one after the other, many at a time and from several threads: the streams of a
+destroyed context are kept for a moment and destroyed by a later call.  J and K are integer sums, so every context's have the same bits; V_xc and
 the gradient come from fixed orders of FP64 sums (atomic ones for the gradient's: 1e-10)."""
 import threading
 
@@ -21,7 +21,7 @@ def _use(eng, b, D, ref, xyz, w, xc):
         assert np.abs(eng.xc_gradient(D) - ref["g"]).max() < 1e-10
 
 
-def test_gpu_streams_pass_from_context_to_context():
+def test_gpu_contexts_in_turn_and_from_threads():
     b = bench_molecule("H2O", "6-31g*")
     rng = np.random.default_rng(1)
     xyz, w = b.xyz[rng.integers(0, b.natom, 500)] + rng.normal(0.0, 1.5, (500, 3)), rng.uniform(0.0, 0.5, 500)
@@ -33,7 +33,7 @@ def test_gpu_streams_pass_from_context_to_context():
     eng.build_grid(30)
     e_ks = eng.ks_scf()["energy_total"]
     eng.close()
-    for alive in (1, 1, 20, 20, 3):  # 20: more than are kept
+    for alive in (1, 1, 20, 20, 3):
         engs = [Engine(b) for _ in range(alive)]
         for i, e in enumerate(engs):
             _use(e, b, D, ref, xyz, w, i % 2 == 0)
