@@ -73,7 +73,9 @@ constexpr int kJkLaneMaxNQ = 81;
 // class with at most two or three parts is the faster one once a launch has lanes enough (default_tiles):
 // (H2O)16 6-31G* FP64 (dp|ds) 0.50 -> 0.18 ms, (dd|ps) 0.29 -> 0.20, (dp|pp) 0.25 -> 0.22, the build 3.40 ->
 // 2.73 ms.  At a total angular momentum of 6 the classes alone are slower ((dp|dp) 0.12 -> 0.28 ms), but run
-// beside others on the four streams they fill the chip better: build 2.80 ms without them, 2.73 with.
+// beside others on the four streams they fill the chip better: build 2.80 ms without them, 2.73 with.  The same
+// with and without them over sizes, FP64 / mixed: (H2O)12 -2 / -1 %, (H2O)16 -4 / -2 %, (H2O)24 -4 / -3 %, dodecane
+// -2 / -1 %, decane 0 / 0, (H2O)8 6-31+G* +1 / +1 %; smaller molecules have too few quartets for parts.
 // Above, (dd|dp) and (dd|dd) would need six or more parts.
 constexpr int kJkPartMaxNQ = 54;
 constexpr int kJkPartMaxL = 6;
