@@ -176,7 +176,7 @@ struct qcg_context {
     // made on its first use for the current grid
     float *d_phi32 = nullptr, *d_aow32 = nullptr, *d_D32 = nullptr;
     float4* d_grid4 = nullptr;  // (Phi, dPhi/dx, dPhi/dy, dPhi/dz) per element, FP32
-    unsigned* d_tile_mask = nullptr;  // per 16 points: tiles of 16 functions that are not zero there
+    unsigned* d_tile_mask = nullptr;  // per 16 points: tiles of 16 functions that reach them
     GridShell* d_gshell = nullptr;
     double *d_gexp = nullptr, *d_gcn = nullptr;
     // The packed FP64 form of the grid (xc_packed.h), made with the grid when the precision option is

@@ -323,7 +323,7 @@ int make_xc32(qcg_context* c, hipStream_t st) {
     HIPCHK(c, launch_to_f32x4(c->d_phi, c->d_dphx, c->d_dphy, c->d_dphz, c->d_grid4, gn, st));
     if (const size_t nm = xc_tile_mask_words((int)c->G, c->basis.nbf)) {
         HIPCHK(c, c->alloc(&c->d_tile_mask, nm));
-        HIPCHK(c, launch_tile_mask((int)c->G, c->basis.nbf, c->d_grid4, c->d_tile_mask, st));
+        HIPCHK(c, launch_tile_mask((int)c->G, c->basis.nbf, c->basis.nshell, c->d_gshell, c->d_pts, c->d_tile_mask, st));
     }
     return QCG_OK;
 }

@@ -24,10 +24,10 @@ hipError_t launch_sym_half(const double* V, double* out, int n, hipStream_t st);
 hipError_t launch_xc_mfma(int G, int nbf, int nchunk, const double* w, const float* phi, const float4* g4,
                           const unsigned* mask, const float* Dm, float* aow, double* exc_sum, double* Vparts,
                           hipStream_t st);
-// words of the FP32 form's tile mask (one per 16 points, padded; 0: this basis takes none) and the kernel
-// that fills it; mask null in launch_xc_mfma: column passes, no skipping
+// words of the FP32 form's tile mask (one per 16 points, padded; 0: this basis takes none) and the kernel that fills it
 size_t xc_tile_mask_words(int G, int nbf);
-hipError_t launch_tile_mask(int G, int nbf, const float4* g4, unsigned* mask, hipStream_t st);
+hipError_t launch_tile_mask(int G, int nbf, int nshell, const GridShell* shells, const double* pts, unsigned* mask,
+                            hipStream_t st);
 hipError_t launch_xc_mfma(int G, int nbf, int nchunk, const double* w, const double* phi, const double* dpx,
                           const double* dpy, const double* dpz, const double* Dm, double* aow, double* exc_sum,
                           double* Vparts, hipStream_t st);

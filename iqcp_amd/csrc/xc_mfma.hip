@@ -313,7 +313,7 @@ __global__ __launch_bounds__(256) void xc_rho_kernel(int G, int nbf, const doubl
 // FP64 products run here in a build that is captured on a grid made for the mixed option (xc_build); they
 // stage D without the look-ahead, whose registers would cost the second block per CU ((H2O)16, 1.05e6 points:
 // 11.2 -> 9.3 ms), and take no mask.
-// mask (FP32): per 16 points the tiles of 16 functions of which Phi or grad Phi has a nonzero element there
+// mask (FP32, more than kRhoMaskNT tiles): per 16 points the tiles of 16 functions that reach one of them
 // (tile_mask_kernel).  K steps that are zero at all 64 points are not staged, and a wavefront multiplies only
 // the K steps and column tiles that its 16 points see: what is left out are exact zeros, so every sum keeps
 // its bits.  (H2O)16, 1.05e6 points, FP32: 2.97 -> 2.50 ms.  (The
@@ -463,28 +463,40 @@ __global__ __launch_bounds__(512) QCG_XC_RHO_ATTR void xc_rho_all_kernel(int G, 
     xc_point_tail<T, 8, (16 * NT + 63) / 64>(G, nbf, wv, l, g0, w, gv, aow, exc_sum, red, coef, part, kMask ? wm : ~0u);
 }
 
-// One wavefront per 16 points: the tiles of 16 functions with a nonzero element there.
-__global__ __launch_bounds__(256) void tile_mask_kernel(int G, int nbf, int n, const float4* __restrict__ g4,
-                                                        unsigned* __restrict__ mask) {
+// One wavefront per 16 points, four lanes to a point: the tiles of 16 functions of the shells that reach one of the points
+// (basis_kernel's cut-off, with room for another rounding of it).  From the points and shells instead of the 16 nbf
+// bytes per point of the arrays: the first mixed build on a grid of (H2O)16, 286081 points, 3.20 -> 2.97 ms
+// (3.04 ms before there was a mask), the same bits of V.
+__global__ __launch_bounds__(256) void tile_mask_kernel(int G, int nshell, int n, const GridShell* __restrict__ shells,
+                                                        const double* __restrict__ pts, unsigned* __restrict__ mask) {
     const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (i >= n) return;
+    const size_t p = 16 * (size_t)i + (lane & 15);
     unsigned m = 0;
-    for (int p = 16 * i; p < min(G, 16 * i + 16); ++p)
-        for (int c = lane; c < nbf; c += 64) {
-            const float4 v = g4[(size_t)p * nbf + c];
-            if (v.x != 0.f || v.y != 0.f || v.z != 0.f || v.w != 0.f) m |= 1u << (c >> 4);
+    if (p < (size_t)G) {
+        const double x = pts[3 * p], y = pts[3 * p + 1], z = pts[3 * p + 2];
+        for (int s = lane >> 4; s < nshell; s += 4) {
+            const double dx = x - shells[s].cx, dy = y - shells[s].cy, dz = z - shells[s].cz;
+            const int f = shells[s].bf;
+            if (!(shells[s].amin * (dx * dx + dy * dy + dz * dz) > kGridCut * (1.0 + 1e-12)))
+                m |= 1u << (f >> 4) | 1u << ((f + ncart(shells[s].l) - 1) >> 4);
         }
+    }
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) m |= __shfl_xor(m, off, 64);
     if (lane == 0) mask[i] = m;
 }
 
-size_t xc_tile_mask_words(int G, int nbf) { return nbf <= 16 * kRhoAllMaxNT ? 4 * ((size_t)(G + 63) / 64) + 4 : 0; }
+size_t xc_tile_mask_words(int G, int nbf) {
+    const int tiles = (nbf + 15) / 16;
+    return tiles > kRhoMaskNT && tiles <= kRhoAllMaxNT ? 4 * ((size_t)(G + 63) / 64) + 4 : 0;
+}
 
-hipError_t launch_tile_mask(int G, int nbf, const float4* g4, unsigned* mask, hipStream_t st) {
+hipError_t launch_tile_mask(int G, int nbf, int nshell, const GridShell* shells, const double* pts, unsigned* mask,
+                            hipStream_t st) {
     const int n = (int)xc_tile_mask_words(G, nbf);
     if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(tile_mask_kernel, dim3((n + 3) / 4), dim3(256), 0, st, G, nbf, n, g4, mask);
+    hipLaunchKernelGGL(tile_mask_kernel, dim3((n + 3) / 4), dim3(256), 0, st, G, nshell, n, shells, pts, mask);
     return hipGetLastError();
 }
 
@@ -1050,7 +1062,8 @@ static hipError_t launch_xc_mfma_t(int G, int nbf, int nchunk, const double* w, 
     const int tiles = (nbf + 15) / 16, passes = (tiles + kMaxNT - 1) / kMaxNT, nt = (tiles + passes - 1) / passes;
     const dim3 grid((G + kRhoBM - 1) / kRhoBM);
     // up to kRhoAllMaxNT column tiles: the all-columns kernel (Phi read once per K step)
-    switch (tiles <= kRhoAllMaxNT && (sizeof(T) == 8 || mask) ? 100 + tiles : nt) {
+    if (sizeof(T) == 4 && !mask && xc_tile_mask_words(G, nbf)) return hipErrorInvalidValue;
+    switch (tiles <= kRhoAllMaxNT ? 100 + tiles : nt) {
 #define QCG_RHO_ALL(n)                                                                                  \
     case 100 + n:                                                                                       \
         hipLaunchKernelGGL((xc_rho_all_kernel<T, n>), grid, dim3(512), 0, st, G, nbf, w, phi, gv, Dm, aow,  \

@@ -219,3 +219,20 @@ def test_gpu_packed_block_sizes(n):
     eng.set_grid(xyz, w)
     V2, _ = eng.xc(D)
     assert np.array_equal(V2, V) and np.abs(eng.xc_gradient(D) - g).max() < 1e-10
+
+
+@pytest.mark.parametrize("n", [10, 11, 16, 18])
+def test_gpu_mixed_tiles_of_any_shell_order(n):
+    """12 to 22 tiles of 16 functions, the shells in a random order (d shells across two tiles), on a row of waters
+    3 angstrom apart, so that most tiles reach few points: the mixed option's V against FP64 products, bounds as
+    above."""
+    b = build_basis(workloads.water_cluster((n, 1, 1), 3.0, 3), "6-31g*", units="angstrom")
+    b = _reordered(b, np.random.default_rng(n).permutation(b.nshell))
+    xyz, w = _points(b, 3001, n)
+    xyz = xyz[np.argsort(xyz[:, 0])]
+    D = random_density(b.nbf, seed=9, nocc=b.n_occ)
+    Vo, Eo, _ = oracle.vxc(*oracle.basis_on_grid(b, xyz), w, D)
+    eng = Engine(b, precision="mixed")
+    eng.set_grid(xyz, w)
+    V, E = eng.xc(D)
+    assert np.abs(V - Vo).max() < 1e-5 and abs(E - Eo) < 1e-6 * max(1.0, abs(Eo))
