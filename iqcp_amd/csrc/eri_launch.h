@@ -274,6 +274,25 @@ inline hipError_t launch_grad(int cb, int ck, const GradLaunch& a, hipStream_t s
 hipError_t launch_schwarz(int c, const PairRec* pairs, int n, const PrimPair<double>* pp, const double* rys,
                           double* Q, hipStream_t st);
 hipError_t launch_fill(double* x, size_t n, double v, hipStream_t st);
+// The kets of all classes as arrays (KetPairs, KetPrims) from the pair records and their primitive pairs: meta is
+// given, the others are written.  jmap: of every matrix element the word of the pair-ordered J arrays, pair i of
+// class k and component ab at jbase[k] + ab * (pairs of the class) + i, -1 where only the transposed element has one.
+struct KetArrays {
+    int np, npr;  // pairs, primitive pairs
+    int off[kNumPairClasses + 1], jbase[kNumPairClasses], nb[kNumPairClasses], nab[kNumPairClasses];
+    const PairRec* pairs;
+    const PrimPair<double>* pp;
+    const PrimPair<float>* ppf;
+    const int4* meta;
+    const int64_t* mat_off;
+    const int* mol_nbf;
+    double2 *cen, *prim;
+    double *hp, *ea;
+    int2* atoms;
+    float4* primf;
+    int* jmap;
+};
+hipError_t launch_ket_arrays(const KetArrays& a, size_t mat_total, hipStream_t st);
 // What the fixed-point scale kernels read (device pointers, packed per molecule): the Schwarz bounds
 // of the shell pairs as nshell x nshell matrices (qsh, offsets qsh_off), their maximum (qmax), the
 // shell of every function (bf_shell, offsets bf_off into the functions of all molecules), the first

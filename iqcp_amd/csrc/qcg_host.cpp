@@ -191,6 +191,12 @@ int qcg_nbf(const qcg_context* c, int* nbf) {
     return QCG_OK;
 }
 
+// Angular momenta of a pair class.
+static void class_l(int k, int& la, int& lb) {
+    la = k == 0 ? 0 : k <= 2 ? 1 : 2;
+    lb = (k == 0 || k == 1 || k == 3) ? 0 : (k == 2 || k == 4) ? 1 : 2;
+}
+
 int qcg_set_basis(qcg_context* c, int nshell, const int* l, const int* nprim, const int* prim_off,
                   const double* exps, const double* coefs, const double* centers, const int* shell_atom,
                   int natom, const int* Z, const double* xyz) {
@@ -430,89 +436,6 @@ int qcg_set_basis_batch(qcg_context* c, int nmol, const int* mol_nshell, const i
         }
     HIPCHK(c, hipMemcpy(c->d_pairs, all.data(), all.size() * sizeof(PairRec), hipMemcpyHostToDevice));
     c->pairs = all;
-    {
-        // the kets as arrays in list order (KetPairs, KetPrims), and the pair order of the J side
-        const int np = npairs, npr = (int)pp.size();
-        std::vector<int4> meta(np);
-        std::vector<double2> cen(3 * (size_t)np), kp(3 * (size_t)npr);
-        std::vector<double> khp(npr), kea(npr);
-        std::vector<int2> katoms(np);
-        std::vector<float4> kpf(2 * (size_t)npr);
-        int first = 0;
-        for (int k = 0; k < kNumPairClasses; ++k)
-            for (int m = 0; m < nmol; ++m) {
-                const std::vector<int>& bnd = c->bucket_bnd[k * nmol + m];
-                const int base = c->class_off[k] + c->ket_off_h[k * nmol + m];
-                for (size_t b = 0; b + 1 < bnd.size(); ++b) {
-                    const int n = bnd[b + 1] - bnd[b], npp = all[base + bnd[b]].npp;
-                    for (int i = 0; i < n; ++i) {
-                        const int g = base + bnd[b] + i;
-                        const PairRec& r = all[g];
-                        meta[g] = make_int4(r.bfa | r.bfb << kKetBfBits | (r.sa == r.sb ? kKetSame : 0), npp, first + i, n);
-                        katoms[g] = make_int2(r.atom_a, r.atom_b);
-                        cen[g] = make_double2(r.ax, r.ay);
-                        cen[(size_t)np + g] = make_double2(r.az, r.abx);
-                        cen[2 * (size_t)np + g] = make_double2(r.aby, r.abz);
-                        for (int j = 0; j < npp; ++j) {
-                            const size_t e = (size_t)first + i + (size_t)j * n;
-                            const PrimPair<double>& q = pp[r.pp_off + j];
-                            const PrimPair<float>& f = ppf[r.pp_off + j];
-                            kp[e] = make_double2(q.px, q.py);
-                            kp[npr + e] = make_double2(q.pz, q.p);
-                            kp[2 * (size_t)npr + e] = make_double2(q.ckp, q.kab);
-                            khp[e] = q.hp;
-                            kea[e] = q.ea;
-                            kpf[e] = make_float4(f.px, f.py, f.pz, f.p);
-                            kpf[npr + e] = make_float4(f.ckp, f.hp, f.kab, f.ea);
-                        }
-                    }
-                    first += n * npp;
-                }
-            }
-        std::vector<int> jmap((size_t)c->mat_total, -1);
-        std::vector<double> bfn;
-        for (const HostBasis& B : c->mols)
-            for (int s = 0; s < B.nshell; ++s)
-                for (int k = 0; k < ncart(B.l[s]); ++k) bfn.push_back(B.l[s] == 2 && (k == 0 || k == 3 || k == 5) ? 0.57735026918962576451 : 1.0);
-        int64_t words = 0;
-        for (int k = 0; k < kNumPairClasses; ++k) {
-            const int na = k == 0 ? 1 : k <= 2 ? 3 : 6, nb = (k == 0 || k == 1 || k == 3) ? 1 : (k == 2 || k == 4) ? 3 : 6;
-            const int n = c->class_off[k + 1] - c->class_off[k];
-            c->jbase[k] = (int)words;
-            for (int i = 0; i < n; ++i) {
-                const PairRec& r = all[c->class_off[k] + i];
-                const int64_t nbf = c->mol_nbf_h[r.mol];
-                for (int a = 0; a < na; ++a)
-                    for (int b = 0; b < nb; ++b)
-                        jmap[c->mat_off_h[r.mol] + (r.bfa + a) * nbf + r.bfb + b] = (int)(words + (int64_t)(a * nb + b) * n + i);
-            }
-            words += (int64_t)na * nb * n;
-        }
-        if (words > INT32_MAX || 3 * (int64_t)npr > INT32_MAX || 3 * (int64_t)np > INT32_MAX)
-            return fail(c, QCG_INVALID_ARG, "basis too large");
-        c->n_kprim = npr;
-        HIPCHK(c, c->alloc(&c->d_kmeta, meta.size()));
-        HIPCHK(c, c->alloc(&c->d_kcen, cen.size()));
-        HIPCHK(c, c->alloc(&c->d_kprim, kp.size()));
-        HIPCHK(c, c->alloc(&c->d_khp, khp.size()));
-        HIPCHK(c, c->alloc(&c->d_kea, kea.size()));
-        HIPCHK(c, c->alloc(&c->d_katoms, katoms.size()));
-        HIPCHK(c, c->alloc(&c->d_kprimf, kpf.size()));
-        HIPCHK(c, c->alloc(&c->d_jmap, jmap.size()));
-        HIPCHK(c, c->alloc(&c->d_bf_norm, bfn.size()));
-        HIPCHK(c, c->alloc(&c->d_Dp, (size_t)words));
-        HIPCHK(c, hipMemcpy(c->d_kmeta, meta.data(), meta.size() * sizeof(int4), hipMemcpyHostToDevice));
-        HIPCHK(c, hipMemcpy(c->d_kcen, cen.data(), cen.size() * sizeof(double2), hipMemcpyHostToDevice));
-        HIPCHK(c, hipMemcpy(c->d_kprim, kp.data(), kp.size() * sizeof(double2), hipMemcpyHostToDevice));
-        HIPCHK(c, hipMemcpy(c->d_khp, khp.data(), khp.size() * sizeof(double), hipMemcpyHostToDevice));
-        HIPCHK(c, hipMemcpy(c->d_kea, kea.data(), kea.size() * sizeof(double), hipMemcpyHostToDevice));
-        HIPCHK(c, hipMemcpy(c->d_katoms, katoms.data(), katoms.size() * sizeof(int2), hipMemcpyHostToDevice));
-        HIPCHK(c, hipMemcpy(c->d_kprimf, kpf.data(), kpf.size() * sizeof(float4), hipMemcpyHostToDevice));
-        HIPCHK(c, hipMemcpy(c->d_jmap, jmap.data(), jmap.size() * sizeof(int), hipMemcpyHostToDevice));
-        HIPCHK(c, hipMemcpy(c->d_bf_norm, bfn.data(), bfn.size() * sizeof(double), hipMemcpyHostToDevice));
-        c->fixdata.jmap = c->d_jmap;
-        c->fixdata.bf_norm = c->d_bf_norm;
-    }
     HIPCHK(c, c->alloc(&c->d_mol_nbf, nmol));
     HIPCHK(c, c->alloc(&c->d_mat_off, nmol));
     HIPCHK(c, c->alloc(&c->d_ket_off, kNumPairClasses * nmol));
@@ -528,6 +451,77 @@ int qcg_set_basis_batch(qcg_context* c, int nmol, const int* mol_nshell, const i
     HIPCHK(c, c->alloc(&c->d_Kacc, n2));
     HIPCHK(c, c->alloc(&c->d_H, n2));
     HIPCHK(c, c->alloc(&c->d_F, n2));
+    {
+        // the kets as arrays in list order (KetPairs, KetPrims), and the pair order of the J side: the host
+        // numbers the primitives of each contraction bucket, the device copies (ket_arrays_kernel)
+        const int np = npairs, npr = (int)pp.size();
+        std::vector<int4> meta(np);
+        int first = 0;
+        for (int k = 0; k < kNumPairClasses; ++k)
+            for (int m = 0; m < nmol; ++m) {
+                const std::vector<int>& bnd = c->bucket_bnd[k * nmol + m];
+                const int base = c->class_off[k] + c->ket_off_h[k * nmol + m];
+                for (size_t b = 0; b + 1 < bnd.size(); ++b) {
+                    const int n = bnd[b + 1] - bnd[b], npp = all[base + bnd[b]].npp;
+                    for (int i = 0; i < n; ++i) {
+                        const PairRec& r = all[base + bnd[b] + i];
+                        meta[base + bnd[b] + i] =
+                            make_int4(r.bfa | r.bfb << kKetBfBits | (r.sa == r.sb ? kKetSame : 0), npp, first + i, n);
+                    }
+                    first += n * npp;
+                }
+            }
+        std::vector<double> bfn;
+        for (const HostBasis& B : c->mols)
+            for (int s = 0; s < B.nshell; ++s)
+                for (int k = 0; k < ncart(B.l[s]); ++k) bfn.push_back(B.l[s] == 2 && (k == 0 || k == 3 || k == 5) ? 0.57735026918962576451 : 1.0);
+        KetArrays ka{};
+        int64_t words = 0;
+        for (int k = 0; k < kNumPairClasses; ++k) {
+            int la, lb;
+            class_l(k, la, lb);
+            c->jbase[k] = ka.jbase[k] = (int)words;
+            ka.off[k] = c->class_off[k];
+            ka.nb[k] = ncart(lb);
+            ka.nab[k] = ncart(la) * ncart(lb);
+            words += (int64_t)ka.nab[k] * (c->class_off[k + 1] - c->class_off[k]);
+        }
+        ka.off[kNumPairClasses] = np;
+        if (words > INT32_MAX || 3 * (int64_t)npr > INT32_MAX || 3 * (int64_t)np > INT32_MAX)
+            return fail(c, QCG_INVALID_ARG, "basis too large");
+        c->n_kprim = npr;
+        HIPCHK(c, c->alloc(&c->d_kmeta, meta.size()));
+        HIPCHK(c, c->alloc(&c->d_kcen, 3 * (size_t)np));
+        HIPCHK(c, c->alloc(&c->d_kprim, 3 * (size_t)npr));
+        HIPCHK(c, c->alloc(&c->d_khp, (size_t)npr));
+        HIPCHK(c, c->alloc(&c->d_kea, (size_t)npr));
+        HIPCHK(c, c->alloc(&c->d_katoms, (size_t)np));
+        HIPCHK(c, c->alloc(&c->d_kprimf, 2 * (size_t)npr));
+        HIPCHK(c, c->alloc(&c->d_jmap, n2));
+        HIPCHK(c, c->alloc(&c->d_bf_norm, bfn.size()));
+        HIPCHK(c, c->alloc(&c->d_Dp, (size_t)words));
+        HIPCHK(c, hipMemcpy(c->d_kmeta, meta.data(), meta.size() * sizeof(int4), hipMemcpyHostToDevice));
+        HIPCHK(c, hipMemcpy(c->d_bf_norm, bfn.data(), bfn.size() * sizeof(double), hipMemcpyHostToDevice));
+        ka.np = np;
+        ka.npr = npr;
+        ka.pairs = c->d_pairs;
+        ka.pp = c->d_pp;
+        ka.ppf = c->d_ppf;
+        ka.meta = c->d_kmeta;
+        ka.mat_off = c->d_mat_off;
+        ka.mol_nbf = c->d_mol_nbf;
+        ka.cen = c->d_kcen;
+        ka.prim = c->d_kprim;
+        ka.hp = c->d_khp;
+        ka.ea = c->d_kea;
+        ka.atoms = c->d_katoms;
+        ka.primf = c->d_kprimf;
+        ka.jmap = c->d_jmap;
+        HIPCHK(c, launch_ket_arrays(ka, n2, c->stream));
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        c->fixdata.jmap = c->d_jmap;
+        c->fixdata.bf_norm = c->d_bf_norm;
+    }
     c->has_basis = true;
     return QCG_OK;
 }
@@ -585,11 +579,7 @@ int qcg::lanes_per_ket(int nb, int nk, double fpq, double chain_us) {
     return lg;
 }
 
-// Angular momenta of a pair class; model flops per primitive quartet (qcg_class_stat).
-static void class_l(int k, int& la, int& lb) {
-    la = k == 0 ? 0 : k <= 2 ? 1 : 2;
-    lb = (k == 0 || k == 1 || k == 3) ? 0 : (k == 2 || k == 4) ? 1 : 2;
-}
+// Model flops per primitive quartet (qcg_class_stat).
 double qcg::model_flops(int cb, int ck) {
     int la, lb, lc, ld;
     class_l(cb, la, lb);

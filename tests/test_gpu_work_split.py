@@ -14,7 +14,7 @@ import oracle
 from helpers import bench_molecule, random_density
 from iqcp_amd import workloads
 from iqcp_amd.basis import BasisSet, build_basis
-from iqcp_amd.engine import Engine, QcgError
+from iqcp_amd.engine import BatchEngine, Engine, QcgError
 
 pytestmark = pytest.mark.gpu
 
@@ -157,3 +157,15 @@ def test_gpu_jk_rows_of_k_out_of_lds(n):
         jk = eng.build_jk(D)
         assert np.abs(jk.J - Jo).max() < 1e-11 * np.abs(Jo).max() and np.abs(jk.K - Ko).max() < 1e-11 * np.abs(Ko).max()
     assert np.abs(eng.build_jk(D, want_j=False).K - Ko).max() < 1e-11 * np.abs(Ko).max()
+
+
+@pytest.mark.parametrize("names", [["H"], ["H", "He"], ["He", "H2O", "H"], ["CH4", "H", "H2O", "NH3", "He", "C6H6"]])
+def test_gpu_batch_ket_arrays(names):
+    """Batches whose classes have none, one and several blocks of 256 pairs, atoms of s shells among them: J and K
+    of every molecule against the oracle, sums of FP64 terms, 1e-11 of the largest element."""
+    bases = [build_basis([(n, (0.1, 0.2, 0.3))], "6-31g*") if n in ("H", "He") else bench_molecule(n, "6-31g*") for n in names]
+    Ds = [random_density(b.nbf, seed=3, nocc=max(1, b.n_occ)) for b in bases]
+    J, K = BatchEngine(bases).build_jk(Ds)
+    for b, D, j, k in zip(bases, Ds, J, K):
+        Jo, Ko, _ = oracle.jk_direct(b, D)
+        assert np.abs(j - Jo).max() < 1e-11 * np.abs(Jo).max() and np.abs(k - Ko).max() < 1e-11 * np.abs(Ko).max()
