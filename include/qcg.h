@@ -84,6 +84,8 @@ typedef struct qcg_scf_iteration {
 
 /* ---- context ---------------------------------------------------------------------------- */
 int qcg_create(qcg_context** ctx, int device);
+/* Frees the context's memory and everything else but its streams: these are idle and are destroyed by a
+ * qcg_create or qcg_destroy that comes a millisecond later or more (qcg_create waits for it). */
 void qcg_destroy(qcg_context* ctx);
 const char* qcg_last_error(const qcg_context* ctx);
 

@@ -62,7 +62,7 @@ Retired& retired() {
     return *p;
 }
 
-// Destroys the sets that are old enough.
+// Destroys the sets that are old enough, with their devices current; the callers set their own again.
 void destroy_retired(Retired& R) {
     const auto now = Clock::now();
     size_t n = 0;
@@ -80,6 +80,7 @@ void retire_streams(StreamSet add) {
     add.since = Clock::now();
     R.sets.push_back(add);
     destroy_retired(R);
+    (void)hipSetDevice(add.device);
 }
 
 // Waits until the sets that are retired now are old enough and destroys them; device: the current one.
